@@ -128,6 +128,20 @@ struct Off16 {
     uint32_t width = 0;
 };
 
+// Node tiles with halo rings (tiles.hip): tile t lists the nodes it owns,
+// then ring by ring the neighbours around them; row i's columns are
+// positions in that list (padding: i itself).
+constexpr uint32_t TILE_WMAX = 12;   // most off-diagonal blocks of a row
+struct Tiles {
+    uint32_t n = 0;                // tiles; 0: none (too wide rows or too large tiles)
+    uint32_t ext = 0;              // list length, the same for every tile (<= 1024, whole waves)
+    uint32_t rings = 0;
+    uint32_t W2 = 0;               // column words per row
+    uint32_t* ids = nullptr;       // [n ext] node ids
+    uint32_t* lcol = nullptr;      // [n W2 ext] two 16-bit positions per word
+    uint32_t* roff = nullptr;      // [n (rings + 1)] rows within r rings
+};
+
 // Symmetric 2x2-block sliced ELL, for a node matrix whose blocks satisfy
 // K(w, v) = K(v, w)^T bit for bit (what the T3 assembly produces).  Row v
 // stores its diagonal block (v, v) as three values (it is symmetric itself),

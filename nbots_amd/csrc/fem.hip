@@ -142,7 +142,7 @@ __global__ void k_scan_add(uint32_t* __restrict__ out, size_t n, const uint32_t*
 }
 
 // out[0..n) = exclusive scan of in; out[n] = total.  out has n+1 entries.
-static int scan_u32(const uint32_t* in, uint32_t* out, size_t n, hipStream_t s) {
+int scan_u32(const uint32_t* in, uint32_t* out, size_t n, hipStream_t s) {
     const size_t tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
     if (tiles <= 1) {
         uint32_t* sums = nullptr;
@@ -592,6 +592,7 @@ int fem_create(FemSys& F, uint32_t nn, const double* nod, uint32_t ne, const uin
     Sell2& S = K.s;
     K.blocked = true;
     K.n = 2 * nn;
+    K.xy = F.nod;
     S.n_nodes = nn;
     S.n_slices = (nn + SLICE - 1) / SLICE;
     NBX_HIP(hipMalloc(&S.rowlen, (size_t)nn + 1));

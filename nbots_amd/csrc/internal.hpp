@@ -61,6 +61,10 @@ struct DevMatrix {
     bool has_off16 = false;    // o's values reflect the current scale
     bool off_packed = false;   // o.pcol holds the columns as 16-bit deltas
     unsigned* off_flag = nullptr;
+    // several Chebyshev steps per launch: tiles of the nodes by position
+    const double2* xy = nullptr;   // node positions (the FEM system's array), or null
+    bool tiles_tried = false;      // t has been attempted
+    Tiles t;                       // of o's pattern, for the Chebyshev preconditioner
 };
 
 // Per-matrix solver scratch (device).  Sized for n scalar rows plus two
@@ -71,8 +75,9 @@ struct DevMatrix {
 //                               v64[5] (the unit diagonal)
 //   flexible CG (CHEB_FCG):     v64[0] r, v64[1] p, v64[2] w; v32[0..3]
 //                               residual, two directions and z of the
-//                               Chebyshev steps (FP64 preconditioner:
-//                               v64[5..8] instead)
+//                               Chebyshev steps, v32[4] the residual's second
+//                               buffer (several steps per launch); FP64
+//                               preconditioner: v64[5..8] instead
 //   FP32 CG (CG_RESTART/RELIABLE): v32[0..3]; a fallback to FP64 PCG takes
 //                               the FP64 slots above
 //   free for callers: v64[3], v64[4] (the drop-in's b and x, the system's
@@ -81,7 +86,7 @@ struct DevMatrix {
 struct Workspace {
     uint32_t n = 0;
     double* v64[9] = {};       // FP64 vectors
-    float* v32[4] = {};        // FP32 vectors
+    float* v32[5] = {};        // FP32 vectors
     double* partials = nullptr;
     float* partials32 = nullptr;
     PcgState* st = nullptr;    // device state (2 slots: outer, inner)
@@ -178,6 +183,13 @@ int mat_make_scaled(DevMatrix& m, hipStream_t s, int bits);
 int mat_make_off16(DevMatrix& m, hipStream_t s);
 // the scaled copy a mixed-precision solve with these options reads
 int mat_prepare_mixed(DevMatrix& m, hipStream_t s, const MixedOpts& o);
+
+// exclusive scan: out[0..n) = scan of in, out[n] = total
+int scan_u32(const uint32_t* in, uint32_t* out, size_t n, hipStream_t s);
+// tiles of the off-diagonal pattern O, whose rows hold at most wmax blocks,
+// by the node positions xy (T.n = 0 when they do not fit)
+int tiles_build(Tiles& T, const Off16& O, uint32_t wmax, const double2* xy, hipStream_t s);
+void tiles_free(Tiles& T);
 
 int spmv(const DevMatrix& m, const double* x, double* y, hipStream_t s);
 

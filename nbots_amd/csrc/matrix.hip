@@ -446,6 +446,7 @@ static void off_free(DevMatrix& m) {
     for (void* p : ps)
         if (p) (void)hipFree(p);
     O = Off16();
+    tiles_free(m.t);
     m.off_flag = nullptr;
     m.off_pattern = m.has_off16 = m.off_packed = false;
 }
@@ -843,7 +844,13 @@ int mat_prepare_mixed(DevMatrix& m, hipStream_t s, const MixedOpts& o) {
     // blocks when the matrix allows it, the full fp16 copy otherwise
     if (m.blocked && o.variant == CHEB_FCG && o.precond_bits == 16) {
         NBX_TRY(mat_make_off16(m, s));
-        if (m.has_off16) return NBX_OK;
+        if (m.has_off16) {
+            if (!m.tiles_tried) {
+                m.tiles_tried = true;
+                NBX_TRY(tiles_build(m.t, m.o, m.s.max_rowlen - 1, m.xy, s));
+            }
+            return NBX_OK;
+        }
     }
     return mat_make_scaled(m, s, o.variant == CHEB_FCG ? o.precond_bits : 32);
 }

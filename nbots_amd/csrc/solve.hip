@@ -22,6 +22,7 @@
 #include <math.h>
 #include <stdio.h>
 #include <string.h>
+#include <algorithm>
 #include <type_traits>
 #include <vector>
 
@@ -560,6 +561,140 @@ static void launch_cheb_step64(uint32_t k, uint32_t last, unsigned G, hipStream_
     else
         hipLaunchKernelGGL((k_cheb_step64<NT, Z_SKIP, M>), dim3(G), dim3(BLOCK), 0, s, K, din, dout,
                            res, z, st, n, c1, c2);
+}
+
+// Several Chebyshev steps in one launch, a workgroup per tile (tiles.hip).
+// Up to about 150k nodes a step of k_cheb_step64 is bound by the launch and
+// the chain of dependent loads (4 us whatever the size), above that by the
+// matrix and vectors it reads; both are paid here once for S steps.  Step
+// t = 1 .. S is taken on the tile's rows within S - t rings of the owned
+// ones, so each row's neighbours were computed by the same workgroup one
+// step earlier; the directions live in LDS (two buffers, widened to FP64
+// once), each thread keeps its row (the fp16 values widened to FP32, 16-bit
+// positions), residual and z in registers, and a step costs one barrier.
+// Halo rows are computed by every tile that lists them.
+// Bound by the FP64 pipe and the barriers on small systems (1.8 us per step
+// at 33k nodes, outer kernels included, against 4.9), by bytes on large ones
+// (about 63 B per node and step against 105: 24.0 against 36.5 us at 2.1M
+// nodes).  Row values held in FP64 registers take 85 VGPRs instead of 63 and
+// leave 5 waves per SIMD instead of 8 (28 us at 2.1M), held as packed fp16
+// they cost a second conversion per product (24.2 us).
+// The arithmetic of a row is k_cheb_step64's: the same sums in the same
+// order, an fp16 value times an FP32 entry being exact in FP64, so that the
+// fused multiply-add rounds as the separate add does.  Results are the same
+// bit for bit.  Residuals and directions are read from one buffer and written
+// to another: the halo rows of a tile are owned by its neighbours.
+// FULL: every row holds W blocks (the uniform layout).
+constexpr uint32_t CHEB_SMAX = 8;   // most rings (steps) of a tile
+struct ChebSteps {
+    uint32_t steps, k0, last;   // steps k0 .. k0 + steps - 1 of 1 .. last
+    double c1[CHEB_SMAX], c2[CHEB_SMAX];
+};
+template <int W, bool FULL>
+__global__ __launch_bounds__(1024) void k_cheb_tiles(Off16 O, Tiles T, ChebSteps cs,
+                                                     const float2* __restrict__ din,
+                                                     float2* __restrict__ dout,
+                                                     const float2* __restrict__ rin,
+                                                     float2* __restrict__ rout,
+                                                     float2* __restrict__ z, const PcgState* st) {
+    if (st->done) return;
+    extern __shared__ double2 sd[];   // [2][T.ext]
+    const uint32_t S = cs.steps, i = threadIdx.x, ext = T.ext;
+    const uint32_t t = xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t* __restrict__ roff = T.roff + (size_t)t * (T.rings + 1);
+    const uint32_t own = roff[0];
+    // a row of ring r takes part in the first S - r steps
+    uint32_t act = 0;
+    for (uint32_t r = 0; r < S; ++r) act += i < roff[r];
+    fv4 av[W];
+    uint32_t pc[(W + 1) / 2];
+    hv2 od = {};
+    float2 rs = {}, zv = {};
+    uint32_t v = 0;
+    int len = W;
+    if (i < roff[S]) {
+        v = T.ids[(size_t)t * ext + i];
+        const float2 d0 = din[v];
+        sd[i] = make_double2((double)d0.x, (double)d0.y);
+        if (act) {
+            size_t g;
+            if (FULL || O.width)
+                g = (size_t)(v >> 6) * SLICE * O.width + (v & 63);
+            else
+                g = (size_t)O.slice_ptr[v >> 6] + (v & 63);
+            if constexpr (!FULL) len = O.width ? (int)O.width : (int)O.rowlen[v];
+            const hv4* __restrict__ val = reinterpret_cast<const hv4*>(O.val);
+#pragma unroll
+            for (int q = 0; q < (W + 1) / 2; ++q)
+                if (FULL || 2 * q < len) pc[q] = T.lcol[((size_t)t * T.W2 + q) * ext + i];
+#pragma unroll
+            for (int k = 0; k < W; ++k)
+                if (FULL || k < len) {
+                    const hv4 h = val[g + (size_t)k * SLICE];
+                    av[k] = fv4{(float)h.x, (float)h.y, (float)h.z, (float)h.w};
+                }
+            od = reinterpret_cast<const hv2*>(O.od)[v];
+            rs = rin[v];
+        }
+        if (i < own) zv = z[v];
+    }
+    __syncthreads();
+    uint32_t cur = 0;
+    for (uint32_t s = 1; s <= S; ++s) {
+        if (s <= act) {
+            const double2* __restrict__ d = sd + cur * ext;
+            const double c1 = cs.c1[s - 1], c2 = cs.c2[s - 1];
+            const uint32_t k = cs.k0 + s - 1;
+            const double2 di = d[i];
+            double s0 = di.x + (double)od.x * di.y;
+            double s1 = (double)od.y * di.x + di.y;
+#pragma unroll
+            for (int q = 0; q < W; ++q) {
+                if (FULL || q < len) {
+                    const double2 xv = d[(pc[q / 2] >> (16 * (q & 1))) & 0xffffu];
+                    // (opaque per step, or FP64 copies of the row are hoisted)
+                    asm volatile("" : "+v"(av[q]));
+                    s0 = fma((double)av[q].x, xv.x, s0);
+                    s0 = fma((double)av[q].y, xv.y, s0);
+                    s1 = fma((double)av[q].z, xv.x, s1);
+                    s1 = fma((double)av[q].w, xv.y, s1);
+                }
+            }
+            const double rx = (double)rs.x - s0, ry = (double)rs.y - s1;
+            const double dx = c1 * di.x + c2 * rx, dy = c1 * di.y + c2 * ry;
+            rs = make_float2((float)rx, (float)ry);
+            sd[(cur ^ 1u) * ext + i] = make_double2((double)(float)dx, (double)(float)dy);
+            // z as launch_cheb_step64 adds it: even steps the pair, the last
+            // odd step its own direction (stored for the owned rows only)
+            const bool pair = (k & 1u) == 0u;
+            if (pair || k == cs.last) {
+                const double ax = pair ? di.x + dx : dx;
+                const double ay = pair ? di.y + dy : dy;
+                zv = make_float2((float)((double)zv.x + ax), (float)((double)zv.y + ay));
+            }
+        }
+        __syncthreads();
+        cur ^= 1u;
+    }
+    if (i < own) {
+        rout[v] = rs;
+        const double2 dn = sd[cur * ext + i];
+        dout[v] = make_float2((float)dn.x, (float)dn.y);
+        z[v] = zv;
+    }
+}
+
+static void launch_cheb_tiles(const Off16& O, const Tiles& T, const ChebSteps& cs,
+                              const float2* din, float2* dout, const float2* rin, float2* rout,
+                              float2* z, const PcgState* st, hipStream_t s) {
+    const dim3 g(T.n), b(T.ext);
+    const size_t lds = 2 * (size_t)T.ext * sizeof(double2);
+    if (O.width == 6)
+        hipLaunchKernelGGL((k_cheb_tiles<6, true>), g, b, lds, s, O, T, cs, din, dout, rin, rout, z,
+                           st);
+    else
+        hipLaunchKernelGGL((k_cheb_tiles<TILE_WMAX, false>), g, b, lds, s, O, T, cs, din, dout, rin,
+                           rout, z, st);
 }
 
 // One V-cycle of the multigrid preconditioner whose finest level is
@@ -1206,6 +1341,7 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
                                     : 12.0 * (double)m.s.n_blocks;
     const bool cheb_cached =
         cheb_mat + (p64 ? 80.0 : 33.0) * (double)nu <= (double)INFINITY_CACHE_BYTES;
+    const bool tiled = off16 && m.t.n;
     const bool amg = opt.variant == AMG_FCG;
     const double2* ones = amg ? (const double2*)amg_ones(m.amg) : nullptr;
     const AmgFine fine = amg ? amg_fine(m.amg) : AmgFine{};
@@ -1268,9 +1404,25 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
         hipLaunchKernelGGL(k_fin_fcg_update, dim3(1), dim3(FIN), 0, s, w.st, w.partials, G, first);
         float2* din = da;
         float2* dout = db;
+        if (tiled) {
+            float2 *rin = res, *rout = (float2*)w.v32[4];
+            ChebSteps cs;
+            cs.last = deg - 1;
+            for (uint32_t k = 1; k < deg; k += cs.steps) {
+                cs.k0 = k;
+                cs.steps = std::min(m.t.rings, deg - k);
+                for (uint32_t t = 0; t < cs.steps; ++t) {
+                    cs.c1[t] = c1d[k + t];
+                    cs.c2[t] = c2d[k + t];
+                }
+                launch_cheb_tiles(m.o, m.t, cs, din, dout, rin, rout, z, w.st, s);
+                std::swap(din, dout);
+                std::swap(rin, rout);
+            }
+        }
         double2* din64 = da64;
         double2* dout64 = db64;
-        for (uint32_t k = 1; k < deg; ++k) {
+        for (uint32_t k = 1; k < deg && !tiled; ++k) {
             auto step = [&](const auto& K) {
                 if (cheb_cached)
                     launch_cheb_step64<false>(k, deg - 1, G, s, K, din, dout, res, z, w.st, nu,

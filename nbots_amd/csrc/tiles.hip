@@ -1,0 +1,316 @@
+// Node tiles with halo rings, for kernels that take several dependent
+// row-product steps of one matrix in a single launch (k_cheb_tiles,
+// solve.hip).
+//
+// A tile owns the nodes of one cell of a uniform grid over the mesh's
+// bounding box (about `own` nodes), so its boundary is short whatever the
+// node numbering: S rings around 256 owned nodes of a triangle mesh hold
+// (16 + 2 S)^2 nodes, where S bandwidths around 256 consecutive ones hold
+// thousands.  The tile lists its nodes ring by ring (the owned ones, then the
+// neighbours of the ring before), ascending within a ring so that reads by
+// node stay nearly coalesced, and each row's columns as positions in that
+// list.  Built on the device, once per pattern.
+#include <hip/hip_runtime.h>
+#include <math.h>
+
+#include <algorithm>
+#include <vector>
+
+#include "rows.hpp"
+
+namespace nbx {
+
+namespace {
+
+constexpr int TILE_TB = 1024;       // threads of the ring kernel = most rows of a tile
+constexpr uint32_t TILE_HASH = 4096;
+constexpr uint32_t NONE = 0xffffffffu;
+
+// per workgroup: smallest and largest x and y
+__global__ __launch_bounds__(BLOCK) void k_tile_bbox(const double2* __restrict__ xy, uint32_t n,
+                                                     double* __restrict__ out) {
+    double v[4] = {INFINITY, INFINITY, INFINITY, INFINITY};   // x, y, -x, -y
+    for (uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += gridDim.x * BLOCK) {
+        const double2 p = xy[i];
+        v[0] = fmin(v[0], p.x);
+        v[1] = fmin(v[1], p.y);
+        v[2] = fmin(v[2], -p.x);
+        v[3] = fmin(v[3], -p.y);
+    }
+    __shared__ double red[4][BLOCK / WAVE];
+    for (int m = 0; m < 4; ++m) {
+        for (int off = WAVE / 2; off > 0; off >>= 1) v[m] = fmin(v[m], __shfl_down(v[m], off, WAVE));
+        if (threadIdx.x % WAVE == 0) red[m][threadIdx.x / WAVE] = v[m];
+    }
+    __syncthreads();
+    if (threadIdx.x < 4) {
+        double m = red[threadIdx.x][0];
+        for (int w = 1; w < BLOCK / WAVE; ++w) m = fmin(m, red[threadIdx.x][w]);
+        out[4 * (size_t)blockIdx.x + threadIdx.x] = m;
+    }
+}
+
+// a node's grid cell
+struct TileGrid {
+    double x0, y0, ix, iy;   // origin, cells per unit length
+    uint32_t nx, ny;
+};
+__device__ __forceinline__ uint32_t tile_cell(const TileGrid& g, double2 p) {
+    // (fmax and fmin return the bound for a NaN)
+    const uint32_t cx = (uint32_t)fmin(fmax((p.x - g.x0) * g.ix, 0.0), (double)(g.nx - 1));
+    const uint32_t cy = (uint32_t)fmin(fmax((p.y - g.y0) * g.iy, 0.0), (double)(g.ny - 1));
+    return cy * g.nx + cx;
+}
+__global__ void k_tile_count(TileGrid g, const double2* __restrict__ xy, uint32_t n,
+                             uint32_t* __restrict__ cell, uint32_t* cnt) {
+    const uint32_t v = blockIdx.x * BLOCK + threadIdx.x;
+    if (v >= n) return;
+    const uint32_t c = tile_cell(g, xy[v]);
+    cell[v] = c;
+    atomicAdd(&cnt[c], 1u);
+}
+__global__ void k_tile_zero(uint32_t* p, uint32_t n) {
+    const uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
+    if (i < n) p[i] = 0u;
+}
+// each cell's nodes, in any order (the ring kernel sorts them)
+__global__ void k_tile_fill(const uint32_t* __restrict__ cell, uint32_t n,
+                            const uint32_t* __restrict__ ptr, uint32_t* pos,
+                            uint32_t* __restrict__ own) {
+    const uint32_t v = blockIdx.x * BLOCK + threadIdx.x;
+    if (v >= n) return;
+    const uint32_t c = cell[v];
+    own[ptr[c] + atomicAdd(&pos[c], 1u)] = v;
+}
+
+__device__ __forceinline__ uint32_t tile_hash(uint32_t id) {
+    return (id * 2654435761u) >> 20;   // 12 bits
+}
+// the table position of id; NONE when it is absent and the table is full
+__device__ uint32_t tile_find(const uint32_t* keys, uint32_t id) {
+    uint32_t h = tile_hash(id);
+    for (uint32_t k = 0; k < TILE_HASH; ++k, h = (h + 1) % TILE_HASH)
+        if (keys[h] == id) return h;
+    return NONE;
+}
+// true when this call put id into the table (bounded probes: a full table
+// takes nothing and the caller's count has overflowed by then)
+__device__ bool tile_insert(uint32_t* keys, uint32_t id) {
+    uint32_t h = tile_hash(id);
+    for (uint32_t k = 0; k < TILE_HASH; ++k, h = (h + 1) % TILE_HASH) {
+        const uint32_t old = atomicCAS(&keys[h], NONE, id);
+        if (old == NONE) return true;
+        if (old == id) return false;
+    }
+    return false;
+}
+// list[b..e) ascending (distinct values): each value to its rank
+__device__ void tile_sort(uint32_t* list, uint32_t* tmp, uint32_t b, uint32_t e) {
+    const uint32_t i = b + threadIdx.x;
+    uint32_t key = 0, rank = 0;
+    if (i < e) {
+        key = list[i];
+        for (uint32_t j = b; j < e; ++j) rank += list[j] < key;
+        tmp[b + rank] = key;
+    }
+    __syncthreads();
+    if (i < e) list[i] = tmp[i];
+    __syncthreads();
+}
+
+// One workgroup per tile.  ext = 0: only info (the largest tile, a flag for
+// one beyond TILE_TB rows).  Otherwise the tile's list, ring
+// offsets and columns (row i's block 2 q + h in half h of word
+// lcol[(t W2 + q) ext + i]; padding names the row itself).
+__global__ __launch_bounds__(TILE_TB) void k_tile_rings(Off16 O, const uint32_t* __restrict__ ptr,
+                                                        const uint32_t* __restrict__ own,
+                                                        uint32_t rings, uint32_t wmax, uint32_t W2,
+                                                        uint32_t ext, uint32_t* __restrict__ ids,
+                                                        uint32_t* __restrict__ lcol,
+                                                        uint32_t* __restrict__ roff,
+                                                        unsigned* info) {
+    __shared__ uint32_t keys[TILE_HASH], list[TILE_TB], tmp[TILE_TB];
+    __shared__ uint16_t slot[TILE_HASH];
+    __shared__ uint32_t cnt;
+    const uint32_t t = blockIdx.x, tid = threadIdx.x;
+    const uint32_t o0 = ptr[t], c0 = ptr[t + 1] - o0;
+    if (c0 > (uint32_t)TILE_TB) {
+        if (tid == 0) info[1] = 1u;
+        return;
+    }
+    for (uint32_t i = tid; i < TILE_HASH; i += TILE_TB) keys[i] = NONE;
+    __syncthreads();
+    if (tid < c0) {
+        const uint32_t id = own[o0 + tid];
+        list[tid] = id;
+        tile_insert(keys, id);
+    }
+    __syncthreads();
+    tile_sort(list, tmp, 0, c0);
+    if (ext && tid == 0) roff[(size_t)t * (rings + 1)] = c0;
+    uint32_t beg = 0, end = c0;
+    for (uint32_t r = 1; r <= rings; ++r) {
+        if (tid == 0) cnt = end;
+        __syncthreads();
+        for (uint32_t f = tid; f < (end - beg) * wmax; f += TILE_TB) {
+            const uint32_t v = list[beg + f / wmax], k = f % wmax;
+            if (k >= O.rowlen[v]) continue;
+            const uint32_t w = O.bcol[(size_t)O.slice_ptr[v >> 6] + (v & 63) + (size_t)k * SLICE];
+            if (tile_insert(keys, w)) {
+                const uint32_t at = atomicAdd(&cnt, 1u);
+                if (at < (uint32_t)TILE_TB) list[at] = w;
+            }
+        }
+        __syncthreads();
+        const uint32_t now = cnt;
+        __syncthreads();
+        if (now > (uint32_t)TILE_TB) {
+            if (tid == 0) info[1] = 1u;
+            return;
+        }
+        tile_sort(list, tmp, end, now);
+        beg = end;
+        end = now;
+        if (ext && tid == 0) roff[(size_t)t * (rings + 1) + r] = end;
+    }
+    if (!ext) {
+        if (tid == 0) atomicMax(&info[0], end);
+        return;
+    }
+    if (tid < end) slot[tile_find(keys, list[tid])] = (uint16_t)tid;
+    __syncthreads();
+    if (tid < end) {
+        const uint32_t v = list[tid];
+        ids[(size_t)t * ext + tid] = v;
+        if (tid < beg) {   // a row whose columns are all in the list
+            const uint32_t len = O.rowlen[v];
+            const size_t g = (size_t)O.slice_ptr[v >> 6] + (v & 63);
+            for (uint32_t q = 0; q < W2; ++q) {
+                uint32_t word = 0;
+                for (uint32_t h = 0; h < 2; ++h) {
+                    const uint32_t k = 2 * q + h;
+                    const uint32_t s = k < len ? slot[tile_find(keys, O.bcol[g + (size_t)k * SLICE])]
+                                               : tid;
+                    word |= s << (16 * h);
+                }
+                lcol[((size_t)t * W2 + q) * ext + tid] = word;
+            }
+        }
+    }
+}
+
+}  // namespace
+
+void tiles_free(Tiles& T) {
+    void* ps[] = {T.ids, T.lcol, T.roff};
+    for (void* p : ps)
+        if (p) (void)hipFree(p);
+    T = Tiles();
+}
+
+// Leaves T.n = 0 (nothing allocated) when the mesh does not divide into
+// tiles of at most TILE_TB rows this way, or without device memory for them:
+// the kernels that take one step per launch then run.
+int tiles_build(Tiles& T, const Off16& O, uint32_t wmax, const double2* xy, hipStream_t s) {
+    const uint32_t n = O.n_nodes;
+    tiles_free(T);
+    if (!xy || n == 0 || wmax == 0 || wmax > TILE_WMAX) return NBX_OK;
+    uint32_t *cell = nullptr, *cnt = nullptr, *ptr = nullptr, *own = nullptr;
+    unsigned* info = nullptr;
+    double* bb = nullptr;
+    auto done = [&](int rc) {
+        void* ps[] = {cell, cnt, ptr, own, info, bb};
+        for (void* p : ps)
+            if (p) (void)hipFree(p);
+        if (rc != NBX_OK) tiles_free(T);
+        return rc;
+    };
+    auto no_memory = [&]() {
+        (void)hipGetLastError();
+        tiles_free(T);
+        return done(NBX_OK);
+    };
+    const unsigned gb = std::min(grid_for(n), 256u);
+    if (hipMalloc(&bb, 4 * (size_t)gb * sizeof(double)) != hipSuccess) return no_memory();
+    hipLaunchKernelGGL(k_tile_bbox, dim3(gb), dim3(BLOCK), 0, s, xy, n, bb);
+    std::vector<double> hb(4 * (size_t)gb);
+    if (copy_on(hb.data(), bb, hb.size() * sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess) {
+        set_last_error("tiles: bounding box");
+        return done(NBX_ERR_HIP);
+    }
+    double lo[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
+    for (size_t i = 0; i < hb.size(); ++i) lo[i % 4] = std::min(lo[i % 4], hb[i]);
+    const double Lx = -lo[2] - lo[0], Ly = -lo[3] - lo[1];
+    if (!(Lx >= 0.0) || !(Ly >= 0.0) || !std::isfinite(Lx) || !std::isfinite(Ly) ||
+        !(Lx + Ly > 0.0))
+        return done(NBX_OK);
+    // Owned nodes per tile and rings (= steps per launch).  Up to about 64k
+    // nodes launches and load latency bound a step, and many short launches
+    // are joined; above 160k the bytes do, and fewer rings read less halo.
+    // us per step of the default solve, outer kernels included, one step per
+    // launch -> (owned, rings): 33k nodes 4.9 -> 1.9 at (128, 8), 2.6 at
+    // (256, 3); 45k 4.9 -> 1.8 at (192, 8); 124k 5.3 -> 2.8 at (256, 5), 3.2 at
+    // (256, 3); 525k 12.3 -> 7.2 at (256, 3), 7.8 at (256, 4); 2.1M 36.5 ->
+    // 24.0 at (256, 3), 28.6 at (256, 4), 29 at (192, 4).
+    const uint32_t rings0 = n <= 65536 ? 8 : n <= 163840 ? 5 : 3;
+    const uint32_t own0 = n <= 65536 ? 160 : 256;
+    if (hipMalloc(&cell, (size_t)n * 4) != hipSuccess ||
+        hipMalloc(&own, (size_t)n * 4) != hipSuccess || hipMalloc(&info, 16) != hipSuccess)
+        return no_memory();
+    const uint32_t W2 = (wmax + 1) / 2;
+    // A mesh of uneven density, or with wider rows, can outgrow TILE_TB in a
+    // few cells: smaller cells with fewer rings then.
+    for (uint32_t attempt = 0; attempt < 3; ++attempt) {
+        const uint32_t rings = std::max(rings0 >> attempt, 2u);
+        const double cells = std::max(1.0, (double)n / (double)(own0 >> attempt));
+        // square cells
+        const double h = Lx > 0.0 && Ly > 0.0 ? sqrt(Lx * Ly / cells) : (Lx + Ly) / cells;
+        const double fx = std::max(1.0, std::round(Lx / h));
+        const double fy = std::max(1.0, std::round(Ly / h));
+        if (!(fx * fy <= 4.0 * cells + 16.0)) return done(NBX_OK);   // a sliver of a mesh
+        TileGrid g{lo[0], lo[1], Lx > 0.0 ? fx / Lx : 0.0, Ly > 0.0 ? fy / Ly : 0.0,
+                   (uint32_t)fx, (uint32_t)fy};
+        const uint32_t nt = g.nx * g.ny;
+        if (cnt) (void)hipFree(cnt);
+        if (ptr) (void)hipFree(ptr);
+        cnt = ptr = nullptr;
+        if (hipMalloc(&cnt, (size_t)nt * 4) != hipSuccess ||
+            hipMalloc(&ptr, ((size_t)nt + 1) * 4) != hipSuccess)
+            return no_memory();
+        hipLaunchKernelGGL(k_tile_zero, dim3(grid_for(nt)), dim3(BLOCK), 0, s, cnt, nt);
+        hipLaunchKernelGGL(k_tile_zero, dim3(1), dim3(BLOCK), 0, s, (uint32_t*)info, 4u);
+        hipLaunchKernelGGL(k_tile_count, dim3(grid_for(n)), dim3(BLOCK), 0, s, g, xy, n, cell, cnt);
+        const int rc = scan_u32(cnt, ptr, nt, s);
+        if (rc) return done(rc);
+        hipLaunchKernelGGL(k_tile_zero, dim3(grid_for(nt)), dim3(BLOCK), 0, s, cnt, nt);
+        hipLaunchKernelGGL(k_tile_fill, dim3(grid_for(n)), dim3(BLOCK), 0, s, cell, n, ptr, cnt, own);
+        hipLaunchKernelGGL(k_tile_rings, dim3(nt), dim3(TILE_TB), 0, s, O, ptr, own, rings, wmax,
+                           W2, 0u, (uint32_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr, info);
+        unsigned hi[2] = {0, 1};   // the largest tile, one beyond TILE_TB rows
+        if (hipGetLastError() != hipSuccess ||
+            copy_on(hi, info, sizeof hi, hipMemcpyDeviceToHost, s) != hipSuccess) {
+            set_last_error("tiles: halo rings");
+            return done(NBX_ERR_HIP);
+        }
+        if (hi[1]) continue;
+        T.n = nt;
+        T.ext = (hi[0] + WAVE - 1) / WAVE * WAVE;
+        T.rings = rings;
+        T.W2 = W2;
+        break;
+    }
+    if (T.n == 0) return done(NBX_OK);
+    if (hipMalloc(&T.ids, (size_t)T.n * T.ext * 4) != hipSuccess ||
+        hipMalloc(&T.lcol, (size_t)T.n * T.ext * W2 * 4) != hipSuccess ||
+        hipMalloc(&T.roff, (size_t)T.n * (T.rings + 1) * 4) != hipSuccess)
+        return no_memory();
+    hipLaunchKernelGGL(k_tile_rings, dim3(T.n), dim3(TILE_TB), 0, s, O, ptr, own, T.rings, wmax, W2,
+                       T.ext, T.ids, T.lcol, T.roff, info);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) {
+        set_last_error("tiles: lists");
+        return done(NBX_ERR_HIP);
+    }
+    return done(NBX_OK);
+}
+
+}  // namespace nbx
