@@ -166,6 +166,10 @@ struct Sym2 {
     uint32_t* l_slice_ptr = nullptr; // [n_slices + 1]
     uint8_t* l_rowlen = nullptr;     // [n_nodes]
     uint32_t* l_idx = nullptr;       // [2 * n_lower]: (w, upper position of (w, v))
+    // > 0: every slice holds that many upper (lower) blocks per row, so row
+    // v's start at (v / 64) 64 width + v % 64; padding may be read (valid
+    // columns and positions, zero values) but is not part of a row
+    uint32_t u_width = 0, l_width = 0;
 };
 
 // index of entry (i, j) of stored block idx in Sell2::val
@@ -201,10 +205,37 @@ __device__ __forceinline__ f32c cadd(f32c x, f32c y) {
     return {t.s, (x.c + y.c) + t.c};
 }
 
+typedef unsigned uv2x __attribute__((ext_vector_type(2)));
+
 // ---- wavefront / workgroup reductions in a fixed order --------------------
+// Lane 0 gets ((v_0 + v_32) + (v_16 + v_48)) + ..., the tree of shuffles down
+// by 32, 16, 8, 4, 2 and 1.  The halves and the rows of 16 meet by lane swaps
+// and the lanes of a row by row shifts, within the vector registers: a
+// shuffle through LDS costs several times as much, and a reduction's six in a
+// row were about 0.25 us of kernels of 2-4 us.
+__device__ __forceinline__ double swap_add32(double v) {
+    const uv2x u = __builtin_bit_cast(uv2x, v);
+    const uv2x a = __builtin_amdgcn_permlane32_swap(u.x, u.x, false, false);
+    const uv2x b = __builtin_amdgcn_permlane32_swap(u.y, u.y, false, false);
+    return __builtin_bit_cast(double, (uv2x){a.x, b.x}) + __builtin_bit_cast(double, (uv2x){a.y, b.y});
+}
+__device__ __forceinline__ double swap_add16(double v) {
+    const uv2x u = __builtin_bit_cast(uv2x, v);
+    const uv2x a = __builtin_amdgcn_permlane16_swap(u.x, u.x, false, false);
+    const uv2x b = __builtin_amdgcn_permlane16_swap(u.y, u.y, false, false);
+    return __builtin_bit_cast(double, (uv2x){a.x, b.x}) + __builtin_bit_cast(double, (uv2x){a.y, b.y});
+}
+template <int N>   // v + v of the lane N above in the same row of 16
+__device__ __forceinline__ double row_add(double v) {
+    const uv2x u = __builtin_bit_cast(uv2x, v);
+    uv2x o;
+    o.x = (unsigned)__builtin_amdgcn_update_dpp(0, (int)u.x, 0x100 + N, 0xf, 0xf, true);
+    o.y = (unsigned)__builtin_amdgcn_update_dpp(0, (int)u.y, 0x100 + N, 0xf, 0xf, true);
+    return v + __builtin_bit_cast(double, o);
+}
 __device__ __forceinline__ double wave_sum(double v) {
-    for (int off = WAVE / 2; off > 0; off >>= 1) v += __shfl_down(v, off, WAVE);
-    return v;
+    v = swap_add16(swap_add32(v));
+    return row_add<1>(row_add<2>(row_add<4>(row_add<8>(v))));
 }
 __device__ __forceinline__ f32c wave_sum(f32c v) {
     for (int off = WAVE / 2; off > 0; off >>= 1) {

@@ -72,7 +72,9 @@ struct DevMatrix {
 // run's b or x):
 //   FP64 Jacobi-PCG (pcg_run):  v64[0] g, v64[1] p_j (j % 4 = 0), v64[2] w,
 //                               v64[6..8] p_j (j % 4 = 1..3); plain CG also
-//                               v64[5] (the unit diagonal)
+//                               v64[5] (the unit diagonal).  In two kernels
+//                               per iteration (pcg2_run): v64[0] g, v64[8] w,
+//                               v64[1..2] and v64[6..7] the (q, p) pairs
 //   flexible CG (CHEB_FCG):     v64[0] r, v64[1] p, v64[2] w; v32[0..3]
 //                               residual, two directions and z of the
 //                               Chebyshev steps, v32[4] the residual's second
@@ -89,7 +91,7 @@ struct Workspace {
     float* v32[5] = {};        // FP32 vectors
     double* partials = nullptr;
     float* partials32 = nullptr;
-    PcgState* st = nullptr;    // device state (2 slots: outer, inner)
+    PcgState* st = nullptr;    // device state (2 slots, which the two-kernel PCG alternates)
     PcgState* h_st = nullptr;  // pinned host mirror
     hipEvent_t ev[4] = {};
     static constexpr int NSAMP = 32;    // sampled SpMV launches per solve, one every
@@ -201,8 +203,9 @@ int pcg_jacobi(const DevMatrix& m, const double* b, double* x, uint32_t max_iter
                hipStream_t s, SolveStats* stats, bool unpreconditioned = false);
 
 // The same on a scalar CSR already in device memory with a caller-made
-// workspace (vectors v64[0..2], v64[6..8], partials, st, a host mirror
-// h_st; no events): nothing is allocated.  diag holds A(i,i).
+// workspace (v64[0], v64[8], two consecutive vectors from v64[1] and from
+// v64[6] on, partials, st, a host mirror h_st; no events): nothing is
+// allocated.  diag holds A(i,i).
 int pcg_jacobi_csr_view(const DevCsr& c, const double* diag, const double* b, double* x,
                         uint32_t max_iter, double tol, uint32_t* niter, double* tol_reached,
                         Workspace& w, hipStream_t s);

@@ -389,7 +389,11 @@ int ws_alloc(Workspace& w, uint32_t n) {
     if (w.n >= n && w.st) return NBX_OK;
     ws_free(w);
     const size_t nn = (size_t)(n ? n : 1) + 2;
-    for (auto& p : w.v64) NBX_HIP(hipMalloc(&p, nn * sizeof(double)));
+    // one array, each vector on a 256-byte boundary: the two-kernel PCG takes
+    // pairs of consecutive vectors
+    const size_t stride = (nn + 31) / 32 * 32;
+    NBX_HIP(hipMalloc(&w.v64[0], 9 * stride * sizeof(double)));
+    for (int i = 1; i < 9; ++i) w.v64[i] = w.v64[0] + (size_t)i * stride;
     for (auto& p : w.v32) NBX_HIP(hipMalloc(&p, nn * sizeof(float)));
     NBX_HIP(hipMalloc(&w.partials, 4 * MAX_GRID * sizeof(double)));
     NBX_HIP(hipMalloc(&w.partials32, 4 * MAX_GRID * sizeof(float)));
@@ -402,10 +406,8 @@ int ws_alloc(Workspace& w, uint32_t n) {
 }
 
 void ws_free(Workspace& w) {
-    for (auto& p : w.v64) {
-        if (p) (void)hipFree(p);
-        p = nullptr;
-    }
+    if (w.v64[0]) (void)hipFree(w.v64[0]);
+    for (auto& p : w.v64) p = nullptr;
     for (auto& p : w.v32) {
         if (p) (void)hipFree(p);
         p = nullptr;
@@ -648,6 +650,18 @@ static int sym_build_pattern(DevMatrix& m, hipStream_t s) {
     NBX_TRY(read_flag(m.sym_flag, s, &bad));
     std::vector<uint32_t> usp, lsp;
     if (bad || !slice_offsets(ul, ns, usp) || !slice_offsets(ll, ns, lsp)) return give_up();
+    // One width for all slices when that adds at most 1/16 of padding: a
+    // product then finds its row without first loading the slice offset.
+    auto uniform = [&](const std::vector<uint8_t>& len, std::vector<uint32_t>& sp) {
+        uint32_t wmax = 0;
+        for (uint8_t l : len) wmax = wmax > l ? wmax : l;
+        const uint64_t uni = (uint64_t)ns * SLICE * wmax;
+        if (wmax == 0 || uni > (uint64_t)sp[ns] + sp[ns] / 16 || uni > 0xffffffffull) return 0u;
+        for (uint32_t sl = 0; sl <= ns; ++sl) sp[sl] = sl * SLICE * wmax;
+        return wmax;
+    };
+    Y.u_width = uniform(ul, usp);
+    Y.l_width = uniform(ll, lsp);
     Y.n_nodes = nn;
     Y.n_slices = ns;
     Y.n_upper = usp[ns];

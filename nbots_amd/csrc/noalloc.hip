@@ -26,7 +26,7 @@ constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 constexpr size_t ST_BYTES = align256(2 * sizeof(nbx::PcgState));
 constexpr size_t PART_BYTES = align256(4 * (size_t)nbx::MAX_GRID * sizeof(double));
 constexpr size_t VEC_BYTES = align256(((size_t)NBX_NOALLOC_MAX_N + 2) * sizeof(double));
-constexpr int NVEC = 7;   // diag, g, w, the four direction buffers
+constexpr int NVEC = 7;   // diag, g, w, two buffers of (q, p) pairs
 constexpr size_t SCRATCH_BYTES = ST_BYTES + PART_BYTES + NVEC * VEC_BYTES;
 
 constexpr int MAX_DEVICES = 64;
@@ -99,11 +99,9 @@ extern "C" int nbx_sparse_solve_CG_precond_Jacobi_noalloc(
     w.n = n;
     w.replay = false;
     w.v64[0] = slot(1);   // g
-    w.v64[1] = slot(2);   // p_j, j % 4 = 0
-    w.v64[2] = slot(3);   // w
-    w.v64[6] = slot(4);   // p_j, j % 4 = 1..3
-    w.v64[7] = slot(5);
-    w.v64[8] = slot(6);
+    w.v64[8] = slot(2);   // w
+    w.v64[1] = slot(3);   // the two buffers of (q, p) pairs, two slots each
+    w.v64[6] = slot(5);
     w.partials = (double*)(base + ST_BYTES);
     w.st = (nbx::PcgState*)base;
     w.h_st = &host_state;

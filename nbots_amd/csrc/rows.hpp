@@ -454,6 +454,7 @@ __device__ __forceinline__ float2 row_scaled(const Sell2& A, uint32_t v, const f
 struct OpS2 {
     Sell2 A;
     using V = double2;
+    __device__ __forceinline__ const Sell2& mat() const { return A; }
     __device__ __forceinline__ double2 row(uint32_t v, const double2* __restrict__ x) const {
         return row64(A, v, x);
     }
@@ -470,6 +471,7 @@ struct OpSym {
 struct OpSymC {
     Sym2 Y;
     using V = double2;
+    __device__ __forceinline__ const Sym2& mat() const { return Y; }
     __device__ __forceinline__ double2 row(uint32_t v, const double2* __restrict__ x) const {
         return row64s<4, 4, false>(Y, v, x);
     }

@@ -221,6 +221,469 @@ __global__ __launch_bounds__(BLOCK) void k_pcg_tail(V* __restrict__ x, PBufs<V> 
 }
 
 // ---------------------------------------------------------------------------
+// FP64 Jacobi PCG in two kernels per iteration (small and medium systems)
+// ---------------------------------------------------------------------------
+// Up to a few hundred thousand rows an iteration of the five kernels above is
+// bound by their launches and by the chains of dependent loads in each (3-4
+// us a kernel), not by bytes.  Two kernels do the same iteration:
+//   k_cg_dir     sums the previous update's partials (g.q and g.g), which
+//                gives beta and the stop decision; forms p_j = -q + beta
+//                p_{j-1} of a row and of its neighbours on the fly, stores
+//                its own, w = A p_j and the partials of p_j.w;
+//   k_cg_update  sums those, which gives alpha; x += alpha p, g += alpha w,
+//                q = g / Aii and the partials of g.q and g.g.
+// Every workgroup sums all partials itself, in the same order, so all have
+// the same scalars and no one-workgroup kernel stands between (G partials
+// read by G workgroups: at most 1,024 of each, a few us of L2 traffic at the
+// largest).  k_cg_dir issues its row's loads before that sum, whose latency
+// then hides them.  The state alternates between two slots: a launch reads
+// one and its first workgroup writes the other, so no workgroup reads what
+// another one of the same launch writes.  Products, vectors, sums (a partial
+// per 256 rows, wave sums of 64 partials, those in index order) and the stop
+// test are formed by the same operations in the same order as in the five
+// kernels, so the results are the same bit for bit.
+constexpr unsigned CG2_PARTS = 1024;   // most partials of a value
+template <int NV>
+__device__ __forceinline__ void all_sum(const double* __restrict__ partials, unsigned np,
+                                        double (&tot)[NV], double (*red)[CG2_PARTS / WAVE]) {
+    constexpr unsigned WAVES = BLOCK / WAVE;
+    const unsigned lane = threadIdx.x % WAVE, wid = threadIdx.x / WAVE;
+    const unsigned groups = (np + WAVE - 1) / WAVE;   // of 64 partials, a wave sum each
+    double v[NV][CG2_PARTS / BLOCK];
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (unsigned j = 0; j < CG2_PARTS / BLOCK; ++j) {
+            const unsigned b = (wid + j * WAVES) * WAVE + lane;
+            v[i][j] = b < np ? partials[(size_t)i * np + b] : 0.0;
+        }
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (unsigned j = 0; j < CG2_PARTS / BLOCK; ++j) {
+            const unsigned g = wid + j * WAVES;
+            if (g < groups) {
+                const double s = wave_sum(v[i][j]);
+                if (lane == 0) red[i][g] = s;
+            }
+        }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        double s = 0.0;
+        for (unsigned g = 0; g < groups; ++g) s += red[i][g];
+        tot[i] = s;
+    }
+}
+
+// q of the coming direction and the direction before it, side by side: the
+// product gathers both of a neighbour in one place.
+template <class V>
+struct __attribute__((aligned(16))) CgPair {
+    V q, p;
+};
+
+// p_j of one row from q and p_{j-1}
+struct CgDir {
+    double beta;
+    bool first;
+    template <class V>
+    __device__ __forceinline__ V operator()(const CgPair<V>& d) const {
+        return first ? negu(d.q) : pupd(d.q, beta, d.p);
+    }
+};
+
+// beta and the stop decision before iteration k (the test of k_fin_init and
+// k_fin_B) from the sums of the update before it; false when the solve has
+// ended.  Called by every thread of every workgroup, with the same results.
+__device__ __forceinline__ bool cg_next(const PcgState* __restrict__ sin, PcgState* sout,
+                                        const double* __restrict__ upd, bool first,
+                                        double (*red)[CG2_PARTS / WAVE], CgDir& dir) {
+    const uint32_t ended = sin->done, max_iter = sin->max_iter;
+    const uint32_t k = first ? 0u : sin->k + 1u;
+    const double tol2 = sin->tol2, rz = sin->rz, gg_cur = sin->gg_cur;
+    double tot[2];
+    all_sum<2>(upd, gridDim.x, tot, red);
+    const double gg_prev = first ? tot[1] : gg_cur;
+    const bool go = gg_prev > tol2 && k < max_iter;
+    dir.beta = first ? 0.0 : tot[0] / rz;
+    dir.first = first;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sout->tol2 = tol2;
+        sout->max_iter = max_iter;
+        sout->gg0 = first ? tot[1] : sin->gg0;
+        if (ended) {   // (the state goes on from slot to slot)
+            sout->k = sin->k;
+            sout->done = 1;
+            sout->status = sin->status;
+            sout->tol_reached = sin->tol_reached;
+        } else {
+            sout->k = k;
+            sout->beta = dir.beta;
+            sout->rz = tot[0];
+            sout->gg_prev = gg_prev;
+            sout->gg_cur = tot[1];
+            sout->done = go ? 0u : 1u;
+            sout->status = gg_prev > tol2 ? 1u : 0u;
+            sout->tol_reached = sqrt(gg_prev);
+        }
+    }
+    return !ended && go;
+}
+
+// A row's loads ahead of beta, then the product with p formed on the fly;
+// blocks beyond the ones held ahead are loaded when they are used.
+template <class Op>
+struct CgRow;
+// the symmetric copy, with U lower and U upper blocks loaded ahead
+template <int U>
+struct OpSymU : OpSymC {};
+template <>
+struct CgRow<OpS2> {
+    static constexpr int U = 7;   // an interior row of a T3 mesh
+    const Sell2& A;
+    size_t base = 0;
+    int len = 0;
+    uint32_t w[U];
+    dv2 a[U], b[U];
+    CgPair<double2> x[U];
+    __device__ __forceinline__ void load(uint32_t v, const CgPair<double2>* __restrict__ d) {
+        const dv2* __restrict__ pa = reinterpret_cast<const dv2*>(A.val);
+        const dv2* __restrict__ pb = reinterpret_cast<const dv2*>(A.val + 2 * A.n_blocks);
+        base = (size_t)A.slice_ptr[v >> 6] + (v & 63);
+        len = A.rowlen[v];
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (k < len) {
+                const size_t i = base + (size_t)k * SLICE;
+                w[k] = A.bcol[i];
+                a[k] = pa[i];
+                b[k] = pb[i];
+            }
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (k < len) x[k] = d[w[k]];
+    }
+    __device__ __forceinline__ double2 product(const CgDir& dir, double2,
+                                               const CgPair<double2>* __restrict__ d) const {
+        double s0 = 0.0, s1 = 0.0;
+        auto add = [&](dv2 ka, dv2 kb, double2 v) {
+            s0 = s0 + ka.x * v.x;
+            s0 = s0 + ka.y * v.y;
+            s1 = s1 + kb.x * v.x;
+            s1 = s1 + kb.y * v.y;
+        };
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (k < len) add(a[k], b[k], dir(x[k]));
+        const dv2* __restrict__ pa = reinterpret_cast<const dv2*>(A.val);
+        const dv2* __restrict__ pb = reinterpret_cast<const dv2*>(A.val + 2 * A.n_blocks);
+        for (int k = U; k < len; ++k) {
+            const size_t i = base + (size_t)k * SLICE;
+            add(pa[i], pb[i], dir(d[A.bcol[i]]));
+        }
+        return make_double2(s0, s1);
+    }
+};
+template <int U>
+struct CgRow<OpSymU<U>> {
+    const Sym2& Y;
+    size_t lbase = 0, ubase = 0;
+    int llen = 0, ulen = 0;
+    dv2 d01;
+    double d11;
+    uv2 e[U];
+    uint32_t w[U];
+    dv2 la[U], lb[U], ua[U], ub[U];
+    CgPair<double2> lx[U], ux[U];
+    __device__ __forceinline__ void load(uint32_t v, const CgPair<double2>* __restrict__ d) {
+        const dv2* __restrict__ pa = reinterpret_cast<const dv2*>(Y.u_val);
+        const dv2* __restrict__ pb = reinterpret_cast<const dv2*>(Y.u_val + 2 * Y.n_upper);
+        const uv2* __restrict__ li = reinterpret_cast<const uv2*>(Y.l_idx);
+        d01 = reinterpret_cast<const dv2*>(Y.d_val)[v];
+        d11 = Y.d_val[2 * (size_t)Y.n_nodes + v];
+        llen = Y.l_rowlen[v];
+        ulen = Y.u_rowlen[v];
+        // the entries to hold: the row's own, or, where every slice is as wide
+        // as the widest row, the slice's, without waiting for the row length
+        int ln = llen, un = ulen;
+        if (Y.l_width) {
+            lbase = (size_t)(v >> 6) * SLICE * Y.l_width + (v & 63);
+            ln = (int)Y.l_width;
+        } else {
+            lbase = (size_t)Y.l_slice_ptr[v >> 6] + (v & 63);
+        }
+        if (Y.u_width) {
+            ubase = (size_t)(v >> 6) * SLICE * Y.u_width + (v & 63);
+            un = (int)Y.u_width;
+        } else {
+            ubase = (size_t)Y.u_slice_ptr[v >> 6] + (v & 63);
+        }
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (k < ln) e[k] = li[lbase + (size_t)k * SLICE];
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (k < un) {
+                const size_t i = ubase + (size_t)k * SLICE;
+                w[k] = Y.u_bcol[i];
+                ua[k] = pa[i];
+                ub[k] = pb[i];
+            }
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (k < ln) {
+                la[k] = pa[e[k].y];
+                lb[k] = pb[e[k].y];
+                lx[k] = d[e[k].x];
+            }
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (k < un) ux[k] = d[w[k]];
+    }
+    __device__ __forceinline__ double2 product(const CgDir& dir, double2 pd,
+                                               const CgPair<double2>* __restrict__ d) const {
+        const dv2* __restrict__ pa = reinterpret_cast<const dv2*>(Y.u_val);
+        const dv2* __restrict__ pb = reinterpret_cast<const dv2*>(Y.u_val + 2 * Y.n_upper);
+        const uv2* __restrict__ li = reinterpret_cast<const uv2*>(Y.l_idx);
+        double s0 = 0.0, s1 = 0.0;
+        auto lower = [&](dv2 a, dv2 b, double2 v) {   // [[a.x, b.x], [a.y, b.y]]
+            s0 = s0 + a.x * v.x;
+            s0 = s0 + b.x * v.y;
+            s1 = s1 + a.y * v.x;
+            s1 = s1 + b.y * v.y;
+        };
+        auto upper = [&](dv2 a, dv2 b, double2 v) {
+            s0 = s0 + a.x * v.x;
+            s0 = s0 + a.y * v.y;
+            s1 = s1 + b.x * v.x;
+            s1 = s1 + b.y * v.y;
+        };
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (k < llen) lower(la[k], lb[k], dir(lx[k]));
+        for (int k = U; k < llen; ++k) {
+            const uv2 c = li[lbase + (size_t)k * SLICE];
+            lower(pa[c.y], pb[c.y], dir(d[c.x]));
+        }
+        s0 = s0 + d01.x * pd.x;
+        s0 = s0 + d01.y * pd.y;
+        s1 = s1 + d01.y * pd.x;
+        s1 = s1 + d11 * pd.y;
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (k < ulen) upper(ua[k], ub[k], dir(ux[k]));
+        for (int k = U; k < ulen; ++k) {
+            const size_t i = ubase + (size_t)k * SLICE;
+            upper(pa[i], pb[i], dir(d[Y.u_bcol[i]]));
+        }
+        return make_double2(s0, s1);
+    }
+};
+
+// g = A x - b; q = g / Aii; partials g.q, g.g  (cg_precond_jacobi.c:33-43)
+template <class Op>
+__global__ __launch_bounds__(BLOCK) void k_cg_init(Op op, const typename Op::V* __restrict__ b,
+                                                   const typename Op::V* __restrict__ x,
+                                                   typename Op::V* __restrict__ g,
+                                                   CgPair<typename Op::V>* __restrict__ d,
+                                                   const typename Op::V* __restrict__ diag,
+                                                   double* partials, uint32_t n) {
+    using V = typename Op::V;
+    double acc[2] = {0.0, 0.0};
+    const Chunk c = my_chunk(n);
+    const size_t u = c.beg + threadIdx.x;
+    if (u < c.end) {
+        const V gv = subu(op.row((uint32_t)u, x), b[u]);
+        const V qv = divu(gv, diag[u]);
+        g[u] = gv;
+        d[u].q = qv;
+        acc[0] = dotu(gv, qv);
+        acc[1] = dotu(gv, gv);
+    }
+    __shared__ double red[2][BLOCK / WAVE];
+    block_sum<2>(acc, red);
+    put_partials<2>(acc, partials);
+}
+
+template <class Op>
+__global__ __launch_bounds__(BLOCK) void k_cg_dir(Op op,
+                                                  const CgPair<typename Op::V>* __restrict__ d,
+                                                  CgPair<typename Op::V>* __restrict__ dnew,
+                                                  typename Op::V* __restrict__ w,
+                                                  const PcgState* __restrict__ sin, PcgState* sout,
+                                                  const double* __restrict__ upd, double* dirp,
+                                                  uint32_t n, bool first) {
+    using V = typename Op::V;
+    __shared__ double red[2][CG2_PARTS / WAVE], red2[2][BLOCK / WAVE];
+    const Chunk c = my_chunk(n);
+    const size_t u = c.beg + threadIdx.x;
+    const bool valid = u < c.end;
+    CgRow<Op> row{op.mat()};
+    CgPair<V> own{};
+    if (valid) {
+        own = d[u];
+        row.load((uint32_t)u, d);
+    }
+    CgDir dir;
+    if (!cg_next(sin, sout, upd, first, red, dir)) return;
+    double acc[1] = {0.0};
+    if (valid) {
+        const V pd = dir(own);
+        dnew[u].p = pd;
+        const V wv = row.product(dir, pd, d);
+        w[u] = wv;
+        acc[0] = dotu(pd, wv);
+    }
+    block_sum<1>(acc, red2);
+    put_partials<1>(acc, dirp);
+}
+
+// The same on scalar CSR.  A workgroup takes 256 rows and walks their entries
+// a tile at a time in storage order, so that columns and values are read in
+// whole cache lines (one thread per row reads them a row apart); the products
+// go through LDS, where each row's thread adds its own in column order, as
+// the reference sums a row.  A tile's loads are issued before the sums of
+// the tile before it.
+// PER entries per thread and tile: 16 take a whole 256-row group of up to 16
+// entries a row at once (168 VGPRs, which is no matter while there is one
+// workgroup per CU or less), 8 leave more waves to a larger matrix.
+// us per iteration (five kernels -> two): 4,290 rows 21 -> 12.4, 41,004 rows
+// 20.6 -> 13.1, 90,902 rows 24 -> 13.9 with 16 and 14.3 with 8, 257,442 rows
+// 94 -> 21 with 8 and 27 with 16.
+constexpr uint32_t CSR_WIDE_ROWS = 131072;   // PER 16 up to here
+template <int PER>
+__global__ __launch_bounds__(BLOCK) void k_cg_dir_csr(DevCsr A,
+                                                      const CgPair<double>* __restrict__ d,
+                                                      CgPair<double>* __restrict__ dnew,
+                                                      double* __restrict__ w,
+                                                      const PcgState* __restrict__ sin,
+                                                      PcgState* sout,
+                                                      const double* __restrict__ upd,
+                                                      double* dirp, uint32_t n, bool first) {
+    constexpr int TILE = PER * BLOCK;
+    __shared__ double red[2][CG2_PARTS / WAVE], prod[TILE], red2[1][BLOCK / WAVE];
+    const Chunk c = my_chunk(n);
+    const size_t u = c.beg + threadIdx.x;
+    const bool valid = u < c.end;
+    const uint32_t e0 = A.rowptr[c.beg], e1 = A.rowptr[c.end];
+    uint32_t r0 = e1, r1 = e1;
+    CgPair<double> own{};
+    if (valid) {
+        r0 = A.rowptr[u];
+        r1 = A.rowptr[u + 1];
+        own = d[u];
+    }
+    double av[PER];
+    CgPair<double> dv[PER];
+    auto fetch = [&](uint64_t base) {
+        uint32_t col[PER];
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const uint64_t e = base + threadIdx.x + (unsigned)i * BLOCK;
+            if (e < e1) {
+                col[i] = A.col[e];
+                av[i] = A.val[e];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if (base + threadIdx.x + (unsigned)i * BLOCK < e1) dv[i] = d[col[i]];
+    };
+    fetch(e0);
+    CgDir dir;
+    if (!cg_next(sin, sout, upd, first, red, dir)) return;
+    double s = 0.0;
+    for (uint64_t base = e0; base < e1; base += TILE) {
+        const uint32_t m = (uint32_t)min((uint64_t)TILE, e1 - base);
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const uint32_t t = threadIdx.x + (unsigned)i * BLOCK;
+            if (t < m) prod[t] = av[i] * dir(dv[i]);
+        }
+        __syncthreads();
+        fetch(base + TILE);   // (nothing past the last entry)
+        const uint32_t lo = r0 > base ? (uint32_t)(r0 - base) : 0u;
+        const uint32_t hi = r1 > base ? (uint32_t)min((uint64_t)m, r1 - base) : 0u;
+        for (uint32_t t = lo; t < hi; t += 8) {   // eight reads in flight, added in order
+            double v[8];
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) v[k] = t + k < hi ? prod[t + k] : 0.0;
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) s = t + k < hi ? s + v[k] : s;
+        }
+        __syncthreads();
+    }
+    double acc[1] = {0.0};
+    if (valid) {
+        const double pd = dir(own);
+        dnew[u].p = pd;
+        w[u] = s;
+        acc[0] = dotu(pd, s);
+    }
+    block_sum<1>(acc, red2);
+    put_partials<1>(acc, dirp);
+}
+template <class Op>
+static void launch_cg_dir(const Op& op, unsigned G, hipStream_t s,
+                          const CgPair<typename Op::V>* d, CgPair<typename Op::V>* dnew,
+                          typename Op::V* w,
+                          const PcgState* sin, PcgState* sout, const double* upd, double* dirp,
+                          uint32_t n, bool first) {
+    if constexpr (std::is_same<Op, OpCsr>::value) {
+        if (n <= CSR_WIDE_ROWS)
+            hipLaunchKernelGGL(k_cg_dir_csr<16>, dim3(G), dim3(BLOCK), 0, s, op.A, d, dnew, w, sin,
+                               sout, upd, dirp, n, first);
+        else
+            hipLaunchKernelGGL(k_cg_dir_csr<8>, dim3(G), dim3(BLOCK), 0, s, op.A, d, dnew, w, sin,
+                               sout, upd, dirp, n, first);
+    } else {
+        hipLaunchKernelGGL(k_cg_dir<Op>, dim3(G), dim3(BLOCK), 0, s, op, d, dnew, w, sin,
+                           sout, upd, dirp, n, first);
+    }
+}
+
+template <class V>
+__global__ __launch_bounds__(BLOCK) void k_cg_update(V* __restrict__ x, V* __restrict__ g,
+                                                     CgPair<V>* __restrict__ d,
+                                                     const V* __restrict__ w,
+                                                     const V* __restrict__ diag,
+                                                     const PcgState* __restrict__ st,
+                                                     const double* __restrict__ dirp, double* upd,
+                                                     uint32_t n) {
+    __shared__ double red[2][CG2_PARTS / WAVE], red2[2][BLOCK / WAVE];
+    const Chunk c = my_chunk(n);
+    const size_t u = c.beg + threadIdx.x;
+    const bool valid = u < c.end;
+    V xv{}, pv{}, gv{}, wv{}, dv{};
+    if (valid) {
+        xv = x[u];
+        pv = d[u].p;
+        gv = g[u];
+        wv = w[u];
+        dv = diag[u];
+    }
+    const uint32_t done = st->done;
+    const double rz = st->rz;
+    double tot[1];
+    all_sum<1>(dirp, gridDim.x, tot, red);
+    if (done) return;
+    const double alpha = rz / tot[0];
+    double acc[2] = {0.0, 0.0};
+    if (valid) {
+        x[u] = axpyu(xv, alpha, pv);
+        gv = axpyu(gv, alpha, wv);
+        g[u] = gv;
+        const V qv = divu(gv, dv);
+        d[u].q = qv;
+        acc[0] = dotu(gv, qv);
+        acc[1] = dotu(gv, gv);
+    }
+    block_sum<2>(acc, red2);
+    put_partials<2>(acc, upd);
+}
+
+// ---------------------------------------------------------------------------
 // mixed precision
 // ---------------------------------------------------------------------------
 // True residual in FP64 and its scaled FP32 image:
@@ -1018,6 +1481,96 @@ static int pcg_run(const Op& op, uint32_t nu, const double* diag_in, const typen
     return NBX_OK;
 }
 
+// The iteration in two kernels (k_cg_dir, k_cg_update), with pcg_run's host
+// cadence.  Node systems take it up to 131,072 nodes: us per iteration, five
+// kernels -> two, 64x32 cantilever 17.8 -> 9.3, 256x128 17 -> 9.1, 400x200 (80k
+// nodes) 17 -> 10.4, 600x300 (181k) 22.3 -> 17.9, 1024x512 (525k) 40 -> 47: a
+// row of the direction kernel gathers twice the bytes and holds 138 VGPRs.
+// Scalar CSR takes it up to 262,144 rows (figures at k_cg_dir_csr).  Both keep
+// the partials, which every workgroup sums, at 1,024 a value at most.
+constexpr uint32_t CG2_MAX_NODES = 131072, CG2_MAX_ROWS = 262144;
+template <class Op>
+static int pcg2_run(const Op& op, uint32_t nu, const double* diag_in, const typename Op::V* b,
+                    typename Op::V* x, uint32_t max_iter, double tol, Workspace& w, hipStream_t s,
+                    SolveStats* stats) {
+    using V = typename Op::V;
+    V* g = (V*)w.v64[0];
+    V* wv = (V*)w.v64[8];
+    // iteration j reads the pairs (q, p_{j-1}) of buffer j % 2 and leaves
+    // (q, p_j) in the other (each takes two consecutive vectors)
+    CgPair<V>* const d[2] = {(CgPair<V>*)w.v64[1], (CgPair<V>*)w.v64[6]};
+    const V* diag = (const V*)diag_in;
+    double* upd = w.partials;                       // of the update: 2 G
+    double* dirp = w.partials + 2 * (size_t)MAX_GRID;   // of the direction: G
+    PcgState h{};
+    h.tol2 = tol * tol;
+    h.max_iter = max_iter;
+    NBX_HIP(hipMemcpyAsync(w.st, &h, sizeof h, hipMemcpyHostToDevice, s));
+    const unsigned G = grid_for(nu);
+    const bool timed = w.ev[0] != nullptr;
+    if (timed) NBX_HIP(hipEventRecord(w.ev[0], s));
+    hipLaunchKernelGGL(k_cg_init<Op>, dim3(G), dim3(BLOCK), 0, s, op, b, x, g, d[0], diag, upd,
+                       nu);
+    NBX_HIP(hipGetLastError());
+    uint32_t nsamp = 0;
+    // iteration j's kernels depend on j only through j % 2 (and j = 0)
+    auto iteration = [&](uint32_t j, bool first, bool samp) {
+        j &= 1u;
+        if (samp) (void)hipEventRecord(w.sev[2 * nsamp], s);
+        launch_cg_dir(op, G, s, d[j], d[j ^ 1u], wv, w.st + j, w.st + (j ^ 1u), upd, dirp, nu,
+                      first);
+        if (samp) (void)hipEventRecord(w.sev[2 * nsamp++ + 1], s);
+        hipLaunchKernelGGL(k_cg_update<V>, dim3(G), dim3(BLOCK), 0, s, x, g, d[j ^ 1u], wv, diag,
+                           w.st + (j ^ 1u), dirp, upd, nu);
+    };
+    Replay four;
+    if (w.replay && s != nullptr)
+        NBX_TRY(capture(s, [&] {
+            for (uint32_t t = 0; t < 4; ++t) iteration(t, false, false);
+        }, four));
+    uint64_t launched = 0;   // 64-bit: max_iter near UINT32_MAX cannot wrap the guard
+    uint32_t batch = 4;
+    for (;;) {
+        for (uint32_t i = 0; i < batch; i += 4) {
+            const uint64_t j0 = launched + i;
+            const bool samp = timed && j0 % Workspace::SAMPLE_EVERY == 0 &&
+                              nsamp < (uint32_t)Workspace::NSAMP;
+            if (four.exec && !samp && j0 != 0) {
+                NBX_HIP(hipGraphLaunch(four.exec, s));
+            } else {
+                for (uint32_t t = 0; t < 4; ++t) iteration(t, j0 == 0 && t == 0, samp && t == 0);
+            }
+        }
+        NBX_HIP(hipGetLastError());
+        launched += batch;
+        // (an even number of iterations: the last state is in slot 0)
+        NBX_TRY(poll_state(w, s));
+        if (w.h_st->done) break;
+        if (launched > (uint64_t)max_iter + 8u) {
+            set_last_error("PCG did not report completion after %llu iterations",
+                           (unsigned long long)launched);
+            return NBX_ERR_BREAKDOWN;
+        }
+        batch = batch < 64 ? batch * 2 : 64;
+    }
+    if (timed) {
+        NBX_HIP(hipEventRecord(w.ev[1], s));
+        NBX_HIP(hipEventSynchronize(w.ev[1]));
+    }
+    if (stats) {
+        stats->iters = stats->fp64_iters = w.h_st->k;
+        stats->res0 = sqrt(w.h_st->gg0);
+        if (timed) {
+            float ms = 0.f;
+            NBX_HIP(hipEventElapsedTime(&ms, w.ev[0], w.ev[1]));
+            stats->ms = ms;
+            const uint32_t ran = (w.h_st->k + Workspace::SAMPLE_EVERY - 1) / Workspace::SAMPLE_EVERY;
+            NBX_TRY(sampled_ms(w, nsamp < ran ? nsamp : ran, &stats->ms_spmv_avg));
+        }
+    }
+    return NBX_OK;
+}
+
 __global__ void k_fill_one(double* __restrict__ v, uint32_t n) {
     const uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
     if (i < n) v[i] = 1.0;
@@ -1051,7 +1604,16 @@ int pcg_jacobi(const DevMatrix& m, const double* b, double* x, uint32_t max_iter
                                                8.0 * (double)m.y.n_lower
                                          : 36.0 * (double)m.s.n_blocks;
     const bool stream = mat_bytes + 40.0 * (double)m.n > (double)INFINITY_CACHE_BYTES;
-    if (m.blocked && m.has_sym && stream)
+    if (m.blocked && m.has_sym && m.s.n_nodes <= CG2_MAX_NODES)
+        rc = m.y.u_width && m.y.u_width <= 3 && m.y.l_width && m.y.l_width <= 3
+                 ? pcg2_run(OpSymU<3>{{m.y}}, m.s.n_nodes, diag, (const double2*)b, (double2*)x,
+                            max_iter, tol, w, s, stats)
+                 : pcg2_run(OpSymU<4>{{m.y}}, m.s.n_nodes, diag, (const double2*)b, (double2*)x,
+                            max_iter, tol, w, s, stats);
+    else if (m.blocked && m.s.n_nodes <= CG2_MAX_NODES)
+        rc = pcg2_run(OpS2{m.s}, m.s.n_nodes, diag, (const double2*)b, (double2*)x, max_iter, tol,
+                      w, s, stats);
+    else if (m.blocked && m.has_sym && stream)
         rc = pcg_run(OpSym{m.y}, m.s.n_nodes, diag, (const double2*)b, (double2*)x, max_iter, tol,
                      stream, w, s, stats);
     else if (m.blocked && m.has_sym)
@@ -1060,6 +1622,8 @@ int pcg_jacobi(const DevMatrix& m, const double* b, double* x, uint32_t max_iter
     else if (m.blocked)
         rc = pcg_run(OpS2{m.s}, m.s.n_nodes, diag, (const double2*)b, (double2*)x, max_iter, tol,
                      stream, w, s, stats);
+    else if (!m.blocked && m.c.n <= CG2_MAX_ROWS)
+        rc = pcg2_run(OpCsr{m.c}, m.c.n, diag, b, x, max_iter, tol, w, s, stats);
     else
         rc = pcg_run(OpCsr{m.c}, m.c.n, diag, b, x, max_iter, tol, stream, w, s, stats);
     if (rc) return -rc;
@@ -1077,7 +1641,11 @@ int pcg_jacobi_csr_view(const DevCsr& c, const double* diag, const double* b, do
         if (tol_reached) *tol_reached = 0.0;
         return 0;
     }
-    const int rc = pcg_run(OpCsr{c}, c.n, diag, b, x, max_iter, tol, false, w, s, nullptr);
+    if (c.n > CG2_MAX_ROWS) {
+        set_last_error("%u rows exceed the two-kernel PCG's %u", c.n, CG2_MAX_ROWS);
+        return -NBX_ERR_ARG;
+    }
+    const int rc = pcg2_run(OpCsr{c}, c.n, diag, b, x, max_iter, tol, w, s, nullptr);
     if (rc) return -rc;
     if (niter) *niter = w.h_st->k;
     if (tol_reached) *tol_reached = w.h_st->tol_reached;
