@@ -331,6 +331,42 @@ __device__ __forceinline__ bool cg_next(const PcgState* __restrict__ sin, PcgSta
     return !ended && go;
 }
 
+// The flexible CG's direction: p = z + beta p (p = z on the first step), beta
+// and the restart from the sums (z.w, r.z) as k_fin_fcg_dots forms them.
+struct FcgDir {
+    double beta;
+    bool first;
+    __device__ __forceinline__ double2 operator()(const CgPair<double2>& d) const {
+        return first ? d.q : axpyu(d.q, beta, d.p);
+    }
+};
+__device__ __forceinline__ bool cg_next(const PcgState* __restrict__ sin, PcgState* sout,
+                                        const double* __restrict__ dots, bool first,
+                                        double (*red)[CG2_PARTS / WAVE], FcgDir& dir) {
+    const uint32_t ended = sin->done;
+    const double alpha = sin->alpha, rz_old = sin->rz;
+    double tot[2];
+    all_sum<2>(dots, gridDim.x, tot, red);
+    const double rz = tot[1];
+    dir.beta = first ? 0.0 : -alpha * tot[0] / rz_old;
+    dir.first = first;
+    const bool restart = !(rz > 0.0) || !isfinite(rz) || !isfinite(dir.beta);
+    if (restart) dir.beta = 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sout->done = ended;
+        if (!ended) {
+            sout->k = sin->k;
+            sout->max_iter = sin->max_iter;
+            sout->tol2 = sin->tol2;
+            sout->gg0 = sin->gg0;
+            sout->beta = dir.beta;
+            sout->rz = rz;
+            sout->breakdown = sin->breakdown + (restart ? 1u : 0u);
+        }
+    }
+    return !ended;
+}
+
 // A row's loads ahead of beta, then the product with p formed on the fly;
 // blocks beyond the ones held ahead are loaded when they are used.
 template <class Op>
@@ -364,7 +400,8 @@ struct CgRow<OpS2> {
         for (int k = 0; k < U; ++k)
             if (k < len) x[k] = d[w[k]];
     }
-    __device__ __forceinline__ double2 product(const CgDir& dir, double2,
+    template <class D>
+    __device__ __forceinline__ double2 product(const D& dir, double2,
                                                const CgPair<double2>* __restrict__ d) const {
         double s0 = 0.0, s1 = 0.0;
         auto add = [&](dv2 ka, dv2 kb, double2 v) {
@@ -441,7 +478,8 @@ struct CgRow<OpSymU<U>> {
         for (int k = 0; k < U; ++k)
             if (k < un) ux[k] = d[w[k]];
     }
-    __device__ __forceinline__ double2 product(const CgDir& dir, double2 pd,
+    template <class D>
+    __device__ __forceinline__ double2 product(const D& dir, double2 pd,
                                                const CgPair<double2>* __restrict__ d) const {
         const dv2* __restrict__ pa = reinterpret_cast<const dv2*>(Y.u_val);
         const dv2* __restrict__ pb = reinterpret_cast<const dv2*>(Y.u_val + 2 * Y.n_upper);
@@ -506,7 +544,7 @@ __global__ __launch_bounds__(BLOCK) void k_cg_init(Op op, const typename Op::V* 
     put_partials<2>(acc, partials);
 }
 
-template <class Op>
+template <class Op, class D>
 __global__ __launch_bounds__(BLOCK) void k_cg_dir(Op op,
                                                   const CgPair<typename Op::V>* __restrict__ d,
                                                   CgPair<typename Op::V>* __restrict__ dnew,
@@ -525,7 +563,7 @@ __global__ __launch_bounds__(BLOCK) void k_cg_dir(Op op,
         own = d[u];
         row.load((uint32_t)u, d);
     }
-    CgDir dir;
+    D dir;
     if (!cg_next(sin, sout, upd, first, red, dir)) return;
     double acc[1] = {0.0};
     if (valid) {
@@ -638,7 +676,7 @@ static void launch_cg_dir(const Op& op, unsigned G, hipStream_t s,
             hipLaunchKernelGGL(k_cg_dir_csr<8>, dim3(G), dim3(BLOCK), 0, s, op.A, d, dnew, w, sin,
                                sout, upd, dirp, n, first);
     } else {
-        hipLaunchKernelGGL(k_cg_dir<Op>, dim3(G), dim3(BLOCK), 0, s, op, d, dnew, w, sin,
+        hipLaunchKernelGGL((k_cg_dir<Op, CgDir>), dim3(G), dim3(BLOCK), 0, s, op, d, dnew, w, sin,
                            sout, upd, dirp, n, first);
     }
 }
@@ -1309,6 +1347,122 @@ __global__ __launch_bounds__(BLOCK) void k_fcg_p(const P* __restrict__ z,
     }
 }
 
+// The flexible CG's outer iteration without one-workgroup kernels, up to
+// FCG2_MAX_NODES: k_cg_dir<.., FcgDir> (the direction and w = K p), this
+// update, the preconditioner, then k_fcg2_dots; 3 kernels in place of 7 around
+// the preconditioner (2-3 us each).  Every workgroup sums the partials of the
+// kernel before it, as in the two-kernel PCG, with the same results bit for
+// bit as the separate kernels.  State slots: k_cg_dir reads s0 and writes s1,
+// the update reads s1 and leaves alpha in s0, the preconditioner's kernels
+// read s1, k_fcg2_dots reads s1 and writes s0 (all but alpha).  The stop test
+// runs in k_fcg2_dots, so the iteration that meets the tolerance still runs
+// its preconditioner.
+// FIRST: r = b - K x; otherwise x += alpha p, r -= alpha w.
+template <bool FIRST>
+__global__ __launch_bounds__(BLOCK) void k_fcg2_update(
+    Sell2 K, const double2* __restrict__ b, double2* __restrict__ x, double2* __restrict__ r,
+    const CgPair<double2>* __restrict__ d, const double2* __restrict__ w,
+    const double2* __restrict__ dis, float2* __restrict__ res, float2* __restrict__ dz,
+    float2* __restrict__ z, PcgState* s0, const PcgState* __restrict__ s1,
+    const double* __restrict__ dirp, double* rrp, uint32_t n, double inv_theta) {
+    __shared__ double red[1][CG2_PARTS / WAVE], red2[1][BLOCK / WAVE];
+    const Chunk c = my_chunk(n);
+    const size_t i = c.beg + threadIdx.x;
+    const bool valid = i < c.end;
+    double2 xv{}, pv{}, rv{}, wv{}, dd{};
+    if (valid) {
+        dd = dis[i];
+        if constexpr (!FIRST) {
+            xv = x[i];
+            pv = d[i].p;
+            rv = r[i];
+            wv = w[i];
+        }
+    }
+    double alpha = 0.0;
+    if constexpr (!FIRST) {
+        const uint32_t done = s1->done;
+        const double rz = s1->rz;
+        double tot[1];
+        all_sum<1>(dirp, gridDim.x, tot, red);
+        if (done) return;
+        alpha = rz / tot[0];
+        if (blockIdx.x == 0 && threadIdx.x == 0) s0->alpha = alpha;
+    }
+    double acc[1] = {0.0};
+    if (valid) {
+        if constexpr (FIRST) {
+            const double2 ku = row64(K, (uint32_t)i, x);
+            const double2 bi = b[i];
+            rv = make_double2(bi.x - ku.x, bi.y - ku.y);
+        } else {
+            x[i] = axpyu(xv, alpha, pv);
+            rv = make_double2(rv.x - alpha * wv.x, rv.y - alpha * wv.y);
+        }
+        r[i] = rv;
+        const float2 sv = make_float2((float)(dd.x * rv.x), (float)(dd.y * rv.y));
+        const float it = (float)inv_theta;
+        res[i] = sv;
+        const float2 dv = make_float2(sv.x * it, sv.y * it);
+        dz[i] = dv;
+        z[i] = dv;
+        acc[0] += rv.x * rv.x + rv.y * rv.y;
+    }
+    block_sum<1>(acc, red2);
+    put_partials<1>(acc, rrp);
+}
+
+// The stop test on r.r (as k_fin_fcg_update); z64 = dis z for the next
+// direction; partials z64.w and r.z64.
+__global__ __launch_bounds__(BLOCK) void k_fcg2_dots(const float2* __restrict__ z,
+                                                     const double2* __restrict__ dis,
+                                                     const double2* __restrict__ w,
+                                                     const double2* __restrict__ r,
+                                                     CgPair<double2>* __restrict__ d, PcgState* s0,
+                                                     const PcgState* __restrict__ s1,
+                                                     const double* __restrict__ rrp, double* dots,
+                                                     uint32_t n, bool first) {
+    __shared__ double red[1][CG2_PARTS / WAVE], red2[2][BLOCK / WAVE];
+    const Chunk c = my_chunk(n);
+    const size_t i = c.beg + threadIdx.x;
+    const bool valid = i < c.end;
+    double2 zz{}, wv{}, rv{};
+    if (valid) {
+        zz = z_unscaled(z, dis, i);
+        if (!first) wv = w[i];
+        rv = r[i];
+    }
+    const uint32_t ended = s1->done, max_iter = s1->max_iter;
+    const uint32_t k = first ? s1->k : s1->k + 1u;
+    const double tol2 = s1->tol2;
+    double tot[1];
+    all_sum<1>(rrp, gridDim.x, tot, red);
+    if (ended) return;   // (s0 holds the end of the solve)
+    const double gg = tot[0];
+    const bool met = !(gg > tol2), stop = met || k >= max_iter || !isfinite(gg);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        s0->k = k;
+        s0->max_iter = max_iter;
+        s0->tol2 = tol2;
+        s0->gg0 = first ? gg : s1->gg0;
+        s0->gg_cur = gg;
+        s0->tol_reached = sqrt(gg);
+        s0->rz = s1->rz;
+        s0->breakdown = s1->breakdown;
+        s0->done = stop ? 1u : 0u;
+        s0->status = met ? 0u : 1u;
+    }
+    if (stop) return;
+    double acc[2] = {0.0, 0.0};
+    if (valid) {
+        d[i].q = zz;
+        if (!first) acc[0] += dotu(zz, wv);
+        acc[1] += dotu(rv, zz);
+    }
+    block_sum<2>(acc, red2);
+    put_partials<2>(acc, dots);
+}
+
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
@@ -1481,6 +1635,12 @@ static int pcg_run(const Op& op, uint32_t nu, const double* diag_in, const typen
     return NBX_OK;
 }
 
+// three lower and three upper blocks a row, every slice alike (an interior
+// row of a T3 mesh)
+static bool sym_u3(const Sym2& y) {
+    return y.u_width && y.u_width <= 3 && y.l_width && y.l_width <= 3;
+}
+
 // The iteration in two kernels (k_cg_dir, k_cg_update), with pcg_run's host
 // cadence.  Node systems take it up to 131,072 nodes: us per iteration, five
 // kernels -> two, 64x32 cantilever 17.8 -> 9.3, 256x128 17 -> 9.1, 400x200 (80k
@@ -1488,6 +1648,7 @@ static int pcg_run(const Op& op, uint32_t nu, const double* diag_in, const typen
 // row of the direction kernel gathers twice the bytes and holds 138 VGPRs.
 // Scalar CSR takes it up to 262,144 rows (figures at k_cg_dir_csr).  Both keep
 // the partials, which every workgroup sums, at 1,024 a value at most.
+constexpr uint32_t FCG2_MAX_NODES = CG2_PARTS * BLOCK;
 constexpr uint32_t CG2_MAX_NODES = 131072, CG2_MAX_ROWS = 262144;
 template <class Op>
 static int pcg2_run(const Op& op, uint32_t nu, const double* diag_in, const typename Op::V* b,
@@ -1605,7 +1766,7 @@ int pcg_jacobi(const DevMatrix& m, const double* b, double* x, uint32_t max_iter
                                          : 36.0 * (double)m.s.n_blocks;
     const bool stream = mat_bytes + 40.0 * (double)m.n > (double)INFINITY_CACHE_BYTES;
     if (m.blocked && m.has_sym && m.s.n_nodes <= CG2_MAX_NODES)
-        rc = m.y.u_width && m.y.u_width <= 3 && m.y.l_width && m.y.l_width <= 3
+        rc = sym_u3(m.y)
                  ? pcg2_run(OpSymU<3>{{m.y}}, m.s.n_nodes, diag, (const double2*)b, (double2*)x,
                             max_iter, tol, w, s, stats)
                  : pcg2_run(OpSymU<4>{{m.y}}, m.s.n_nodes, diag, (const double2*)b, (double2*)x,
@@ -1856,7 +2017,8 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
     PcgState h{};
     h.tol2 = rtol * rtol * bb;
     h.max_iter = max_iter;
-    NBX_HIP(hipMemcpyAsync(w.st, &h, sizeof h, hipMemcpyHostToDevice, s));
+    const PcgState h2[2] = {h, h};
+    NBX_HIP(hipMemcpyAsync(w.st, h2, sizeof h2, hipMemcpyHostToDevice, s));
     // Chebyshev coefficients on [lmax/ratio, lmax] (Saad, Alg. 12.1)
     const uint32_t deg = opt.cheb_degree < 1 ? 1 : opt.cheb_degree;
     const double lmax = m.lambda_max, lmin = lmax / opt.cheb_ratio;
@@ -1892,6 +2054,15 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
     const unsigned G = red_grid(nu);
     OpS2 op{m.s};
     OpSym ops{m.y};
+    // three kernels around the preconditioner (k_fcg2_update) or seven; the
+    // preconditioner's kernels test `done` in stp
+    const bool fold = !p64 && nu <= FCG2_MAX_NODES;
+    PcgState* const stp = fold ? w.st + 1 : w.st;
+    CgPair<double2>* const pair[2] = {(CgPair<double2>*)w.v64[1], (CgPair<double2>*)w.v64[6]};
+    if (fold) wv = (double2*)w.v64[8];
+    double* const dots = w.partials;                             // 2 G
+    double* const dirp = w.partials + 2 * (size_t)MAX_GRID;      // G
+    double* const rrp = w.partials + 3 * (size_t)MAX_GRID;       // G
     // The fp16 preconditioner's working set (matrix + four FP32 vectors) is
     // read by each of the degree - 1 steps in a row: when it fits in the
     // Infinity Cache, cached loads keep it there between steps (at 4.2M DOF,
@@ -1918,15 +2089,43 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
                                                4.0 * (double)m.o.n_pairs + 4.0 * (double)nu
                                          : 12.0 * (double)m.o.n_blocks + 4.0 * (double)nu;
     const bool fine_cached = fine_mat + 41.0 * (double)nu <= (double)INFINITY_CACHE_BYTES;
-    auto precondition_amg16 = [&](int first) {
-        hipLaunchKernelGGL(k_fcg_update<float2>, dim3(G), dim3(BLOCK), 0, s, m.s, bv, xv, r, p, wv,
-                           dis, res, da, z, w.st, w.partials, nu, first, fine.inv_theta);
-        hipLaunchKernelGGL(k_fin_fcg_update, dim3(1), dim3(FIN), 0, s, w.st, w.partials, G, first);
+    // What precedes and follows the preconditioner in the step that leaves
+    // z_j (first: z_0); dscale: the diagonal scaling (ones: none).
+    auto before = [&](int first, uint32_t j, const double2* dscale, double theta_inv) {
+        if (!fold) {
+            hipLaunchKernelGGL(k_fcg_update<float2>, dim3(G), dim3(BLOCK), 0, s, m.s, bv, xv, r, p,
+                               wv, dscale, res, da, z, w.st, w.partials, nu, first, theta_inv);
+            hipLaunchKernelGGL(k_fin_fcg_update, dim3(1), dim3(FIN), 0, s, w.st, w.partials, G,
+                               first);
+        } else if (first) {
+            hipLaunchKernelGGL(k_fcg2_update<true>, dim3(G), dim3(BLOCK), 0, s, m.s, bv, xv, r,
+                               pair[j & 1], wv, dscale, res, da, z, w.st, stp, dirp, rrp, nu,
+                               theta_inv);
+        } else {
+            hipLaunchKernelGGL(k_fcg2_update<false>, dim3(G), dim3(BLOCK), 0, s, m.s, bv, xv, r,
+                               pair[j & 1], wv, dscale, res, da, z, w.st, stp, dirp, rrp, nu,
+                               theta_inv);
+        }
+    };
+    auto after = [&](int first, uint32_t j, const double2* dscale) {
+        if (fold) {
+            hipLaunchKernelGGL(k_fcg2_dots, dim3(G), dim3(BLOCK), 0, s, z, dscale, wv, r,
+                               pair[j & 1], w.st, stp, rrp, dots, nu, first != 0);
+            return;
+        }
+        hipLaunchKernelGGL(k_fcg_dots<float2>, dim3(G), dim3(BLOCK), 0, s, z, dscale, wv, r, w.st,
+                           w.partials, nu, first);
+        hipLaunchKernelGGL(k_fin_fcg_dots, dim3(1), dim3(FIN), 0, s, w.st, w.partials, G, first);
+        hipLaunchKernelGGL(k_fcg_p<float2>, dim3(G), dim3(BLOCK), 0, s, z, dscale, p, w.st, nu,
+                           first);
+    };
+    auto precondition_amg16 = [&](int first, uint32_t j) {
+        before(first, j, dis, fine.inv_theta);
         auto cycle = [&](const auto& K) {
             if (fine_cached)
-                amg16_cycle<false>(K, fine, m.amg, res, da, db, z, w.st, nu, G, s);
+                amg16_cycle<false>(K, fine, m.amg, res, da, db, z, stp, nu, G, s);
             else
-                amg16_cycle<true>(K, fine, m.amg, res, da, db, z, w.st, nu, G, s);
+                amg16_cycle<true>(K, fine, m.amg, res, da, db, z, stp, nu, G, s);
         };
         if (m.off_packed && m.o.width)
             cycle(Off16U{m.o});
@@ -1934,42 +2133,33 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
             cycle(Off16P{m.o});
         else
             cycle(m.o);
-        hipLaunchKernelGGL(k_fcg_dots<float2>, dim3(G), dim3(BLOCK), 0, s, z, dis, wv, r, w.st,
-                           w.partials, nu, first);
-        hipLaunchKernelGGL(k_fin_fcg_dots, dim3(1), dim3(FIN), 0, s, w.st, w.partials, G, first);
-        hipLaunchKernelGGL(k_fcg_p<float2>, dim3(G), dim3(BLOCK), 0, s, z, dis, p, w.st, nu, first);
+        after(first, j, dis);
     };
-    auto precondition_amg = [&](int first) {
+    auto precondition_amg = [&](int first, uint32_t j) {
         // a one-level hierarchy: the update with a unit scaling writes r in
         // FP32 (res), the dense solve z = C^-1 r, the dot products and
         // direction read z unscaled
-        hipLaunchKernelGGL(k_fcg_update<float2>, dim3(G), dim3(BLOCK), 0, s, m.s, bv, xv, r, p, wv,
-                           ones, res, da, z, w.st, w.partials, nu, first, 1.0);
-        hipLaunchKernelGGL(k_fin_fcg_update, dim3(1), dim3(FIN), 0, s, w.st, w.partials, G, first);
-        (void)amg_vcycle(m.amg, (const float*)res, (float*)z, w.st, s);
-        hipLaunchKernelGGL(k_fcg_dots<float2>, dim3(G), dim3(BLOCK), 0, s, z, ones, wv, r, w.st,
-                           w.partials, nu, first);
-        hipLaunchKernelGGL(k_fin_fcg_dots, dim3(1), dim3(FIN), 0, s, w.st, w.partials, G, first);
-        hipLaunchKernelGGL(k_fcg_p<float2>, dim3(G), dim3(BLOCK), 0, s, z, ones, p, w.st, nu,
-                           first);
+        before(first, j, ones, 1.0);
+        (void)amg_vcycle(m.amg, (const float*)res, (float*)z, stp, s);
+        after(first, j, ones);
     };
-    auto precondition = [&](int first) {
+    auto precondition = [&](int first, uint32_t j) {
         if (amg && fine.scaled16) {
-            precondition_amg16(first);
+            precondition_amg16(first, j);
             return;
         }
         if (amg) {
-            precondition_amg(first);
+            precondition_amg(first, j);
             return;
         }
         if (p64) {
             hipLaunchKernelGGL(k_fcg_update<double2>, dim3(G), dim3(BLOCK), 0, s, m.s, bv, xv, r, p,
                                wv, dis, res64, da64, z64, w.st, w.partials, nu, first, inv_theta);
+            hipLaunchKernelGGL(k_fin_fcg_update, dim3(1), dim3(FIN), 0, s, w.st, w.partials, G,
+                               first);
         } else {
-            hipLaunchKernelGGL(k_fcg_update<float2>, dim3(G), dim3(BLOCK), 0, s, m.s, bv, xv, r, p,
-                               wv, dis, res, da, z, w.st, w.partials, nu, first, inv_theta);
+            before(first, j, dis, inv_theta);
         }
-        hipLaunchKernelGGL(k_fin_fcg_update, dim3(1), dim3(FIN), 0, s, w.st, w.partials, G, first);
         float2* din = da;
         float2* dout = db;
         if (tiled) {
@@ -1983,7 +2173,7 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
                     cs.c1[t] = c1d[k + t];
                     cs.c2[t] = c2d[k + t];
                 }
-                launch_cheb_tiles(m.o, m.t, cs, din, dout, rin, rout, z, w.st, s);
+                launch_cheb_tiles(m.o, m.t, cs, din, dout, rin, rout, z, stp, s);
                 std::swap(din, dout);
                 std::swap(rin, rout);
             }
@@ -1993,10 +2183,10 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
         for (uint32_t k = 1; k < deg && !tiled; ++k) {
             auto step = [&](const auto& K) {
                 if (cheb_cached)
-                    launch_cheb_step64<false>(k, deg - 1, G, s, K, din, dout, res, z, w.st, nu,
+                    launch_cheb_step64<false>(k, deg - 1, G, s, K, din, dout, res, z, stp, nu,
                                               c1d[k], c2d[k]);
                 else
-                    launch_cheb_step64<true>(k, deg - 1, G, s, K, din, dout, res, z, w.st, nu,
+                    launch_cheb_step64<true>(k, deg - 1, G, s, K, din, dout, res, z, stp, nu,
                                              c1d[k], c2d[k]);
             };
             if (p64 && m.has_sym && cheb_cached)
@@ -2018,27 +2208,22 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
                 step(m.s);
             else
                 hipLaunchKernelGGL(k_cheb_step<32>, dim3(G), dim3(BLOCK), 0, s, m.s, din, dout, res, z,
-                                   w.st, nu, c1[k], c2[k]);
+                                   stp, nu, c1[k], c2[k]);
             std::swap(din, dout);
             std::swap(din64, dout64);
         }
-        if (p64) {
-            hipLaunchKernelGGL(k_fcg_dots<double2>, dim3(G), dim3(BLOCK), 0, s, z64, dis, wv, r,
-                               w.st, w.partials, nu, first);
-        } else {
-            hipLaunchKernelGGL(k_fcg_dots<float2>, dim3(G), dim3(BLOCK), 0, s, z, dis, wv, r, w.st,
-                               w.partials, nu, first);
+        if (!p64) {
+            after(first, j, dis);
+            return;
         }
+        hipLaunchKernelGGL(k_fcg_dots<double2>, dim3(G), dim3(BLOCK), 0, s, z64, dis, wv, r, w.st,
+                           w.partials, nu, first);
         hipLaunchKernelGGL(k_fin_fcg_dots, dim3(1), dim3(FIN), 0, s, w.st, w.partials, G, first);
-        if (p64)
-            hipLaunchKernelGGL(k_fcg_p<double2>, dim3(G), dim3(BLOCK), 0, s, z64, dis, p, w.st, nu,
-                               first);
-        else
-            hipLaunchKernelGGL(k_fcg_p<float2>, dim3(G), dim3(BLOCK), 0, s, z, dis, p, w.st, nu,
-                               first);
+        hipLaunchKernelGGL(k_fcg_p<double2>, dim3(G), dim3(BLOCK), 0, s, z64, dis, p, w.st, nu,
+                           first);
     };
     NBX_HIP(hipEventRecord(w.ev[0], s));
-    precondition(1);
+    precondition(1, 0);
     NBX_HIP(hipGetLastError());
     NBX_TRY(poll_state(w, s));
     // Iterations launched between polls of the device state.  Kernels
@@ -2057,30 +2242,45 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
     }
     uint64_t launched = 0;   // 64-bit: max_iter near UINT32_MAX cannot wrap the guard
     constexpr uint32_t every = 8;   // sample one outer iteration in eight
-    // An outer iteration: the FP64 product, then the preconditioner and the
-    // flexible-CG updates; the same kernels and arguments every time.
-    auto outer = [&](bool samp) {
+    // Outer iteration j: the FP64 product, then the preconditioner and the
+    // flexible-CG updates; the same kernels and arguments every second time
+    // (but for j = 0).
+    auto outer = [&](uint32_t j, bool head, bool samp) {
         if (samp) (void)hipEventRecord(w.sev[2 * nsamp], s);
-        if (m.has_sym)
+        auto dir = [&](const auto& o) {
+            using Op = std::decay_t<decltype(o)>;
+            hipLaunchKernelGGL((k_cg_dir<Op, FcgDir>), dim3(G), dim3(BLOCK), 0, s, o, pair[j & 1],
+                               pair[(j + 1) & 1], wv, w.st, stp, dots, dirp, nu, head);
+        };
+        if (fold && m.has_sym && sym_u3(m.y))
+            dir(OpSymU<3>{{m.y}});
+        else if (fold && m.has_sym)
+            dir(OpSymU<4>{{m.y}});
+        else if (fold)
+            dir(op);
+        else if (m.has_sym)
             hipLaunchKernelGGL(k_pcg_A<OpSym>, dim3(G), dim3(BLOCK), 0, s, ops,
                                (const double2*)p, wv, w.st, w.partials, nu);
         else
             hipLaunchKernelGGL(k_pcg_A<OpS2>, dim3(G), dim3(BLOCK), 0, s, op,
                                (const double2*)p, wv, w.st, w.partials, nu);
         if (samp) (void)hipEventRecord(w.sev[2 * nsamp++ + 1], s);
-        hipLaunchKernelGGL(k_fin_A, dim3(1), dim3(FIN), 0, s, w.st, w.partials, G);
-        precondition(0);
+        if (!fold)
+            hipLaunchKernelGGL(k_fin_A, dim3(1), dim3(FIN), 0, s, w.st, w.partials, G);
+        precondition(0, j + 1);
     };
-    Replay one;
+    Replay two[2];
     if (w.replay && s != nullptr && !w.h_st->done)
-        NBX_TRY(capture(s, [&] { outer(false); }, one));
+        for (uint32_t j = 0; j < 2; ++j)
+            NBX_TRY(capture(s, [&] { outer(j, false, false); }, two[j]));
     while (!w.h_st->done) {
         for (uint32_t i = 0; i < batch; ++i) {
             const bool samp = (launched + i) % every == 0 && nsamp < (uint32_t)Workspace::NSAMP;
-            if (one.exec && !samp)
-                NBX_HIP(hipGraphLaunch(one.exec, s));
+            const uint64_t j = launched + i;
+            if (two[j & 1].exec && !samp && j != 0)
+                NBX_HIP(hipGraphLaunch(two[j & 1].exec, s));
             else
-                outer(samp);
+                outer((uint32_t)(j & 1), j == 0, samp);
         }
         NBX_HIP(hipGetLastError());
         launched += batch;
