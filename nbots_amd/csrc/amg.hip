@@ -33,6 +33,7 @@ namespace nbx {
 struct BellDev {
     uint32_t rows = 0;
     int lanes = 1;             // lanes per block row in the V-cycle's products
+    uint32_t wmax = 0;         // blocks of the longest row
     size_t slots = 0;
     uint32_t* slice_ptr = nullptr;
     uint16_t* len = nullptr;
@@ -78,6 +79,7 @@ struct AmgDev {
     // scaled copy, in scaled variables, and its P values are stored as
     // D^1/2 P (FP32)
     bool scaled16 = false;
+    size_t bottom = 0;              // the level k_amg_bottom starts from, or 0
 };
 
 namespace {
@@ -688,6 +690,227 @@ __global__ __launch_bounds__(DENSE_BLOCK) void k_amg_dense(const float* __restri
     }
 }
 
+// ---- the bottom of the V-cycle in one workgroup -------------------------------
+// A smoothing step on a level of a few hundred unknowns costs a launch and a
+// chain of dependent loads (3.5-4 us), and the last smoothed level takes 8-13
+// such launches per cycle with the dense solve below it.  One workgroup of
+// 512 threads does them all, down to the dense solve and back up, when that
+// level has at most 1,024 unknowns.  Its operator is read once and kept in
+// registers (a thread holds one or two scalar rows, padded with zero blocks
+// to HELD, so that a product's LDS reads go out together), every vector lives
+// in LDS, and a step costs one barrier; the products (0.5-1 us) and the loads
+// of P, P^T and C^-1 bound it.  Every sum keeps the order of the kernels of
+// one step each, so the cycle's result is the same to the bit.  The kernel and the outer iteration around it,
+// with the launches it replaces and with it (cantilevers): 357 unknowns
+// (150x75) 14 us, 104 -> 71; 726 (64x32) 62 -> 44; 969 (256x128) 27 us,
+// 118 -> 95; 288 (512x256) 18 us, 184 -> 150; 312 (2048x1024) 25 us,
+// 661 -> 630.  With 1,024 threads the rows spill (128 VGPRs): 20 us at 357.
+// Threads take the scalar rows of equal component r of consecutive block
+// rows, so that a wavefront's loads of a block position are coalesced.
+constexpr int BOTTOM_TB = 512;
+struct BottomLevel {
+    Bell<3, 3> A, P, T;
+    const float* dinv;
+    int p_lanes, t_lanes;               // lanes per row of P and T
+    uint32_t rows, degree;              // block rows
+    float inv_theta, c1[AMG_MAX_DEGREE], c2[AMG_MAX_DEGREE];
+};
+struct Bottom {
+    BottomLevel lv;
+    uint32_t nco;
+    const float* cinv;
+    const float* b;
+    float* x;
+};
+// the scalar rows of one thread on a level: row j is component r of block
+// row I, q = r rows + I = threadIdx.x + 512 j
+template <int RP, int HELD, int LANES>   // HELD: blocks of a row, none longer
+struct BottomRows {
+    uint32_t i[RP];   // the scalar row 3 I + r, or none
+    float dinv[RP];
+    static constexpr uint32_t NO_ROW = 0xffffffffu;
+    __device__ __forceinline__ bool on(int j) const { return i[j] != NO_ROW; }
+    float v[RP][HELD][3];
+    uint32_t col[RP][HELD / 2];   // two 16-bit positions (3 J) per word
+    __device__ __forceinline__ void load(const BottomLevel& L) {
+#pragma unroll
+        for (int j = 0; j < RP; ++j) {
+            const uint32_t q = threadIdx.x + (uint32_t)j * BOTTOM_TB;
+            const uint32_t r = q / L.rows, I = q - r * L.rows;
+            const bool valid = r < 3;
+            i[j] = valid ? 3 * I + r : NO_ROW;
+            dinv[j] = valid ? L.dinv[i[j]] : 0.f;
+            const size_t base = valid ? (size_t)L.A.slice_ptr[I >> 6] + (I & 63) : 0;
+            const int len = valid ? L.A.len[I] : 0;
+#pragma unroll
+            for (int k = 0; k < HELD / 2; ++k) col[j][k] = 0;
+#pragma unroll
+            for (int k = 0; k < HELD; ++k) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) v[j][k][c] = 0.f;
+                if (k < len) {
+                    const size_t sl = base + (size_t)k * SLICE;
+                    col[j][k / 2] |= (3 * L.A.bcol[sl]) << (16 * (k & 1));
+#pragma unroll
+                    for (int c = 0; c < 3; ++c)
+                        v[j][k][c] = L.A.val[(size_t)(3 * r + c) * L.A.slots + sl];
+                }
+            }
+        }
+    }
+    // (A x) of row j, summed as bell_row's LANES lanes sum it
+    __device__ __forceinline__ float product(int j, const float* x) const {
+        float y[LANES] = {};
+#pragma unroll
+        for (int k = 0; k < HELD; ++k) {
+            const float* xk = x + ((col[j][k / 2] >> (16 * (k & 1))) & 0xffffu);
+            float& t = y[k % LANES];
+            t += v[j][k][0] * xk[0];
+            t += v[j][k][1] * xk[1];
+            t += v[j][k][2] * xk[2];
+        }
+#pragma unroll
+        for (int o = LANES / 2; o > 0; o >>= 1)
+#pragma unroll
+            for (int l = 0; l < o; ++l) y[l] += y[l + o];
+        return y[0];
+    }
+};
+// Vectors of a level in LDS: right-hand side, solution, residual (or the
+// second direction), direction.
+struct BottomVec {
+    float *b, *x, *r, *d;
+};
+// x = 0 start and degree - 1 steps, then the residual b - A x into v.r
+template <int RP, int HELD, int LANES>
+__device__ __forceinline__ void bottom_down(const BottomLevel& L, const BottomRows<RP, HELD, LANES>& R,
+                                            const BottomVec& v) {
+    float rr[RP], xx[RP], dd[RP];
+#pragma unroll
+    for (int j = 0; j < RP; ++j)
+        if (R.on(j)) {
+            const uint32_t i = R.i[j];
+            rr[j] = R.dinv[j] * v.b[i];
+            dd[j] = rr[j] * L.inv_theta;
+            xx[j] = dd[j];
+            v.d[i] = dd[j];
+        }
+    float *din = v.d, *dout = v.r;
+    for (uint32_t k = 1; k < L.degree; ++k) {
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < RP; ++j)
+            if (R.on(j)) {
+                rr[j] -= R.dinv[j] * R.product(j, din);
+                dd[j] = L.c1[k] * dd[j] + L.c2[k] * rr[j];
+                xx[j] += dd[j];
+                dout[R.i[j]] = dd[j];
+            }
+        float* t = din;
+        din = dout;
+        dout = t;
+    }
+#pragma unroll
+    for (int j = 0; j < RP; ++j)
+        if (R.on(j)) v.x[R.i[j]] = xx[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < RP; ++j)
+        if (R.on(j)) {
+            const uint32_t i = R.i[j];
+            v.r[i] = v.b[i] - R.product(j, v.x);
+        }
+    __syncthreads();
+}
+// post-smoothing from v.x
+template <int RP, int HELD, int LANES>
+__device__ __forceinline__ void bottom_up(const BottomLevel& L, const BottomRows<RP, HELD, LANES>& R,
+                                          const BottomVec& v) {
+    float rr[RP], xx[RP], dd[RP];
+#pragma unroll
+    for (int j = 0; j < RP; ++j)
+        if (R.on(j)) {
+            const uint32_t i = R.i[j];
+            xx[j] = v.x[i];
+            rr[j] = R.dinv[j] * (v.b[i] - R.product(j, v.x));
+            dd[j] = rr[j] * L.inv_theta;
+            v.d[i] = dd[j];
+        }
+    float *din = v.d, *dout = v.r;
+    for (uint32_t k = 1; k < L.degree; ++k) {
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < RP; ++j)
+            if (R.on(j)) {
+                rr[j] -= R.dinv[j] * R.product(j, din);
+                const float dn = L.c1[k] * dd[j] + L.c2[k] * rr[j];
+                xx[j] += k == 1 ? dd[j] + dn : dn;
+                dd[j] = dn;
+                dout[R.i[j]] = dn;
+            }
+        float* t = din;
+        din = dout;
+        dout = t;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < RP; ++j)
+        if (R.on(j)) v.x[R.i[j]] = xx[j];
+    __syncthreads();
+}
+// y = B x, or y += B x (ADD); LANES lanes per block row
+template <bool ADD, int LANES>
+__device__ __forceinline__ void bottom_apply(const Bell<3, 3>& B, uint32_t rows, const float* x,
+                                             float* y) {
+    const uint32_t lane = threadIdx.x % LANES;
+    for (uint32_t I = threadIdx.x / LANES; I < rows; I += BOTTOM_TB / LANES) {
+        float t[3];
+        bell_row<3, 3, LANES>(B, I, lane, x, t);
+        if (lane == 0)
+#pragma unroll
+            for (int r = 0; r < 3; ++r) y[3 * I + r] = ADD ? y[3 * I + r] + t[r] : t[r];
+    }
+    __syncthreads();
+}
+template <bool ADD>
+__device__ __forceinline__ void bottom_apply(const Bell<3, 3>& B, int lanes, uint32_t rows,
+                                             const float* x, float* y) {
+    switch (lanes) {
+        case 1: bottom_apply<ADD, 1>(B, rows, x, y); break;
+        case 2: bottom_apply<ADD, 2>(B, rows, x, y); break;
+        case 4: bottom_apply<ADD, 4>(B, rows, x, y); break;
+        case 8: bottom_apply<ADD, 8>(B, rows, x, y); break;
+        default: bottom_apply<ADD, 16>(B, rows, x, y); break;
+    }
+}
+template <int RP, int HELD, int LANES>
+__global__ __launch_bounds__(BOTTOM_TB) void k_amg_bottom(Bottom B, const PcgState* st) {
+    if (st->done) return;
+    extern __shared__ float lds[];
+    const BottomLevel& L0 = B.lv;
+    const uint32_t n = 3 * L0.rows;
+    const BottomVec v{lds, lds + n, lds + 2 * n, lds + 3 * n};
+    float *bc = lds + 4 * n, *xc = bc + B.nco;
+    BottomRows<RP, HELD, LANES> R0;
+    R0.load(L0);
+    for (uint32_t i = threadIdx.x; i < n; i += BOTTOM_TB) v.b[i] = B.b[i];
+    __syncthreads();
+    bottom_down(L0, R0, v);
+    bottom_apply<false>(L0.T, L0.t_lanes, B.nco / 3, v.r, bc);
+    // x = C^-1 b (C^-1 is symmetric: its columns are read as rows)
+    if (threadIdx.x < B.nco) {
+        const float* c = B.cinv + threadIdx.x;
+        float t = 0.f;
+#pragma unroll 24
+        for (uint32_t j = 0; j < B.nco; ++j) t += c[(size_t)j * B.nco] * bc[j];
+        xc[threadIdx.x] = t;
+    }
+    __syncthreads();
+    bottom_apply<true>(L0.P, L0.p_lanes, L0.rows, xc, v.x);
+    bottom_up(L0, R0, v);
+    for (uint32_t i = threadIdx.x; i < n; i += BOTTOM_TB) B.x[i] = v.x[i];
+}
+
 }  // namespace
 
 
@@ -743,6 +966,7 @@ static int bell_upload(uint32_t rows, Len len_of, Col col_of, BellDev& B, size_t
             bcol[sp[I / SLICE] + (size_t)k * SLICE + I % SLICE] = col_of(I, k);
     B.rows = rows;
     B.slots = sp[ns];
+    for (uint16_t l : len) B.wmax = std::max<uint32_t>(B.wmax, l);
     // about three blocks per lane (1, 2, 4, 8 or 16 lanes)
     size_t used = 0;
     for (uint32_t I = 0; I < rows; ++I) used += len[I];
@@ -774,6 +998,20 @@ static bool grouped(uint32_t rows, int R, int C, const HostVec<uint32_t>& ptr,
                 if (col[b0 + q + c] != col[b0 + q] + c || col[b0 + q] % C) return false;
     }
     return true;
+}
+
+// k_amg_bottom's form for level L: 1 or 2 scalar rows per thread of up to 14
+// blocks (the coarse levels of structured T3 meshes have 11-13), 3: one row
+// of up to 24; 0 none.  Three rows per thread do not fit the registers (37
+// spilled) and take 57 us at 1,050 unknowns, as long as the launches they
+// replace.  Rows of 5 to 20 blocks on average, that is 2 or 4 lanes in the
+// kernels of one step: thinner and denser levels are too rare to pay for more
+// forms.
+static int bottom_kind(const AmgDevLevel& L) {
+    if (L.ab.lanes != 2 && L.ab.lanes != 4) return 0;
+    const uint32_t rows = (L.n + BOTTOM_TB - 1) / BOTTOM_TB;
+    if (L.ab.wmax <= 14 && rows <= 2) return (int)rows;
+    return L.ab.wmax <= 24 && rows == 1 ? 3 : 0;
 }
 
 // Symbolic hierarchy of the system's current K (pattern, Dirichlet rows,
@@ -911,6 +1149,8 @@ static int amg_symbolic(FemSys& S) {
             NBX_TRY(up(&L.pt_pos, h.pt_pos, A->bytes));
         }
     }
+    // the last smoothed level in one workgroup with the dense solve
+    if (nl >= 3 && bottom_kind(A->lv[nl - 2])) A->bottom = nl - 2;
     const uint32_t nco = A->lv.back().n;
     NBX_TRY(alloc(&A->cinv, (size_t)nco * nco, A->bytes));
     NBX_TRY(alloc(&A->ones, n, A->bytes));
@@ -1146,7 +1386,7 @@ uint32_t amg_levels(const AmgDev* A) { return (uint32_t)A->lv.size(); }
 static void restrict_to(AmgDev* A, size_t l, const float* r, const PcgState* st, hipStream_t s) {
     AmgDevLevel& V = A->lv[l];
     AmgDevLevel& W = A->lv[l + 1];
-    const bool init = l + 2 < A->lv.size();
+    const bool init = l + 2 < A->lv.size() && l + 1 != A->bottom;
     with_bs(V.bs, [&](auto R) {
         constexpr int RR = decltype(R)::value;
         with_bl(V.tb.lanes, [&](auto ln) {
@@ -1184,6 +1424,43 @@ static void prolong_from(AmgDev* A, size_t l, float* x, bool add, const PcgState
     });
 }
 
+// The one-workgroup part: level A->bottom and the dense solve below it.
+static void bottom_cycle(AmgDev* A, const float* b, float* x, const PcgState* st, hipStream_t s) {
+    Bottom B{};
+    const AmgDevLevel& C = A->lv.back();
+    const AmgDevLevel& V = A->lv[A->bottom];
+    BottomLevel& L = B.lv;
+    L.A = bell<3, 3>(V.ab);
+    L.P = bell<3, 3>(V.pb);
+    L.T = bell<3, 3>(V.tb);
+    L.dinv = V.dinv32;
+    L.p_lanes = V.pb.lanes;
+    L.t_lanes = V.tb.lanes;
+    L.rows = V.n / 3;
+    L.degree = (uint32_t)V.degree;
+    L.inv_theta = V.inv_theta;
+    std::copy(V.c1, V.c1 + AMG_MAX_DEGREE, L.c1);
+    std::copy(V.c2, V.c2 + AMG_MAX_DEGREE, L.c2);
+    B.nco = C.n;
+    B.cinv = A->cinv;
+    B.b = b;
+    B.x = x;
+    const size_t lds = (4 * (size_t)V.n + 2 * (size_t)C.n) * sizeof(float);
+    const dim3 g(1), t(BOTTOM_TB);
+    auto launch = [&](auto ln) {
+        constexpr int LN = decltype(ln)::value;
+        switch (bottom_kind(V)) {
+            case 1: hipLaunchKernelGGL((k_amg_bottom<1, 14, LN>), g, t, lds, s, B, st); break;
+            case 2: hipLaunchKernelGGL((k_amg_bottom<2, 14, LN>), g, t, lds, s, B, st); break;
+            default: hipLaunchKernelGGL((k_amg_bottom<1, 24, LN>), g, t, lds, s, B, st); break;
+        }
+    };
+    if (V.ab.lanes == 2)
+        launch(std::integral_constant<int, 2>{});
+    else
+        launch(std::integral_constant<int, 4>{});
+}
+
 // The V-cycle from level l0 >= 1 down, x = M^-1 b on that level (b, x: that
 // level's arrays; the finest level is smoothed by the flexible CG's own
 // kernels on the fp16 copy).  The restriction has already started each
@@ -1192,7 +1469,8 @@ static void prolong_from(AmgDev* A, size_t l, float* x, bool add, const PcgState
 static void cycle_from(AmgDev* A, size_t l0, const float* b, float* x, const PcgState* st,
                        hipStream_t s) {
     const size_t L = A->lv.size();
-    for (size_t l = l0; l + 1 < L; ++l) {
+    const size_t low = A->bottom ? std::max(A->bottom, l0) : L - 1;   // the last part's level
+    for (size_t l = l0; l < low; ++l) {
         AmgDevLevel& V = A->lv[l];
         const float* bl = l == l0 ? b : V.b;
         float* xl = l == l0 ? x : V.x;
@@ -1211,12 +1489,15 @@ static void cycle_from(AmgDev* A, size_t l0, const float* b, float* x, const Pcg
         });
         restrict_to(A, l, V.r, st, s);
     }
-    {
+    if (A->bottom) {
+        AmgDevLevel& V = A->lv[low];
+        bottom_cycle(A, low == l0 ? b : V.b, low == l0 ? x : V.x, st, s);
+    } else {
         AmgDevLevel& C = A->lv[L - 1];
         hipLaunchKernelGGL(k_amg_dense, dim3(1), dim3(DENSE_BLOCK), 0, s, A->cinv,
                            L == l0 + 1 ? b : C.b, L == l0 + 1 ? x : C.x, st, C.n);
     }
-    for (size_t l = L - 1; l-- > l0;) {
+    for (size_t l = low; l-- > l0;) {
         AmgDevLevel& V = A->lv[l];
         const float* bl = l == l0 ? b : V.b;
         float* xl = l == l0 ? x : V.x;
