@@ -2332,13 +2332,16 @@ static int solve_fcg_cheb(const DevMatrix& m, const double* b, double* x, double
     SolveStats tot{};
     int status = NBX_NOT_CONVERGED;
     uint32_t used = 0;
+    // per preconditioner: a Chebyshev adjoint solve's 147 iterations are no
+    // guess for the multigrid state solve's 39 (6 ms of launched kernels that
+    // returned at once, of 16, at 256x128)
+    uint32_t& hint = w.fcg_hint[opt.variant == AMG_FCG];
     double prev = 0.0;
     const int passes = opt.true_residual ? SOLVE_PASSES : 1;
     for (int pass = 0; pass < passes; ++pass) {
         SolveStats ps{};
-        rc = fcg_cheb_pass(m, b, x, rtol, opt, max_iter - used, pass == 0 ? w.fcg_hint : 0u, w,
-                           s, &ps);
-        if (pass == 0) w.fcg_hint = rc == NBX_OK ? ps.iters : 0u;
+        rc = fcg_cheb_pass(m, b, x, rtol, opt, max_iter - used, pass == 0 ? hint : 0u, w, s, &ps);
+        if (pass == 0) hint = rc == NBX_OK ? ps.iters : 0u;
         if (rc != NBX_OK && rc != NBX_NOT_CONVERGED) return rc;
         used += ps.iters;
         add_pass(tot, ps, pass);
