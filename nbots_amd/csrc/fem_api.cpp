@@ -390,12 +390,13 @@ int nbx_simp_get(const nbx_simp_t* h, double* x, double* xphys, double* dc, uint
 int nbx_simp_filter(const nbx_simp_t* h, uint64_t* n_entries, uint32_t* Hptr, uint32_t* Hidx,
                     double* Hval, double* Hs) {
     const nbx::Simp& o = h->o;
-    if (n_entries) *n_entries = o.h_idx.size();
-    if (Hptr) std::copy(o.h_ptr.begin(), o.h_ptr.end(), Hptr);
-    if (Hidx) std::copy(o.h_idx.begin(), o.h_idx.end(), Hidx);
-    if (Hval) std::copy(o.h_val.begin(), o.h_val.end(), Hval);
-    if (Hs) std::copy(o.h_hs.begin(), o.h_hs.end(), Hs);
-    return nbx::NBX_OK;
+    if (n_entries) *n_entries = o.H.n_ent;
+    try {
+        return nbx::simp_filter_csr(o, Hptr, Hidx, Hval, Hs);
+    } catch (const std::bad_alloc&) {
+        nbx::set_last_error("out of host memory");
+        return nbx::NBX_ERR_ARG;
+    }
 }
 
 }  // extern "C"

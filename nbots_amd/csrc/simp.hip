@@ -21,6 +21,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <new>
 
 #include "simp.hpp"
 
@@ -199,70 +200,191 @@ __global__ __launch_bounds__(FIN) void k_fin_absmax(const double* partials, unsi
     }
 }
 
+// ---- building H -------------------------------------------------------------
+// Bins of edge >= rmin over the centroid bounding box: the entries of a row
+// are in the 3x3 bins around its element's.  Each bin lists its elements in
+// ascending order, so a row in ascending columns is a merge of nine lists:
+// one thread per row, no sorting and no limit on a row's length.  The host
+// loop with a sort per row, the layout and the upload took 54-77 ms at
+// 512x256 (262,144 elements, a radius of 1.5 edges), this takes 1.9 ms with
+// the allocations (96x48: 1.5 -> 0.3): bound by the gathers of the candidates'
+// centroids.  The arithmetic is the host's, so is every bit of H.
+struct Bins {
+    double x0, y0, edge;
+    uint32_t nx, ny;
+    __host__ __device__ size_t count() const { return (size_t)nx * ny; }
+};
+
+// Centroids, areas, and each workgroup's bounding box of the centroids
+__global__ __launch_bounds__(BLOCK) void k_simp_geom(const double2* __restrict__ nod,
+                                                     const uint32_t* __restrict__ conn,
+                                                     uint32_t ne, double2* __restrict__ c,
+                                                     double* __restrict__ area,
+                                                     double* __restrict__ box) {
+    const size_t e = (size_t)blockIdx.x * BLOCK + threadIdx.x;
+    double b[4] = {INFINITY, INFINITY, INFINITY, INFINITY};   // min of x, y, -x, -y
+    if (e < ne) {
+        const double2 p = nod[conn[3 * e]], q = nod[conn[3 * e + 1]], r = nod[conn[3 * e + 2]];
+        const double2 m = make_double2((p.x + q.x + r.x) / 3.0, (p.y + q.y + r.y) / 3.0);
+        c[e] = m;
+        area[e] = 0.5 * ((q.x - p.x) * (r.y - p.y) - (r.x - p.x) * (q.y - p.y));
+        b[0] = m.x;
+        b[1] = m.y;
+        b[2] = -m.x;
+        b[3] = -m.y;
+    }
+    __shared__ double red[4][BLOCK / WAVE];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        for (int off = WAVE / 2; off > 0; off >>= 1) b[i] = fmin(b[i], __shfl_xor(b[i], off));
+        if (threadIdx.x % WAVE == 0) red[i][threadIdx.x / WAVE] = b[i];
+    }
+    __syncthreads();
+    if (threadIdx.x < 4) {
+        double v = red[threadIdx.x][0];
+        for (int w = 1; w < BLOCK / WAVE; ++w) v = fmin(v, red[threadIdx.x][w]);
+        box[4 * (size_t)blockIdx.x + threadIdx.x] = v;
+    }
+}
+
+// Each element's bin and a place in it (in the order of arrival)
+__global__ __launch_bounds__(BLOCK) void k_bin_count(const double2* __restrict__ c, uint32_t ne,
+                                                     Bins B, uint32_t* __restrict__ bin,
+                                                     uint32_t* __restrict__ place, uint32_t* cnt) {
+    const size_t e = (size_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (e >= ne) return;
+    const uint32_t bx = min((uint32_t)((c[e].x - B.x0) / B.edge), B.nx - 1);
+    const uint32_t by = min((uint32_t)((c[e].y - B.y0) / B.edge), B.ny - 1);
+    const uint32_t b = by * B.nx + bx;
+    bin[e] = b;
+    place[e] = atomicAdd(&cnt[b], 1u);
+}
+__global__ __launch_bounds__(BLOCK) void k_bin_fill(const uint32_t* __restrict__ bin,
+                                                    const uint32_t* __restrict__ place,
+                                                    uint32_t ne, const uint32_t* __restrict__ ptr,
+                                                    uint32_t* __restrict__ list) {
+    const size_t e = (size_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (e < ne) list[ptr[bin[e]] + place[e]] = (uint32_t)e;
+}
+// An element's place in ascending order: how many of its bin come before it
+__global__ __launch_bounds__(BLOCK) void k_bin_order(const uint32_t* __restrict__ bin, uint32_t ne,
+                                                     const uint32_t* __restrict__ ptr,
+                                                     const uint32_t* __restrict__ list,
+                                                     uint32_t* __restrict__ out) {
+    const size_t e = (size_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (e >= ne) return;
+    const uint32_t beg = ptr[bin[e]], end = ptr[bin[e] + 1];
+    uint32_t r = 0;
+    for (uint32_t t = beg; t < end; ++t) r += list[t] < (uint32_t)e;
+    out[beg + r] = (uint32_t)e;
+}
+
+// rmin - |c_e - c_j|
+__device__ __forceinline__ double filt_weight(double2 ce, double2 cj, double rmin) {
+    const double dx = ce.x - cj.x, dy = ce.y - cj.y;
+    return rmin - sqrt(dx * dx + dy * dy);
+}
+
+// Row lengths, and each slice's (a wavefront's) longest row and entries
+__global__ __launch_bounds__(BLOCK) void k_filt_count(const double2* __restrict__ c, uint32_t ne,
+                                                      Bins B, const uint32_t* __restrict__ bin,
+                                                      const uint32_t* __restrict__ ptr,
+                                                      const uint32_t* __restrict__ list,
+                                                      double rmin, uint32_t* __restrict__ width,
+                                                      uint32_t* __restrict__ entries) {
+    const size_t e = (size_t)blockIdx.x * BLOCK + threadIdx.x;
+    uint32_t len = 0;
+    if (e < ne) {
+        const double2 ce = c[e];
+        const uint32_t bx = bin[e] % B.nx, by = bin[e] / B.nx;
+        // the bins of one row of bins lie side by side
+        for (uint32_t jy = by ? by - 1 : 0; jy <= min(by + 1, B.ny - 1); ++jy) {
+            const uint32_t end = ptr[(size_t)jy * B.nx + min(bx + 1, B.nx - 1) + 1];
+            for (uint32_t t = ptr[(size_t)jy * B.nx + (bx ? bx - 1 : 0)]; t < end; ++t)
+                len += filt_weight(ce, c[list[t]], rmin) > 0.0;
+        }
+    }
+    uint32_t w = len, n = len;
+    for (int off = WAVE / 2; off > 0; off >>= 1) {
+        w = max(w, __shfl_xor(w, off));
+        n += __shfl_xor(n, off);
+    }
+    if (threadIdx.x % WAVE == 0 && e < ne) {
+        width[e / SLICE] = w;
+        entries[e / SLICE] = n;
+    }
+}
+
+// Rows of H (columns ascending, padded with weight 0), their lengths and sums
+__global__ __launch_bounds__(BLOCK) void k_filt_rows(const double2* __restrict__ c, DevFilter H,
+                                                     Bins B, const uint32_t* __restrict__ bin,
+                                                     const uint32_t* __restrict__ ptr,
+                                                     const uint32_t* __restrict__ list,
+                                                     double rmin) {
+    const size_t e = (size_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (e >= H.ne) return;
+    constexpr uint32_t NONE = 0xffffffffu;
+    const double2 ce = c[e];
+    const uint32_t bx = bin[e] % B.nx, by = bin[e] / B.nx;
+    uint32_t cur[9], end[9], head[9];
+    auto next = [&](int q) {   // the list's next element within rmin
+        head[q] = NONE;
+        for (; cur[q] < end[q]; ++cur[q]) {
+            const uint32_t j = list[cur[q]];
+            if (filt_weight(ce, c[j], rmin) > 0.0) {
+                head[q] = j;
+                break;
+            }
+        }
+    };
+#pragma unroll
+    for (int q = 0; q < 9; ++q) {
+        const int64_t jx = (int64_t)bx + q % 3 - 1, jy = (int64_t)by + q / 3 - 1;
+        cur[q] = end[q] = 0;
+        if (jx >= 0 && jx < B.nx && jy >= 0 && jy < B.ny) {
+            cur[q] = ptr[(size_t)jy * B.nx + jx];
+            end[q] = ptr[(size_t)jy * B.nx + jx + 1];
+        }
+        next(q);
+    }
+    const size_t beg = (size_t)H.slice_ptr[e / SLICE] + e % SLICE;
+    const size_t stop = H.slice_ptr[e / SLICE + 1];
+    size_t i = beg;
+    double sum = 0.0;
+    for (;;) {
+        uint32_t j = NONE;
+#pragma unroll
+        for (int q = 0; q < 9; ++q) j = min(j, head[q]);
+        if (j == NONE || i >= stop) break;   // (a row never has more than its slice's width)
+        const double h = filt_weight(ce, c[j], rmin);
+        H.idx[i] = j;
+        H.val[i] = h;
+        sum += h;
+        i += SLICE;
+#pragma unroll
+        for (int q = 0; q < 9; ++q)
+            if (head[q] == j) {
+                ++cur[q];
+                next(q);
+            }
+    }
+    H.rowlen[e] = (uint16_t)((i - beg) / SLICE);
+    H.Hs[e] = sum;
+    for (; i < stop; i += SLICE) {
+        H.idx[i] = (uint32_t)e;
+        H.val[i] = 0.0;
+    }
+}
+
 // ---- host -------------------------------------------------------------------
 namespace {
 
-// H by uniform bins of size rmin over the centroid bounding box: candidates
-// of element e are the elements of the 3x3 bins around its own; a row lists
-// its columns in ascending order.
-void filter_csr(uint32_t ne, const std::vector<double>& cx, const std::vector<double>& cy,
-                double rmin, std::vector<uint32_t>& ptr, std::vector<uint32_t>& idx,
-                std::vector<double>& val, std::vector<double>& hs) {
-    double x0 = cx[0], x1 = cx[0], y0 = cy[0], y1 = cy[0];
-    for (uint32_t e = 0; e < ne; ++e) {
-        x0 = std::min(x0, cx[e]);
-        x1 = std::max(x1, cx[e]);
-        y0 = std::min(y0, cy[e]);
-        y1 = std::max(y1, cy[e]);
-    }
-    const uint32_t nbx = (uint32_t)((x1 - x0) / rmin) + 1;
-    const uint32_t nby = (uint32_t)((y1 - y0) / rmin) + 1;
-    const size_t nb = (size_t)nbx * nby;
-    std::vector<uint32_t> bin(ne), bptr(nb + 1, 0), bidx(ne);
-    for (uint32_t e = 0; e < ne; ++e) {
-        uint32_t bx = (uint32_t)((cx[e] - x0) / rmin);
-        uint32_t by = (uint32_t)((cy[e] - y0) / rmin);
-        bx = std::min(bx, nbx - 1);
-        by = std::min(by, nby - 1);
-        bin[e] = by * nbx + bx;
-        bptr[bin[e] + 1]++;
-    }
-    for (size_t b = 0; b < nb; ++b) bptr[b + 1] += bptr[b];
-    {
-        std::vector<uint32_t> fill(bptr.begin(), bptr.end() - 1);
-        for (uint32_t e = 0; e < ne; ++e) bidx[fill[bin[e]]++] = e;
-    }
-    ptr.assign(ne + 1, 0);
-    idx.clear();
-    val.clear();
-    hs.assign(ne, 0.0);
-    std::vector<uint32_t> cand;
-    for (uint32_t e = 0; e < ne; ++e) {
-        const int64_t bx = bin[e] % nbx, by = bin[e] / nbx;
-        cand.clear();
-        for (int64_t jy = std::max<int64_t>(by - 1, 0); jy <= std::min<int64_t>(by + 1, nby - 1); ++jy)
-            for (int64_t jx = std::max<int64_t>(bx - 1, 0); jx <= std::min<int64_t>(bx + 1, nbx - 1);
-                 ++jx) {
-                const size_t b = (size_t)jy * nbx + jx;
-                for (uint32_t t = bptr[b]; t < bptr[b + 1]; ++t) {
-                    const uint32_t j = bidx[t];
-                    const double dx = cx[e] - cx[j], dy = cy[e] - cy[j];
-                    if (rmin - std::sqrt(dx * dx + dy * dy) > 0.0) cand.push_back(j);
-                }
-            }
-        std::sort(cand.begin(), cand.end());
-        double s = 0.0;
-        for (uint32_t j : cand) {
-            const double dx = cx[e] - cx[j], dy = cy[e] - cy[j];
-            const double h = rmin - std::sqrt(dx * dx + dy * dy);
-            idx.push_back(j);
-            val.push_back(h);
-            s += h;
-        }
-        hs[e] = s;
-        ptr[e + 1] = (uint32_t)idx.size();
-    }
-}
+struct DevBuf {   // device scratch of one call
+    void* p = nullptr;
+    ~DevBuf() { if (p) (void)hipFree(p); }
+    template <class T>
+    T* at(size_t byte) const { return (T*)((char*)p + byte); }
+};
 
 template <class T>
 int upload(T** d, const std::vector<T>& h, hipStream_t s) {
@@ -271,7 +393,111 @@ int upload(T** d, const std::vector<T>& h, hipStream_t s) {
     return NBX_OK;
 }
 
+// H, Hs, the element areas and their sum (in element order)
+int build_filter(Simp& o, FemSys& S) {
+    const uint32_t ne = S.ne;
+    const hipStream_t s = S.s;
+    const unsigned g = grid_for(ne);
+    const uint32_t ns = (ne + SLICE - 1) / SLICE;
+    // scratch: centroids, boxes, bins, places, two lists, widths, entries
+    DevBuf t, u;
+    const size_t at_box = (size_t)ne * 16, at_bin = at_box + (size_t)g * 32, n4 = (size_t)ne * 4;
+    const size_t at_width = at_bin + 4 * n4;
+    NBX_HIP(hipMalloc(&t.p, at_width + 2 * (size_t)ns * 4));
+    double2* c = t.at<double2>(0);
+    double* box = t.at<double>(at_box);
+    uint32_t *bin = t.at<uint32_t>(at_bin), *place = bin + ne, *list0 = place + ne,
+             *list = list0 + ne, *width = list + ne;
+    NBX_HIP(hipMalloc(&o.area, (size_t)ne * 8 + 8));
+    hipLaunchKernelGGL(k_simp_geom, dim3(g), dim3(BLOCK), 0, s, S.nod, S.conn, ne, c, o.area, box);
+    NBX_HIP(hipGetLastError());
+    std::vector<double> area(ne), hb(4 * (size_t)g);
+    NBX_HIP(hipMemcpyAsync(area.data(), o.area, area.size() * 8, hipMemcpyDeviceToHost, s));
+    NBX_HIP(copy_on(hb.data(), box, hb.size() * 8, hipMemcpyDeviceToHost, s));
+    double b[4] = {hb[0], hb[1], hb[2], hb[3]};
+    for (size_t i = 4; i < hb.size(); ++i) b[i % 4] = std::min(b[i % 4], hb[i]);
+    // at most about 2 ne bins, however small rmin is
+    const double lx = -b[2] - b[0], ly = -b[3] - b[1];
+    Bins B{b[0], b[1], o.rmin, 1, 1};
+    if (std::isfinite(lx) && std::isfinite(ly)) {
+        B.edge = std::max({o.rmin, std::sqrt(lx * ly / ne), (lx + ly) / ne});
+        B.nx = (uint32_t)(lx / B.edge) + 1;
+        B.ny = (uint32_t)(ly / B.edge) + 1;
+    }
+    const size_t nb = B.count();
+    NBX_HIP(hipMalloc(&u.p, (2 * nb + 1) * sizeof(uint32_t)));
+    uint32_t *cnt = u.at<uint32_t>(0), *ptr = cnt + nb;
+    NBX_HIP(hipMemsetAsync(cnt, 0, nb * sizeof(uint32_t), s));
+    hipLaunchKernelGGL(k_bin_count, dim3(g), dim3(BLOCK), 0, s, c, ne, B, bin, place, cnt);
+    NBX_TRY(scan_u32(cnt, ptr, nb, s));
+    hipLaunchKernelGGL(k_bin_fill, dim3(g), dim3(BLOCK), 0, s, bin, place, ne, ptr, list0);
+    hipLaunchKernelGGL(k_bin_order, dim3(g), dim3(BLOCK), 0, s, bin, ne, ptr, list0, list);
+    hipLaunchKernelGGL(k_filt_count, dim3(g), dim3(BLOCK), 0, s, c, ne, B, bin, ptr, list, o.rmin,
+                       width, width + ns);
+    NBX_HIP(hipGetLastError());
+    std::vector<uint32_t> we(2 * (size_t)ns), sptr(ns + 1, 0);
+    NBX_HIP(hipMemcpyAsync(we.data(), width, we.size() * 4, hipMemcpyDeviceToHost, s));
+    // (the sum while the device counts)
+    double atot = 0.0;
+    for (uint32_t e = 0; e < ne; ++e) atot += area[e];
+    o.atot = atot;
+    NBX_HIP(hipStreamSynchronize(s));
+    DevFilter& H = o.H;
+    H.ne = ne;
+    H.n_slices = ns;
+    H.n_ent = 0;
+    size_t tot = 0;
+    for (uint32_t sl = 0; sl < ns; ++sl) {
+        if (we[sl] > 0xffffu) {
+            set_last_error("simp: filter row of %u entries (rmin too large)", we[sl]);
+            return NBX_ERR_ARG;
+        }
+        H.n_ent += we[ns + sl];
+        tot += (size_t)we[sl] * SLICE;
+        if (tot > 0xffffffffull) {
+            set_last_error("simp: filter too large");
+            return NBX_ERR_ARG;
+        }
+        sptr[sl + 1] = (uint32_t)tot;
+    }
+    H.n_stored = tot;
+    NBX_TRY(upload(&H.slice_ptr, sptr, s));
+    NBX_HIP(hipMalloc(&H.rowlen, (size_t)ne * 2 + 8));
+    NBX_HIP(hipMalloc(&H.idx, tot * 4 + 8));
+    NBX_HIP(hipMalloc(&H.val, tot * 8 + 8));
+    NBX_HIP(hipMalloc(&H.Hs, (size_t)ne * 8 + 8));
+    hipLaunchKernelGGL(k_filt_rows, dim3(g), dim3(BLOCK), 0, s, c, H, B, bin, ptr, list, o.rmin);
+    NBX_HIP(hipGetLastError());
+    NBX_HIP(hipStreamSynchronize(s));
+    return NBX_OK;
+}
+
 }  // namespace
+
+// H and Hs as host CSR
+int simp_filter_csr(const Simp& o, uint32_t* ptr, uint32_t* idx, double* val, double* Hs) {
+    const DevFilter& H = o.H;
+    if (Hs) NBX_HIP(hipMemcpy(Hs, H.Hs, (size_t)H.ne * 8, hipMemcpyDeviceToHost));
+    if (!ptr && !idx && !val) return NBX_OK;
+    std::vector<uint32_t> sptr(H.n_slices + 1), ei(idx ? H.n_stored : 0);
+    std::vector<uint16_t> len(H.ne);
+    std::vector<double> ev(val ? H.n_stored : 0);
+    NBX_HIP(hipMemcpy(sptr.data(), H.slice_ptr, sptr.size() * 4, hipMemcpyDeviceToHost));
+    NBX_HIP(hipMemcpy(len.data(), H.rowlen, len.size() * 2, hipMemcpyDeviceToHost));
+    if (!ei.empty()) NBX_HIP(hipMemcpy(ei.data(), H.idx, ei.size() * 4, hipMemcpyDeviceToHost));
+    if (!ev.empty()) NBX_HIP(hipMemcpy(ev.data(), H.val, ev.size() * 8, hipMemcpyDeviceToHost));
+    size_t at = 0;
+    for (uint32_t e = 0; e < H.ne; ++e) {
+        if (ptr) ptr[e] = (uint32_t)at;
+        size_t i = (size_t)sptr[e / SLICE] + e % SLICE;
+        for (uint32_t k = 0; k < len[e]; ++k, ++at, i += SLICE) {
+            if (idx) idx[at] = ei[i];
+            if (val) val[at] = ev[i];
+        }
+    }
+    if (ptr) ptr[H.ne] = (uint32_t)at;
+    return NBX_OK;
+}
 
 int simp_create(Simp& o, FemSys& S, double rmin, double volfrac, double penal, double E0,
                 double Emin, double move, const double* x0_host) {
@@ -291,70 +517,8 @@ int simp_create(Simp& o, FemSys& S, double rmin, double volfrac, double penal, d
     o.E0 = E0;
     o.Emin = Emin;
     o.move = move;
-    // centroids and areas from the system's mesh
-    std::vector<double> nod(2 * (size_t)S.nn);
-    std::vector<uint32_t> conn(3 * (size_t)ne);
-    NBX_HIP(copy_on(nod.data(), S.nod, nod.size() * 8, hipMemcpyDeviceToHost, s));
-    NBX_HIP(copy_on(conn.data(), S.conn, conn.size() * 4, hipMemcpyDeviceToHost, s));
-    std::vector<double> cx(ne), cy(ne), area(ne);
-    for (uint32_t e = 0; e < ne; ++e) {
-        const uint32_t a = conn[3 * (size_t)e], b = conn[3 * (size_t)e + 1], c = conn[3 * (size_t)e + 2];
-        const double xa = nod[2 * (size_t)a], ya = nod[2 * (size_t)a + 1];
-        const double xb = nod[2 * (size_t)b], yb = nod[2 * (size_t)b + 1];
-        const double xc = nod[2 * (size_t)c], yc = nod[2 * (size_t)c + 1];
-        cx[e] = (xa + xb + xc) / 3.0;
-        cy[e] = (ya + yb + yc) / 3.0;
-        area[e] = 0.5 * ((xb - xa) * (yc - ya) - (xc - xa) * (yb - ya));
-    }
-    double atot = 0.0;
-    for (uint32_t e = 0; e < ne; ++e) atot += area[e];
-    o.atot = atot;
-    filter_csr(ne, cx, cy, rmin, o.h_ptr, o.h_idx, o.h_val, o.h_hs);
-    // sliced ELL
-    DevFilter& H = o.H;
-    H.ne = ne;
-    H.n_slices = (ne + SLICE - 1) / SLICE;
-    H.n_ent = o.h_idx.size();
-    std::vector<uint32_t> sptr(H.n_slices + 1, 0);
-    std::vector<uint16_t> rowlen(ne);
-    size_t tot = 0;
-    for (uint32_t sl = 0; sl < H.n_slices; ++sl) {
-        uint32_t w = 0;
-        for (uint32_t e = sl * SLICE; e < std::min<uint32_t>(ne, (sl + 1) * SLICE); ++e) {
-            const uint32_t len = o.h_ptr[e + 1] - o.h_ptr[e];
-            if (len > 0xffffu) {
-                set_last_error("simp: filter row of %u entries (rmin too large)", len);
-                return NBX_ERR_ARG;
-            }
-            rowlen[e] = (uint16_t)len;
-            w = std::max(w, len);
-        }
-        sptr[sl] = (uint32_t)tot;
-        tot += (size_t)w * SLICE;
-        if (tot > 0xffffffffull) {
-            set_last_error("simp: filter too large");
-            return NBX_ERR_ARG;
-        }
-    }
-    sptr[H.n_slices] = (uint32_t)tot;
-    H.n_stored = tot;
-    std::vector<uint32_t> eidx(tot);
-    std::vector<double> eval(tot, 0.0);
-    for (uint32_t e = 0; e < ne; ++e) {
-        const size_t base = sptr[e / SLICE] + (e % SLICE);
-        const uint32_t len = rowlen[e];
-        const uint32_t w = (sptr[e / SLICE + 1] - sptr[e / SLICE]) / SLICE;
-        for (uint32_t k = 0; k < w; ++k) {
-            eidx[base + (size_t)k * SLICE] = k < len ? o.h_idx[o.h_ptr[e] + k] : e;
-            eval[base + (size_t)k * SLICE] = k < len ? o.h_val[o.h_ptr[e] + k] : 0.0;
-        }
-    }
-    NBX_TRY(upload(&H.slice_ptr, sptr, s));
-    NBX_TRY(upload(&H.rowlen, rowlen, s));
-    NBX_TRY(upload(&H.idx, eidx, s));
-    NBX_TRY(upload(&H.val, eval, s));
-    NBX_TRY(upload(&H.Hs, o.h_hs, s));
-    NBX_TRY(upload(&o.area, area, s));
+    NBX_TRY(build_filter(o, S));
+    const DevFilter& H = o.H;
     // design, filtered densities (xPhys = x at the start), sensitivities
     std::vector<double> x0(ne, volfrac);
     if (x0_host) std::copy(x0_host, x0_host + ne, x0.begin());

@@ -28,8 +28,6 @@ struct OcState {
 
 struct Simp {
     DevFilter H;
-    std::vector<uint32_t> h_ptr, h_idx;   // CSR copy of H (host)
-    std::vector<double> h_val, h_hs;
     double* x = nullptr;       // design variables
     double* xnew = nullptr;
     double* xphys = nullptr;   // filtered densities
@@ -46,6 +44,8 @@ struct Simp {
 int simp_create(Simp& o, FemSys& S, double rmin, double volfrac, double penal, double E0,
                 double Emin, double move, const double* x0_host);
 void simp_free(Simp& o);
+// H as host CSR (columns ascending) and Hs; null: not wanted
+int simp_filter_csr(const Simp& o, uint32_t* ptr, uint32_t* idx, double* val, double* Hs);
 // E_e = Emin + xPhys_e^p (E0 - Emin) into the system's per-element moduli
 int simp_moduli(Simp& o, FemSys& S);
 // sensitivity filter, OC update with bisection, change = max |x_new - x|
