@@ -34,6 +34,7 @@ struct BellDev {
     uint32_t rows = 0;
     int lanes = 1;             // lanes per block row in the V-cycle's products
     uint32_t wmax = 0;         // blocks of the longest row
+    uint32_t width = 0;        // the width of every slice where they are alike, or 0
     size_t slots = 0;
     uint32_t* slice_ptr = nullptr;
     uint16_t* len = nullptr;
@@ -518,7 +519,7 @@ __device__ __forceinline__ float group_sum(float s) {
 
 template <int R, int C>
 struct Bell {
-    size_t slots;
+    uint32_t slots, width;
     const uint32_t* __restrict__ slice_ptr;
     const uint16_t* __restrict__ len;
     const uint32_t* __restrict__ bcol;
@@ -526,40 +527,83 @@ struct Bell {
 };
 template <int R, int C>
 Bell<R, C> bell(const BellDev& B) {
-    return Bell<R, C>{B.slots, B.slice_ptr, B.len, B.bcol, B.val};
+    return Bell<R, C>{(uint32_t)B.slots, B.width, B.slice_ptr, B.len, B.bcol, B.val};
 }
 
-// y = (block row I) x, x indexed by C per block column, by a group of LANES
-// lanes: lane l takes blocks l, l + LANES, ..., two at a time (their columns
+// What a kernel of the cycle reads before its product.  On the coarse levels
+// such a kernel is a chain of dependent loads, each a trip past the L2 (the
+// kernel before it has just written them): the stop flag, the slice and
+// length, the columns and values, x, and what the update of the row reads.
+// They go out in three rounds: the flag with the slice, the length and the
+// row's own values (KEEP holds them before the branch on the flag, below
+// which the compiler would sink them), four blocks of a lane at once, their
+// x; on a level of one slice width the first round needs no slice or length,
+// and the blocks' loads follow it without a wait.  Outer iteration, five or
+// six trips before -> this, us: 96x48 56.5 -> 53, 150x75 67.5 -> 62.6,
+// 512x256 141 -> 127, 1024x512 260 -> 237, 2048x1024 628 -> 598 (there bound
+// by the bytes of its two finest levels).
+#define KEEP(v) asm volatile("" : "+v"(v))
+struct BellHead {
+    uint32_t slice, row, len, done;   // the slice's first slot, the row in it
+};
+template <int R, int C>
+__device__ __forceinline__ BellHead bell_head(const Bell<R, C>& B, uint32_t I, const PcgState* st) {
+    uint32_t slice = (I >> 6) * SLICE * B.width, len = B.width;
+    if (!B.width) {
+        slice = B.slice_ptr[I >> 6];
+        len = B.len[I];
+    }
+    uint32_t zero = 0;   // in a vector register: the flag goes out with the other loads, not
+    KEEP(zero);          // through the scalar cache, whose trip the branch would wait for
+    return {slice, I & 63, len, (&st->done)[zero]};
+}
+template <int R>
+__device__ __forceinline__ void load_rows(const float* __restrict__ p, uint32_t I, float (&v)[R]) {
+#pragma unroll
+    for (int m = 0; m < R; ++m) v[m] = p[(size_t)R * I + m];
+}
+__device__ __forceinline__ void keep(BellHead& h) {
+    KEEP(h.len);
+    KEEP(h.slice);
+    KEEP(h.done);
+}
+template <int R, class... Rest>
+__device__ __forceinline__ void keep(BellHead& h, float (&v)[R], Rest&... rest) {
+#pragma unroll
+    for (int m = 0; m < R; ++m) KEEP(v[m]);
+    keep(h, rest...);
+}
+
+// y = (block row) x, x indexed by C per block column, by a group of LANES
+// lanes: lane l takes blocks l, l + LANES, ..., four at a time (their columns
 // and values loaded before the dependent gathers), and the group adds the
 // lanes' sums by a butterfly; every lane gets the result.
-template <int R, int C, int LANES>
-__device__ __forceinline__ void bell_row(const Bell<R, C>& B, uint32_t I, uint32_t lane,
+template <int R, int C, int LANES, int DEPTH = 4>
+__device__ __forceinline__ void bell_row(const Bell<R, C>& B, const BellHead& h, uint32_t lane,
                                          const float* __restrict__ x, float (&y)[R]) {
 #pragma unroll
     for (int r = 0; r < R; ++r) y[r] = 0.f;
-    const size_t base = (size_t)B.slice_ptr[I >> 6] + (I & 63);
-    const int len = B.len[I];
-    for (int k0 = (int)lane; k0 < len; k0 += 2 * LANES) {
-        uint32_t J[2];
-        float a[2][R * C], xv[2][C];
+    const uint32_t base = h.slice + h.row;
+    for (uint32_t k0 = lane; k0 < h.len; k0 += DEPTH * LANES) {
+        uint32_t J[DEPTH];
+        float a[DEPTH][R * C], xv[DEPTH][C];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            if (k0 + u * LANES < len) {
-                const size_t sl = base + (size_t)(k0 + u * LANES) * SLICE;
+        for (int u = 0; u < DEPTH; ++u) {
+            if (k0 + u * LANES < h.len) {
+                const uint32_t sl = base + (k0 + u * LANES) * SLICE;
                 J[u] = B.bcol[sl];
 #pragma unroll
                 for (int m = 0; m < R * C; ++m) a[u][m] = B.val[(size_t)m * B.slots + sl];
             }
         }
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-            if (k0 + u * LANES < len)
+        for (int u = 0; u < DEPTH; ++u)
+            if (k0 + u * LANES < h.len)
 #pragma unroll
                 for (int c = 0; c < C; ++c) xv[u][c] = x[(size_t)C * J[u] + c];
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-            if (k0 + u * LANES < len)
+        for (int u = 0; u < DEPTH; ++u)
+            if (k0 + u * LANES < h.len)
 #pragma unroll
                 for (int r = 0; r < R; ++r)
 #pragma unroll
@@ -569,12 +613,14 @@ __device__ __forceinline__ void bell_row(const Bell<R, C>& B, uint32_t I, uint32
     for (int r = 0; r < R; ++r) y[r] = group_sum<LANES>(y[r]);
 }
 
-// the group's block row and lane (a group's lanes share its validity, so a
-// group leaves as a whole)
-#define BELL_ROW(LANES, rows)                                                       \
-    const size_t gid_ = (size_t)blockIdx.x * BLOCK + threadIdx.x;                  \
-    const uint32_t I = (uint32_t)(gid_ / LANES), lane = (uint32_t)(gid_ % LANES); \
-    if (I >= (rows)) return
+// the group's block row and lane; groups past the last row take that row
+// again without storing it (rows >= 1: a branch here would put another trip
+// before the first loads)
+#define BELL_ROW(LANES, rows)                                       \
+    const size_t gid_ = (size_t)blockIdx.x * BLOCK + threadIdx.x;  \
+    const uint32_t lane = (uint32_t)(gid_ % LANES);                \
+    const bool store = lane == 0 && gid_ / LANES < (rows);         \
+    const uint32_t I = min((uint32_t)(gid_ / LANES), (rows) - 1u)
 
 // Chebyshev smoothing below the finest level, a group per aggregate (3
 // rows).  The start (r = D^-1 b, d = r / theta, x = d) rides in the
@@ -586,15 +632,19 @@ __global__ __launch_bounds__(BLOCK) void k_bsm_init(Bell<3, 3> A, const float* _
                                                     float* __restrict__ r, float* __restrict__ d,
                                                     float inv_theta, const PcgState* st,
                                                     uint32_t rows) {
-    if (st->done) return;
     BELL_ROW(LANES, rows);
-    float ax[3];
-    bell_row<3, 3, LANES>(A, I, lane, x, ax);
-    if (lane != 0) return;
+    BellHead h = bell_head(A, I, st);
+    float ax[3], di[3], bi[3];
+    load_rows(dinv, I, di);
+    load_rows(b, I, bi);
+    keep(h, di, bi);
+    if (__builtin_amdgcn_readfirstlane(h.done)) return;
+    bell_row<3, 3, LANES>(A, h, lane, x, ax);
+    if (!store) return;
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
         const size_t i = 3 * (size_t)I + m;
-        const float ri = dinv[i] * (b[i] - ax[m]);
+        const float ri = di[m] * (bi[m] - ax[m]);
         r[i] = ri;
         d[i] = ri * inv_theta;
     }
@@ -608,20 +658,25 @@ __global__ __launch_bounds__(BLOCK) void k_bsm_step(Bell<3, 3> A, const float* _
                                                     float* __restrict__ r, float* __restrict__ x,
                                                     float c1, float c2, const PcgState* st,
                                                     uint32_t rows) {
-    if (st->done) return;
     BELL_ROW(LANES, rows);
-    float ad[3];
-    bell_row<3, 3, LANES>(A, I, lane, din, ad);
-    if (lane != 0) return;
+    BellHead h = bell_head(A, I, st);
+    float ad[3], dv[3], d0[3], r0[3], x0[3];
+    load_rows(dinv, I, dv);
+    load_rows(din, I, d0);
+    load_rows(r, I, r0);
+    load_rows(x, I, x0);
+    keep(h, dv, d0, r0, x0);
+    if (__builtin_amdgcn_readfirstlane(h.done)) return;
+    bell_row<3, 3, LANES>(A, h, lane, din, ad);
+    if (!store) return;
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
         const size_t i = 3 * (size_t)I + m;
-        const float di = din[i];
-        const float ri = r[i] - dinv[i] * ad[m];
-        const float dn = c1 * di + c2 * ri;
+        const float ri = r0[m] - dv[m] * ad[m];
+        const float dn = c1 * d0[m] + c2 * ri;
         r[i] = ri;
         dout[i] = dn;
-        x[i] += ADD_IN ? di + dn : dn;
+        x[i] = x0[m] + (ADD_IN ? d0[m] + dn : dn);
     }
 }
 
@@ -630,16 +685,16 @@ __global__ __launch_bounds__(BLOCK) void k_bresidual(Bell<3, 3> A, const float* 
                                                      const float* __restrict__ x,
                                                      float* __restrict__ r, const PcgState* st,
                                                      uint32_t rows) {
-    if (st->done) return;
     BELL_ROW(LANES, rows);
-    float ax[3];
-    bell_row<3, 3, LANES>(A, I, lane, x, ax);
-    if (lane != 0) return;
+    BellHead h = bell_head(A, I, st);
+    float ax[3], bi[3];
+    load_rows(b, I, bi);
+    keep(h, bi);
+    if (__builtin_amdgcn_readfirstlane(h.done)) return;
+    bell_row<3, 3, LANES>(A, h, lane, x, ax);
+    if (!store) return;
 #pragma unroll
-    for (int m = 0; m < 3; ++m) {
-        const size_t i = 3 * (size_t)I + m;
-        r[i] = b[i] - ax[m];
-    }
+    for (int m = 0; m < 3; ++m) r[3 * (size_t)I + m] = bi[m] - ax[m];
 }
 
 // b_c = P^T r, a group per aggregate; INIT: also the next level's
@@ -652,21 +707,28 @@ __global__ __launch_bounds__(BLOCK) void k_brestrict(Bell<3, R> T, const float* 
                                                      float* __restrict__ rc,
                                                      float* __restrict__ dc, float inv_theta_c,
                                                      const PcgState* st, uint32_t aggs) {
-    if (st->done) return;
     BELL_ROW(LANES, aggs);
-    float y[3];
-    bell_row<3, R, LANES>(T, I, lane, r, y);
-    if (lane != 0) return;
+    BellHead h = bell_head(T, I, st);
+    float y[3], di[3] = {};
+    if constexpr (INIT) {
+        load_rows(dinv_c, I, di);
+        keep(h, di);
+    } else {
+        keep(h);
+    }
+    if (__builtin_amdgcn_readfirstlane(h.done)) return;
+    bell_row<3, R, LANES>(T, h, lane, r, y);
+    if (!store) return;
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
         const size_t i = 3 * (size_t)I + m;
         bc[i] = y[m];
         if constexpr (INIT) {
-            const float ri = dinv_c[i] * y[m];
-            const float di = ri * inv_theta_c;
+            const float ri = di[m] * y[m];
+            const float d = ri * inv_theta_c;
             rc[i] = ri;
-            dc[i] = di;
-            xc[i] = di;
+            dc[i] = d;
+            xc[i] = d;
         }
     }
 }
@@ -676,16 +738,20 @@ template <int R, bool ADD, int LANES>
 __global__ __launch_bounds__(BLOCK) void k_bprolong(Bell<R, 3> P, const float* __restrict__ xc,
                                                     float* __restrict__ x, const PcgState* st,
                                                     uint32_t rows) {
-    if (st->done) return;
     BELL_ROW(LANES, rows);
-    float y[R];
-    bell_row<R, 3, LANES>(P, I, lane, xc, y);
-    if (lane != 0) return;
-#pragma unroll
-    for (int m = 0; m < R; ++m) {
-        const size_t i = (size_t)R * I + m;
-        x[i] = ADD ? x[i] + y[m] : y[m];
+    BellHead h = bell_head(P, I, st);
+    float y[R], x0[R] = {};
+    if constexpr (ADD) {
+        load_rows(x, I, x0);
+        keep(h, x0);
+    } else {
+        keep(h);
     }
+    if (__builtin_amdgcn_readfirstlane(h.done)) return;
+    bell_row<R, 3, LANES>(P, h, lane, xc, y);
+    if (!store) return;
+#pragma unroll
+    for (int m = 0; m < R; ++m) x[(size_t)R * I + m] = ADD ? x0[m] + y[m] : y[m];
 }
 
 // x = C^-1 b on the coarsest level (n <= AMG_COARSEST), one workgroup
@@ -880,7 +946,8 @@ __device__ __forceinline__ void bottom_apply(const Bell<3, 3>& B, uint32_t rows,
     const uint32_t lane = threadIdx.x % LANES;
     for (uint32_t I = threadIdx.x / LANES; I < rows; I += BOTTOM_TB / LANES) {
         float t[3];
-        bell_row<3, 3, LANES>(B, I, lane, x, t);
+        bell_row<3, 3, LANES, 2>(B, 
+                                  BellHead{B.slice_ptr[I >> 6], I & 63, B.len[I], 0}, lane, x, t);
         if (lane == 0)
 #pragma unroll
             for (int r = 0; r < 3; ++r) y[3 * I + r] = ADD ? y[3 * I + r] + t[r] : t[r];
@@ -950,6 +1017,8 @@ void amg_free(AmgDev* A) {
     delete A;
 }
 
+constexpr size_t BELL_SMALL = 65536;   // slots (2.6 MB)
+
 // The block sliced-ELL pattern of `rows` block rows: len_of(I) blocks in
 // row I, col_of(I, k) the k-th block's column; uploaded with room for R x C
 // FP32 values per slot.  NBX_ERR_ARG when a row has more blocks than the
@@ -977,12 +1046,25 @@ static int bell_upload(uint32_t rows, Len len_of, Col col_of, BellDev& B, size_t
         sp[sl + 1] = sp[sl] + w * SLICE;
     }
     std::vector<uint32_t> bcol(sp[ns], 0);
-    for (uint32_t I = 0; I < rows; ++I)
-        for (uint32_t k = 0; k < len[I]; ++k)
-            bcol[sp[I / SLICE] + (size_t)k * SLICE + I % SLICE] = col_of(I, k);
+    // One width for all slices where that adds little or the level is small:
+    // a row's place then follows from its index, without the loads of its
+    // slice and length before its blocks' (96x48 58 -> 53 us per outer
+    // iteration, 512x256 130 -> 127, 2048x1024 608 -> 598).  Padding blocks are zero, on the
+    // row's own first column: they add +0 to sums that are never -0.
+    for (uint16_t l : len) B.wmax = std::max<uint32_t>(B.wmax, l);
+    const size_t same = (size_t)ns * SLICE * B.wmax;
+    if (same <= 0xffffffffull && (same <= sp[ns] + (size_t)sp[ns] / 8 || same <= BELL_SMALL)) {
+        B.width = B.wmax;
+        for (uint32_t sl = 0; sl <= ns; ++sl) sp[sl] = sl * SLICE * B.width;
+        bcol.assign(same, 0);
+    }
+    for (uint32_t I = 0; I < rows; ++I) {
+        const uint32_t w = (sp[I / SLICE + 1] - sp[I / SLICE]) / SLICE;
+        for (uint32_t k = 0; k < w && len[I]; ++k)
+            bcol[sp[I / SLICE] + (size_t)k * SLICE + I % SLICE] = col_of(I, k < len[I] ? k : 0);
+    }
     B.rows = rows;
     B.slots = sp[ns];
-    for (uint16_t l : len) B.wmax = std::max<uint32_t>(B.wmax, l);
     // about three blocks per lane (1, 2, 4, 8 or 16 lanes)
     size_t used = 0;
     for (uint32_t I = 0; I < rows; ++I) used += len[I];
@@ -993,6 +1075,7 @@ static int bell_upload(uint32_t rows, Len len_of, Col col_of, BellDev& B, size_t
     NBX_TRY(up(&B.len, len, bytes));
     NBX_TRY(up(&B.bcol, bcol, bytes));
     NBX_TRY(alloc(&B.val, B.slots * R * C, bytes));
+    NBX_HIP(hipMemset(B.val, 0, B.slots * R * C * sizeof(float)));
     return NBX_OK;
 }
 
