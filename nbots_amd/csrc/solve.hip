@@ -1656,14 +1656,16 @@ static bool sym_u3(const Sym2& y) {
 }
 
 // The iteration in two kernels (k_cg_dir, k_cg_update), with pcg_run's host
-// cadence.  Node systems take it up to 131,072 nodes: us per iteration, five
-// kernels -> two, 64x32 cantilever 17.8 -> 9.3, 256x128 17 -> 9.1, 400x200 (80k
-// nodes) 17 -> 10.4, 600x300 (181k) 22.3 -> 17.9, 1024x512 (525k) 40 -> 47: a
-// row of the direction kernel gathers twice the bytes and holds 138 VGPRs.
+// cadence.  Node systems with the symmetric copy take it up to 196,608 nodes:
+// us per iteration, five kernels -> two, 64x32 cantilever 17.8 -> 9.3, 256x128
+// 17 -> 9.1, 400x200 (80k nodes) 17 -> 10.4, 540x270 (147k) 22.3 -> 17.1,
+// 600x300 (181k) 23.3 -> 19.5, 640x320 (206k) 24.4 -> 24.7, 1024x512 (525k)
+// 40 -> 47: a row of the direction kernel gathers twice the bytes and holds
+// 138 VGPRs.  The full layout, with twice the blocks a row, stops at 131,072.
 // Scalar CSR takes it up to 262,144 rows (figures at k_cg_dir_csr).  Both keep
 // the partials, which every workgroup sums, at 1,024 a value at most.
 constexpr uint32_t FCG2_MAX_NODES = CG2_PARTS * BLOCK;
-constexpr uint32_t CG2_MAX_NODES = 131072, CG2_MAX_ROWS = 262144;
+constexpr uint32_t CG2_MAX_NODES = 196608, CG2_MAX_FULL = 131072, CG2_MAX_ROWS = 262144;
 template <class Op>
 static int pcg2_run(const Op& op, uint32_t nu, const double* diag_in, const typename Op::V* b,
                     typename Op::V* x, uint32_t max_iter, double tol, Workspace& w, hipStream_t s,
@@ -1785,7 +1787,7 @@ int pcg_jacobi(const DevMatrix& m, const double* b, double* x, uint32_t max_iter
                             max_iter, tol, w, s, stats)
                  : pcg2_run(OpSymU<4>{{m.y}}, m.s.n_nodes, diag, (const double2*)b, (double2*)x,
                             max_iter, tol, w, s, stats);
-    else if (m.blocked && m.s.n_nodes <= CG2_MAX_NODES)
+    else if (m.blocked && !m.has_sym && m.s.n_nodes <= CG2_MAX_FULL)
         rc = pcg2_run(OpS2{m.s}, m.s.n_nodes, diag, (const double2*)b, (double2*)x, max_iter, tol,
                       w, s, stats);
     else if (m.blocked && m.has_sym && stream)

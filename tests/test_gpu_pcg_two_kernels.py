@@ -142,10 +142,10 @@ def test_scalar_limits(n):
     A.destroy()
 
 
-@pytest.mark.parametrize("n", [(361, 361), (362, 361)])
+@pytest.mark.parametrize("n", [(361, 361), (362, 361), (442, 442), (443, 443)])
 def test_node_limits(n):
-    """131,044 nodes (two kernels) and 131,406 (five), through the device
-    system in reference mode."""
+    """131,044 and 131,406 nodes, 196,249 (two kernels) and 197,136 (five),
+    through the device system in reference mode."""
     import oracle
     from nbots_amd import synth
     from nbots_amd.fem import Fem, SOLVE_REFERENCE
