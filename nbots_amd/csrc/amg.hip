@@ -72,9 +72,9 @@ struct AmgDev {
     double* ones = nullptr;         // [finest n + 2] the flexible CG's unit scaling
     double* pow_x = nullptr;        // power iteration: [finest n + 2] x, y
     double* pow_y = nullptr;
-    double* scal = nullptr;         // [2] device scalars
+    double* scal = nullptr;         // [2 levels] 1 / norm and norm of the power iteration
     double* partials = nullptr;     // [MAX_GRID] reduction partials
-    std::vector<double> host_inv;
+    double* dense = nullptr;        // the coarsest matrix, n x n
     size_t bytes = 0;
     // more than one level: the finest is smoothed on the matrix's fp16
     // scaled copy, in scaled variables, and its P values are stored as
@@ -185,29 +185,30 @@ __global__ __launch_bounds__(BLOCK) void k_amg_pow_init(double* __restrict__ x, 
     h ^= h >> 13;
     x[i] = (h & 1u) ? 1.0 : -1.0;
 }
-// x.x partials
-__global__ __launch_bounds__(BLOCK) void k_amg_sq(const double* __restrict__ x, double* partials,
-                                                  uint32_t n) {
-    double acc[1] = {0.0};
-    const uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i < n) acc[0] = x[i] * x[i];
-    __shared__ double red[1][BLOCK / WAVE];
-    block_sum<1>(acc, red);
-    put_partials<1>(acc, partials);
-}
-// y = D^-1 A (x * s), s = *scale (1 / ||x|| of the previous step); y.y
-// partials.  Eight lanes per row, rows strided over the grid (at most
-// MAX_GRID workgroups, one partial each).
+// y = D^-1 A (x * s) and the y.y partials.  s = 1 / ||x||: from the step
+// before's partials (prev), which every workgroup sums itself; on levels of
+// more than ALL_PARTS workgroups from *scale, left by k_amg_pow_fin; or, on the
+// first step, s0.  Eight lanes per row, rows strided over the grid (at most
+// MAX_GRID workgroups, one partial each).  A step of a small level is a launch
+// and a chain of loads, so the summing kernel between two steps cost as much
+// again (15 of 2.3 us and their launches a level, of 4.5 us steps).
 constexpr int POW_LANES = 8;
-__global__ __launch_bounds__(BLOCK) void k_amg_pow_step(const uint32_t* __restrict__ ptr,
-                                                        const uint32_t* __restrict__ col,
-                                                        const double* __restrict__ a,
-                                                        const double* __restrict__ dinv,
-                                                        const double* __restrict__ x,
-                                                        double* __restrict__ y,
-                                                        const double* __restrict__ scale,
-                                                        double* partials, uint32_t n) {
-    const double sc = *scale;
+constexpr int POW_STEPS = 15;
+__global__ __launch_bounds__(BLOCK) void k_amg_pow_step(
+    const uint32_t* __restrict__ ptr, const uint32_t* __restrict__ col,
+    const double* __restrict__ a, const double* __restrict__ dinv, const double* __restrict__ x,
+    double* __restrict__ y, const double* __restrict__ prev, const double* __restrict__ scale,
+    double s0, double* __restrict__ partials, uint32_t n) {
+    double sc = s0;
+    if (prev) {
+        __shared__ double sums[1][ALL_PARTS / WAVE];
+        double tot[1];
+        all_sum<1>(prev, gridDim.x, tot, sums);
+        const double nr = sqrt(tot[0]);
+        sc = nr > 0.0 ? 1.0 / nr : 0.0;
+    } else if (scale) {
+        sc = *scale;
+    }
     double acc[1] = {0.0};
     const size_t gid = (size_t)blockIdx.x * BLOCK + threadIdx.x;
     const uint32_t lane = (uint32_t)(gid % POW_LANES);
@@ -242,6 +243,114 @@ __global__ __launch_bounds__(FIN) void k_amg_pow_fin(const double* partials, uns
     }
 }
 
+// ---- the coarsest level's inverse --------------------------------------------
+// A^-1 of the coarsest level (at most AMG_COARSEST unknowns) by symmetric
+// sweeps (Goodnight 1979): sweeping k turns a_kk into -1 / a_kk, a_ik into
+// a_ik / a_kk and a_ij into a_ij - a_ik a_kj / a_kk; all swept, A is -A^-1.
+// The pivots are the Cholesky factor's, and an unknown whose pivot is not
+// above 1e-13 of the largest diagonal entry is dropped as amg_dense_inverse
+// drops it (zero row and column).  One workgroup holds the matrix in
+// registers, NB x NB entries a thread; a step passes column k through LDS and
+// costs one barrier.  Bound by its n steps of LDS reads, a division and a
+// barrier: 190 us at 162 unknowns.  The host function took 0.6 ms there besides
+// the copies and the wait; with the folded power iteration above, the numeric
+// phase went from 1.13 to 0.78 ms at 96x48 (162 unknowns), 0.95 -> 0.78 at
+// 150x75 (36), 1.74 -> 1.52 at 512x256 (24).  The same Cholesky factor and
+// products on the device, bit for bit the host's, take 445 us at 162.  Against
+// extended precision the inverse's error is the host's within a factor of three
+// either way (1e-14 to 1e-10 at condition numbers of 1e4 to 1e9; FP32 rounding
+// is 2e-8).
+constexpr int SWEEP_SIDE = 32, SWEEP_TB = SWEEP_SIDE * SWEEP_SIDE;
+constexpr int SWEEP_NB = (AMG_COARSEST + SWEEP_SIDE - 1) / SWEEP_SIDE;
+
+// The dense matrix from its CSR rows, a wavefront per row
+__global__ __launch_bounds__(WAVE) void k_dense_rows(const uint32_t* __restrict__ ptr,
+                                                     const uint32_t* __restrict__ col,
+                                                     const double* __restrict__ a,
+                                                     double* __restrict__ out, uint32_t n) {
+    __shared__ double row[AMG_COARSEST];
+    const uint32_t i = blockIdx.x;
+    for (uint32_t j = threadIdx.x; j < n; j += WAVE) row[j] = 0.0;
+    __syncthreads();
+    for (uint32_t e = ptr[i] + threadIdx.x; e < ptr[i + 1]; e += WAVE) row[col[e]] = a[e];
+    __syncthreads();
+    for (uint32_t j = threadIdx.x; j < n; j += WAVE) out[(size_t)i * n + j] = row[j];
+}
+
+// inv = A^-1 in FP32, of A symmetrised (P^T A P rounds slightly
+// unsymmetrically).  Thread (tx, ty) holds the entries (ty + 32 p, tx + 32 q).
+template <int NB>
+__global__ __launch_bounds__(SWEEP_TB) void k_dense_sweep(const double* __restrict__ a,
+                                                          float* __restrict__ inv, uint32_t n) {
+    __shared__ double colk[2][NB * SWEEP_SIDE], big[SWEEP_TB / WAVE];
+    const uint32_t tx = threadIdx.x % SWEEP_SIDE, ty = threadIdx.x / SWEEP_SIDE;
+    double v[NB][NB], dmax = 0.0;
+#pragma unroll
+    for (int p = 0; p < NB; ++p)
+#pragma unroll
+        for (int q = 0; q < NB; ++q) {
+            const uint32_t i = ty + p * SWEEP_SIDE, j = tx + q * SWEEP_SIDE;
+            v[p][q] = 0.0;
+            if (i < n && j < n)
+                v[p][q] = i == j ? a[(size_t)i * n + i]
+                                 : 0.5 * (a[(size_t)i * n + j] + a[(size_t)j * n + i]);
+            if (i == j) dmax = fmax(dmax, v[p][q]);
+        }
+    for (int off = WAVE / 2; off > 0; off >>= 1) dmax = fmax(dmax, __shfl_xor(dmax, off));
+    if (threadIdx.x % WAVE == 0) big[threadIdx.x / WAVE] = dmax;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < SWEEP_TB / WAVE; ++w) dmax = fmax(dmax, big[w]);
+    for (uint32_t k = 0; k < n; ++k) {
+        double* const ck = colk[k & 1];
+        const uint32_t kq = k / SWEEP_SIDE, kt = k % SWEEP_SIDE;
+        if (tx == kt)
+#pragma unroll
+            for (int q = 0; q < NB; ++q)
+                if (q == (int)kq)
+#pragma unroll
+                    for (int p = 0; p < NB; ++p) ck[ty + p * SWEEP_SIDE] = v[p][q];
+        __syncthreads();
+        const double piv = ck[k];
+        const bool drop = !(piv > 1e-13 * dmax);
+        const double d = drop ? 0.0 : 1.0 / piv;
+        double cj[NB];
+#pragma unroll
+        for (int q = 0; q < NB; ++q) cj[q] = ck[tx + q * SWEEP_SIDE];
+#pragma unroll
+        for (int p = 0; p < NB; ++p) {
+            const double f = ck[ty + p * SWEEP_SIDE] * d;
+#pragma unroll
+            for (int q = 0; q < NB; ++q) v[p][q] = fma(-f, cj[q], v[p][q]);
+        }
+        // row and column k
+        if (ty == kt)
+#pragma unroll
+            for (int p = 0; p < NB; ++p)
+                if (p == (int)kq)
+#pragma unroll
+                    for (int q = 0; q < NB; ++q) v[p][q] = cj[q] * d;
+        if (tx == kt)
+#pragma unroll
+            for (int q = 0; q < NB; ++q)
+                if (q == (int)kq)
+#pragma unroll
+                    for (int p = 0; p < NB; ++p) {
+                        const uint32_t i = ty + p * SWEEP_SIDE;
+                        v[p][q] = i == k ? -d : ck[i] * d;
+                    }
+    }
+    // (one of the two entries that rounding may leave different for both)
+#pragma unroll
+    for (int p = 0; p < NB; ++p)
+#pragma unroll
+        for (int q = 0; q < NB; ++q) {
+            const uint32_t i = ty + p * SWEEP_SIDE, j = tx + q * SWEEP_SIDE;
+            if (i < n && j <= i)
+                inv[(size_t)i * n + j] = inv[(size_t)j * n + i] = (float)-v[p][q];
+        }
+}
+
 // P = T - omega D^-1 A T: SMOOTH_SLOTS threads per node, each taking every
 // SMOOTH_SLOTS-th aggregate column group of the node's P rows (its R rows
 // share one A and one P pattern; a group is the three columns of one
@@ -253,7 +362,9 @@ __global__ __launch_bounds__(BLOCK) void k_amg_smooth_p(
     const uint32_t* __restrict__ a_ptr, const uint32_t* __restrict__ a_col,
     const double* __restrict__ a, const double* __restrict__ dinv, const double* __restrict__ t,
     const uint32_t* __restrict__ agg, const uint32_t* __restrict__ p_ptr,
-    const uint32_t* __restrict__ p_col, double* __restrict__ p, double omega, uint32_t nodes) {
+    const uint32_t* __restrict__ p_col, double* __restrict__ p, const double* __restrict__ lmax,
+    uint32_t nodes) {
+    const double omega = 4.0 / (3.0 * *lmax);
     const size_t tid = (size_t)blockIdx.x * BLOCK + threadIdx.x;
     const uint32_t I = (uint32_t)(tid / SMOOTH_SLOTS);
     if (I >= nodes) return;
@@ -1011,7 +1122,7 @@ void amg_free(AmgDev* A) {
         }
     }
     void* ps[] = {A->cinv, A->ones,     A->pow_x,  A->pow_y,
-                  A->scal, A->partials, A->nzbits, A->differ};
+                  A->scal, A->partials, A->nzbits, A->differ, A->dense};
     for (void* p : ps)
         if (p) (void)hipFree(p);
     delete A;
@@ -1252,11 +1363,11 @@ static int amg_symbolic(FemSys& S) {
     NBX_TRY(alloc(&A->ones, n, A->bytes));
     NBX_TRY(alloc(&A->pow_x, n, A->bytes));
     NBX_TRY(alloc(&A->pow_y, n, A->bytes));
-    NBX_TRY(alloc(&A->scal, 2, A->bytes));
+    NBX_TRY(alloc(&A->scal, 2 * nl, A->bytes));
+    NBX_TRY(alloc(&A->dense, (size_t)nco * nco, A->bytes));
     NBX_TRY(alloc(&A->partials, (size_t)MAX_GRID, A->bytes));
     std::vector<double> ones(n + 2, 1.0);
     NBX_HIP(hipMemcpy(A->ones, ones.data(), ones.size() * sizeof(double), hipMemcpyHostToDevice));
-    A->host_inv.assign((size_t)nco * nco, 0.0);
     NBX_TRY(alloc(&A->differ, 1, A->bytes));
     std::swap(A->nzbits, dbits.d);
     return NBX_OK;
@@ -1310,6 +1421,23 @@ static void with_out_lanes(size_t blocks, F&& f) {
         f(std::integral_constant<int, 16>{});
 }
 
+// cinv of the coarsest level's current values
+template <int NB>
+static void launch_sweep(AmgDev* A, uint32_t n, hipStream_t s) {
+    if constexpr (NB < SWEEP_NB)
+        if (n > NB * SWEEP_SIDE) return launch_sweep<NB + 1>(A, n, s);
+    hipLaunchKernelGGL(k_dense_sweep<NB>, dim3(1), dim3(SWEEP_TB), 0, s, A->dense, A->cinv, n);
+}
+static int coarsest_inverse(AmgDev* A, hipStream_t s) {
+    const AmgDevLevel& L = A->lv.back();
+    if (!L.n) return NBX_OK;
+    hipLaunchKernelGGL(k_dense_rows, dim3(L.n), dim3(WAVE), 0, s, L.a_ptr, L.a_col, L.a64, A->dense,
+                       L.n);
+    launch_sweep<1>(A, L.n, s);
+    NBX_HIP(hipGetLastError());
+    return NBX_OK;
+}
+
 // Numeric phase for the current values of K.
 static int amg_numeric(FemSys& S) {
     AmgDev* A = S.K.amg;
@@ -1326,73 +1454,32 @@ static int amg_numeric(FemSys& S) {
         // (the finest level's smoothing reads the fp16 scaled copy; the
         // coarser levels' operators are filled in block form by the level
         // above)
-        // lambda_max(D^-1 A): 15 power steps from a fixed start (the
-        // coarsest level, solved directly, needs none)
-        if (l + 1 < A->lv.size()) {
+        if (l + 1 == A->lv.size()) break;
+        // lambda_max(D^-1 A): POW_STEPS power steps from a fixed start, x.x = n
+        // (the coarsest level, solved directly, needs none)
         hipLaunchKernelGGL(k_amg_pow_init, dim3(g), dim3(BLOCK), 0, s, A->pow_x, L.n);
-        hipLaunchKernelGGL(k_amg_sq, dim3(g), dim3(BLOCK), 0, s, A->pow_x, A->partials, L.n);
-        hipLaunchKernelGGL(k_amg_pow_fin, dim3(1), dim3(FIN), 0, s, A->partials, g, A->scal);
-        double *px = A->pow_x, *py = A->pow_y;
+        double *px = A->pow_x, *py = A->pow_y, *scal = A->scal + 2 * l;
         const unsigned gp = std::min<size_t>(grid_for((size_t)L.n * POW_LANES), (size_t)MAX_GRID);
-        for (int it = 0; it < 15; ++it) {
+        const bool fold = gp <= ALL_PARTS;
+        const double s0 = 1.0 / sqrt((double)L.n);
+        for (int it = 0; it < POW_STEPS; ++it) {
+            double* const part = A->partials + (fold ? (it & 1) * ALL_PARTS : 0);
+            const double* const prev =
+                fold && it ? A->partials + ((it - 1) & 1) * ALL_PARTS : nullptr;
             hipLaunchKernelGGL(k_amg_pow_step, dim3(gp), dim3(BLOCK), 0, s, L.a_ptr, L.a_col, L.a64,
-                               L.dinv64, px, py, A->scal, A->partials, L.n);
-            hipLaunchKernelGGL(k_amg_pow_fin, dim3(1), dim3(FIN), 0, s, A->partials, gp, A->scal);
+                               L.dinv64, px, py, prev, it ? scal : nullptr, s0, part, L.n);
+            if (!fold || it + 1 == POW_STEPS)
+                hipLaunchKernelGGL(k_amg_pow_fin, dim3(1), dim3(FIN), 0, s, part, gp, scal);
             std::swap(px, py);
         }
         NBX_HIP(hipGetLastError());
-        double sc[2];
-        NBX_HIP(copy_on(sc, A->scal, sizeof sc, hipMemcpyDeviceToHost, s));
-        L.lmax = sc[1];
-        if (!(L.lmax > 0.0) || !std::isfinite(L.lmax)) {
-            set_last_error("AMG: lambda_max(D^-1 A) of level %zu is %g", l, L.lmax);
-            return NBX_ERR_BREAKDOWN;
-        }
-        {
-            const double hi = 1.1 * L.lmax, lo = L.lmax / 30.0;
-            const double theta = 0.5 * (hi + lo), delta = 0.5 * (hi - lo), sigma = theta / delta;
-            double rho = 1.0 / sigma;
-            L.inv_theta = (float)(1.0 / theta);
-            for (int k = 1; k < L.degree; ++k) {
-                const double rn = 1.0 / (2.0 * sigma - rho);
-                L.c1[k] = (float)(rn * rho);
-                L.c2[k] = (float)(2.0 * rn / delta);
-                rho = rn;
-            }
-        }
-        }
-        if (l + 1 == A->lv.size()) {
-            // coarsest: its inverse, on the host (at most AMG_COARSEST^2 entries)
-            std::vector<uint32_t> ptr(L.n + 1), col(L.a_nnz);
-            std::vector<double> a(L.a_nnz);
-            NBX_HIP(hipMemcpyAsync(ptr.data(), L.a_ptr, ptr.size() * 4, hipMemcpyDeviceToHost, s));
-            NBX_HIP(hipMemcpyAsync(col.data(), L.a_col, col.size() * 4, hipMemcpyDeviceToHost, s));
-            NBX_HIP(copy_on(a.data(), L.a64, a.size() * 8, hipMemcpyDeviceToHost, s));
-            std::vector<double>& inv = A->host_inv;
-            std::fill(inv.begin(), inv.end(), 0.0);
-            for (uint32_t i = 0; i < L.n; ++i)
-                for (uint32_t e = ptr[i]; e < ptr[i + 1]; ++e) inv[(size_t)i * L.n + col[e]] = a[e];
-            // symmetrise (P^T A P rounds slightly unsymmetrically)
-            for (uint32_t i = 0; i < L.n; ++i)
-                for (uint32_t j = 0; j < i; ++j) {
-                    const double m = 0.5 * (inv[(size_t)i * L.n + j] + inv[(size_t)j * L.n + i]);
-                    inv[(size_t)i * L.n + j] = inv[(size_t)j * L.n + i] = m;
-                }
-            amg_dense_inverse(L.n, inv.data());
-            std::vector<float> f(inv.size());
-            for (size_t k = 0; k < inv.size(); ++k) f[k] = (float)inv[k];
-            NBX_HIP(hipMemcpyAsync(A->cinv, f.data(), f.size() * 4, hipMemcpyHostToDevice, s));
-            NBX_HIP(hipStreamSynchronize(s));
-            break;
-        }
         AmgDevLevel& C = A->lv[l + 1];
-        const double omega = 4.0 / (3.0 * L.lmax);
         with_bs(L.bs, [&](auto rr) {
             constexpr int R = decltype(rr)::value;
             hipLaunchKernelGGL(k_amg_smooth_p<R>,
                                dim3(grid_for((size_t)(L.n / R) * SMOOTH_SLOTS)), dim3(BLOCK), 0,
                                s, L.a_ptr, L.a_col, L.a64, L.dinv64, L.t, L.agg, L.p_ptr,
-                               L.p_col, L.p64, omega, L.n / R);
+                               L.p_col, L.p64, scal + 1, L.n / R);
         });
         // P and P^T in block form (D^1/2 P on the finest level when it is
         // smoothed in the scaled variables)
@@ -1433,6 +1520,28 @@ static int amg_numeric(FemSys& S) {
             hipLaunchKernelGGL((k_bell_fill<3, 3>), dim3(grid_for(C.ab.rows)), dim3(BLOCK), 0, s,
                                C.ab, C.a_ptr, C.a64, (const double*)nullptr);
         NBX_HIP(hipGetLastError());
+    }
+    NBX_TRY(coarsest_inverse(A, s));
+    // the smoothers' coefficients, from all levels' lambda_max at once
+    std::vector<double> scal(2 * A->lv.size());
+    NBX_HIP(copy_on(scal.data(), A->scal, scal.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+    for (size_t l = 0; l + 1 < A->lv.size(); ++l) {
+        AmgDevLevel& L = A->lv[l];
+        L.lmax = scal[2 * l + 1];
+        if (!(L.lmax > 0.0) || !std::isfinite(L.lmax)) {
+            set_last_error("AMG: lambda_max(D^-1 A) of level %zu is %g", l, L.lmax);
+            return NBX_ERR_BREAKDOWN;
+        }
+        const double hi = 1.1 * L.lmax, lo = L.lmax / 30.0;
+        const double theta = 0.5 * (hi + lo), delta = 0.5 * (hi - lo), sigma = theta / delta;
+        double rho = 1.0 / sigma;
+        L.inv_theta = (float)(1.0 / theta);
+        for (int k = 1; k < L.degree; ++k) {
+            const double rn = 1.0 / (2.0 * sigma - rho);
+            L.c1[k] = (float)(rn * rho);
+            L.c2[k] = (float)(2.0 * rn / delta);
+            rho = rn;
+        }
     }
     return NBX_OK;
 }

@@ -242,39 +242,6 @@ __global__ __launch_bounds__(BLOCK) void k_pcg_tail(V* __restrict__ x, PBufs<V> 
 // per 256 rows, wave sums of 64 partials, those in index order) and the stop
 // test are formed by the same operations in the same order as in the five
 // kernels, so the results are the same bit for bit.
-constexpr unsigned CG2_PARTS = 1024;   // most partials of a value
-template <int NV>
-__device__ __forceinline__ void all_sum(const double* __restrict__ partials, unsigned np,
-                                        double (&tot)[NV], double (*red)[CG2_PARTS / WAVE]) {
-    constexpr unsigned WAVES = BLOCK / WAVE;
-    const unsigned lane = threadIdx.x % WAVE, wid = threadIdx.x / WAVE;
-    const unsigned groups = (np + WAVE - 1) / WAVE;   // of 64 partials, a wave sum each
-    double v[NV][CG2_PARTS / BLOCK];
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
-#pragma unroll
-        for (unsigned j = 0; j < CG2_PARTS / BLOCK; ++j) {
-            const unsigned b = (wid + j * WAVES) * WAVE + lane;
-            v[i][j] = b < np ? partials[(size_t)i * np + b] : 0.0;
-        }
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
-#pragma unroll
-        for (unsigned j = 0; j < CG2_PARTS / BLOCK; ++j) {
-            const unsigned g = wid + j * WAVES;
-            if (g < groups) {
-                const double s = wave_sum(v[i][j]);
-                if (lane == 0) red[i][g] = s;
-            }
-        }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        double s = 0.0;
-        for (unsigned g = 0; g < groups; ++g) s += red[i][g];
-        tot[i] = s;
-    }
-}
 
 // q of the coming direction and the direction before it, side by side: the
 // product gathers both of a neighbour in one place.
@@ -298,7 +265,7 @@ struct CgDir {
 // ended.  Called by every thread of every workgroup, with the same results.
 __device__ __forceinline__ bool cg_next(const PcgState* __restrict__ sin, PcgState* sout,
                                         const double* __restrict__ upd, bool first,
-                                        double (*red)[CG2_PARTS / WAVE], CgDir& dir) {
+                                        double (*red)[ALL_PARTS / WAVE], CgDir& dir) {
     const uint32_t ended = sin->done, max_iter = sin->max_iter;
     const uint32_t k = first ? 0u : sin->k + 1u;
     const double tol2 = sin->tol2, rz = sin->rz, gg_cur = sin->gg_cur;
@@ -342,7 +309,7 @@ struct FcgDir {
 };
 __device__ __forceinline__ bool cg_next(const PcgState* __restrict__ sin, PcgState* sout,
                                         const double* __restrict__ dots, bool first,
-                                        double (*red)[CG2_PARTS / WAVE], FcgDir& dir) {
+                                        double (*red)[ALL_PARTS / WAVE], FcgDir& dir) {
     const uint32_t ended = sin->done;
     const double alpha = sin->alpha, rz_old = sin->rz;
     double tot[2];
@@ -553,7 +520,7 @@ __global__ __launch_bounds__(BLOCK) void k_cg_dir(Op op,
                                                   const double* __restrict__ upd, double* dirp,
                                                   uint32_t n, bool first) {
     using V = typename Op::V;
-    __shared__ double red[2][CG2_PARTS / WAVE], red2[2][BLOCK / WAVE];
+    __shared__ double red[2][ALL_PARTS / WAVE], red2[2][BLOCK / WAVE];
     const Chunk c = my_chunk(n);
     const size_t u = c.beg + threadIdx.x;
     const bool valid = u < c.end;
@@ -600,7 +567,7 @@ __global__ __launch_bounds__(BLOCK) void k_cg_dir_csr(DevCsr A,
                                                       const double* __restrict__ upd,
                                                       double* dirp, uint32_t n, bool first) {
     constexpr int TILE = PER * BLOCK;
-    __shared__ double red[2][CG2_PARTS / WAVE], prod[TILE], red2[1][BLOCK / WAVE];
+    __shared__ double red[2][ALL_PARTS / WAVE], prod[TILE], red2[1][BLOCK / WAVE];
     const Chunk c = my_chunk(n);
     const size_t u = c.beg + threadIdx.x;
     const bool valid = u < c.end;
@@ -689,7 +656,7 @@ __global__ __launch_bounds__(BLOCK) void k_cg_update(V* __restrict__ x, V* __res
                                                      const PcgState* __restrict__ st,
                                                      const double* __restrict__ dirp, double* upd,
                                                      uint32_t n) {
-    __shared__ double red[2][CG2_PARTS / WAVE], red2[2][BLOCK / WAVE];
+    __shared__ double red[2][ALL_PARTS / WAVE], red2[2][BLOCK / WAVE];
     const Chunk c = my_chunk(n);
     const size_t u = c.beg + threadIdx.x;
     const bool valid = u < c.end;
@@ -1379,7 +1346,7 @@ __global__ __launch_bounds__(BLOCK) void k_fcg2_update(
     const double2* __restrict__ dis, float2* __restrict__ res, float2* __restrict__ dz,
     float2* __restrict__ z, PcgState* s0, const PcgState* __restrict__ s1,
     const double* __restrict__ dirp, double* rrp, uint32_t n, double inv_theta) {
-    __shared__ double red[1][CG2_PARTS / WAVE], red2[1][BLOCK / WAVE];
+    __shared__ double red[1][ALL_PARTS / WAVE], red2[1][BLOCK / WAVE];
     const Chunk c = my_chunk(n);
     const size_t i = c.beg + threadIdx.x;
     const bool valid = i < c.end;
@@ -1436,7 +1403,7 @@ __global__ __launch_bounds__(BLOCK) void k_fcg2_dots(const float2* __restrict__ 
                                                      const PcgState* __restrict__ s1,
                                                      const double* __restrict__ rrp, double* dots,
                                                      uint32_t n, bool first) {
-    __shared__ double red[1][CG2_PARTS / WAVE], red2[2][BLOCK / WAVE];
+    __shared__ double red[1][ALL_PARTS / WAVE], red2[2][BLOCK / WAVE];
     const Chunk c = my_chunk(n);
     const size_t i = c.beg + threadIdx.x;
     const bool valid = i < c.end;
@@ -1664,7 +1631,7 @@ static bool sym_u3(const Sym2& y) {
 // 138 VGPRs.  The full layout, with twice the blocks a row, stops at 131,072.
 // Scalar CSR takes it up to 262,144 rows (figures at k_cg_dir_csr).  Both keep
 // the partials, which every workgroup sums, at 1,024 a value at most.
-constexpr uint32_t FCG2_MAX_NODES = CG2_PARTS * BLOCK;
+constexpr uint32_t FCG2_MAX_NODES = ALL_PARTS * BLOCK;
 constexpr uint32_t CG2_MAX_NODES = 196608, CG2_MAX_FULL = 131072, CG2_MAX_ROWS = 262144;
 template <class Op>
 static int pcg2_run(const Op& op, uint32_t nu, const double* diag_in, const typename Op::V* b,
