@@ -348,40 +348,46 @@ __device__ __forceinline__ void fin_sum(const double* partials, unsigned np, dou
 }
 // fin_sum's result in every thread of a workgroup of BLOCK threads, for up to
 // ALL_PARTS partials a value: kernels that would follow a finalize kernel sum
-// the partials themselves.
+// the partials themselves.  load() goes before the kernel's own loads, which
+// are then still under way while total() adds (loads complete in order).
 constexpr unsigned ALL_PARTS = 1024;
 template <int NV>
-__device__ __forceinline__ void all_sum(const double* __restrict__ partials, unsigned np,
-                                        double (&tot)[NV], double (*red)[ALL_PARTS / WAVE]) {
-    constexpr unsigned WAVES = BLOCK / WAVE;
-    const unsigned lane = threadIdx.x % WAVE, wid = threadIdx.x / WAVE;
-    const unsigned groups = (np + WAVE - 1) / WAVE;   // of 64 partials, a wave sum each
+struct AllSum {
+    static constexpr unsigned WAVES = BLOCK / WAVE;
     double v[NV][ALL_PARTS / BLOCK];
+    __device__ __forceinline__ void load(const double* __restrict__ partials, unsigned np) {
+        const unsigned lane = threadIdx.x % WAVE, wid = threadIdx.x / WAVE;
 #pragma unroll
-    for (int i = 0; i < NV; ++i)
+        for (int i = 0; i < NV; ++i)
 #pragma unroll
-        for (unsigned j = 0; j < ALL_PARTS / BLOCK; ++j) {
-            const unsigned b = (wid + j * WAVES) * WAVE + lane;
-            v[i][j] = b < np ? partials[(size_t)i * np + b] : 0.0;
-        }
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
-#pragma unroll
-        for (unsigned j = 0; j < ALL_PARTS / BLOCK; ++j) {
-            const unsigned g = wid + j * WAVES;
-            if (g < groups) {
-                const double s = wave_sum(v[i][j]);
-                if (lane == 0) red[i][g] = s;
+            for (unsigned j = 0; j < ALL_PARTS / BLOCK; ++j) {
+                const unsigned b = (wid + j * WAVES) * WAVE + lane;
+                v[i][j] = b < np ? partials[(size_t)i * np + b] : 0.0;
             }
-        }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        double s = 0.0;
-        for (unsigned g = 0; g < groups; ++g) s += red[i][g];
-        tot[i] = s;
     }
-}
+    __device__ __forceinline__ void total(unsigned np, double (&tot)[NV],
+                                          double (*red)[ALL_PARTS / WAVE]) const {
+        const unsigned lane = threadIdx.x % WAVE, wid = threadIdx.x / WAVE;
+        const unsigned groups = (np + WAVE - 1) / WAVE;   // of 64 partials, a wave sum each
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (unsigned j = 0; j < ALL_PARTS / BLOCK; ++j) {
+                const unsigned g = wid + j * WAVES;
+                if (g < groups) {
+                    const double s = wave_sum(v[i][j]);
+                    if (lane == 0) red[i][g] = s;
+                }
+            }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            double s = 0.0;
+            for (unsigned g = 0; g < groups; ++g) s += red[i][g];
+            tot[i] = s;
+        }
+    }
+};
 template <int NV>
 __device__ __forceinline__ void fin_sum(const float* partials, unsigned np, f32c (&tot)[NV]) {
     __shared__ f32c red[NV][FIN / WAVE];

@@ -264,13 +264,13 @@ struct CgDir {
 // k_fin_B) from the sums of the update before it; false when the solve has
 // ended.  Called by every thread of every workgroup, with the same results.
 __device__ __forceinline__ bool cg_next(const PcgState* __restrict__ sin, PcgState* sout,
-                                        const double* __restrict__ upd, bool first,
+                                        const AllSum<2>& upd, bool first,
                                         double (*red)[ALL_PARTS / WAVE], CgDir& dir) {
     const uint32_t ended = sin->done, max_iter = sin->max_iter;
     const uint32_t k = first ? 0u : sin->k + 1u;
     const double tol2 = sin->tol2, rz = sin->rz, gg_cur = sin->gg_cur;
     double tot[2];
-    all_sum<2>(upd, gridDim.x, tot, red);
+    upd.total(gridDim.x, tot, red);
     const double gg_prev = first ? tot[1] : gg_cur;
     const bool go = gg_prev > tol2 && k < max_iter;
     dir.beta = first ? 0.0 : tot[0] / rz;
@@ -308,12 +308,12 @@ struct FcgDir {
     }
 };
 __device__ __forceinline__ bool cg_next(const PcgState* __restrict__ sin, PcgState* sout,
-                                        const double* __restrict__ dots, bool first,
+                                        const AllSum<2>& dots, bool first,
                                         double (*red)[ALL_PARTS / WAVE], FcgDir& dir) {
     const uint32_t ended = sin->done;
     const double alpha = sin->alpha, rz_old = sin->rz;
     double tot[2];
-    all_sum<2>(dots, gridDim.x, tot, red);
+    dots.total(gridDim.x, tot, red);
     const double rz = tot[1];
     dir.beta = first ? 0.0 : -alpha * tot[0] / rz_old;
     dir.first = first;
@@ -524,6 +524,8 @@ __global__ __launch_bounds__(BLOCK) void k_cg_dir(Op op,
     const Chunk c = my_chunk(n);
     const size_t u = c.beg + threadIdx.x;
     const bool valid = u < c.end;
+    AllSum<2> sums;
+    sums.load(upd, gridDim.x);
     CgRow<Op> row{op.mat()};
     CgPair<V> own{};
     if (valid) {
@@ -531,7 +533,7 @@ __global__ __launch_bounds__(BLOCK) void k_cg_dir(Op op,
         row.load((uint32_t)u, d);
     }
     D dir;
-    if (!cg_next(sin, sout, upd, first, red, dir)) return;
+    if (!cg_next(sin, sout, sums, first, red, dir)) return;
     double acc[1] = {0.0};
     if (valid) {
         const V pd = dir(own);
@@ -571,6 +573,8 @@ __global__ __launch_bounds__(BLOCK) void k_cg_dir_csr(DevCsr A,
     const Chunk c = my_chunk(n);
     const size_t u = c.beg + threadIdx.x;
     const bool valid = u < c.end;
+    AllSum<2> sums;
+    sums.load(upd, gridDim.x);
     const uint32_t e0 = A.rowptr[c.beg], e1 = A.rowptr[c.end];
     uint32_t r0 = e1, r1 = e1;
     CgPair<double> own{};
@@ -597,7 +601,7 @@ __global__ __launch_bounds__(BLOCK) void k_cg_dir_csr(DevCsr A,
     };
     fetch(e0);
     CgDir dir;
-    if (!cg_next(sin, sout, upd, first, red, dir)) return;
+    if (!cg_next(sin, sout, sums, first, red, dir)) return;
     double s = 0.0;
     for (uint64_t base = e0; base < e1; base += TILE) {
         const uint32_t m = (uint32_t)min((uint64_t)TILE, e1 - base);
@@ -660,6 +664,8 @@ __global__ __launch_bounds__(BLOCK) void k_cg_update(V* __restrict__ x, V* __res
     const Chunk c = my_chunk(n);
     const size_t u = c.beg + threadIdx.x;
     const bool valid = u < c.end;
+    AllSum<1> sums;
+    sums.load(dirp, gridDim.x);
     V xv{}, pv{}, gv{}, wv{}, dv{};
     if (valid) {
         xv = x[u];
@@ -671,7 +677,7 @@ __global__ __launch_bounds__(BLOCK) void k_cg_update(V* __restrict__ x, V* __res
     const uint32_t done = st->done;
     const double rz = st->rz;
     double tot[1];
-    all_sum<1>(dirp, gridDim.x, tot, red);
+    sums.total(gridDim.x, tot, red);
     if (done) return;
     const double alpha = rz / tot[0];
     double acc[2] = {0.0, 0.0};
@@ -1350,6 +1356,8 @@ __global__ __launch_bounds__(BLOCK) void k_fcg2_update(
     const Chunk c = my_chunk(n);
     const size_t i = c.beg + threadIdx.x;
     const bool valid = i < c.end;
+    AllSum<1> sums;
+    if constexpr (!FIRST) sums.load(dirp, gridDim.x);
     double2 xv{}, pv{}, rv{}, wv{}, dd{};
     if (valid) {
         dd = dis[i];
@@ -1365,7 +1373,7 @@ __global__ __launch_bounds__(BLOCK) void k_fcg2_update(
         const uint32_t done = s1->done;
         const double rz = s1->rz;
         double tot[1];
-        all_sum<1>(dirp, gridDim.x, tot, red);
+        sums.total(gridDim.x, tot, red);
         if (done) return;
         alpha = rz / tot[0];
         if (blockIdx.x == 0 && threadIdx.x == 0) s0->alpha = alpha;
@@ -1407,6 +1415,8 @@ __global__ __launch_bounds__(BLOCK) void k_fcg2_dots(const float2* __restrict__ 
     const Chunk c = my_chunk(n);
     const size_t i = c.beg + threadIdx.x;
     const bool valid = i < c.end;
+    AllSum<1> sums;
+    sums.load(rrp, gridDim.x);
     double2 zz{}, wv{}, rv{};
     if (valid) {
         zz = z_unscaled(z, dis, i);
@@ -1417,7 +1427,7 @@ __global__ __launch_bounds__(BLOCK) void k_fcg2_dots(const float2* __restrict__ 
     const uint32_t k = first ? s1->k : s1->k + 1u;
     const double tol2 = s1->tol2;
     double tot[1];
-    all_sum<1>(rrp, gridDim.x, tot, red);
+    sums.total(gridDim.x, tot, red);
     if (ended) return;   // (s0 holds the end of the solve)
     const double gg = tot[0];
     const bool met = !(gg > tol2), stop = met || k >= max_iter || !isfinite(gg);
