@@ -1047,12 +1047,16 @@ static void launch_cheb_step64(uint32_t k, uint32_t last, unsigned G, hipStream_
 // once), each thread keeps its row (the fp16 values widened to FP32, 16-bit
 // positions), residual and z in registers, and a step costs one barrier.
 // Halo rows are computed by every tile that lists them.
-// Bound by the FP64 pipe and the barriers on small systems (1.8 us per step
+// Bound by the FP64 pipe and the barriers on small systems (1.35 us per step
 // at 33k nodes, outer kernels included, against 4.9), by bytes on large ones
 // (about 63 B per node and step against 105: 24.0 against 36.5 us at 2.1M
-// nodes).  Row values held in FP64 registers take 85 VGPRs instead of 63 and
-// leave 5 waves per SIMD instead of 8 (28 us at 2.1M), held as packed fp16
-// they cost a second conversion per product (24.2 us).
+// nodes).  Where one tile a CU is all there is, the row's values are widened to
+// FP64 once, which saves 24 conversions of some 66 FP64 operations a row and
+// step (33k nodes 59.1 -> 54.9 us per outer iteration); that takes 84 VGPRs
+// instead of 62 and leaves 5 waves per SIMD instead of 8, so more tiles hold
+// FP32 (2.1M nodes: 24.0 against 28 us a step, 45k in 283 tiles 71.6 against
+// 80.3 per outer iteration).  Held as packed fp16 they cost a second
+// conversion per product (24.2 us).
 // The arithmetic of a row is k_cheb_step64's: the same sums in the same
 // order, an fp16 value times an FP32 entry being exact in FP64, so that the
 // fused multiply-add rounds as the separate add does.  Results are the same
@@ -1064,7 +1068,8 @@ struct ChebSteps {
     uint32_t steps, k0, last;   // steps k0 .. k0 + steps - 1 of 1 .. last
     double c1[CHEB_SMAX], c2[CHEB_SMAX];
 };
-template <int W, bool FULL>
+// V: the components that a row's values are held in.
+template <int W, bool FULL, class V>
 __global__ __launch_bounds__(1024) void k_cheb_tiles(Off16 O, Tiles T, ChebSteps cs,
                                                      const float2* __restrict__ din,
                                                      float2* __restrict__ dout,
@@ -1096,7 +1101,8 @@ __global__ __launch_bounds__(1024) void k_cheb_tiles(Off16 O, Tiles T, ChebSteps
     // a row of ring r takes part in the first S - r steps
     uint32_t act = 0;
     for (uint32_t r = 0; r < S; ++r) act += i < (uint32_t)__builtin_amdgcn_readlane(ro, r);
-    fv4 av[W];
+    typedef V V4 __attribute__((ext_vector_type(4)));
+    V4 av[W];
     hv2 od = {};
     float2 rs = {}, zv = {};
     int len = W;
@@ -1119,7 +1125,7 @@ __global__ __launch_bounds__(1024) void k_cheb_tiles(Off16 O, Tiles T, ChebSteps
             for (int k = 0; k < W; ++k)
                 if (FULL || k < len) {
                     const hv4 h = val[g + (size_t)k * SLICE];
-                    av[k] = fv4{(float)h.x, (float)h.y, (float)h.z, (float)h.w};
+                    av[k] = V4{(V)h.x, (V)h.y, (V)h.z, (V)h.w};
                 }
             od = reinterpret_cast<const hv2*>(O.od)[v];
             rs = rin[v];
@@ -1141,7 +1147,7 @@ __global__ __launch_bounds__(1024) void k_cheb_tiles(Off16 O, Tiles T, ChebSteps
                 if (FULL || q < len) {
                     const double2 xv = d[(pc[q / 2] >> (16 * (q & 1))) & 0xffffu];
                     // (opaque per step, or FP64 copies of the row are hoisted)
-                    asm volatile("" : "+v"(av[q]));
+                    if constexpr (sizeof(V) == 4) asm volatile("" : "+v"(av[q]));
                     s0 = fma((double)av[q].x, xv.x, s0);
                     s0 = fma((double)av[q].y, xv.y, s0);
                     s1 = fma((double)av[q].z, xv.x, s1);
@@ -1177,12 +1183,15 @@ static void launch_cheb_tiles(const Off16& O, const Tiles& T, const ChebSteps& c
                               float2* z, const PcgState* st, hipStream_t s) {
     const dim3 g(T.n), b(T.ext);
     const size_t lds = 2 * (size_t)T.ext * sizeof(double2);
-    if (O.width == 6)
-        hipLaunchKernelGGL((k_cheb_tiles<6, true>), g, b, lds, s, O, T, cs, din, dout, rin, rout, z,
-                           st);
-    else
-        hipLaunchKernelGGL((k_cheb_tiles<TILE_WMAX, false>), g, b, lds, s, O, T, cs, din, dout, rin,
+    if (O.width == 6 && T.n <= NUM_CU)
+        hipLaunchKernelGGL((k_cheb_tiles<6, true, double>), g, b, lds, s, O, T, cs, din, dout, rin,
                            rout, z, st);
+    else if (O.width == 6)
+        hipLaunchKernelGGL((k_cheb_tiles<6, true, float>), g, b, lds, s, O, T, cs, din, dout, rin,
+                           rout, z, st);
+    else
+        hipLaunchKernelGGL((k_cheb_tiles<TILE_WMAX, false, float>), g, b, lds, s, O, T, cs, din,
+                           dout, rin, rout, z, st);
 }
 
 // One V-cycle of the multigrid preconditioner whose finest level is

@@ -244,30 +244,54 @@ int tiles_build(Tiles& T, const Off16& O, uint32_t wmax, const double2* xy, hipS
     if (!(Lx >= 0.0) || !(Ly >= 0.0) || !std::isfinite(Lx) || !std::isfinite(Ly) ||
         !(Lx + Ly > 0.0))
         return done(NBX_OK);
-    // Owned nodes per tile and rings (= steps per launch).  Up to about 64k
-    // nodes launches and load latency bound a step, and many short launches
-    // are joined; above 160k the bytes do, and fewer rings read less halo.
-    // us per step of the default solve, outer kernels included, one step per
-    // launch -> (owned, rings): 33k nodes 4.9 -> 1.9 at (128, 8), 2.6 at
-    // (256, 3); 45k 4.9 -> 1.8 at (192, 8); 124k 5.3 -> 2.8 at (256, 5), 3.2 at
-    // (256, 3); 525k 12.3 -> 7.2 at (256, 3), 7.8 at (256, 4); 2.1M 36.5 ->
-    // 24.0 at (256, 3), 28.6 at (256, 4), 29 at (192, 4).
-    const uint32_t rings0 = n <= 65536 ? 8 : n <= 163840 ? 5 : 3;
-    const uint32_t own0 = n <= 65536 ? 160 : 256;
+    // Tiles and rings (= steps per launch).  A launch takes as long as its
+    // fullest CU, so the tiles are as many as run at once, or twice that, with
+    // as many rings as a tile's TILE_TB rows leave room for; from 540k nodes
+    // bytes bound a step, and 256 nodes with three rings read least per node.
+    // At once: 256 tiles (one a CU: a row's values in FP64 registers, or the
+    // rows of up to TILE_WMAX blocks), or 512 (two a CU, values in FP32).
+    // us per outer iteration of the default solve (39 steps), with about 160 or
+    // 256 owned nodes and 8, 5 or 3 rings before -> now.  Rows of six blocks,
+    // 256 tiles: 64x32 54.9 -> 43.5, 150x75 56.7 -> 46.0, 256x128 58.9 -> 52.9,
+    // 300x150 71.3 -> 55.8, 400x200 89.6 -> 73.4 (78.0 with 512 tiles); 512
+    // tiles: 450x225 93.2 -> 85.6, 501x247 97.4 -> 93.9 (95 with 256), 570x285
+    // 128 -> 104, 700x350 158 -> 131, 800x400 196 -> 180; 1,024: 900x450 271 ->
+    // 249, 1024x512 279 -> 268; 2048x1024 937 (979 in rounds of 512).  Longer
+    // rows: 33k nodes 74.5 -> 73.8, 80k 151 -> 97, 136k 230 -> 127, 193k 325 ->
+    // 207.
+    const bool six = O.width == 6;
+    uint32_t tiles = 256;
+    if (six && n > 98304) tiles = n <= 512 * 640 ? 512 : 1024;
+    if (!six && n > 256 * 640) tiles = 512;
+    uint32_t own0 = std::max((n + tiles - 1) / tiles, 16u), rings0 = 3;
+    if (n > (six ? 1024 : 512) * 528u) {
+        own0 = 256;
+        tiles = (n + own0 - 1) / own0;
+    } else {
+        // the rows of r rings around a square of own0 nodes of a triangle mesh
+        auto rows = [&](uint32_t r) { return own0 + 4.0 * r * sqrt((double)own0) + 3.0 * r * r; };
+        while (rings0 < 8 && rows(rings0 + 1) <= TILE_TB) ++rings0;
+    }
+    const uint32_t cells0 = std::max(std::min(tiles, n / own0), 1u);
     if (hipMalloc(&cell, (size_t)n * 4) != hipSuccess ||
         hipMalloc(&own, (size_t)n * 4) != hipSuccess || hipMalloc(&info, 16) != hipSuccess)
         return no_memory();
     const uint32_t W2 = (wmax + 1) / 2;
     // A mesh of uneven density, or with wider rows, can outgrow TILE_TB in a
-    // few cells: smaller cells with fewer rings then.
-    for (uint32_t attempt = 0; attempt < 3; ++attempt) {
-        const uint32_t rings = std::max(rings0 >> attempt, 2u);
-        const double cells = std::max(1.0, (double)n / (double)(own0 >> attempt));
-        // square cells
-        const double h = Lx > 0.0 && Ly > 0.0 ? sqrt(Lx * Ly / cells) : (Lx + Ly) / cells;
-        const double fx = std::max(1.0, std::round(Lx / h));
-        const double fy = std::max(1.0, std::round(Ly / h));
-        if (!(fx * fy <= 4.0 * cells + 16.0)) return done(NBX_OK);   // a sliver of a mesh
+    // few cells: fewer rings then, and more cells.
+    const struct { uint32_t cells, rings; } attempts[] = {{cells0, rings0},
+                                                          {cells0, rings0 - 1},
+                                                          {cells0, rings0 / 2},
+                                                          {2 * cells0, rings0 / 2},
+                                                          {4 * cells0, rings0 / 4}};
+    for (const auto& at : attempts) {
+        const uint32_t rings = std::max(at.rings, 2u);
+        // at most so many cells, about square
+        const double cells = (double)at.cells;
+        const double fx = Lx > 0.0 && Ly > 0.0
+                              ? std::min(std::max(1.0, std::round(sqrt(cells * Lx / Ly))), cells)
+                              : (Lx > 0.0 ? cells : 1.0);
+        const double fy = Ly > 0.0 ? std::max(1.0, std::floor(cells / fx)) : 1.0;
         TileGrid g{lo[0], lo[1], Lx > 0.0 ? fx / Lx : 0.0, Ly > 0.0 ? fy / Ly : 0.0,
                    (uint32_t)fx, (uint32_t)fy};
         const uint32_t nt = g.nx * g.ny;

@@ -76,10 +76,11 @@ def test_tiles_equal_single_steps(mesh, degree):
     f.destroy()
 
 
-@pytest.mark.parametrize("n", [(362, 181), (363, 181), (570, 287)])
+@pytest.mark.parametrize("n", [(362, 181), (363, 181), (442, 220), (446, 220), (570, 287),
+                               (811, 403), (810, 402)])
 def test_tiles_equal_single_steps_at_the_rules_edges(n):
-    """Either side of 65,536 nodes and beyond 163,840 (other tile sizes and
-    ring counts): a solve of two outer iterations."""
+    """Around 65,536, 98,304, 163,840 and 327,680 nodes (tile counts, ring
+    counts and the form of the rows' values): two outer iterations."""
     import nbots_amd as nb
     from nbots_amd.fem import Fem, SOLVE_MIXED
     p = _grid(*n)
