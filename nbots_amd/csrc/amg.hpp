@@ -90,8 +90,7 @@ constexpr int amg_level_degree(size_t l) {
 }
 constexpr uint32_t AMG_COARSEST = 200; // unknowns of the directly solved level
 constexpr int AMG_MAX_LEVELS = 12;
-static_assert(AMG_FINE_DEGREE >= 1 && AMG_FINE_DEGREE <= AMG_MAX_DEGREE,
-              "AmgFine holds the coefficients of at most AMG_MAX_DEGREE steps");
+static_assert(AMG_FINE_DEGREE == 1, "the finest level's kernels (k_amg_residual, k_amg_post)");
 static_assert(AMG_LEVEL1_DEGREE >= 2 && AMG_LEVEL2_DEGREE >= 2 && AMG_DEGREE >= 2 &&
               AMG_LEVEL1_DEGREE <= AMG_MAX_DEGREE && AMG_LEVEL2_DEGREE <= AMG_MAX_DEGREE &&
               AMG_DEGREE <= AMG_MAX_DEGREE,

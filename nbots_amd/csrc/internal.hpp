@@ -156,8 +156,6 @@ uint32_t amg_levels(const AmgDev* a);
 struct AmgFine {
     bool scaled16 = false;
     double inv_theta = 0.0;
-    double c1[8] = {}, c2[8] = {};   // steps 1 .. degree - 1
-    uint32_t degree = 0;
     float* c = nullptr;              // [finest n]
 };
 AmgFine amg_fine(const AmgDev* a);

@@ -351,9 +351,9 @@ __device__ __forceinline__ double2 row16d(const Sell2& A, uint32_t v, const floa
 // two blocks, instead of A.bcol.
 // U: the uniform-width layout (A.width > 0), whose rows run over the full
 // width, padding included (value 0, column v: adds 0).
-template <bool NT, bool P, bool U = false>
-__device__ __forceinline__ double2 row16od(const Off16& A, uint32_t v, const float2* __restrict__ x,
-                                           float2 xo) {
+// x: a vector, or one scaled as it is read (Scaled32).
+template <bool NT, bool P, bool U = false, class X>
+__device__ __forceinline__ double2 row16od(const Off16& A, uint32_t v, X x, float2 xo) {
     const size_t base = U ? (size_t)(v >> 6) * SLICE * A.width + (v & 63)
                           : (size_t)A.slice_ptr[v >> 6] + (v & 63);
     const int len = U ? (int)A.width : (int)A.rowlen[v];
@@ -412,33 +412,40 @@ __device__ __forceinline__ double2 row16od(const Off16& A, uint32_t v, const flo
     return make_double2(s0, s1);
 }
 
+// x[i] s
+struct Scaled32 {
+    const float2* __restrict__ x;
+    float s;
+    __device__ __forceinline__ float2 operator[](size_t i) const {
+        const float2 v = x[i];
+        return make_float2(v.x * s, v.y * s);
+    }
+};
+
 // the Chebyshev step's row on either fp16 layout
 template <bool NT>
 __device__ __forceinline__ double2 cheb_row(const Sell2& A, uint32_t v, const float2* __restrict__ x,
                                             float2) {
     return row16d<NT>(A, v, x);
 }
-template <bool NT>
-__device__ __forceinline__ double2 cheb_row(const Off16& A, uint32_t v, const float2* __restrict__ x,
-                                            float2 xo) {
+template <bool NT, class X>
+__device__ __forceinline__ double2 cheb_row(const Off16& A, uint32_t v, X x, float2 xo) {
     return row16od<NT, false>(A, v, x, xo);
 }
 // the copy without diagonal blocks read through its packed column deltas
 struct Off16P {
     Off16 O;
 };
-template <bool NT>
-__device__ __forceinline__ double2 cheb_row(const Off16P& A, uint32_t v, const float2* __restrict__ x,
-                                            float2 xo) {
+template <bool NT, class X>
+__device__ __forceinline__ double2 cheb_row(const Off16P& A, uint32_t v, X x, float2 xo) {
     return row16od<NT, true>(A.O, v, x, xo);
 }
 // ... in the uniform-width layout
 struct Off16U {
     Off16 O;
 };
-template <bool NT>
-__device__ __forceinline__ double2 cheb_row(const Off16U& A, uint32_t v, const float2* __restrict__ x,
-                                            float2 xo) {
+template <bool NT, class X>
+__device__ __forceinline__ double2 cheb_row(const Off16U& A, uint32_t v, X x, float2 xo) {
     return row16od<NT, true, true>(A.O, v, x, xo);
 }
 

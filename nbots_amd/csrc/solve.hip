@@ -881,7 +881,7 @@ __global__ __launch_bounds__(BLOCK) void k_mix_update(double2* __restrict__ u,
 
 // first: r = b - K x; otherwise x += alpha p, r -= alpha w.  Then the
 // preconditioner's start, P = float2 (scaled, FP32): s = fl32(dis r),
-// res = s, d = z = s / theta; P = double2 (unscaled, FP64): res = r,
+// res = s, d = z = s / theta (d null: neither); P = double2 (unscaled, FP64): res = r,
 // d = z = D^-1 r / theta.
 template <class P>
 __global__ __launch_bounds__(BLOCK) void k_fcg_update(Sell2 K, const double2* __restrict__ b,
@@ -916,9 +916,11 @@ __global__ __launch_bounds__(BLOCK) void k_fcg_update(Sell2 K, const double2* __
             const float2 sv = make_float2((float)(dd.x * rv.x), (float)(dd.y * rv.y));
             const float it = (float)inv_theta;
             res[i] = sv;
-            const float2 dv = make_float2(sv.x * it, sv.y * it);
-            d[i] = dv;
-            z[i] = dv;
+            if (d) {
+                const float2 dv = make_float2(sv.x * it, sv.y * it);
+                d[i] = dv;
+                z[i] = dv;
+            }
         } else {
             res[i] = rv;
             const double2 dv = make_double2(dd.x * dd.x * rv.x * inv_theta,
@@ -1194,38 +1196,6 @@ static void launch_cheb_tiles(const Off16& O, const Tiles& T, const ChebSteps& c
                            dout, rin, rout, z, st);
 }
 
-// One V-cycle of the multigrid preconditioner whose finest level is
-// smoothed on the fp16 scaled copy K~ = D^-1/2 K D^-1/2, in scaled variables
-// (z~ = D^1/2 z, res~ = D^-1/2 res): Chebyshev smoothing in K~ is Chebyshev
-// smoothing in D^-1 K.  On entry the flexible-CG update has written
-// res = r~, din = r~ / theta, z = din (the first smoothing step from 0).
-//   pre-smoothing: steps 1 .. degree - 1;
-//   res = r~ - K~ z (a step with c1 = c2 = 0 completes the residual);
-//   c = P~ M_c^-1 P~^T res, the coarse levels' V-cycle (P~ = D^1/2 P);
-//   post-smoothing from z + c: its first step takes res -= K~ c,
-//   d = res / theta, z += c + d; then steps 1 .. degree - 1.
-template <bool NT, class M>
-static void amg16_cycle(const M& K, const AmgFine& f, AmgDev* amg, float2* res, float2* da,
-                        float2* db, float2* z, PcgState* st, uint32_t nu, unsigned G,
-                        hipStream_t s) {
-    const uint32_t last = f.degree - 1;
-    auto smooth = [&]() {
-        float2 *din = da, *dout = db;
-        for (uint32_t k = 1; k <= last; ++k) {
-            launch_cheb_step64<NT>(k, last, G, s, K, din, dout, res, z, st, nu, f.c1[k], f.c2[k]);
-            std::swap(din, dout);
-        }
-        return din;
-    };
-    const float2* dl = smooth();
-    hipLaunchKernelGGL((k_cheb_step64<NT, Z_SKIP, M>), dim3(G), dim3(BLOCK), 0, s, K, dl,
-                       dl == da ? db : da, res, z, st, nu, 0.0, 0.0);
-    (void)amg_coarse_correction(amg, (const float*)res, f.c, st, s);
-    hipLaunchKernelGGL((k_cheb_step64<NT, Z_PAIR, M>), dim3(G), dim3(BLOCK), 0, s, K,
-                       (const float2*)f.c, da, res, z, st, nu, 0.0, f.inv_theta);
-    (void)smooth();
-}
-
 // One step of the all-FP64 preconditioner (precond_bits = 64): the same
 // Chebyshev recurrence on the FP64 matrix itself (the symmetric copy the
 // FP64 products read, or the full one), vectors and arithmetic in FP64, in
@@ -1401,17 +1371,44 @@ __global__ __launch_bounds__(BLOCK) void k_fcg2_update(
         const float2 sv = make_float2((float)(dd.x * rv.x), (float)(dd.y * rv.y));
         const float it = (float)inv_theta;
         res[i] = sv;
-        const float2 dv = make_float2(sv.x * it, sv.y * it);
-        dz[i] = dv;
-        z[i] = dv;
+        if (dz) {
+            const float2 dv = make_float2(sv.x * it, sv.y * it);
+            dz[i] = dv;
+            z[i] = dv;
+        }
         acc[0] += rv.x * rv.x + rv.y * rv.y;
     }
     block_sum<1>(acc, red2);
     put_partials<1>(acc, rrp);
 }
 
-// The stop test on r.r (as k_fin_fcg_update); z64 = dis z for the next
-// direction; partials z64.w and r.z64.
+// The stop test on r.r (as k_fin_fcg_update); false when the solve has ended
+__device__ __forceinline__ bool fcg2_goes_on(PcgState* s0, const PcgState* __restrict__ s1,
+                                             const AllSum<1>& sums, double (&tot)[1],
+                                             double (*red)[ALL_PARTS / WAVE], bool first) {
+    const uint32_t ended = s1->done, max_iter = s1->max_iter;
+    const uint32_t k = first ? s1->k : s1->k + 1u;
+    const double tol2 = s1->tol2;
+    sums.total(gridDim.x, tot, red);
+    if (ended) return false;   // (s0 holds the end of the solve)
+    const double gg = tot[0];
+    const bool met = !(gg > tol2), stop = met || k >= max_iter || !isfinite(gg);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        s0->k = k;
+        s0->max_iter = max_iter;
+        s0->tol2 = tol2;
+        s0->gg0 = first ? gg : s1->gg0;
+        s0->gg_cur = gg;
+        s0->tol_reached = sqrt(gg);
+        s0->rz = s1->rz;
+        s0->breakdown = s1->breakdown;
+        s0->done = stop ? 1u : 0u;
+        s0->status = met ? 0u : 1u;
+    }
+    return !stop;
+}
+
+// ... and z64 = dis z for the next direction; partials z64.w and r.z64.
 __global__ __launch_bounds__(BLOCK) void k_fcg2_dots(const float2* __restrict__ z,
                                                      const double2* __restrict__ dis,
                                                      const double2* __restrict__ w,
@@ -1432,27 +1429,90 @@ __global__ __launch_bounds__(BLOCK) void k_fcg2_dots(const float2* __restrict__ 
         if (!first) wv = w[i];
         rv = r[i];
     }
-    const uint32_t ended = s1->done, max_iter = s1->max_iter;
-    const uint32_t k = first ? s1->k : s1->k + 1u;
-    const double tol2 = s1->tol2;
     double tot[1];
-    sums.total(gridDim.x, tot, red);
-    if (ended) return;   // (s0 holds the end of the solve)
-    const double gg = tot[0];
-    const bool met = !(gg > tol2), stop = met || k >= max_iter || !isfinite(gg);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        s0->k = k;
-        s0->max_iter = max_iter;
-        s0->tol2 = tol2;
-        s0->gg0 = first ? gg : s1->gg0;
-        s0->gg_cur = gg;
-        s0->tol_reached = sqrt(gg);
-        s0->rz = s1->rz;
-        s0->breakdown = s1->breakdown;
-        s0->done = stop ? 1u : 0u;
-        s0->status = met ? 0u : 1u;
+    if (!fcg2_goes_on(s0, s1, sums, tot, red, first)) return;
+    double acc[2] = {0.0, 0.0};
+    if (valid) {
+        d[i].q = zz;
+        if (!first) acc[0] += dotu(zz, wv);
+        acc[1] += dotu(rv, zz);
     }
-    if (stop) return;
+    block_sum<2>(acc, red2);
+    put_partials<2>(acc, dots);
+}
+
+// One V-cycle of the multigrid preconditioner whose finest level is
+// smoothed on the fp16 scaled copy K~ = D^-1/2 K D^-1/2, in scaled variables
+// (z~ = D^1/2 z, res~ = D^-1/2 res): Chebyshev smoothing of degree 1 in K~ is
+// that in D^-1 K.  The flexible-CG update leaves res = r~ alone; then
+//   k_amg_residual  r1 = r~ - K~ z0, the first smoothing step z0 = r~ / theta
+//                   formed from r~ wherever it is read;
+//   the coarse levels  c = P~ M_c^-1 P~^T r1 (P~ = D^1/2 P);
+//   k_amg_post      z = z0 + c + d with d = (r1 - K~ c) / theta, the post-
+//                   smoothing; k_amg_post2 does k_fcg2_dots's work as well.
+// As steps of the general Chebyshev kernel these wrote z0 and d, a direction
+// of zeros and the last residual: 84 MB more at 2.1M nodes (598 -> 587 us per
+// outer iteration).  Up to 262,144 nodes, where a launch costs 3.3 us: 64x32
+// 43.4 -> 41.5, 96x48 58.4 -> 55.1, 150x75 67.8 -> 64.2, 512x256 141 -> 135.
+// The dot products in k_amg_post of the large systems too: 603 (82 VGPRs, or
+// their vectors' loads after the product).
+template <bool NT, class M>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_amg_residual(M K, const float2* __restrict__ res,
+                                                        float2* __restrict__ r1, float it,
+                                                        const PcgState* __restrict__ st,
+                                                        uint32_t n) {
+    if (st->done) return;
+    const Chunk c = my_chunk(n);
+    for (size_t i = c.beg + threadIdx.x; i < c.end; i += BLOCK) {
+        const float2 r0 = res[i];
+        const double2 t = cheb_row<NT>(K, (uint32_t)i, Scaled32{res, it},
+                                       make_float2(r0.x * it, r0.y * it));
+        r1[i] = make_float2((float)((double)r0.x - t.x), (float)((double)r0.y - t.y));
+    }
+}
+template <bool NT, class M>
+__device__ __forceinline__ float2 amg_post_row(const M& K, size_t i, const float2* __restrict__ cc,
+                                               float2 r0, float2 r1, double inv_theta) {
+    const float it = (float)inv_theta;
+    const float2 ci = cc[i];
+    const double2 t = cheb_row<NT>(K, (uint32_t)i, cc, ci);
+    const double dx = inv_theta * ((double)r1.x - t.x), dy = inv_theta * ((double)r1.y - t.y);
+    return make_float2((float)((double)(r0.x * it) + ((double)ci.x + dx)),
+                       (float)((double)(r0.y * it) + ((double)ci.y + dy)));
+}
+template <bool NT, class M>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_amg_post(
+    M K, const float2* __restrict__ cc, const float2* __restrict__ res,
+    const float2* __restrict__ r1, float2* __restrict__ z, const PcgState* __restrict__ st,
+    uint32_t n, double inv_theta) {
+    if (st->done) return;
+    const Chunk c = my_chunk(n);
+    for (size_t i = c.beg + threadIdx.x; i < c.end; i += BLOCK)
+        z[i] = amg_post_row<NT>(K, i, cc, res[i], r1[i], inv_theta);
+}
+template <bool NT, class M>
+__global__ __launch_bounds__(BLOCK) void k_amg_post2(
+    M K, const float2* __restrict__ cc, const float2* __restrict__ res,
+    const float2* __restrict__ r1, const double2* __restrict__ dis, const double2* __restrict__ w,
+    const double2* __restrict__ r, CgPair<double2>* __restrict__ d, PcgState* s0,
+    const PcgState* __restrict__ s1, const double* __restrict__ rrp, double* dots, uint32_t n,
+    bool first, double inv_theta) {
+    __shared__ double red[1][ALL_PARTS / WAVE], red2[2][BLOCK / WAVE];
+    const Chunk c = my_chunk(n);
+    const size_t i = c.beg + threadIdx.x;
+    const bool valid = i < c.end;
+    AllSum<1> sums;
+    sums.load(rrp, gridDim.x);
+    double2 zz{}, wv{}, rv{};
+    if (valid) {
+        const double2 dd = dis[i];
+        if (!first) wv = w[i];
+        rv = r[i];
+        const float2 zv = amg_post_row<NT>(K, i, cc, res[i], r1[i], inv_theta);
+        zz = make_double2(dd.x * (double)zv.x, dd.y * (double)zv.y);
+    }
+    double tot[1];
+    if (!fcg2_goes_on(s0, s1, sums, tot, red, first)) return;
     double acc[2] = {0.0, 0.0};
     if (valid) {
         d[i].q = zz;
@@ -2093,19 +2153,21 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
     const bool fine_cached = fine_mat + 41.0 * (double)nu <= (double)INFINITY_CACHE_BYTES;
     // What precedes and follows the preconditioner in the step that leaves
     // z_j (first: z_0); dscale: the diagonal scaling (ones: none).
-    auto before = [&](int first, uint32_t j, const double2* dscale, double theta_inv) {
+    // d0, z0: where the preconditioner's first direction goes, or null.
+    auto before = [&](int first, uint32_t j, const double2* dscale, double theta_inv, float2* d0,
+                      float2* z0) {
         if (!fold) {
             hipLaunchKernelGGL(k_fcg_update<float2>, dim3(G), dim3(BLOCK), 0, s, m.s, bv, xv, r, p,
-                               wv, dscale, res, da, z, w.st, w.partials, nu, first, theta_inv);
+                               wv, dscale, res, d0, z0, w.st, w.partials, nu, first, theta_inv);
             hipLaunchKernelGGL(k_fin_fcg_update, dim3(1), dim3(FIN), 0, s, w.st, w.partials, G,
                                first);
         } else if (first) {
             hipLaunchKernelGGL(k_fcg2_update<true>, dim3(G), dim3(BLOCK), 0, s, m.s, bv, xv, r,
-                               pair[j & 1], wv, dscale, res, da, z, w.st, stp, dirp, rrp, nu,
+                               pair[j & 1], wv, dscale, res, d0, z0, w.st, stp, dirp, rrp, nu,
                                theta_inv);
         } else {
             hipLaunchKernelGGL(k_fcg2_update<false>, dim3(G), dim3(BLOCK), 0, s, m.s, bv, xv, r,
-                               pair[j & 1], wv, dscale, res, da, z, w.st, stp, dirp, rrp, nu,
+                               pair[j & 1], wv, dscale, res, d0, z0, w.st, stp, dirp, rrp, nu,
                                theta_inv);
         }
     };
@@ -2122,26 +2184,42 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
                            first);
     };
     auto precondition_amg16 = [&](int first, uint32_t j) {
-        before(first, j, dis, fine.inv_theta);
-        auto cycle = [&](const auto& K) {
-            if (fine_cached)
-                amg16_cycle<false>(K, fine, m.amg, res, da, db, z, stp, nu, G, s);
-            else
-                amg16_cycle<true>(K, fine, m.amg, res, da, db, z, stp, nu, G, s);
+        before(first, j, dis, fine.inv_theta, nullptr, nullptr);
+        auto cycle = [&](auto nt, const auto& K) {
+            constexpr bool NT = decltype(nt)::value;
+            using M = std::decay_t<decltype(K)>;
+            hipLaunchKernelGGL((k_amg_residual<NT, M>), dim3(G), dim3(BLOCK), 0, s, K, res, da,
+                               (float)fine.inv_theta, stp, nu);
+            (void)amg_coarse_correction(m.amg, (const float*)da, fine.c, stp, s);
+            const float2* cc = (const float2*)fine.c;
+            if (fold) {
+                hipLaunchKernelGGL((k_amg_post2<NT, M>), dim3(G), dim3(BLOCK), 0, s, K, cc, res, da,
+                                   dis, wv, r, pair[j & 1], w.st, stp, rrp, dots, nu, first != 0,
+                                   fine.inv_theta);
+                return;
+            }
+            hipLaunchKernelGGL((k_amg_post<NT, M>), dim3(G), dim3(BLOCK), 0, s, K, cc, res, da, z,
+                               stp, nu, fine.inv_theta);
+            after(first, j, dis);
         };
-        if (m.off_packed && m.o.width)
-            cycle(Off16U{m.o});
-        else if (m.off_packed)
-            cycle(Off16P{m.o});
+        auto layout = [&](auto nt) {
+            if (m.off_packed && m.o.width)
+                cycle(nt, Off16U{m.o});
+            else if (m.off_packed)
+                cycle(nt, Off16P{m.o});
+            else
+                cycle(nt, m.o);
+        };
+        if (fine_cached)
+            layout(std::false_type{});
         else
-            cycle(m.o);
-        after(first, j, dis);
+            layout(std::true_type{});
     };
     auto precondition_amg = [&](int first, uint32_t j) {
         // a one-level hierarchy: the update with a unit scaling writes r in
         // FP32 (res), the dense solve z = C^-1 r, the dot products and
         // direction read z unscaled
-        before(first, j, ones, 1.0);
+        before(first, j, ones, 1.0, nullptr, nullptr);
         (void)amg_vcycle(m.amg, (const float*)res, (float*)z, stp, s);
         after(first, j, ones);
     };
@@ -2160,7 +2238,7 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
             hipLaunchKernelGGL(k_fin_fcg_update, dim3(1), dim3(FIN), 0, s, w.st, w.partials, G,
                                first);
         } else {
-            before(first, j, dis, inv_theta);
+            before(first, j, dis, inv_theta, da, z);
         }
         float2* din = da;
         float2* dout = db;
