@@ -687,23 +687,25 @@ __device__ __forceinline__ void keep(BellHead& h, float (&v)[R], Rest&... rest) 
     keep(h, rest...);
 }
 
-// y = (block row) x, x indexed by C per block column, by a group of LANES
-// lanes: lane l takes blocks l, l + LANES, ..., four at a time (their columns
-// and values loaded before the dependent gathers), and the group adds the
-// lanes' sums by a butterfly; every lane gets the result.
-template <int R, int C, int LANES, int DEPTH = 4>
+// y = (block row) x, x indexed by C per block column, as a group of LANES
+// lanes sums it: lane l adds blocks l, l + LANES, ..., and a butterfly the
+// lanes' sums.  PHYS lanes do it, each the sums of LANES / PHYS of them, with
+// DEPTH blocks (their columns and values) loaded before the dependent gathers;
+// every lane of the group gets the result.
+template <int R, int C, int LANES, int PHYS = LANES, int DEPTH = 4>
 __device__ __forceinline__ void bell_row(const Bell<R, C>& B, const BellHead& h, uint32_t lane,
                                          const float* __restrict__ x, float (&y)[R]) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) y[r] = 0.f;
+    constexpr int V = LANES / PHYS;
+    static_assert(DEPTH % V == 0, "a block's accumulator follows from its place");
+    float s[V][R] = {};
     const uint32_t base = h.slice + h.row;
-    for (uint32_t k0 = lane; k0 < h.len; k0 += DEPTH * LANES) {
+    for (uint32_t k0 = lane; k0 < h.len; k0 += DEPTH * PHYS) {
         uint32_t J[DEPTH];
         float a[DEPTH][R * C], xv[DEPTH][C];
 #pragma unroll
         for (int u = 0; u < DEPTH; ++u) {
-            if (k0 + u * LANES < h.len) {
-                const uint32_t sl = base + (k0 + u * LANES) * SLICE;
+            if (k0 + u * PHYS < h.len) {
+                const uint32_t sl = base + (k0 + u * PHYS) * SLICE;
                 J[u] = B.bcol[sl];
 #pragma unroll
                 for (int m = 0; m < R * C; ++m) a[u][m] = B.val[(size_t)m * B.slots + sl];
@@ -711,19 +713,25 @@ __device__ __forceinline__ void bell_row(const Bell<R, C>& B, const BellHead& h,
         }
 #pragma unroll
         for (int u = 0; u < DEPTH; ++u)
-            if (k0 + u * LANES < h.len)
+            if (k0 + u * PHYS < h.len)
 #pragma unroll
                 for (int c = 0; c < C; ++c) xv[u][c] = x[(size_t)C * J[u] + c];
 #pragma unroll
         for (int u = 0; u < DEPTH; ++u)
-            if (k0 + u * LANES < h.len)
+            if (k0 + u * PHYS < h.len)
 #pragma unroll
                 for (int r = 0; r < R; ++r)
 #pragma unroll
-                    for (int c = 0; c < C; ++c) y[r] += a[u][r * C + c] * xv[u][c];
+                    for (int c = 0; c < C; ++c) s[u % V][r] += a[u][r * C + c] * xv[u][c];
     }
 #pragma unroll
-    for (int r = 0; r < R; ++r) y[r] = group_sum<LANES>(y[r]);
+    for (int o = V / 2; o > 0; o >>= 1)
+#pragma unroll
+        for (int v = 0; v < o; ++v)
+#pragma unroll
+            for (int r = 0; r < R; ++r) s[v][r] += s[v + o][r];
+#pragma unroll
+    for (int r = 0; r < R; ++r) y[r] = group_sum<PHYS>(s[0][r]);
 }
 
 // the group's block row and lane; groups past the last row take that row
@@ -738,21 +746,21 @@ __device__ __forceinline__ void bell_row(const Bell<R, C>& B, const BellHead& h,
 // Chebyshev smoothing below the finest level, a group per aggregate (3
 // rows).  The start (r = D^-1 b, d = r / theta, x = d) rides in the
 // restriction that writes b; the post-smoothing start takes A x.
-template <int LANES>
+template <int LANES, int PHYS>
 __global__ __launch_bounds__(BLOCK) void k_bsm_init(Bell<3, 3> A, const float* __restrict__ dinv,
                                                     const float* __restrict__ b,
                                                     const float* __restrict__ x,
                                                     float* __restrict__ r, float* __restrict__ d,
                                                     float inv_theta, const PcgState* st,
                                                     uint32_t rows) {
-    BELL_ROW(LANES, rows);
+    BELL_ROW(PHYS, rows);
     BellHead h = bell_head(A, I, st);
     float ax[3], di[3], bi[3];
     load_rows(dinv, I, di);
     load_rows(b, I, bi);
     keep(h, di, bi);
     if (__builtin_amdgcn_readfirstlane(h.done)) return;
-    bell_row<3, 3, LANES>(A, h, lane, x, ax);
+    bell_row<3, 3, LANES, PHYS, (LANES / PHYS > 4 ? LANES / PHYS : 4)>(A, h, lane, x, ax);
     if (!store) return;
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
@@ -764,14 +772,14 @@ __global__ __launch_bounds__(BLOCK) void k_bsm_init(Bell<3, 3> A, const float* _
 }
 
 // r -= D^-1 A d_in; d_out = c1 d_in + c2 r; x += d_out (and d_in when ADD_IN)
-template <bool ADD_IN, int LANES>
+template <bool ADD_IN, int LANES, int PHYS>
 __global__ __launch_bounds__(BLOCK) void k_bsm_step(Bell<3, 3> A, const float* __restrict__ dinv,
                                                     const float* __restrict__ din,
                                                     float* __restrict__ dout,
                                                     float* __restrict__ r, float* __restrict__ x,
                                                     float c1, float c2, const PcgState* st,
                                                     uint32_t rows) {
-    BELL_ROW(LANES, rows);
+    BELL_ROW(PHYS, rows);
     BellHead h = bell_head(A, I, st);
     float ad[3], dv[3], d0[3], r0[3], x0[3];
     load_rows(dinv, I, dv);
@@ -780,7 +788,7 @@ __global__ __launch_bounds__(BLOCK) void k_bsm_step(Bell<3, 3> A, const float* _
     load_rows(x, I, x0);
     keep(h, dv, d0, r0, x0);
     if (__builtin_amdgcn_readfirstlane(h.done)) return;
-    bell_row<3, 3, LANES>(A, h, lane, din, ad);
+    bell_row<3, 3, LANES, PHYS, (LANES / PHYS > 4 ? LANES / PHYS : 4)>(A, h, lane, din, ad);
     if (!store) return;
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
@@ -793,18 +801,18 @@ __global__ __launch_bounds__(BLOCK) void k_bsm_step(Bell<3, 3> A, const float* _
     }
 }
 
-template <int LANES>
+template <int LANES, int PHYS>
 __global__ __launch_bounds__(BLOCK) void k_bresidual(Bell<3, 3> A, const float* __restrict__ b,
                                                      const float* __restrict__ x,
                                                      float* __restrict__ r, const PcgState* st,
                                                      uint32_t rows) {
-    BELL_ROW(LANES, rows);
+    BELL_ROW(PHYS, rows);
     BellHead h = bell_head(A, I, st);
     float ax[3], bi[3];
     load_rows(b, I, bi);
     keep(h, bi);
     if (__builtin_amdgcn_readfirstlane(h.done)) return;
-    bell_row<3, 3, LANES>(A, h, lane, x, ax);
+    bell_row<3, 3, LANES, PHYS, (LANES / PHYS > 4 ? LANES / PHYS : 4)>(A, h, lane, x, ax);
     if (!store) return;
 #pragma unroll
     for (int m = 0; m < 3; ++m) r[3 * (size_t)I + m] = bi[m] - ax[m];
@@ -812,7 +820,7 @@ __global__ __launch_bounds__(BLOCK) void k_bresidual(Bell<3, 3> A, const float* 
 
 // b_c = P^T r, a group per aggregate; INIT: also the next level's
 // smoothing start from x = 0 (r_c = D_c^-1 b_c, d_c = r_c / theta_c, x_c = d_c)
-template <int R, bool INIT, int LANES>
+template <int R, bool INIT, int LANES, int PHYS>
 __global__ __launch_bounds__(BLOCK) void k_brestrict(Bell<3, R> T, const float* __restrict__ r,
                                                      float* __restrict__ bc,
                                                      const float* __restrict__ dinv_c,
@@ -820,7 +828,7 @@ __global__ __launch_bounds__(BLOCK) void k_brestrict(Bell<3, R> T, const float* 
                                                      float* __restrict__ rc,
                                                      float* __restrict__ dc, float inv_theta_c,
                                                      const PcgState* st, uint32_t aggs) {
-    BELL_ROW(LANES, aggs);
+    BELL_ROW(PHYS, aggs);
     BellHead h = bell_head(T, I, st);
     float y[3], di[3] = {};
     if constexpr (INIT) {
@@ -830,7 +838,7 @@ __global__ __launch_bounds__(BLOCK) void k_brestrict(Bell<3, R> T, const float* 
         keep(h);
     }
     if (__builtin_amdgcn_readfirstlane(h.done)) return;
-    bell_row<3, R, LANES>(T, h, lane, r, y);
+    bell_row<3, R, LANES, PHYS, (LANES / PHYS > 4 ? LANES / PHYS : 4)>(T, h, lane, r, y);
     if (!store) return;
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
@@ -847,11 +855,11 @@ __global__ __launch_bounds__(BLOCK) void k_brestrict(Bell<3, R> T, const float* 
 }
 
 // x += P x_c (ADD), or x = P x_c; a group per node
-template <int R, bool ADD, int LANES>
+template <int R, bool ADD, int LANES, int PHYS>
 __global__ __launch_bounds__(BLOCK) void k_bprolong(Bell<R, 3> P, const float* __restrict__ xc,
                                                     float* __restrict__ x, const PcgState* st,
                                                     uint32_t rows) {
-    BELL_ROW(LANES, rows);
+    BELL_ROW(PHYS, rows);
     BellHead h = bell_head(P, I, st);
     float y[R], x0[R] = {};
     if constexpr (ADD) {
@@ -861,7 +869,7 @@ __global__ __launch_bounds__(BLOCK) void k_bprolong(Bell<R, 3> P, const float* _
         keep(h);
     }
     if (__builtin_amdgcn_readfirstlane(h.done)) return;
-    bell_row<R, 3, LANES>(P, h, lane, xc, y);
+    bell_row<R, 3, LANES, PHYS, (LANES / PHYS > 4 ? LANES / PHYS : 4)>(P, h, lane, xc, y);
     if (!store) return;
 #pragma unroll
     for (int m = 0; m < R; ++m) x[(size_t)R * I + m] = ADD ? x0[m] + y[m] : y[m];
@@ -1059,7 +1067,7 @@ __device__ __forceinline__ void bottom_apply(const Bell<3, 3>& B, uint32_t rows,
     const uint32_t lane = threadIdx.x % LANES;
     for (uint32_t I = threadIdx.x / LANES; I < rows; I += BOTTOM_TB / LANES) {
         float t[3];
-        bell_row<3, 3, LANES, 2>(B, 
+        bell_row<3, 3, LANES, LANES, 2>(B, 
                                   BellHead{B.slice_ptr[I >> 6], I & 63, B.len[I], 0}, lane, x, t);
         if (lane == 0)
 #pragma unroll
@@ -1131,6 +1139,7 @@ void amg_free(AmgDev* A) {
 }
 
 constexpr size_t BELL_SMALL = 65536;   // slots (2.6 MB)
+constexpr uint32_t BELL_LARGE = 32768;   // block rows
 
 // The block sliced-ELL pattern of `rows` block rows: len_of(I) blocks in
 // row I, col_of(I, k) the k-th block's column; uploaded with room for R x C
@@ -1391,15 +1400,28 @@ static int amg_same_entries(FemSys& S, bool* same) {
     return NBX_OK;
 }
 
-// f(integral_constant LANES) for a block layout's lanes per row
+// f(LANES, PHYS) for a block layout: the lanes a row's sum is formed by, and
+// the lanes that form it.  Large levels are bound by bytes: there one lane
+// takes a row, so that a wavefront reads 256 bytes in a row of each plane
+// instead of 32 or 64 (2048x1024: the finest restriction 51.5 -> 44 us, level
+// 1's products 5% less, 586 -> 572 us per outer iteration, 1024x512 239 -> 231).
+// Smaller levels need the wavefronts.
 template <class F>
-static void with_bl(int lanes, F&& f) {
-    switch (lanes) {
-        case 1: f(std::integral_constant<int, 1>{}); break;
-        case 2: f(std::integral_constant<int, 2>{}); break;
-        case 4: f(std::integral_constant<int, 4>{}); break;
-        case 8: f(std::integral_constant<int, 8>{}); break;
-        default: f(std::integral_constant<int, 16>{}); break;
+static void with_bl(const BellDev& B, F&& f) {
+    std::integral_constant<int, 1> one;
+    const bool large = B.rows >= BELL_LARGE;
+    auto go = [&](auto ln) {
+        if (large)
+            f(ln, one);
+        else
+            f(ln, ln);
+    };
+    switch (B.lanes) {
+        case 1: f(one, one); break;
+        case 2: go(std::integral_constant<int, 2>{}); break;
+        case 4: go(std::integral_constant<int, 4>{}); break;
+        case 8: go(std::integral_constant<int, 8>{}); break;
+        default: f(std::integral_constant<int, 16>{}, std::integral_constant<int, 16>{}); break;
     }
 }
 // f(integral_constant R) for a level's rows per node
@@ -1611,15 +1633,15 @@ static void restrict_to(AmgDev* A, size_t l, const float* r, const PcgState* st,
     const bool init = l + 2 < A->lv.size() && l + 1 != A->bottom;
     with_bs(V.bs, [&](auto R) {
         constexpr int RR = decltype(R)::value;
-        with_bl(V.tb.lanes, [&](auto ln) {
-            constexpr int LN = decltype(ln)::value;
-            const unsigned g = grid_for((size_t)V.tb.rows * LN);
+        with_bl(V.tb, [&](auto ln, auto ph) {
+            constexpr int LN = decltype(ln)::value, PH = decltype(ph)::value;
+            const unsigned g = grid_for((size_t)V.tb.rows * PH);
             if (init)
-                hipLaunchKernelGGL((k_brestrict<RR, true, LN>), dim3(g), dim3(BLOCK), 0, s,
+                hipLaunchKernelGGL((k_brestrict<RR, true, LN, PH>), dim3(g), dim3(BLOCK), 0, s,
                                    bell<3, RR>(V.tb), r, W.b, W.dinv32, W.x, W.r, W.d0,
                                    W.inv_theta, st, V.tb.rows);
             else
-                hipLaunchKernelGGL((k_brestrict<RR, false, LN>), dim3(g), dim3(BLOCK), 0, s,
+                hipLaunchKernelGGL((k_brestrict<RR, false, LN, PH>), dim3(g), dim3(BLOCK), 0, s,
                                    bell<3, RR>(V.tb), r, W.b, W.dinv32, W.x, W.r, W.d0,
                                    W.inv_theta, st, V.tb.rows);
         });
@@ -1633,14 +1655,14 @@ static void prolong_from(AmgDev* A, size_t l, float* x, bool add, const PcgState
     const float* xc = A->lv[l + 1].x;
     with_bs(V.bs, [&](auto R) {
         constexpr int RR = decltype(R)::value;
-        with_bl(V.pb.lanes, [&](auto ln) {
-            constexpr int LN = decltype(ln)::value;
-            const unsigned g = grid_for((size_t)V.pb.rows * LN);
+        with_bl(V.pb, [&](auto ln, auto ph) {
+            constexpr int LN = decltype(ln)::value, PH = decltype(ph)::value;
+            const unsigned g = grid_for((size_t)V.pb.rows * PH);
             if (add)
-                hipLaunchKernelGGL((k_bprolong<RR, true, LN>), dim3(g), dim3(BLOCK), 0, s,
+                hipLaunchKernelGGL((k_bprolong<RR, true, LN, PH>), dim3(g), dim3(BLOCK), 0, s,
                                    bell<RR, 3>(V.pb), xc, x, st, V.pb.rows);
             else
-                hipLaunchKernelGGL((k_bprolong<RR, false, LN>), dim3(g), dim3(BLOCK), 0, s,
+                hipLaunchKernelGGL((k_bprolong<RR, false, LN, PH>), dim3(g), dim3(BLOCK), 0, s,
                                    bell<RR, 3>(V.pb), xc, x, st, V.pb.rows);
         });
     });
@@ -1697,16 +1719,16 @@ static void cycle_from(AmgDev* A, size_t l0, const float* b, float* x, const Pcg
         const float* bl = l == l0 ? b : V.b;
         float* xl = l == l0 ? x : V.x;
         float *din = V.d0, *dout = V.d1;
-        with_bl(V.ab.lanes, [&](auto ln) {
-            constexpr int LN = decltype(ln)::value;
-            const unsigned g = grid_for((size_t)V.ab.rows * LN);
+        with_bl(V.ab, [&](auto ln, auto ph) {
+            constexpr int LN = decltype(ln)::value, PH = decltype(ph)::value;
+            const unsigned g = grid_for((size_t)V.ab.rows * PH);
             for (int k = 1; k < V.degree; ++k) {
-                hipLaunchKernelGGL((k_bsm_step<false, LN>), dim3(g), dim3(BLOCK), 0, s,
+                hipLaunchKernelGGL((k_bsm_step<false, LN, PH>), dim3(g), dim3(BLOCK), 0, s,
                                    bell<3, 3>(V.ab), V.dinv32, din, dout, V.r, xl, V.c1[k],
                                    V.c2[k], st, V.ab.rows);
                 std::swap(din, dout);
             }
-            hipLaunchKernelGGL(k_bresidual<LN>, dim3(g), dim3(BLOCK), 0, s, bell<3, 3>(V.ab), bl,
+            hipLaunchKernelGGL((k_bresidual<LN, PH>), dim3(g), dim3(BLOCK), 0, s, bell<3, 3>(V.ab), bl,
                                xl, V.r, st, V.ab.rows);
         });
         restrict_to(A, l, V.r, st, s);
@@ -1725,18 +1747,18 @@ static void cycle_from(AmgDev* A, size_t l0, const float* b, float* x, const Pcg
         float* xl = l == l0 ? x : V.x;
         prolong_from(A, l, xl, true, st, s);
         float *din = V.d0, *dout = V.d1;
-        with_bl(V.ab.lanes, [&](auto ln) {
-            constexpr int LN = decltype(ln)::value;
-            const unsigned g = grid_for((size_t)V.ab.rows * LN);
-            hipLaunchKernelGGL(k_bsm_init<LN>, dim3(g), dim3(BLOCK), 0, s, bell<3, 3>(V.ab),
+        with_bl(V.ab, [&](auto ln, auto ph) {
+            constexpr int LN = decltype(ln)::value, PH = decltype(ph)::value;
+            const unsigned g = grid_for((size_t)V.ab.rows * PH);
+            hipLaunchKernelGGL((k_bsm_init<LN, PH>), dim3(g), dim3(BLOCK), 0, s, bell<3, 3>(V.ab),
                                V.dinv32, bl, xl, V.r, V.d0, V.inv_theta, st, V.ab.rows);
             for (int k = 1; k < V.degree; ++k) {
                 if (k == 1)
-                    hipLaunchKernelGGL((k_bsm_step<true, LN>), dim3(g), dim3(BLOCK), 0, s,
+                    hipLaunchKernelGGL((k_bsm_step<true, LN, PH>), dim3(g), dim3(BLOCK), 0, s,
                                        bell<3, 3>(V.ab), V.dinv32, din, dout, V.r, xl, V.c1[k],
                                        V.c2[k], st, V.ab.rows);
                 else
-                    hipLaunchKernelGGL((k_bsm_step<false, LN>), dim3(g), dim3(BLOCK), 0, s,
+                    hipLaunchKernelGGL((k_bsm_step<false, LN, PH>), dim3(g), dim3(BLOCK), 0, s,
                                        bell<3, 3>(V.ab), V.dinv32, din, dout, V.r, xl, V.c1[k],
                                        V.c2[k], st, V.ab.rows);
                 std::swap(din, dout);
