@@ -58,6 +58,10 @@ struct AmgDevLevel {
     double* w64 = nullptr;
     uint32_t *pt_ptr = nullptr, *pt_row = nullptr, *pt_pos = nullptr;
     BellDev ab, pb, tb;        // the operator (below the finest level), P, P^T
+    // tiles for the level's smoothing in two launches, or none; the cycle then
+    // leaves its correction in d0 instead of x
+    Tiles tiles;
+    float* out() const { return tiles.n ? d0 : x; }
     // V-cycle vectors: right-hand side and solution of this level (the
     // finest level's come from the caller), residual, two directions
     float *b = nullptr, *x = nullptr, *r = nullptr, *d0 = nullptr, *d1 = nullptr;
@@ -928,12 +932,37 @@ struct Bottom {
 // row I, q = r rows + I = threadIdx.x + 512 j
 template <int RP, int HELD, int LANES>   // HELD: blocks of a row, none longer
 struct BottomRows {
-    uint32_t i[RP];   // the scalar row 3 I + r, or none
+    uint32_t i[RP];   // the scalar row's place in LDS (3 I + r), or none
     float dinv[RP];
     static constexpr uint32_t NO_ROW = 0xffffffffu;
     __device__ __forceinline__ bool on(int j) const { return i[j] != NO_ROW; }
     float v[RP][HELD][3];
-    uint32_t col[RP][HELD / 2];   // two 16-bit positions (3 J) per word
+    uint32_t col[RP][HELD / 2];   // two 16-bit places (3 J) per word
+    // component r of block row I into row j: its values, and with COLS the
+    // columns as they stand
+    template <bool COLS>
+    __device__ __forceinline__ void load_row(const BottomLevel& L, int j, uint32_t I, uint32_t r,
+                                             bool valid) {
+        dinv[j] = valid ? L.dinv[3 * (size_t)I + r] : 0.f;
+        size_t base = (size_t)(I >> 6) * SLICE * L.A.width + (I & 63);
+        int len = valid ? (int)L.A.width : 0;
+        if (valid && !L.A.width) {
+            base = (size_t)L.A.slice_ptr[I >> 6] + (I & 63);
+            len = L.A.len[I];
+        }
+#pragma unroll
+        for (int k = 0; k < HELD; ++k) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) v[j][k][c] = 0.f;
+            if (k < len) {
+                const size_t sl = base + (size_t)k * SLICE;
+                if constexpr (COLS) col[j][k / 2] |= (3 * L.A.bcol[sl]) << (16 * (k & 1));
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    v[j][k][c] = L.A.val[(size_t)(3 * r + c) * L.A.slots + sl];
+            }
+        }
+    }
     __device__ __forceinline__ void load(const BottomLevel& L) {
 #pragma unroll
         for (int j = 0; j < RP; ++j) {
@@ -941,23 +970,9 @@ struct BottomRows {
             const uint32_t r = q / L.rows, I = q - r * L.rows;
             const bool valid = r < 3;
             i[j] = valid ? 3 * I + r : NO_ROW;
-            dinv[j] = valid ? L.dinv[i[j]] : 0.f;
-            const size_t base = valid ? (size_t)L.A.slice_ptr[I >> 6] + (I & 63) : 0;
-            const int len = valid ? L.A.len[I] : 0;
 #pragma unroll
             for (int k = 0; k < HELD / 2; ++k) col[j][k] = 0;
-#pragma unroll
-            for (int k = 0; k < HELD; ++k) {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) v[j][k][c] = 0.f;
-                if (k < len) {
-                    const size_t sl = base + (size_t)k * SLICE;
-                    col[j][k / 2] |= (3 * L.A.bcol[sl]) << (16 * (k & 1));
-#pragma unroll
-                    for (int c = 0; c < 3; ++c)
-                        v[j][k][c] = L.A.val[(size_t)(3 * r + c) * L.A.slots + sl];
-                }
-            }
+            load_row<true>(L, j, I, r, valid);
         }
     }
     // (A x) of row j, summed as bell_row's LANES lanes sum it
@@ -1114,6 +1129,163 @@ __global__ __launch_bounds__(BOTTOM_TB) void k_amg_bottom(Bottom B, const PcgSta
     for (uint32_t i = threadIdx.x; i < n; i += BOTTOM_TB) B.x[i] = v.x[i];
 }
 
+// ---- a level between the finest and the bottom, on tiles ------------------------
+// Such a level takes 2 degree + 3 launches of one step each per cycle. On tiles
+// (tiles.hip) of its graph with `degree` rings it takes two, with the
+// restriction between them: k_amg_down all steps before the coarse correction
+// and the residual, k_amg_up the prolongation and all steps after.  A tile's
+// rows are held as k_amg_bottom holds its own; a step is taken on the rows whose
+// neighbours' last step this workgroup has, so each leaves a ring behind.
+// Sums keep the order of the kernels of one step: same bits.
+// Bound by the launch and the loads of the rows (about 200 listed for 57 owned
+// at degree 2, 300 for 20 at degree 4).  One scalar row a thread: with two in
+// 512 threads 120 us per outer iteration at 512x256 instead of 115.  Launch per
+// step -> tiles, us per outer iteration: 96x48 56.1 -> 49.1, 150x75 64.7 ->
+// 56.6, 256x128 84.1 -> 78.0, 512x256 137 -> 115, 1024x512 232 -> 210,
+// 2048x1024 572 -> 563.
+template <int HELD, int LANES>
+struct TileHeld : BottomRows<1, HELD, LANES> {
+    uint32_t I, r, act;  // block row, component, rings inside (0: the outermost)
+    uint32_t own, all;   // rows owned, rows listed
+    // false: the solve has ended, or the tile owns nothing
+    __device__ __forceinline__ bool load(const BottomLevel& L, const Tiles& T, const PcgState* st) {
+        const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
+        uint32_t zero = 0;
+        KEEP(zero);
+        uint32_t ro = T.roff[(size_t)tile * (T.rings + 1) + min(threadIdx.x % WAVE, T.rings)];
+        uint32_t done = (&st->done)[zero];
+        KEEP(ro);
+        KEEP(done);
+        own = __builtin_amdgcn_readlane(ro, 0);
+        all = __builtin_amdgcn_readlane(ro, T.rings);
+        if (__builtin_amdgcn_readfirstlane(done) || !own) return false;
+        r = threadIdx.x / all;
+        const uint32_t e = threadIdx.x - r * all;
+        const bool valid = r < 3;
+        act = 0;   // rings that hold the row, so products it may take
+        for (uint32_t k = 0; k < T.rings; ++k)
+            act += e < (uint32_t)__builtin_amdgcn_readlane(ro, k);
+        if (!valid) act = 0;
+        this->i[0] = valid ? 3 * e + r : this->NO_ROW;
+        I = valid ? T.ids[(size_t)tile * T.ext + e] : 0;
+#pragma unroll
+        for (int k = 0; k < HELD / 2; ++k) {
+            uint32_t w = 0;
+            if (act && k < (int)T.W2) w = T.lcol[((size_t)tile * T.W2 + k) * T.ext + e];
+            this->col[0][k] = (3 * (w & 0xffffu)) | ((3 * (w >> 16)) << 16);
+        }
+        this->template load_row<false>(L, 0, I, r, act != 0);
+        if (valid) this->dinv[0] = L.dinv[3 * (size_t)I + r];
+        return true;
+    }
+    __device__ __forceinline__ bool owned() const { return this->on(0) && this->i[0] < 3 * own; }
+    __device__ __forceinline__ size_t global() const { return 3 * (size_t)I + r; }
+    __device__ __forceinline__ uint32_t at() const { return this->i[0]; }
+    __device__ __forceinline__ float scaled(const float* x) const {   // (D^-1 A x) of the row
+        return this->dinv[0] * this->product(0, x);
+    }
+};
+template <int TB, int HELD, int LANES>
+__global__ __launch_bounds__(TB) void k_amg_down(BottomLevel L, Tiles T,
+                                                 const float* __restrict__ b,
+                                                 float* __restrict__ x, float* __restrict__ r,
+                                                 const PcgState* st) {
+    extern __shared__ float lds[];
+    TileHeld<HELD, LANES> R;
+    if (!R.load(L, T, st)) return;
+    float *din = lds, *dout = lds + 3 * R.all, *xs = lds + 6 * R.all;
+    float bb = 0.f, rr = 0.f, xx = 0.f, dd = 0.f;
+    if (R.on(0)) {
+        bb = b[R.global()];
+        rr = R.dinv[0] * bb;
+        dd = rr * L.inv_theta;
+        xx = dd;
+        din[R.at()] = dd;
+    }
+    for (uint32_t k = 1; k < L.degree; ++k) {
+        __syncthreads();
+        if (k <= R.act) {
+            rr -= R.scaled(din);
+            dd = L.c1[k] * dd + L.c2[k] * rr;
+            xx += dd;
+            dout[R.at()] = dd;
+        }
+        float* t = din;
+        din = dout;
+        dout = t;
+    }
+    if (R.on(0)) xs[R.at()] = xx;
+    __syncthreads();
+    if (R.owned()) {
+        r[R.global()] = bb - R.product(0, xs);
+        x[R.global()] = xx;
+    }
+}
+template <int TB, int HELD, int LANES>
+__global__ __launch_bounds__(TB) void k_amg_up(BottomLevel L, Tiles T,
+                                               const float* __restrict__ b,
+                                               const float* __restrict__ x,
+                                               const float* __restrict__ xc,
+                                               float* __restrict__ out, const PcgState* st) {
+    extern __shared__ float lds[];
+    TileHeld<HELD, LANES> R;
+    if (!R.load(L, T, st)) return;
+    float *din = lds, *dout = lds + 3 * R.all, *xs = lds + 6 * R.all;
+    float rr = 0.f, xx = 0.f, dd = 0.f;
+    if (R.on(0)) {   // x + P xc, by one lane a row
+        const uint32_t I = R.I;
+        const Bell<3, 3>& P = L.P;
+        uint32_t base = (I >> 6) * SLICE * P.width + (I & 63), len = P.width;
+        if (!P.width) {
+            base = P.slice_ptr[I >> 6] + (I & 63);
+            len = P.len[I];
+        }
+        const float* const val = P.val + (size_t)(3 * R.r) * P.slots;
+        float y = 0.f;
+        for (uint32_t k0 = 0; k0 < len; k0 += 4) {
+            float a[4][3], v[4][3];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u)
+                if (k0 + u < len) {
+                    const uint32_t sl = base + (k0 + u) * SLICE;
+                    const float* const xj = xc + 3 * (size_t)P.bcol[sl];
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        a[u][c] = val[(size_t)c * P.slots + sl];
+                        v[u][c] = xj[c];
+                    }
+                }
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u)
+                if (k0 + u < len)
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) y += a[u][c] * v[u][c];
+        }
+        xx = x[R.global()] + y;
+        xs[R.at()] = xx;
+    }
+    __syncthreads();
+    if (R.act) {
+        rr = R.dinv[0] * (b[R.global()] - R.product(0, xs));
+        dd = rr * L.inv_theta;
+        din[R.at()] = dd;
+    }
+    for (uint32_t k = 1; k < L.degree; ++k) {
+        __syncthreads();
+        if (k < R.act) {
+            rr -= R.scaled(din);
+            const float dn = L.c1[k] * dd + L.c2[k] * rr;
+            xx += k == 1 ? dd + dn : dn;
+            dd = dn;
+            dout[R.at()] = dn;
+        }
+        float* t = din;
+        din = dout;
+        dout = t;
+    }
+    if (R.owned()) out[R.global()] = xx;
+}
+
 }  // namespace
 
 
@@ -1130,6 +1302,7 @@ void amg_free(AmgDev* A) {
             for (void* q : qs)
                 if (q) (void)hipFree(q);
         }
+        tiles_free(L.tiles);
     }
     void* ps[] = {A->cinv, A->ones,     A->pow_x,  A->pow_y,
                   A->scal, A->partials, A->nzbits, A->differ, A->dense};
@@ -1235,6 +1408,48 @@ static int bottom_kind(const AmgDevLevel& L) {
     return L.ab.wmax <= 24 && rows == 1 ? 3 : 0;
 }
 
+// The mean place of each aggregate's nodes (the next level's nodes)
+static std::vector<double> mean_places(const AmgHostLevel& h, const std::vector<double>& xy) {
+    std::vector<double> out(2 * (size_t)(h.nc / 3), 0.0), cnt(h.nc / 3, 0.0);
+    for (uint32_t i = 0; i < h.n / h.bs; ++i) {
+        const uint32_t a = h.agg[i];
+        if (a >= h.nc / 3) continue;   // in no aggregate
+        out[2 * (size_t)a] += xy[2 * (size_t)i];
+        out[2 * (size_t)a + 1] += xy[2 * (size_t)i + 1];
+        cnt[a] += 1.0;
+    }
+    for (size_t a = 0; a < cnt.size(); ++a)
+        for (int c = 0; c < 2; ++c) out[2 * a + c] /= std::max(cnt[a], 1.0);
+    return out;
+}
+
+// Most block rows of a tile of level L, 0: its rows do not fit the kernels'
+// forms (those of k_amg_bottom, a row's P by one lane).
+static uint32_t tile_limit(const AmgDevLevel& L) {
+    if ((L.ab.lanes != 2 && L.ab.lanes != 4) || L.pb.lanes != 1) return 0;
+    return L.ab.wmax <= 14 ? 1024 / 3 : L.ab.wmax <= 24 ? 512 / 3 : 0;
+}
+// Tiles of a level of fewer than BELL_LARGE block rows (larger ones are bound by
+// bytes, of which the rings read more), at most 256, which run at once (a tile
+// takes a CU: 19,608 rows of degree 4 in 990 tiles take 644 us per outer
+// iteration instead of 563 with a launch per step), of about 8 rows at least
+// (a launch takes as long as its largest tile: 16 rows 1-2 us more).
+static int level_tiles(AmgDevLevel& L, const std::vector<double>& xy, hipStream_t s) {
+    const uint32_t rows = L.n / 3, limit = tile_limit(L), rings = (uint32_t)L.degree;
+    if (!limit || rows >= BELL_LARGE || rows < 64) return NBX_OK;
+    const uint32_t cells = std::max(std::min(256u, rows / 8), 1u);
+    double2* d = nullptr;
+    NBX_HIP(hipMalloc(&d, (size_t)rows * sizeof(double2)));
+    hipError_t e = copy_on(d, xy.data(), (size_t)rows * sizeof(double2), hipMemcpyHostToDevice, s);
+    int rc = NBX_OK;
+    if (e == hipSuccess)
+        rc = tiles_build(L.tiles, TileRows<uint16_t>{L.ab.slice_ptr, L.ab.len, L.ab.bcol}, rows,
+                         L.ab.wmax, d, {{cells, rings}, {std::min(256u, 2 * cells), rings}}, limit, s);
+    (void)hipFree(d);
+    NBX_HIP(e);
+    return rc;
+}
+
 // Symbolic hierarchy of the system's current K (pattern, Dirichlet rows,
 // node coordinates), uploaded; replaces any previous one.
 static int amg_symbolic(FemSys& S) {
@@ -1311,6 +1526,7 @@ static int amg_symbolic(FemSys& S) {
     for (size_t l = 0; l < nl; ++l) {
         const AmgHostLevel& h = H.lv[l];
         AmgDevLevel& L = A->lv[l];
+        if (l > 0) xy = mean_places(H.lv[l - 1], xy);
         L.n = h.n;
         L.nc = h.nc;
         L.bs = l == 0 ? 2 : 3;
@@ -1353,6 +1569,8 @@ static int amg_symbolic(FemSys& S) {
             } else {
                 NBX_TRY((bell_upload<3, 3>(L.n / 3, plen, pcol, L.pb, A->bytes)));
                 NBX_TRY((bell_upload<3, 3>(L.nc / 3, tlen, tcol, L.tb, A->bytes)));
+                // (the last smoothed level: with the dense solve, where it can)
+                if (l + 2 < nl || !bottom_kind(L)) NBX_TRY(level_tiles(L, xy, S.s));
             }
             NBX_TRY(up(&L.t, h.t, A->bytes));
             NBX_TRY(up(&L.agg, h.agg, A->bytes));
@@ -1630,7 +1848,7 @@ uint32_t amg_levels(const AmgDev* A) { return (uint32_t)A->lv.size(); }
 static void restrict_to(AmgDev* A, size_t l, const float* r, const PcgState* st, hipStream_t s) {
     AmgDevLevel& V = A->lv[l];
     AmgDevLevel& W = A->lv[l + 1];
-    const bool init = l + 2 < A->lv.size() && l + 1 != A->bottom;
+    const bool init = l + 2 < A->lv.size() && l + 1 != A->bottom && !W.tiles.n;
     with_bs(V.bs, [&](auto R) {
         constexpr int RR = decltype(R)::value;
         with_bl(V.tb, [&](auto ln, auto ph) {
@@ -1652,7 +1870,7 @@ static void restrict_to(AmgDev* A, size_t l, const float* r, const PcgState* st,
 static void prolong_from(AmgDev* A, size_t l, float* x, bool add, const PcgState* st,
                          hipStream_t s) {
     AmgDevLevel& V = A->lv[l];
-    const float* xc = A->lv[l + 1].x;
+    const float* xc = A->lv[l + 1].out();
     with_bs(V.bs, [&](auto R) {
         constexpr int RR = decltype(R)::value;
         with_bl(V.pb, [&](auto ln, auto ph) {
@@ -1668,12 +1886,8 @@ static void prolong_from(AmgDev* A, size_t l, float* x, bool add, const PcgState
     });
 }
 
-// The one-workgroup part: level A->bottom and the dense solve below it.
-static void bottom_cycle(AmgDev* A, const float* b, float* x, const PcgState* st, hipStream_t s) {
-    Bottom B{};
-    const AmgDevLevel& C = A->lv.back();
-    const AmgDevLevel& V = A->lv[A->bottom];
-    BottomLevel& L = B.lv;
+static BottomLevel level_args(const AmgDevLevel& V) {
+    BottomLevel L{};
     L.A = bell<3, 3>(V.ab);
     L.P = bell<3, 3>(V.pb);
     L.T = bell<3, 3>(V.tb);
@@ -1685,6 +1899,51 @@ static void bottom_cycle(AmgDev* A, const float* b, float* x, const PcgState* st
     L.inv_theta = V.inv_theta;
     std::copy(V.c1, V.c1 + AMG_MAX_DEGREE, L.c1);
     std::copy(V.c2, V.c2 + AMG_MAX_DEGREE, L.c2);
+    return L;
+}
+
+// f(TB, HELD, LANES) of k_amg_down and k_amg_up for a level on tiles
+template <class F>
+static void with_tile_form(const AmgDevLevel& V, F&& f) {
+    using std::integral_constant;
+    auto lanes = [&](auto tb, auto held) {
+        if (V.ab.lanes == 2)
+            f(tb, held, integral_constant<int, 2>{});
+        else
+            f(tb, held, integral_constant<int, 4>{});
+    };
+    if (V.ab.wmax > 14)
+        lanes(integral_constant<int, 512>{}, integral_constant<int, 24>{});
+    else if (3 * V.tiles.most <= 512)
+        lanes(integral_constant<int, 512>{}, integral_constant<int, 14>{});
+    else
+        lanes(integral_constant<int, 1024>{}, integral_constant<int, 14>{});
+}
+static void tile_down(const AmgDevLevel& V, const float* b, float* x, const PcgState* st,
+                      hipStream_t s) {
+    const size_t lds = 9 * (size_t)V.tiles.most * sizeof(float);
+    with_tile_form(V, [&](auto tb, auto held, auto ln) {
+        constexpr int TB = decltype(tb)::value, HELD = decltype(held)::value;
+        hipLaunchKernelGGL((k_amg_down<TB, HELD, decltype(ln)::value>), dim3(V.tiles.n), dim3(TB),
+                           lds, s, level_args(V), V.tiles, b, x, V.r, st);
+    });
+}
+static void tile_up(const AmgDevLevel& V, const float* b, const float* x, const float* xc,
+                    const PcgState* st, hipStream_t s) {
+    const size_t lds = 9 * (size_t)V.tiles.most * sizeof(float);
+    with_tile_form(V, [&](auto tb, auto held, auto ln) {
+        constexpr int TB = decltype(tb)::value, HELD = decltype(held)::value;
+        hipLaunchKernelGGL((k_amg_up<TB, HELD, decltype(ln)::value>), dim3(V.tiles.n), dim3(TB),
+                           lds, s, level_args(V), V.tiles, b, x, xc, V.d0, st);
+    });
+}
+
+// The one-workgroup part: level A->bottom and the dense solve below it.
+static void bottom_cycle(AmgDev* A, const float* b, float* x, const PcgState* st, hipStream_t s) {
+    Bottom B{};
+    const AmgDevLevel& C = A->lv.back();
+    const AmgDevLevel& V = A->lv[A->bottom];
+    B.lv = level_args(V);
     B.nco = C.n;
     B.cinv = A->cinv;
     B.b = b;
@@ -1707,9 +1966,11 @@ static void bottom_cycle(AmgDev* A, const float* b, float* x, const PcgState* st
 
 // The V-cycle from level l0 >= 1 down, x = M^-1 b on that level (b, x: that
 // level's arrays; the finest level is smoothed by the flexible CG's own
-// kernels on the fp16 copy).  The restriction has already started each
-// level's pre-smoothing (r, d0, x).  A one-level hierarchy is its dense
-// solve alone (l0 = 0).
+// kernels on the fp16 copy).  The restriction has already started the
+// pre-smoothing (r, d0, x) of each level that takes a launch per step; levels
+// on tiles take two launches, and the last ones one workgroup.  A level's
+// correction is in its out().  A one-level hierarchy is its dense solve alone
+// (l0 = 0).
 static void cycle_from(AmgDev* A, size_t l0, const float* b, float* x, const PcgState* st,
                        hipStream_t s) {
     const size_t L = A->lv.size();
@@ -1718,6 +1979,11 @@ static void cycle_from(AmgDev* A, size_t l0, const float* b, float* x, const Pcg
         AmgDevLevel& V = A->lv[l];
         const float* bl = l == l0 ? b : V.b;
         float* xl = l == l0 ? x : V.x;
+        if (V.tiles.n) {
+            tile_down(V, bl, xl, st, s);
+            restrict_to(A, l, V.r, st, s);
+            continue;
+        }
         float *din = V.d0, *dout = V.d1;
         with_bl(V.ab, [&](auto ln, auto ph) {
             constexpr int LN = decltype(ln)::value, PH = decltype(ph)::value;
@@ -1745,6 +2011,10 @@ static void cycle_from(AmgDev* A, size_t l0, const float* b, float* x, const Pcg
         AmgDevLevel& V = A->lv[l];
         const float* bl = l == l0 ? b : V.b;
         float* xl = l == l0 ? x : V.x;
+        if (V.tiles.n) {
+            tile_up(V, bl, xl, A->lv[l + 1].out(), st, s);
+            continue;
+        }
         prolong_from(A, l, xl, true, st, s);
         float *din = V.d0, *dout = V.d1;
         with_bl(V.ab, [&](auto ln, auto ph) {

@@ -138,6 +138,7 @@ struct Tiles {
     uint32_t ext = 0;              // list length, the same for every tile (<= 1024, whole waves)
     uint32_t rings = 0;
     uint32_t W2 = 0;               // column words per row
+    uint32_t most = 0;             // rows of the largest tile (ext: to whole waves)
     uint32_t* ids = nullptr;       // [n ext] node ids
     uint32_t* lcol = nullptr;      // [n W2 ext] two 16-bit positions per word
     uint32_t* roff = nullptr;      // [n (rings + 1)] rows within r rings

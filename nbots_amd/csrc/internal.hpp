@@ -1,6 +1,8 @@
 // Host-side interfaces between the C-ABI layer and the HIP kernels.
 #pragma once
 
+#include <vector>
+
 #include "common.hpp"
 
 namespace nbx {
@@ -189,7 +191,21 @@ int mat_prepare_mixed(DevMatrix& m, hipStream_t s, const MixedOpts& o);
 int scan_u32(const uint32_t* in, uint32_t* out, size_t n, hipStream_t s);
 // tiles of the off-diagonal pattern O, whose rows hold at most wmax blocks,
 // by the node positions xy (T.n = 0 when they do not fit)
+// Tiles of the fp16 copy's rows for the Chebyshev preconditioner, or (the second
+// form) of any sliced rows: the first of `attempts` (cells, rings) whose tiles
+// have at most `limit` rows; T.n = 0 when none has.
 int tiles_build(Tiles& T, const Off16& O, uint32_t wmax, const double2* xy, hipStream_t s);
+struct TileAttempt {
+    uint32_t cells, rings;
+};
+template <class Len>
+struct TileRows {   // block k of row v at slice_ptr[v / 64] + 64 k + v % 64
+    const uint32_t* slice_ptr;
+    const Len* rowlen;
+    const uint32_t* bcol;
+};
+int tiles_build(Tiles& T, const TileRows<uint16_t>& O, uint32_t n, uint32_t wmax, const double2* xy,
+                const std::vector<TileAttempt>& attempts, uint32_t limit, hipStream_t s);
 void tiles_free(Tiles& T);
 
 int spmv(const DevMatrix& m, const double* x, double* y, hipStream_t s);

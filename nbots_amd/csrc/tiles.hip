@@ -119,13 +119,16 @@ __device__ void tile_sort(uint32_t* list, uint32_t* tmp, uint32_t b, uint32_t e)
 }
 
 // One workgroup per tile.  ext = 0: only info (the largest tile, a flag for
-// one beyond TILE_TB rows).  Otherwise the tile's list, ring
+// one beyond `limit` rows).  Otherwise the tile's list, ring
 // offsets and columns (row i's block 2 q + h in half h of word
 // lcol[(t W2 + q) ext + i]; padding names the row itself).
-__global__ __launch_bounds__(TILE_TB) void k_tile_rings(Off16 O, const uint32_t* __restrict__ ptr,
+template <class Len>
+__global__ __launch_bounds__(TILE_TB) void k_tile_rings(TileRows<Len> O,
+                                                        const uint32_t* __restrict__ ptr,
                                                         const uint32_t* __restrict__ own,
-                                                        uint32_t rings, uint32_t wmax, uint32_t W2,
-                                                        uint32_t ext, uint32_t* __restrict__ ids,
+                                                        uint32_t limit, uint32_t rings,
+                                                        uint32_t wmax, uint32_t W2, uint32_t ext,
+                                                        uint32_t* __restrict__ ids,
                                                         uint32_t* __restrict__ lcol,
                                                         uint32_t* __restrict__ roff,
                                                         unsigned* info) {
@@ -134,7 +137,7 @@ __global__ __launch_bounds__(TILE_TB) void k_tile_rings(Off16 O, const uint32_t*
     __shared__ uint32_t cnt;
     const uint32_t t = blockIdx.x, tid = threadIdx.x;
     const uint32_t o0 = ptr[t], c0 = ptr[t + 1] - o0;
-    if (c0 > (uint32_t)TILE_TB) {
+    if (c0 > limit) {
         if (tid == 0) info[1] = 1u;
         return;
     }
@@ -158,13 +161,13 @@ __global__ __launch_bounds__(TILE_TB) void k_tile_rings(Off16 O, const uint32_t*
             const uint32_t w = O.bcol[(size_t)O.slice_ptr[v >> 6] + (v & 63) + (size_t)k * SLICE];
             if (tile_insert(keys, w)) {
                 const uint32_t at = atomicAdd(&cnt, 1u);
-                if (at < (uint32_t)TILE_TB) list[at] = w;
+                if (at < limit) list[at] = w;
             }
         }
         __syncthreads();
         const uint32_t now = cnt;
         __syncthreads();
-        if (now > (uint32_t)TILE_TB) {
+        if (now > limit) {
             if (tid == 0) info[1] = 1u;
             return;
         }
@@ -208,13 +211,13 @@ void tiles_free(Tiles& T) {
     T = Tiles();
 }
 
-// Leaves T.n = 0 (nothing allocated) when the mesh does not divide into
-// tiles of at most TILE_TB rows this way, or without device memory for them:
-// the kernels that take one step per launch then run.
-int tiles_build(Tiles& T, const Off16& O, uint32_t wmax, const double2* xy, hipStream_t s) {
-    const uint32_t n = O.n_nodes;
-    tiles_free(T);
-    if (!xy || n == 0 || wmax == 0 || wmax > TILE_WMAX) return NBX_OK;
+// Cuts the n rows at positions xy into the first of `attempts` whose tiles have
+// at most `limit` rows.  Leaves T.n = 0 (nothing allocated) when none has, or
+// without device memory for them: the kernels that take one step per launch
+// then run.
+template <class Len>
+static int tiles_cut(Tiles& T, const TileRows<Len>& O, uint32_t n, uint32_t wmax, const double2* xy,
+                     const std::vector<TileAttempt>& attempts, uint32_t limit, hipStream_t s) {
     uint32_t *cell = nullptr, *cnt = nullptr, *ptr = nullptr, *own = nullptr;
     unsigned* info = nullptr;
     double* bb = nullptr;
@@ -244,6 +247,68 @@ int tiles_build(Tiles& T, const Off16& O, uint32_t wmax, const double2* xy, hipS
     if (!(Lx >= 0.0) || !(Ly >= 0.0) || !std::isfinite(Lx) || !std::isfinite(Ly) ||
         !(Lx + Ly > 0.0))
         return done(NBX_OK);
+    if (hipMalloc(&cell, (size_t)n * 4) != hipSuccess ||
+        hipMalloc(&own, (size_t)n * 4) != hipSuccess || hipMalloc(&info, 16) != hipSuccess)
+        return no_memory();
+    const uint32_t W2 = (wmax + 1) / 2;
+    for (const auto& at : attempts) {
+        const uint32_t rings = std::max(at.rings, 2u);
+        // at most so many cells, about square
+        const double cells = (double)at.cells;
+        const double fx = Lx > 0.0 && Ly > 0.0
+                              ? std::min(std::max(1.0, std::round(sqrt(cells * Lx / Ly))), cells)
+                              : (Lx > 0.0 ? cells : 1.0);
+        const double fy = Ly > 0.0 ? std::max(1.0, std::floor(cells / fx)) : 1.0;
+        TileGrid g{lo[0], lo[1], Lx > 0.0 ? fx / Lx : 0.0, Ly > 0.0 ? fy / Ly : 0.0,
+                   (uint32_t)fx, (uint32_t)fy};
+        const uint32_t nt = g.nx * g.ny;
+        if (cnt) (void)hipFree(cnt);
+        if (ptr) (void)hipFree(ptr);
+        cnt = ptr = nullptr;
+        if (hipMalloc(&cnt, (size_t)nt * 4) != hipSuccess ||
+            hipMalloc(&ptr, ((size_t)nt + 1) * 4) != hipSuccess)
+            return no_memory();
+        hipLaunchKernelGGL(k_tile_zero, dim3(grid_for(nt)), dim3(BLOCK), 0, s, cnt, nt);
+        hipLaunchKernelGGL(k_tile_zero, dim3(1), dim3(BLOCK), 0, s, (uint32_t*)info, 4u);
+        hipLaunchKernelGGL(k_tile_count, dim3(grid_for(n)), dim3(BLOCK), 0, s, g, xy, n, cell, cnt);
+        const int rc = scan_u32(cnt, ptr, nt, s);
+        if (rc) return done(rc);
+        hipLaunchKernelGGL(k_tile_zero, dim3(grid_for(nt)), dim3(BLOCK), 0, s, cnt, nt);
+        hipLaunchKernelGGL(k_tile_fill, dim3(grid_for(n)), dim3(BLOCK), 0, s, cell, n, ptr, cnt, own);
+        hipLaunchKernelGGL(k_tile_rings<Len>, dim3(nt), dim3(TILE_TB), 0, s, O, ptr, own, limit, rings,
+                           wmax, W2, 0u, (uint32_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr, info);
+        unsigned hi[2] = {0, 1};   // the largest tile, one beyond TILE_TB rows
+        if (hipGetLastError() != hipSuccess ||
+            copy_on(hi, info, sizeof hi, hipMemcpyDeviceToHost, s) != hipSuccess) {
+            set_last_error("tiles: halo rings");
+            return done(NBX_ERR_HIP);
+        }
+        if (hi[1]) continue;
+        T.n = nt;
+        T.most = hi[0];
+        T.ext = (hi[0] + WAVE - 1) / WAVE * WAVE;
+        T.rings = rings;
+        T.W2 = W2;
+        break;
+    }
+    if (T.n == 0) return done(NBX_OK);
+    if (hipMalloc(&T.ids, (size_t)T.n * T.ext * 4) != hipSuccess ||
+        hipMalloc(&T.lcol, (size_t)T.n * T.ext * W2 * 4) != hipSuccess ||
+        hipMalloc(&T.roff, (size_t)T.n * (T.rings + 1) * 4) != hipSuccess)
+        return no_memory();
+    hipLaunchKernelGGL(k_tile_rings<Len>, dim3(T.n), dim3(TILE_TB), 0, s, O, ptr, own, limit, T.rings, wmax, W2,
+                       T.ext, T.ids, T.lcol, T.roff, info);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) {
+        set_last_error("tiles: lists");
+        return done(NBX_ERR_HIP);
+    }
+    return done(NBX_OK);
+}
+
+int tiles_build(Tiles& T, const Off16& O, uint32_t wmax, const double2* xy, hipStream_t s) {
+    const uint32_t n = O.n_nodes;
+    tiles_free(T);
+    if (!xy || n == 0 || wmax == 0 || wmax > TILE_WMAX) return NBX_OK;
     // Tiles and rings (= steps per launch).  A launch takes as long as its
     // fullest CU, so the tiles are as many as run at once, or twice that, with
     // as many rings as a tile's TILE_TB rows leave room for; from 540k nodes
@@ -273,68 +338,22 @@ int tiles_build(Tiles& T, const Off16& O, uint32_t wmax, const double2* xy, hipS
         while (rings0 < 8 && rows(rings0 + 1) <= TILE_TB) ++rings0;
     }
     const uint32_t cells0 = std::max(std::min(tiles, n / own0), 1u);
-    if (hipMalloc(&cell, (size_t)n * 4) != hipSuccess ||
-        hipMalloc(&own, (size_t)n * 4) != hipSuccess || hipMalloc(&info, 16) != hipSuccess)
-        return no_memory();
-    const uint32_t W2 = (wmax + 1) / 2;
     // A mesh of uneven density, or with wider rows, can outgrow TILE_TB in a
     // few cells: fewer rings then, and more cells.
-    const struct { uint32_t cells, rings; } attempts[] = {{cells0, rings0},
-                                                          {cells0, rings0 - 1},
-                                                          {cells0, rings0 / 2},
-                                                          {2 * cells0, rings0 / 2},
-                                                          {4 * cells0, rings0 / 4}};
-    for (const auto& at : attempts) {
-        const uint32_t rings = std::max(at.rings, 2u);
-        // at most so many cells, about square
-        const double cells = (double)at.cells;
-        const double fx = Lx > 0.0 && Ly > 0.0
-                              ? std::min(std::max(1.0, std::round(sqrt(cells * Lx / Ly))), cells)
-                              : (Lx > 0.0 ? cells : 1.0);
-        const double fy = Ly > 0.0 ? std::max(1.0, std::floor(cells / fx)) : 1.0;
-        TileGrid g{lo[0], lo[1], Lx > 0.0 ? fx / Lx : 0.0, Ly > 0.0 ? fy / Ly : 0.0,
-                   (uint32_t)fx, (uint32_t)fy};
-        const uint32_t nt = g.nx * g.ny;
-        if (cnt) (void)hipFree(cnt);
-        if (ptr) (void)hipFree(ptr);
-        cnt = ptr = nullptr;
-        if (hipMalloc(&cnt, (size_t)nt * 4) != hipSuccess ||
-            hipMalloc(&ptr, ((size_t)nt + 1) * 4) != hipSuccess)
-            return no_memory();
-        hipLaunchKernelGGL(k_tile_zero, dim3(grid_for(nt)), dim3(BLOCK), 0, s, cnt, nt);
-        hipLaunchKernelGGL(k_tile_zero, dim3(1), dim3(BLOCK), 0, s, (uint32_t*)info, 4u);
-        hipLaunchKernelGGL(k_tile_count, dim3(grid_for(n)), dim3(BLOCK), 0, s, g, xy, n, cell, cnt);
-        const int rc = scan_u32(cnt, ptr, nt, s);
-        if (rc) return done(rc);
-        hipLaunchKernelGGL(k_tile_zero, dim3(grid_for(nt)), dim3(BLOCK), 0, s, cnt, nt);
-        hipLaunchKernelGGL(k_tile_fill, dim3(grid_for(n)), dim3(BLOCK), 0, s, cell, n, ptr, cnt, own);
-        hipLaunchKernelGGL(k_tile_rings, dim3(nt), dim3(TILE_TB), 0, s, O, ptr, own, rings, wmax,
-                           W2, 0u, (uint32_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr, info);
-        unsigned hi[2] = {0, 1};   // the largest tile, one beyond TILE_TB rows
-        if (hipGetLastError() != hipSuccess ||
-            copy_on(hi, info, sizeof hi, hipMemcpyDeviceToHost, s) != hipSuccess) {
-            set_last_error("tiles: halo rings");
-            return done(NBX_ERR_HIP);
-        }
-        if (hi[1]) continue;
-        T.n = nt;
-        T.ext = (hi[0] + WAVE - 1) / WAVE * WAVE;
-        T.rings = rings;
-        T.W2 = W2;
-        break;
-    }
-    if (T.n == 0) return done(NBX_OK);
-    if (hipMalloc(&T.ids, (size_t)T.n * T.ext * 4) != hipSuccess ||
-        hipMalloc(&T.lcol, (size_t)T.n * T.ext * W2 * 4) != hipSuccess ||
-        hipMalloc(&T.roff, (size_t)T.n * (T.rings + 1) * 4) != hipSuccess)
-        return no_memory();
-    hipLaunchKernelGGL(k_tile_rings, dim3(T.n), dim3(TILE_TB), 0, s, O, ptr, own, T.rings, wmax, W2,
-                       T.ext, T.ids, T.lcol, T.roff, info);
-    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) {
-        set_last_error("tiles: lists");
-        return done(NBX_ERR_HIP);
-    }
-    return done(NBX_OK);
+    return tiles_cut(T, TileRows<uint8_t>{O.slice_ptr, O.rowlen, O.bcol}, n, wmax, xy,
+                     {{cells0, rings0},
+                      {cells0, rings0 - 1},
+                      {cells0, rings0 / 2},
+                      {2 * cells0, rings0 / 2},
+                      {4 * cells0, rings0 / 4}},
+                     TILE_TB, s);
+}
+
+int tiles_build(Tiles& T, const TileRows<uint16_t>& O, uint32_t n, uint32_t wmax, const double2* xy,
+                const std::vector<TileAttempt>& attempts, uint32_t limit, hipStream_t s) {
+    tiles_free(T);
+    if (!xy || n == 0 || wmax == 0) return NBX_OK;
+    return tiles_cut(T, O, n, wmax, xy, attempts, std::min(limit, (uint32_t)TILE_TB), s);
 }
 
 }  // namespace nbx
