@@ -256,11 +256,12 @@ __global__ __launch_bounds__(FIN) void k_amg_pow_fin(const double* partials, uns
 // The pivots are the Cholesky factor's, and an unknown whose pivot is not
 // above 1e-13 of the largest diagonal entry is dropped as amg_dense_inverse
 // drops it (zero row and column).  One workgroup holds the matrix in
-// registers, NB x NB entries a thread; a step passes column k through LDS and
-// costs one barrier.  Bound by its n steps of LDS reads, a division and a
-// barrier: 190 us at 162 unknowns.  The host function took 0.6 ms there besides
+// registers, the lower half of its 32 x 32 blocks; a step passes column k
+// through LDS and costs one barrier.  Bound by its n steps of LDS reads, a
+// division and a barrier: 142 us at 162 unknowns (190 with all entries).  The
+// host function took 0.6 ms there besides
 // the copies and the wait; with the folded power iteration above, the numeric
-// phase went from 1.13 to 0.78 ms at 96x48 (162 unknowns), 0.95 -> 0.78 at
+// phase went from 1.13 to 0.71 ms at 96x48 (162 unknowns), 0.95 -> 0.78 at
 // 150x75 (36), 1.74 -> 1.52 at 512x256 (24).  The same Cholesky factor and
 // products on the device, bit for bit the host's, take 445 us at 162.  Against
 // extended precision the inverse's error is as often below the host's as above
@@ -284,17 +285,19 @@ __global__ __launch_bounds__(WAVE) void k_dense_rows(const uint32_t* __restrict_
 }
 
 // inv = A^-1 in FP32, of A symmetrised (P^T A P rounds slightly
-// unsymmetrically).  Thread (tx, ty) holds the entries (ty + 32 p, tx + 32 q).
+// unsymmetrically).  Thread (tx, ty) holds the entries (ty + 32 p, tx + 32 q)
+// with q <= p; column k is those of the column from row block k / 32 on and
+// those of row k before it.
 template <int NB>
 __global__ __launch_bounds__(SWEEP_TB) void k_dense_sweep(const double* __restrict__ a,
                                                           float* __restrict__ inv, uint32_t n) {
     __shared__ double colk[2][NB * SWEEP_SIDE], big[SWEEP_TB / WAVE];
     const uint32_t tx = threadIdx.x % SWEEP_SIDE, ty = threadIdx.x / SWEEP_SIDE;
-    double v[NB][NB], dmax = 0.0;
+    double v[NB][NB], dmax = 0.0;   // (the entries q > p are never used)
 #pragma unroll
     for (int p = 0; p < NB; ++p)
 #pragma unroll
-        for (int q = 0; q < NB; ++q) {
+        for (int q = 0; q <= p; ++q) {
             const uint32_t i = ty + p * SWEEP_SIDE, j = tx + q * SWEEP_SIDE;
             v[p][q] = 0.0;
             if (i < n && j < n)
@@ -307,51 +310,44 @@ __global__ __launch_bounds__(SWEEP_TB) void k_dense_sweep(const double* __restri
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < SWEEP_TB / WAVE; ++w) dmax = fmax(dmax, big[w]);
-    for (uint32_t k = 0; k < n; ++k) {
-        double* const ck = colk[k & 1];
-        const uint32_t kq = k / SWEEP_SIDE, kt = k % SWEEP_SIDE;
-        if (tx == kt)
 #pragma unroll
-            for (int q = 0; q < NB; ++q)
-                if (q == (int)kq)
+    for (int kq = 0; kq < NB; ++kq)
+        for (uint32_t kt = 0; kt < SWEEP_SIDE; ++kt) {
+            const uint32_t k = kq * SWEEP_SIDE + kt;
+            if (k >= n) break;
+            double* const ck = colk[k & 1];
+            if (tx == kt)
 #pragma unroll
-                    for (int p = 0; p < NB; ++p) ck[ty + p * SWEEP_SIDE] = v[p][q];
-        __syncthreads();
-        const double piv = ck[k];
-        const bool drop = !(piv > 1e-13 * dmax);
-        const double d = drop ? 0.0 : 1.0 / piv;
-        double cj[NB];
+                for (int p = kq; p < NB; ++p) ck[ty + p * SWEEP_SIDE] = v[p][kq];
+            if (ty == kt)
 #pragma unroll
-        for (int q = 0; q < NB; ++q) cj[q] = ck[tx + q * SWEEP_SIDE];
+                for (int q = 0; q < kq; ++q) ck[tx + q * SWEEP_SIDE] = v[kq][q];
+            __syncthreads();
+            const double piv = ck[k];
+            const bool drop = !(piv > 1e-13 * dmax);
+            const double d = drop ? 0.0 : 1.0 / piv;
+            double cj[NB];
 #pragma unroll
-        for (int p = 0; p < NB; ++p) {
-            const double f = ck[ty + p * SWEEP_SIDE] * d;
+            for (int q = 0; q < NB; ++q) cj[q] = ck[tx + q * SWEEP_SIDE];
 #pragma unroll
-            for (int q = 0; q < NB; ++q) v[p][q] = fma(-f, cj[q], v[p][q]);
+            for (int p = 0; p < NB; ++p) {
+                const double f = ck[ty + p * SWEEP_SIDE] * d;
+#pragma unroll
+                for (int q = 0; q <= p; ++q) v[p][q] = fma(-f, cj[q], v[p][q]);
+                if (p >= kq && tx == kt) v[p][kq] = ty + p * SWEEP_SIDE == k ? -d : f;   // column k
+            }
+            if (ty == kt)   // row k
+#pragma unroll
+                for (int q = 0; q <= kq; ++q)
+                    if (tx + q * SWEEP_SIDE != k) v[kq][q] = cj[q] * d;
         }
-        // row and column k
-        if (ty == kt)
-#pragma unroll
-            for (int p = 0; p < NB; ++p)
-                if (p == (int)kq)
-#pragma unroll
-                    for (int q = 0; q < NB; ++q) v[p][q] = cj[q] * d;
-        if (tx == kt)
-#pragma unroll
-            for (int q = 0; q < NB; ++q)
-                if (q == (int)kq)
-#pragma unroll
-                    for (int p = 0; p < NB; ++p) {
-                        const uint32_t i = ty + p * SWEEP_SIDE;
-                        v[p][q] = i == k ? -d : ck[i] * d;
-                    }
-    }
-    // (one of the two entries that rounding may leave different for both)
 #pragma unroll
     for (int p = 0; p < NB; ++p)
 #pragma unroll
-        for (int q = 0; q < NB; ++q) {
+        for (int q = 0; q <= p; ++q) {
             const uint32_t i = ty + p * SWEEP_SIDE, j = tx + q * SWEEP_SIDE;
+            // (of a diagonal block's two entries that rounding may leave
+            // different, the lower one for both)
             if (i < n && j <= i)
                 inv[(size_t)i * n + j] = inv[(size_t)j * n + i] = (float)-v[p][q];
         }
