@@ -895,21 +895,22 @@ __global__ __launch_bounds__(DENSE_BLOCK) void k_amg_dense(const float* __restri
 // ---- the bottom of the V-cycle in one workgroup -------------------------------
 // A smoothing step on a level of a few hundred unknowns costs a launch and a
 // chain of dependent loads (3.5-4 us), and the last smoothed level takes 8-13
-// such launches per cycle with the dense solve below it.  One workgroup of
-// 512 threads does them all, down to the dense solve and back up, when that
-// level has at most 1,024 unknowns.  Its operator is read once and kept in
-// registers (a thread holds one or two scalar rows, padded with zero blocks
-// to HELD, so that a product's LDS reads go out together), every vector lives
-// in LDS, and a step costs one barrier; the products (0.5-1 us) and the loads
-// of P, P^T and C^-1 bound it.  Every sum keeps the order of the kernels of
-// one step each, so the cycle's result is the same to the bit.  The kernel and the outer iteration around it,
-// with the launches it replaces and with it (cantilevers): 357 unknowns
-// (150x75) 14 us, 104 -> 71; 726 (64x32) 62 -> 44; 969 (256x128) 27 us,
-// 118 -> 95; 288 (512x256) 18 us, 184 -> 150; 312 (2048x1024) 25 us,
-// 661 -> 630.  With 1,024 threads the rows spill (128 VGPRs): 20 us at 357.
+// such launches per cycle with the dense solve below it.  One workgroup of 512
+// or 1,024 threads does them all, down to the dense solve and back up, when
+// that level has at most 1,024 unknowns.  Its operator is read once and kept in
+// registers (a thread holds a scalar row, padded with zero blocks to HELD, so
+// that a product's LDS reads go out together), every vector lives in LDS, and a
+// step costs one barrier; the products (0.5 us) and the loads of P, P^T and C^-1
+// bound it.  Every sum keeps the order of the kernels of one step each, so the
+// cycle's result is the same to the bit.  The kernel and the outer iteration
+// around it, with the launches it replaces and with it (cantilevers): 357
+// unknowns (150x75) 14 us, 104 -> 71; 726 (64x32) 62 -> 43; 969 (256x128)
+// 118 -> 95; 288 (512x256) 17 us, 184 -> 150; 312 (2048x1024) 25 us,
+// 661 -> 630.  With two rows a thread in 512 threads 64x32 42.1 instead of
+// 40.6 now, 256x128 78.4 instead of 76; more unknowns than that (three rows a
+// thread spill) take as long as the launches.
 // Threads take the scalar rows of equal component r of consecutive block
 // rows, so that a wavefront's loads of a block position are coalesced.
-constexpr int BOTTOM_TB = 512;
 struct BottomLevel {
     Bell<3, 3> A, P, T;
     const float* dinv;
@@ -924,22 +925,22 @@ struct Bottom {
     const float* b;
     float* x;
 };
-// the scalar rows of one thread on a level: row j is component r of block
-// row I, q = r rows + I = threadIdx.x + 512 j
-template <int RP, int HELD, int LANES>   // HELD: blocks of a row, none longer
+// one thread's scalar row on a level: component r of block row I, thread
+// r rows + I
+template <int HELD, int LANES>   // HELD: blocks of a row, none longer
 struct BottomRows {
-    uint32_t i[RP];   // the scalar row's place in LDS (3 I + r), or none
-    float dinv[RP];
+    uint32_t at;   // the scalar row's place in LDS (3 I + r), or none
+    float dinv;
     static constexpr uint32_t NO_ROW = 0xffffffffu;
-    __device__ __forceinline__ bool on(int j) const { return i[j] != NO_ROW; }
-    float v[RP][HELD][3];
-    uint32_t col[RP][HELD / 2];   // two 16-bit places (3 J) per word
-    // component r of block row I into row j: its values, and with COLS the
-    // columns as they stand
+    __device__ __forceinline__ bool on() const { return at != NO_ROW; }
+    float v[HELD][3];
+    uint32_t col[HELD / 2];   // two 16-bit places (3 J) per word
+    // component r of block row I: its values, and with COLS the columns as
+    // they stand
     template <bool COLS>
-    __device__ __forceinline__ void load_row(const BottomLevel& L, int j, uint32_t I, uint32_t r,
+    __device__ __forceinline__ void load_row(const BottomLevel& L, uint32_t I, uint32_t r,
                                              bool valid) {
-        dinv[j] = valid ? L.dinv[3 * (size_t)I + r] : 0.f;
+        dinv = valid ? L.dinv[3 * (size_t)I + r] : 0.f;
         size_t base = (size_t)(I >> 6) * SLICE * L.A.width + (I & 63);
         int len = valid ? (int)L.A.width : 0;
         if (valid && !L.A.width) {
@@ -949,38 +950,33 @@ struct BottomRows {
 #pragma unroll
         for (int k = 0; k < HELD; ++k) {
 #pragma unroll
-            for (int c = 0; c < 3; ++c) v[j][k][c] = 0.f;
+            for (int c = 0; c < 3; ++c) v[k][c] = 0.f;
             if (k < len) {
                 const size_t sl = base + (size_t)k * SLICE;
-                if constexpr (COLS) col[j][k / 2] |= (3 * L.A.bcol[sl]) << (16 * (k & 1));
+                if constexpr (COLS) col[k / 2] |= (3 * L.A.bcol[sl]) << (16 * (k & 1));
 #pragma unroll
-                for (int c = 0; c < 3; ++c)
-                    v[j][k][c] = L.A.val[(size_t)(3 * r + c) * L.A.slots + sl];
+                for (int c = 0; c < 3; ++c) v[k][c] = L.A.val[(size_t)(3 * r + c) * L.A.slots + sl];
             }
         }
     }
     __device__ __forceinline__ void load(const BottomLevel& L) {
+        const uint32_t r = threadIdx.x / L.rows, I = threadIdx.x - r * L.rows;
+        const bool valid = r < 3;
+        at = valid ? 3 * I + r : NO_ROW;
 #pragma unroll
-        for (int j = 0; j < RP; ++j) {
-            const uint32_t q = threadIdx.x + (uint32_t)j * BOTTOM_TB;
-            const uint32_t r = q / L.rows, I = q - r * L.rows;
-            const bool valid = r < 3;
-            i[j] = valid ? 3 * I + r : NO_ROW;
-#pragma unroll
-            for (int k = 0; k < HELD / 2; ++k) col[j][k] = 0;
-            load_row<true>(L, j, I, r, valid);
-        }
+        for (int k = 0; k < HELD / 2; ++k) col[k] = 0;
+        load_row<true>(L, I, r, valid);
     }
-    // (A x) of row j, summed as bell_row's LANES lanes sum it
-    __device__ __forceinline__ float product(int j, const float* x) const {
+    // (A x) of the row, summed as bell_row's LANES lanes sum it
+    __device__ __forceinline__ float product(const float* x) const {
         float y[LANES] = {};
 #pragma unroll
         for (int k = 0; k < HELD; ++k) {
-            const float* xk = x + ((col[j][k / 2] >> (16 * (k & 1))) & 0xffffu);
+            const float* xk = x + ((col[k / 2] >> (16 * (k & 1))) & 0xffffu);
             float& t = y[k % LANES];
-            t += v[j][k][0] * xk[0];
-            t += v[j][k][1] * xk[1];
-            t += v[j][k][2] * xk[2];
+            t += v[k][0] * xk[0];
+            t += v[k][1] * xk[1];
+            t += v[k][2] * xk[2];
         }
 #pragma unroll
         for (int o = LANES / 2; o > 0; o >>= 1)
@@ -988,6 +984,7 @@ struct BottomRows {
             for (int l = 0; l < o; ++l) y[l] += y[l + o];
         return y[0];
     }
+    __device__ __forceinline__ float scaled(const float* x) const { return dinv * product(x); }
 };
 // Vectors of a level in LDS: right-hand side, solution, residual (or the
 // second direction), direction.
@@ -995,80 +992,61 @@ struct BottomVec {
     float *b, *x, *r, *d;
 };
 // x = 0 start and degree - 1 steps, then the residual b - A x into v.r
-template <int RP, int HELD, int LANES>
-__device__ __forceinline__ void bottom_down(const BottomLevel& L, const BottomRows<RP, HELD, LANES>& R,
-                                            const BottomVec& v) {
-    float rr[RP], xx[RP], dd[RP];
-#pragma unroll
-    for (int j = 0; j < RP; ++j)
-        if (R.on(j)) {
-            const uint32_t i = R.i[j];
-            rr[j] = R.dinv[j] * v.b[i];
-            dd[j] = rr[j] * L.inv_theta;
-            xx[j] = dd[j];
-            v.d[i] = dd[j];
-        }
+template <int HELD, int LANES>
+__device__ __forceinline__ void bottom_down(const BottomLevel& L,
+                                            const BottomRows<HELD, LANES>& R, const BottomVec& v) {
+    float rr = 0.f, xx = 0.f, dd = 0.f;
+    if (R.on()) {
+        rr = R.dinv * v.b[R.at];
+        dd = rr * L.inv_theta;
+        xx = dd;
+        v.d[R.at] = dd;
+    }
     float *din = v.d, *dout = v.r;
     for (uint32_t k = 1; k < L.degree; ++k) {
         __syncthreads();
-#pragma unroll
-        for (int j = 0; j < RP; ++j)
-            if (R.on(j)) {
-                rr[j] -= R.dinv[j] * R.product(j, din);
-                dd[j] = L.c1[k] * dd[j] + L.c2[k] * rr[j];
-                xx[j] += dd[j];
-                dout[R.i[j]] = dd[j];
-            }
+        if (R.on()) {
+            rr -= R.scaled(din);
+            dd = L.c1[k] * dd + L.c2[k] * rr;
+            xx += dd;
+            dout[R.at] = dd;
+        }
         float* t = din;
         din = dout;
         dout = t;
     }
-#pragma unroll
-    for (int j = 0; j < RP; ++j)
-        if (R.on(j)) v.x[R.i[j]] = xx[j];
+    if (R.on()) v.x[R.at] = xx;
     __syncthreads();
-#pragma unroll
-    for (int j = 0; j < RP; ++j)
-        if (R.on(j)) {
-            const uint32_t i = R.i[j];
-            v.r[i] = v.b[i] - R.product(j, v.x);
-        }
+    if (R.on()) v.r[R.at] = v.b[R.at] - R.product(v.x);
     __syncthreads();
 }
 // post-smoothing from v.x
-template <int RP, int HELD, int LANES>
-__device__ __forceinline__ void bottom_up(const BottomLevel& L, const BottomRows<RP, HELD, LANES>& R,
+template <int HELD, int LANES>
+__device__ __forceinline__ void bottom_up(const BottomLevel& L, const BottomRows<HELD, LANES>& R,
                                           const BottomVec& v) {
-    float rr[RP], xx[RP], dd[RP];
-#pragma unroll
-    for (int j = 0; j < RP; ++j)
-        if (R.on(j)) {
-            const uint32_t i = R.i[j];
-            xx[j] = v.x[i];
-            rr[j] = R.dinv[j] * (v.b[i] - R.product(j, v.x));
-            dd[j] = rr[j] * L.inv_theta;
-            v.d[i] = dd[j];
-        }
+    float rr = 0.f, xx = 0.f, dd = 0.f;
+    if (R.on()) {
+        xx = v.x[R.at];
+        rr = R.dinv * (v.b[R.at] - R.product(v.x));
+        dd = rr * L.inv_theta;
+        v.d[R.at] = dd;
+    }
     float *din = v.d, *dout = v.r;
     for (uint32_t k = 1; k < L.degree; ++k) {
         __syncthreads();
-#pragma unroll
-        for (int j = 0; j < RP; ++j)
-            if (R.on(j)) {
-                rr[j] -= R.dinv[j] * R.product(j, din);
-                const float dn = L.c1[k] * dd[j] + L.c2[k] * rr[j];
-                xx[j] += k == 1 ? dd[j] + dn : dn;
-                dd[j] = dn;
-                dout[R.i[j]] = dn;
-            }
+        if (R.on()) {
+            rr -= R.scaled(din);
+            const float dn = L.c1[k] * dd + L.c2[k] * rr;
+            xx += k == 1 ? dd + dn : dn;
+            dd = dn;
+            dout[R.at] = dn;
+        }
         float* t = din;
         din = dout;
         dout = t;
     }
     __syncthreads();
-#pragma unroll
-    for (int j = 0; j < RP; ++j)
-        if (R.on(j)) v.x[R.i[j]] = xx[j];
+    if (R.on()) v.x[R.at] = xx;
     __syncthreads();
 }
 // y = B x, or y += B x (ADD); LANES lanes per block row
@@ -1076,10 +1054,10 @@ template <bool ADD, int LANES>
 __device__ __forceinline__ void bottom_apply(const Bell<3, 3>& B, uint32_t rows, const float* x,
                                              float* y) {
     const uint32_t lane = threadIdx.x % LANES;
-    for (uint32_t I = threadIdx.x / LANES; I < rows; I += BOTTOM_TB / LANES) {
+    for (uint32_t I = threadIdx.x / LANES; I < rows; I += blockDim.x / LANES) {
         float t[3];
-        bell_row<3, 3, LANES, LANES, 2>(B, 
-                                  BellHead{B.slice_ptr[I >> 6], I & 63, B.len[I], 0}, lane, x, t);
+        bell_row<3, 3, LANES, LANES, 2>(B, BellHead{B.slice_ptr[I >> 6], I & 63, B.len[I], 0}, lane,
+                                        x, t);
         if (lane == 0)
 #pragma unroll
             for (int r = 0; r < 3; ++r) y[3 * I + r] = ADD ? y[3 * I + r] + t[r] : t[r];
@@ -1097,17 +1075,17 @@ __device__ __forceinline__ void bottom_apply(const Bell<3, 3>& B, int lanes, uin
         default: bottom_apply<ADD, 16>(B, rows, x, y); break;
     }
 }
-template <int RP, int HELD, int LANES>
-__global__ __launch_bounds__(BOTTOM_TB) void k_amg_bottom(Bottom B, const PcgState* st) {
+template <int TB, int HELD, int LANES>
+__global__ __launch_bounds__(TB) void k_amg_bottom(Bottom B, const PcgState* st) {
     if (st->done) return;
     extern __shared__ float lds[];
     const BottomLevel& L0 = B.lv;
     const uint32_t n = 3 * L0.rows;
     const BottomVec v{lds, lds + n, lds + 2 * n, lds + 3 * n};
     float *bc = lds + 4 * n, *xc = bc + B.nco;
-    BottomRows<RP, HELD, LANES> R0;
+    BottomRows<HELD, LANES> R0;
     R0.load(L0);
-    for (uint32_t i = threadIdx.x; i < n; i += BOTTOM_TB) v.b[i] = B.b[i];
+    for (uint32_t i = threadIdx.x; i < n; i += TB) v.b[i] = B.b[i];
     __syncthreads();
     bottom_down(L0, R0, v);
     bottom_apply<false>(L0.T, L0.t_lanes, B.nco / 3, v.r, bc);
@@ -1122,7 +1100,7 @@ __global__ __launch_bounds__(BOTTOM_TB) void k_amg_bottom(Bottom B, const PcgSta
     __syncthreads();
     bottom_apply<true>(L0.P, L0.p_lanes, L0.rows, xc, v.x);
     bottom_up(L0, R0, v);
-    for (uint32_t i = threadIdx.x; i < n; i += BOTTOM_TB) B.x[i] = v.x[i];
+    for (uint32_t i = threadIdx.x; i < n; i += TB) B.x[i] = v.x[i];
 }
 
 // ---- a level between the finest and the bottom, on tiles ------------------------
@@ -1140,7 +1118,7 @@ __global__ __launch_bounds__(BOTTOM_TB) void k_amg_bottom(Bottom B, const PcgSta
 // 56.6, 256x128 84.1 -> 78.0, 512x256 137 -> 115, 1024x512 232 -> 210,
 // 2048x1024 572 -> 563.
 template <int HELD, int LANES>
-struct TileHeld : BottomRows<1, HELD, LANES> {
+struct TileHeld : BottomRows<HELD, LANES> {
     uint32_t I, r, act;  // block row, component, rings inside (0: the outermost)
     uint32_t own, all;   // rows owned, rows listed
     // false: the solve has ended, or the tile owns nothing
@@ -1162,24 +1140,20 @@ struct TileHeld : BottomRows<1, HELD, LANES> {
         for (uint32_t k = 0; k < T.rings; ++k)
             act += e < (uint32_t)__builtin_amdgcn_readlane(ro, k);
         if (!valid) act = 0;
-        this->i[0] = valid ? 3 * e + r : this->NO_ROW;
+        this->at = valid ? 3 * e + r : this->NO_ROW;
         I = valid ? T.ids[(size_t)tile * T.ext + e] : 0;
 #pragma unroll
         for (int k = 0; k < HELD / 2; ++k) {
             uint32_t w = 0;
             if (act && k < (int)T.W2) w = T.lcol[((size_t)tile * T.W2 + k) * T.ext + e];
-            this->col[0][k] = (3 * (w & 0xffffu)) | ((3 * (w >> 16)) << 16);
+            this->col[k] = (3 * (w & 0xffffu)) | ((3 * (w >> 16)) << 16);
         }
-        this->template load_row<false>(L, 0, I, r, act != 0);
-        if (valid) this->dinv[0] = L.dinv[3 * (size_t)I + r];
+        this->template load_row<false>(L, I, r, act != 0);
+        if (valid) this->dinv = L.dinv[3 * (size_t)I + r];
         return true;
     }
-    __device__ __forceinline__ bool owned() const { return this->on(0) && this->i[0] < 3 * own; }
+    __device__ __forceinline__ bool owned() const { return this->on() && this->at < 3 * own; }
     __device__ __forceinline__ size_t global() const { return 3 * (size_t)I + r; }
-    __device__ __forceinline__ uint32_t at() const { return this->i[0]; }
-    __device__ __forceinline__ float scaled(const float* x) const {   // (D^-1 A x) of the row
-        return this->dinv[0] * this->product(0, x);
-    }
 };
 template <int TB, int HELD, int LANES>
 __global__ __launch_bounds__(TB) void k_amg_down(BottomLevel L, Tiles T,
@@ -1191,12 +1165,12 @@ __global__ __launch_bounds__(TB) void k_amg_down(BottomLevel L, Tiles T,
     if (!R.load(L, T, st)) return;
     float *din = lds, *dout = lds + 3 * R.all, *xs = lds + 6 * R.all;
     float bb = 0.f, rr = 0.f, xx = 0.f, dd = 0.f;
-    if (R.on(0)) {
+    if (R.on()) {
         bb = b[R.global()];
-        rr = R.dinv[0] * bb;
+        rr = R.dinv * bb;
         dd = rr * L.inv_theta;
         xx = dd;
-        din[R.at()] = dd;
+        din[R.at] = dd;
     }
     for (uint32_t k = 1; k < L.degree; ++k) {
         __syncthreads();
@@ -1204,16 +1178,16 @@ __global__ __launch_bounds__(TB) void k_amg_down(BottomLevel L, Tiles T,
             rr -= R.scaled(din);
             dd = L.c1[k] * dd + L.c2[k] * rr;
             xx += dd;
-            dout[R.at()] = dd;
+            dout[R.at] = dd;
         }
         float* t = din;
         din = dout;
         dout = t;
     }
-    if (R.on(0)) xs[R.at()] = xx;
+    if (R.on()) xs[R.at] = xx;
     __syncthreads();
     if (R.owned()) {
-        r[R.global()] = bb - R.product(0, xs);
+        r[R.global()] = bb - R.product(xs);
         x[R.global()] = xx;
     }
 }
@@ -1228,7 +1202,7 @@ __global__ __launch_bounds__(TB) void k_amg_up(BottomLevel L, Tiles T,
     if (!R.load(L, T, st)) return;
     float *din = lds, *dout = lds + 3 * R.all, *xs = lds + 6 * R.all;
     float rr = 0.f, xx = 0.f, dd = 0.f;
-    if (R.on(0)) {   // x + P xc, by one lane a row
+    if (R.on()) {   // x + P xc, by one lane a row
         const uint32_t I = R.I;
         const Bell<3, 3>& P = L.P;
         uint32_t base = (I >> 6) * SLICE * P.width + (I & 63), len = P.width;
@@ -1258,13 +1232,13 @@ __global__ __launch_bounds__(TB) void k_amg_up(BottomLevel L, Tiles T,
                     for (int c = 0; c < 3; ++c) y += a[u][c] * v[u][c];
         }
         xx = x[R.global()] + y;
-        xs[R.at()] = xx;
+        xs[R.at] = xx;
     }
     __syncthreads();
     if (R.act) {
-        rr = R.dinv[0] * (b[R.global()] - R.product(0, xs));
+        rr = R.dinv * (b[R.global()] - R.product(xs));
         dd = rr * L.inv_theta;
-        din[R.at()] = dd;
+        din[R.at] = dd;
     }
     for (uint32_t k = 1; k < L.degree; ++k) {
         __syncthreads();
@@ -1273,7 +1247,7 @@ __global__ __launch_bounds__(TB) void k_amg_up(BottomLevel L, Tiles T,
             const float dn = L.c1[k] * dd + L.c2[k] * rr;
             xx += k == 1 ? dd + dn : dn;
             dd = dn;
-            dout[R.at()] = dn;
+            dout[R.at] = dn;
         }
         float* t = din;
         din = dout;
@@ -1390,18 +1364,32 @@ static bool grouped(uint32_t rows, int R, int C, const HostVec<uint32_t>& ptr,
     return true;
 }
 
-// k_amg_bottom's form for level L: 1 or 2 scalar rows per thread of up to 14
-// blocks (the coarse levels of structured T3 meshes have 11-13), 3: one row
-// of up to 24; 0 none.  Three rows per thread do not fit the registers (37
-// spilled) and take 57 us at 1,050 unknowns, as long as the launches they
-// replace.  Rows of 5 to 20 blocks on average, that is 2 or 4 lanes in the
-// kernels of one step: thinner and denser levels are too rare to pay for more
-// forms.
-static int bottom_kind(const AmgDevLevel& L) {
+// Most scalar rows of level L that a workgroup holds, one a thread: 1,024 of up
+// to 14 blocks (the coarse levels of structured T3 meshes have 11-13), 512 of
+// up to 24; 0 where the rows do not fit.  Rows of 5 to 20 blocks on average,
+// that is 2 or 4 lanes in the kernels of one step: thinner and denser levels
+// are too rare to pay for more forms.
+static uint32_t held_rows(const AmgDevLevel& L) {
     if (L.ab.lanes != 2 && L.ab.lanes != 4) return 0;
-    const uint32_t rows = (L.n + BOTTOM_TB - 1) / BOTTOM_TB;
-    if (L.ab.wmax <= 14 && rows <= 2) return (int)rows;
-    return L.ab.wmax <= 24 && rows == 1 ? 3 : 0;
+    return L.ab.wmax <= 14 ? 1024 : L.ab.wmax <= 24 ? 512 : 0;
+}
+static bool bottom_fits(const AmgDevLevel& L) { return L.n <= held_rows(L); }
+// f(threads, HELD, LANES) for a workgroup of `rows` scalar rows of level V
+template <class F>
+static void with_row_form(const AmgDevLevel& V, uint32_t rows, F&& f) {
+    using std::integral_constant;
+    auto lanes = [&](auto tb, auto held) {
+        if (V.ab.lanes == 2)
+            f(tb, held, integral_constant<int, 2>{});
+        else
+            f(tb, held, integral_constant<int, 4>{});
+    };
+    if (V.ab.wmax > 14)
+        lanes(integral_constant<int, 512>{}, integral_constant<int, 24>{});
+    else if (rows <= 512)
+        lanes(integral_constant<int, 512>{}, integral_constant<int, 14>{});
+    else
+        lanes(integral_constant<int, 1024>{}, integral_constant<int, 14>{});
 }
 
 // The mean place of each aggregate's nodes (the next level's nodes)
@@ -1419,19 +1407,15 @@ static std::vector<double> mean_places(const AmgHostLevel& h, const std::vector<
     return out;
 }
 
-// Most block rows of a tile of level L, 0: its rows do not fit the kernels'
-// forms (those of k_amg_bottom, a row's P by one lane).
-static uint32_t tile_limit(const AmgDevLevel& L) {
-    if ((L.ab.lanes != 2 && L.ab.lanes != 4) || L.pb.lanes != 1) return 0;
-    return L.ab.wmax <= 14 ? 1024 / 3 : L.ab.wmax <= 24 ? 512 / 3 : 0;
-}
 // Tiles of a level of fewer than BELL_LARGE block rows (larger ones are bound by
 // bytes, of which the rings read more), at most 256, which run at once (a tile
 // takes a CU: 19,608 rows of degree 4 in 990 tiles take 644 us per outer
 // iteration instead of 563 with a launch per step), of about 8 rows at least
 // (a launch takes as long as its largest tile: 16 rows 1-2 us more).
 static int level_tiles(AmgDevLevel& L, const std::vector<double>& xy, hipStream_t s) {
-    const uint32_t rows = L.n / 3, limit = tile_limit(L), rings = (uint32_t)L.degree;
+    // (a row's P by one lane, as the prolongation's kernel sums it)
+    const uint32_t limit = L.pb.lanes == 1 ? held_rows(L) / 3 : 0;
+    const uint32_t rows = L.n / 3, rings = (uint32_t)L.degree;
     if (!limit || rows >= BELL_LARGE || rows < 64) return NBX_OK;
     const uint32_t cells = std::max(std::min(256u, rows / 8), 1u);
     double2* d = nullptr;
@@ -1566,7 +1550,7 @@ static int amg_symbolic(FemSys& S) {
                 NBX_TRY((bell_upload<3, 3>(L.n / 3, plen, pcol, L.pb, A->bytes)));
                 NBX_TRY((bell_upload<3, 3>(L.nc / 3, tlen, tcol, L.tb, A->bytes)));
                 // (the last smoothed level: with the dense solve, where it can)
-                if (l + 2 < nl || !bottom_kind(L)) NBX_TRY(level_tiles(L, xy, S.s));
+                if (l + 2 < nl || !bottom_fits(L)) NBX_TRY(level_tiles(L, xy, S.s));
             }
             NBX_TRY(up(&L.t, h.t, A->bytes));
             NBX_TRY(up(&L.agg, h.agg, A->bytes));
@@ -1582,7 +1566,7 @@ static int amg_symbolic(FemSys& S) {
         }
     }
     // the last smoothed level in one workgroup with the dense solve
-    if (nl >= 3 && bottom_kind(A->lv[nl - 2])) A->bottom = nl - 2;
+    if (nl >= 3 && bottom_fits(A->lv[nl - 2])) A->bottom = nl - 2;
     const uint32_t nco = A->lv.back().n;
     NBX_TRY(alloc(&A->cinv, (size_t)nco * nco, A->bytes));
     NBX_TRY(alloc(&A->ones, n, A->bytes));
@@ -1898,27 +1882,10 @@ static BottomLevel level_args(const AmgDevLevel& V) {
     return L;
 }
 
-// f(TB, HELD, LANES) of k_amg_down and k_amg_up for a level on tiles
-template <class F>
-static void with_tile_form(const AmgDevLevel& V, F&& f) {
-    using std::integral_constant;
-    auto lanes = [&](auto tb, auto held) {
-        if (V.ab.lanes == 2)
-            f(tb, held, integral_constant<int, 2>{});
-        else
-            f(tb, held, integral_constant<int, 4>{});
-    };
-    if (V.ab.wmax > 14)
-        lanes(integral_constant<int, 512>{}, integral_constant<int, 24>{});
-    else if (3 * V.tiles.most <= 512)
-        lanes(integral_constant<int, 512>{}, integral_constant<int, 14>{});
-    else
-        lanes(integral_constant<int, 1024>{}, integral_constant<int, 14>{});
-}
 static void tile_down(const AmgDevLevel& V, const float* b, float* x, const PcgState* st,
                       hipStream_t s) {
     const size_t lds = 9 * (size_t)V.tiles.most * sizeof(float);
-    with_tile_form(V, [&](auto tb, auto held, auto ln) {
+    with_row_form(V, 3 * V.tiles.most, [&](auto tb, auto held, auto ln) {
         constexpr int TB = decltype(tb)::value, HELD = decltype(held)::value;
         hipLaunchKernelGGL((k_amg_down<TB, HELD, decltype(ln)::value>), dim3(V.tiles.n), dim3(TB),
                            lds, s, level_args(V), V.tiles, b, x, V.r, st);
@@ -1927,7 +1894,7 @@ static void tile_down(const AmgDevLevel& V, const float* b, float* x, const PcgS
 static void tile_up(const AmgDevLevel& V, const float* b, const float* x, const float* xc,
                     const PcgState* st, hipStream_t s) {
     const size_t lds = 9 * (size_t)V.tiles.most * sizeof(float);
-    with_tile_form(V, [&](auto tb, auto held, auto ln) {
+    with_row_form(V, 3 * V.tiles.most, [&](auto tb, auto held, auto ln) {
         constexpr int TB = decltype(tb)::value, HELD = decltype(held)::value;
         hipLaunchKernelGGL((k_amg_up<TB, HELD, decltype(ln)::value>), dim3(V.tiles.n), dim3(TB),
                            lds, s, level_args(V), V.tiles, b, x, xc, V.d0, st);
@@ -1945,19 +1912,11 @@ static void bottom_cycle(AmgDev* A, const float* b, float* x, const PcgState* st
     B.b = b;
     B.x = x;
     const size_t lds = (4 * (size_t)V.n + 2 * (size_t)C.n) * sizeof(float);
-    const dim3 g(1), t(BOTTOM_TB);
-    auto launch = [&](auto ln) {
-        constexpr int LN = decltype(ln)::value;
-        switch (bottom_kind(V)) {
-            case 1: hipLaunchKernelGGL((k_amg_bottom<1, 14, LN>), g, t, lds, s, B, st); break;
-            case 2: hipLaunchKernelGGL((k_amg_bottom<2, 14, LN>), g, t, lds, s, B, st); break;
-            default: hipLaunchKernelGGL((k_amg_bottom<1, 24, LN>), g, t, lds, s, B, st); break;
-        }
-    };
-    if (V.ab.lanes == 2)
-        launch(std::integral_constant<int, 2>{});
-    else
-        launch(std::integral_constant<int, 4>{});
+    with_row_form(V, V.n, [&](auto tb, auto held, auto ln) {
+        constexpr int TB = decltype(tb)::value, HELD = decltype(held)::value;
+        hipLaunchKernelGGL((k_amg_bottom<TB, HELD, decltype(ln)::value>), dim3(1), dim3(TB), lds, s,
+                           B, st);
+    });
 }
 
 // The V-cycle from level l0 >= 1 down, x = M^-1 b on that level (b, x: that
