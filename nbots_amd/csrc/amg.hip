@@ -1314,8 +1314,8 @@ static int bell_upload(uint32_t rows, Len len_of, Col col_of, BellDev& B, size_t
     // One width for all slices where that adds little or the level is small:
     // a row's place then follows from its index, without the loads of its
     // slice and length before its blocks' (96x48 58 -> 53 us per outer
-    // iteration, 512x256 130 -> 127, 2048x1024 608 -> 598).  Padding blocks are zero, on the
-    // row's own first column: they add +0 to sums that are never -0.
+    // iteration, 512x256 130 -> 127, 2048x1024 608 -> 598).  Padding blocks are
+    // zero, on the row's own first column: they add +0 to sums that are never -0.
     for (uint16_t l : len) B.wmax = std::max<uint32_t>(B.wmax, l);
     const size_t same = (size_t)ns * SLICE * B.wmax;
     if (same <= 0xffffffffull && (same <= sp[ns] + (size_t)sp[ns] / 8 || same <= BELL_SMALL)) {
@@ -1324,8 +1324,8 @@ static int bell_upload(uint32_t rows, Len len_of, Col col_of, BellDev& B, size_t
         bcol.assign(same, 0);
     }
     for (uint32_t I = 0; I < rows; ++I) {
-        const uint32_t w = (sp[I / SLICE + 1] - sp[I / SLICE]) / SLICE;
-        for (uint32_t k = 0; k < w && len[I]; ++k)
+        const uint32_t w = len[I] ? std::max<uint32_t>(B.width, len[I]) : 0;
+        for (uint32_t k = 0; k < w; ++k)
             bcol[sp[I / SLICE] + (size_t)k * SLICE + I % SLICE] = col_of(I, k < len[I] ? k : 0);
     }
     B.rows = rows;
@@ -1340,7 +1340,7 @@ static int bell_upload(uint32_t rows, Len len_of, Col col_of, BellDev& B, size_t
     NBX_TRY(up(&B.len, len, bytes));
     NBX_TRY(up(&B.bcol, bcol, bytes));
     NBX_TRY(alloc(&B.val, B.slots * R * C, bytes));
-    NBX_HIP(hipMemset(B.val, 0, B.slots * R * C * sizeof(float)));
+    if (B.width) NBX_HIP(hipMemset(B.val, 0, B.slots * R * C * sizeof(float)));
     return NBX_OK;
 }
 
