@@ -4,11 +4,13 @@
 //   (solver_bot/sparse/solvers/cg_precond_jacobi.c:13-90).  Three kernels per
 //   iteration: SpMV + p.w, the g update + g.q and g.g, and the x and
 //   direction update (x += alpha p reads the p that the direction update
-//   reads anyway, so the vectors cross HBM 12 times per iteration, not 13).  Reducing kernels write one partial per workgroup; a one-
-//   workgroup finalize kernel sums them in index order and computes alpha,
-//   beta and the stop decision on the GPU (runs are reproducible, and no
-//   device-scope fence or atomic sits in the loop); the host only polls a
-//   done flag between batches of iterations.
+//   reads anyway, so the vectors cross HBM 12 times per iteration, not 13).
+//   Reducing kernels write one partial per workgroup; a one-workgroup
+//   finalize kernel sums them in index order and computes alpha, beta and the
+//   stop decision on the GPU (runs are reproducible, and no device-scope fence
+//   or atomic sits in the loop); the host only polls a done flag between
+//   batches of iterations.  Small and medium systems take two kernels per
+//   iteration, whose workgroups each add the partials themselves (k_cg_dir).
 // * Mixed precision: CG on the Jacobi-scaled FP32 copy D^-1/2 K D^-1/2 with
 //   FP32 vectors and compensated FP32 dot products, and FP64 reliable updates
 //   (Sleijpen & van der Vorst 1996): when the iterated residual has dropped
