@@ -141,10 +141,18 @@ __device__ __forceinline__ double2 row64(const Sell2& A, uint32_t v, const doubl
 // Lower and upper blocks are taken UL and UU at a time; few registers per
 // row keep many waves resident, which hides the dependent loads better than
 // longer batches.  An interior row of a T3 mesh has 3 lower and 3 upper
-// blocks: the streamed product takes them 3 and 3 (70 VGPRs, 7 waves per
-// SIMD), the cached one 4 and 4 (84 VGPRs, 5 waves), which measured faster
-// where the matrix is read from cache.  Issuing the diagonal loads after the
-// lower blocks instead saves registers but exposes their latency.
+// blocks: the streamed product takes them 3 and 3 (76 VGPRs, 6 waves per
+// SIMD), the cached one 4 and 4 (94 VGPRs, 5 waves; 3 and 3 measure the same).
+// Bound by the chain of dependent loads below the Infinity Cache's size: row
+// lengths, the indexes of both parts and, without waiting for the offsets
+// where every slice has one width, the first batch's places come in one trip,
+// then the lower blocks with x, then the upper blocks with x: three trips
+// instead of six.  us per iteration of the FP64 PCG, before -> after: 800x400
+// 28.4 -> 26.9, 1024x512 39.2 -> 36.3, 1200x600 49.5 -> 45.3, 1430x720 66.4 ->
+// 61.9; streamed, 2048x1024 119.0 -> 118.2.  The widths alone: 1024x512 37.7;
+// the first upper values in the first trip as well (100 VGPRs, 4 waves): 36.7,
+// and 134 at 2048x1024.  Issuing the diagonal loads after the lower blocks
+// saves registers but exposes their latency.
 // NT: non-temporal loads of the matrix stream (when the working set exceeds
 // the Infinity Cache); otherwise ordinary loads, so that the matrix stays
 // cached from one product to the next.
@@ -159,38 +167,60 @@ template <int UL, int UU, bool NT = true>
 __device__ __forceinline__ double2 row64s(const Sym2& Y, uint32_t v, const double2* __restrict__ x) {
     const dv2* __restrict__ pa = reinterpret_cast<const dv2*>(Y.u_val);
     const dv2* __restrict__ pb = reinterpret_cast<const dv2*>(Y.u_val + 2 * Y.n_upper);
+    const uv2* __restrict__ li = reinterpret_cast<const uv2*>(Y.l_idx);
+    const int llen = Y.l_rowlen[v], ulen = Y.u_rowlen[v];
     const dv2 d01 = ldm<NT>(reinterpret_cast<const dv2*>(Y.d_val) + v);
     const double d11 = ldm<NT>(Y.d_val + 2 * (size_t)Y.n_nodes + v);
     const double2 xd = x[v];
+    size_t lbase = v & 63, ubase = v & 63;
+    int ln = llen, un = ulen;
+    if (Y.l_width) {
+        lbase += (size_t)(v >> 6) * SLICE * Y.l_width;
+        ln = (int)Y.l_width;
+    } else {
+        lbase += (size_t)Y.l_slice_ptr[v >> 6];
+    }
+    if (Y.u_width) {
+        ubase += (size_t)(v >> 6) * SLICE * Y.u_width;
+        un = (int)Y.u_width;
+    } else {
+        ubase += (size_t)Y.u_slice_ptr[v >> 6];
+    }
+    uv2 e[UL];
+    uint32_t w[UU];
+    auto lower_idx = [&](int k0, int n) {
+#pragma unroll
+        for (int k = 0; k < UL; ++k)
+            if (k0 + k < n) e[k] = ldm<NT>(&li[lbase + (size_t)(k0 + k) * SLICE]);
+    };
+    auto upper_idx = [&](int k0, int n) {
+#pragma unroll
+        for (int k = 0; k < UU; ++k)
+            if (k0 + k < n) w[k] = ldm<NT>(&Y.u_bcol[ubase + (size_t)(k0 + k) * SLICE]);
+    };
+    lower_idx(0, ln);
+    upper_idx(0, un);
     double s0 = 0.0, s1 = 0.0;
-    {
-        const uv2* __restrict__ li = reinterpret_cast<const uv2*>(Y.l_idx);
-        const size_t base = (size_t)Y.l_slice_ptr[v >> 6] + (v & 63);
-        const int len = Y.l_rowlen[v];
-        for (int k0 = 0; k0 < len; k0 += UL) {
-            uv2 e[UL];
-            dv2 a[UL], b[UL];
-            double2 xv[UL];
+    for (int k0 = 0; k0 < llen; k0 += UL) {
+        dv2 a[UL], b[UL];
+        double2 xv[UL];
+        if (k0) lower_idx(k0, llen);
 #pragma unroll
-            for (int k = 0; k < UL; ++k)
-                if (k0 + k < len) e[k] = ldm<NT>(&li[base + (size_t)(k0 + k) * SLICE]);
-#pragma unroll
-            for (int k = 0; k < UL; ++k) {
-                if (k0 + k < len) {
-                    a[k] = pa[e[k].y];
-                    b[k] = pb[e[k].y];
-                    xv[k] = x[e[k].x];
-                }
+        for (int k = 0; k < UL; ++k) {
+            if (k0 + k < llen) {
+                a[k] = pa[e[k].y];
+                b[k] = pb[e[k].y];
+                xv[k] = x[e[k].x];
             }
-            // block (v, w) = [[a.x, b.x], [a.y, b.y]]
+        }
+        // block (v, w) = [[a.x, b.x], [a.y, b.y]]
 #pragma unroll
-            for (int k = 0; k < UL; ++k) {
-                if (k0 + k < len) {
-                    s0 = s0 + a[k].x * xv[k].x;
-                    s0 = s0 + b[k].x * xv[k].y;
-                    s1 = s1 + a[k].y * xv[k].x;
-                    s1 = s1 + b[k].y * xv[k].y;
-                }
+        for (int k = 0; k < UL; ++k) {
+            if (k0 + k < llen) {
+                s0 = s0 + a[k].x * xv[k].x;
+                s0 = s0 + b[k].x * xv[k].y;
+                s1 = s1 + a[k].y * xv[k].x;
+                s1 = s1 + b[k].y * xv[k].y;
             }
         }
     }
@@ -199,33 +229,26 @@ __device__ __forceinline__ double2 row64s(const Sym2& Y, uint32_t v, const doubl
     s0 = s0 + d01.y * xd.y;
     s1 = s1 + d01.y * xd.x;
     s1 = s1 + d11 * xd.y;
-    {
-        const size_t base = (size_t)Y.u_slice_ptr[v >> 6] + (v & 63);
-        const int len = Y.u_rowlen[v];
-        for (int k0 = 0; k0 < len; k0 += UU) {
-            uint32_t w[UU];
-            dv2 a[UU], b[UU];
-            double2 xv[UU];
+    for (int k0 = 0; k0 < ulen; k0 += UU) {
+        dv2 a[UU], b[UU];
+        double2 xv[UU];
+        if (k0) upper_idx(k0, ulen);
 #pragma unroll
-            for (int k = 0; k < UU; ++k) {
-                if (k0 + k < len) {
-                    const size_t i = base + (size_t)(k0 + k) * SLICE;
-                    w[k] = ldm<NT>(&Y.u_bcol[i]);
-                    a[k] = ldm<NT>(&pa[i]);
-                    b[k] = ldm<NT>(&pb[i]);
-                }
+        for (int k = 0; k < UU; ++k) {
+            if (k0 + k < ulen) {
+                const size_t i = ubase + (size_t)(k0 + k) * SLICE;
+                a[k] = ldm<NT>(&pa[i]);
+                b[k] = ldm<NT>(&pb[i]);
+                xv[k] = x[w[k]];
             }
+        }
 #pragma unroll
-            for (int k = 0; k < UU; ++k)
-                if (k0 + k < len) xv[k] = x[w[k]];
-#pragma unroll
-            for (int k = 0; k < UU; ++k) {
-                if (k0 + k < len) {
-                    s0 = s0 + a[k].x * xv[k].x;
-                    s0 = s0 + a[k].y * xv[k].y;
-                    s1 = s1 + b[k].x * xv[k].x;
-                    s1 = s1 + b[k].y * xv[k].y;
-                }
+        for (int k = 0; k < UU; ++k) {
+            if (k0 + k < ulen) {
+                s0 = s0 + a[k].x * xv[k].x;
+                s0 = s0 + a[k].y * xv[k].y;
+                s1 = s1 + b[k].x * xv[k].x;
+                s1 = s1 + b[k].y * xv[k].y;
             }
         }
     }
