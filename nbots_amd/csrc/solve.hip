@@ -555,12 +555,72 @@ __global__ __launch_bounds__(BLOCK) void k_cg_dir(Op op,
 // the reference sums a row.  A tile's loads are issued before the sums of
 // the tile before it.
 // PER entries per thread and tile: 16 take a whole 256-row group of up to 16
-// entries a row at once (168 VGPRs, which is no matter while there is one
-// workgroup per CU or less), 8 leave more waves to a larger matrix.
+// entries a row at once (182 VGPRs, which is no matter while there are two
+// workgroups per CU or less), 8 leave more waves to a larger matrix.
 // us per iteration (five kernels -> two): 4,290 rows 21 -> 12.4, 41,004 rows
 // 20.6 -> 13.1, 90,902 rows 24 -> 13.9 with 16 and 14.3 with 8, 257,442 rows
 // 94 -> 21 with 8 and 27 with 16.
+// A tile holds few long rows, whose threads add thousands of entries one after
+// another while the others wait.  Where a workgroup's rows have 64 entries or
+// more on average and none is much longer than the rest, it takes STRIP entries
+// of every row at a time instead (8 of 8 bytes are half a cache line, and the
+// rest of the line is still cached for the next strip).  us per iteration, five
+// kernels -> two with tiles -> with strips: 2,001 rows of 33 entries 29.7 -> 22.3
+// (tiles), of 129 59 -> 76 -> 31, of 2,001 1,526 -> 8,297 -> 467; 20,001 of 65 43
+// -> 36 -> 22, of 513 365 -> 704 -> 114; 100,001 of 129 197 -> 112 -> 77; every
+// tenth of 2,001 rows full, the others of 5 entries, 337 -> 871 -> 310.  Beyond
+// CSR_WIDE_ROWS four workgroups a CU hide each other's sums and strips of 4, all
+// that their registers leave room for, lose the lines to one another: 250,001 of
+// 65 633 -> 89 -> 190, of 257 2,429 -> 466 -> 674; they keep the tiles.  One row
+// of 9,000 entries among short ones: 1,183 -> 306 with tiles.
 constexpr uint32_t CSR_WIDE_ROWS = 131072;   // PER 16 up to here
+constexpr int STRIP = 8;
+constexpr uint32_t STRIP_MIN = 64 * BLOCK;   // a workgroup's entries from which strips are taken
+constexpr uint32_t STRIP_EVEN = 16;          // ... if they are so many times its longest row's
+// The thread's row of a workgroup's 256, by strips (rp: where the rows begin,
+// the last one's end after them; prod: STRIP + 1 values a row)
+__device__ __forceinline__ double strip_sum(const DevCsr& A, const CgPair<double>* __restrict__ d,
+                                            const CgDir& dir, const uint32_t* rp, uint32_t longest,
+                                            double* prod) {
+    constexpr unsigned AT_ONCE = BLOCK / STRIP, STRIDE = STRIP + 1;   // (a row apart, off the banks)
+    const unsigned row0 = threadIdx.x / STRIP, lane = threadIdx.x % STRIP;
+    const uint32_t len = rp[threadIdx.x + 1] - rp[threadIdx.x];
+    double av[STRIP], s = 0.0;
+    CgPair<double> dv[STRIP];
+    auto fetch = [&](uint32_t base) {   // (zeros past a row's end)
+        uint32_t col[STRIP];
+#pragma unroll
+        for (int i = 0; i < STRIP; ++i) {
+            const unsigned row = row0 + (unsigned)i * AT_ONCE;
+            const uint32_t beg = rp[row];
+            col[i] = 0;
+            av[i] = 0.0;
+            if (base + lane < rp[row + 1] - beg) {
+                col[i] = A.col[(size_t)beg + base + lane];
+                av[i] = A.val[(size_t)beg + base + lane];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < STRIP; ++i) dv[i] = d[col[i]];
+    };
+    fetch(0);
+    for (uint32_t base = 0; base < longest; base += STRIP) {
+#pragma unroll
+        for (int i = 0; i < STRIP; ++i)
+            prod[(row0 + (unsigned)i * AT_ONCE) * STRIDE + lane] = av[i] * dir(dv[i]);
+        __syncthreads();
+        if (base + STRIP < longest) fetch(base + STRIP);
+        for (unsigned t = 0; t < STRIP && base + t < len; t += 4) {   // four reads in flight
+            double v[4];
+#pragma unroll
+            for (unsigned k = 0; k < 4; ++k) v[k] = prod[threadIdx.x * STRIDE + t + k];
+#pragma unroll
+            for (unsigned k = 0; k < 4; ++k) s = base + t + k < len ? s + v[k] : s;
+        }
+        __syncthreads();
+    }
+    return s;
+}
 template <int PER>
 __global__ __launch_bounds__(BLOCK) void k_cg_dir_csr(DevCsr A,
                                                       const CgPair<double>* __restrict__ d,
@@ -571,7 +631,10 @@ __global__ __launch_bounds__(BLOCK) void k_cg_dir_csr(DevCsr A,
                                                       const double* __restrict__ upd,
                                                       double* dirp, uint32_t n, bool first) {
     constexpr int TILE = PER * BLOCK;
+    constexpr bool STRIPS = PER == 16;
+    static_assert(!STRIPS || (STRIP + 1) * BLOCK <= TILE, "a strip's products lie in prod");
     __shared__ double red[2][ALL_PARTS / WAVE], prod[TILE], red2[1][BLOCK / WAVE];
+    __shared__ uint32_t rp[STRIPS ? BLOCK + 1 : 1], wlen[BLOCK / WAVE];
     const Chunk c = my_chunk(n);
     const size_t u = c.beg + threadIdx.x;
     const bool valid = u < c.end;
@@ -584,6 +647,21 @@ __global__ __launch_bounds__(BLOCK) void k_cg_dir_csr(DevCsr A,
         r0 = A.rowptr[u];
         r1 = A.rowptr[u + 1];
         own = d[u];
+    }
+    uint32_t longest = 0;   // the longest row's entries where strips are taken
+    if constexpr (STRIPS) {
+        if (e1 - e0 >= STRIP_MIN) {
+            uint32_t m = r1 - r0;
+            for (int off = WAVE / 2; off > 0; off >>= 1)
+                m = max(m, (uint32_t)__shfl_xor((int)m, off));
+            if (threadIdx.x % WAVE == 0) wlen[threadIdx.x / WAVE] = m;
+            rp[threadIdx.x] = r0;
+            if (threadIdx.x == 0) rp[BLOCK] = e1;
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < BLOCK / WAVE; ++k) longest = max(longest, wlen[k]);
+            if ((uint64_t)longest * STRIP_EVEN > e1 - e0) longest = 0;
+        }
     }
     double av[PER];
     CgPair<double> dv[PER];
@@ -601,29 +679,33 @@ __global__ __launch_bounds__(BLOCK) void k_cg_dir_csr(DevCsr A,
         for (int i = 0; i < PER; ++i)
             if (base + threadIdx.x + (unsigned)i * BLOCK < e1) dv[i] = d[col[i]];
     };
-    fetch(e0);
+    if (!longest) fetch(e0);
     CgDir dir;
     if (!cg_next(sin, sout, sums, first, red, dir)) return;
     double s = 0.0;
-    for (uint64_t base = e0; base < e1; base += TILE) {
-        const uint32_t m = (uint32_t)min((uint64_t)TILE, e1 - base);
+    if (longest) {
+        s = strip_sum(A, d, dir, rp, longest, prod);
+    } else {
+        for (uint64_t base = e0; base < e1; base += TILE) {
+            const uint32_t m = (uint32_t)min((uint64_t)TILE, e1 - base);
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const uint32_t t = threadIdx.x + (unsigned)i * BLOCK;
-            if (t < m) prod[t] = av[i] * dir(dv[i]);
+            for (int i = 0; i < PER; ++i) {
+                const uint32_t t = threadIdx.x + (unsigned)i * BLOCK;
+                if (t < m) prod[t] = av[i] * dir(dv[i]);
+            }
+            __syncthreads();
+            fetch(base + TILE);   // (nothing past the last entry)
+            const uint32_t lo = r0 > base ? (uint32_t)(r0 - base) : 0u;
+            const uint32_t hi = r1 > base ? (uint32_t)min((uint64_t)m, r1 - base) : 0u;
+            for (uint32_t t = lo; t < hi; t += 8) {   // eight reads in flight, added in order
+                double v[8];
+#pragma unroll
+                for (uint32_t k = 0; k < 8; ++k) v[k] = t + k < hi ? prod[t + k] : 0.0;
+#pragma unroll
+                for (uint32_t k = 0; k < 8; ++k) s = t + k < hi ? s + v[k] : s;
+            }
+            __syncthreads();
         }
-        __syncthreads();
-        fetch(base + TILE);   // (nothing past the last entry)
-        const uint32_t lo = r0 > base ? (uint32_t)(r0 - base) : 0u;
-        const uint32_t hi = r1 > base ? (uint32_t)min((uint64_t)m, r1 - base) : 0u;
-        for (uint32_t t = lo; t < hi; t += 8) {   // eight reads in flight, added in order
-            double v[8];
-#pragma unroll
-            for (uint32_t k = 0; k < 8; ++k) v[k] = t + k < hi ? prod[t + k] : 0.0;
-#pragma unroll
-            for (uint32_t k = 0; k < 8; ++k) s = t + k < hi ? s + v[k] : s;
-        }
-        __syncthreads();
     }
     double acc[1] = {0.0};
     if (valid) {
