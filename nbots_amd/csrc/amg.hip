@@ -1422,9 +1422,11 @@ static int level_tiles(AmgDevLevel& L, const std::vector<double>& xy, hipStream_
     NBX_HIP(hipMalloc(&d, (size_t)rows * sizeof(double2)));
     hipError_t e = copy_on(d, xy.data(), (size_t)rows * sizeof(double2), hipMemcpyHostToDevice, s);
     int rc = NBX_OK;
+    std::vector<TileAttempt> attempts{{cells, rings, rings}};
+    if (cells < 256) attempts.push_back({std::min(256u, 2 * cells), rings, rings});
     if (e == hipSuccess)
         rc = tiles_build(L.tiles, TileRows<uint16_t>{L.ab.slice_ptr, L.ab.len, L.ab.bcol}, rows,
-                         L.ab.wmax, d, {{cells, rings}, {std::min(256u, 2 * cells), rings}}, limit, s);
+                         L.ab.wmax, d, attempts, limit, s);
     (void)hipFree(d);
     NBX_HIP(e);
     return rc;

@@ -196,7 +196,7 @@ int scan_u32(const uint32_t* in, uint32_t* out, size_t n, hipStream_t s);
 // have at most `limit` rows; T.n = 0 when none has.
 int tiles_build(Tiles& T, const Off16& O, uint32_t wmax, const double2* xy, hipStream_t s);
 struct TileAttempt {
-    uint32_t cells, rings;
+    uint32_t cells, rings, least;   // `rings` rings, or as many as fit but `least` at least
 };
 template <class Len>
 struct TileRows {   // block k of row v at slice_ptr[v / 64] + 64 k + v % 64

@@ -25,6 +25,8 @@ namespace {
 constexpr int TILE_TB = 1024;       // threads of the ring kernel = most rows of a tile
 constexpr uint32_t TILE_HASH = 4096;
 constexpr uint32_t NONE = 0xffffffffu;
+constexpr unsigned TOO_MANY = 0xffffffffu;
+constexpr uint32_t RINGS_MAX = 8;
 
 // per workgroup: smallest and largest x and y
 __global__ __launch_bounds__(BLOCK) void k_tile_bbox(const double2* __restrict__ xy, uint32_t n,
@@ -118,9 +120,10 @@ __device__ void tile_sort(uint32_t* list, uint32_t* tmp, uint32_t b, uint32_t e)
     __syncthreads();
 }
 
-// One workgroup per tile.  ext = 0: only info (the largest tile, a flag for
-// one beyond `limit` rows).  Otherwise the tile's list, ring
-// offsets and columns (row i's block 2 q + h in half h of word
+// One workgroup per tile.  ext = 0: only info[0], set by a tile that owns more
+// than `limit` rows, and info[r], r = 1 .. rings, the rows of the largest tile
+// of r rings (TOO_MANY: more than `limit`).  Otherwise the
+// tile's list, ring offsets and columns (row i's block 2 q + h in half h of word
 // lcol[(t W2 + q) ext + i]; padding names the row itself).
 template <class Len>
 __global__ __launch_bounds__(TILE_TB) void k_tile_rings(TileRows<Len> O,
@@ -138,7 +141,7 @@ __global__ __launch_bounds__(TILE_TB) void k_tile_rings(TileRows<Len> O,
     const uint32_t t = blockIdx.x, tid = threadIdx.x;
     const uint32_t o0 = ptr[t], c0 = ptr[t + 1] - o0;
     if (c0 > limit) {
-        if (tid == 0) info[1] = 1u;
+        if (tid == 0) info[0] = 1u;
         return;
     }
     for (uint32_t i = tid; i < TILE_HASH; i += TILE_TB) keys[i] = NONE;
@@ -168,18 +171,17 @@ __global__ __launch_bounds__(TILE_TB) void k_tile_rings(TileRows<Len> O,
         const uint32_t now = cnt;
         __syncthreads();
         if (now > limit) {
-            if (tid == 0) info[1] = 1u;
+            if (tid == 0)
+                for (uint32_t q = r; q <= rings; ++q) atomicMax(&info[q], TOO_MANY);
             return;
         }
+        if (!ext && tid == 0) atomicMax(&info[r], now);
         tile_sort(list, tmp, end, now);
         beg = end;
         end = now;
         if (ext && tid == 0) roff[(size_t)t * (rings + 1) + r] = end;
     }
-    if (!ext) {
-        if (tid == 0) atomicMax(&info[0], end);
-        return;
-    }
+    if (!ext) return;
     if (tid < end) slot[tile_find(keys, list[tid])] = (uint16_t)tid;
     __syncthreads();
     if (tid < end) {
@@ -212,7 +214,8 @@ void tiles_free(Tiles& T) {
 }
 
 // Cuts the n rows at positions xy into the first of `attempts` whose tiles have
-// at most `limit` rows.  Leaves T.n = 0 (nothing allocated) when none has, or
+// at most `limit` rows with `least` rings or more (as many of its `rings` as
+// fit).  Leaves T.n = 0 (nothing allocated) when none has, or
 // without device memory for them: the kernels that take one step per launch
 // then run.
 template <class Len>
@@ -248,11 +251,12 @@ static int tiles_cut(Tiles& T, const TileRows<Len>& O, uint32_t n, uint32_t wmax
         !(Lx + Ly > 0.0))
         return done(NBX_OK);
     if (hipMalloc(&cell, (size_t)n * 4) != hipSuccess ||
-        hipMalloc(&own, (size_t)n * 4) != hipSuccess || hipMalloc(&info, 16) != hipSuccess)
+        hipMalloc(&own, (size_t)n * 4) != hipSuccess ||
+        hipMalloc(&info, (RINGS_MAX + 1) * sizeof(unsigned)) != hipSuccess)
         return no_memory();
     const uint32_t W2 = (wmax + 1) / 2;
     for (const auto& at : attempts) {
-        const uint32_t rings = std::max(at.rings, 2u);
+        const uint32_t rings = std::min(at.rings, RINGS_MAX);
         // at most so many cells, about square
         const double cells = (double)at.cells;
         const double fx = Lx > 0.0 && Ly > 0.0
@@ -269,7 +273,7 @@ static int tiles_cut(Tiles& T, const TileRows<Len>& O, uint32_t n, uint32_t wmax
             hipMalloc(&ptr, ((size_t)nt + 1) * 4) != hipSuccess)
             return no_memory();
         hipLaunchKernelGGL(k_tile_zero, dim3(grid_for(nt)), dim3(BLOCK), 0, s, cnt, nt);
-        hipLaunchKernelGGL(k_tile_zero, dim3(1), dim3(BLOCK), 0, s, (uint32_t*)info, 4u);
+        hipLaunchKernelGGL(k_tile_zero, dim3(1), dim3(BLOCK), 0, s, (uint32_t*)info, RINGS_MAX + 1);
         hipLaunchKernelGGL(k_tile_count, dim3(grid_for(n)), dim3(BLOCK), 0, s, g, xy, n, cell, cnt);
         const int rc = scan_u32(cnt, ptr, nt, s);
         if (rc) return done(rc);
@@ -277,17 +281,19 @@ static int tiles_cut(Tiles& T, const TileRows<Len>& O, uint32_t n, uint32_t wmax
         hipLaunchKernelGGL(k_tile_fill, dim3(grid_for(n)), dim3(BLOCK), 0, s, cell, n, ptr, cnt, own);
         hipLaunchKernelGGL(k_tile_rings<Len>, dim3(nt), dim3(TILE_TB), 0, s, O, ptr, own, limit, rings,
                            wmax, W2, 0u, (uint32_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr, info);
-        unsigned hi[2] = {0, 1};   // the largest tile, one beyond TILE_TB rows
+        unsigned hi[RINGS_MAX + 1];
         if (hipGetLastError() != hipSuccess ||
             copy_on(hi, info, sizeof hi, hipMemcpyDeviceToHost, s) != hipSuccess) {
             set_last_error("tiles: halo rings");
             return done(NBX_ERR_HIP);
         }
-        if (hi[1]) continue;
+        uint32_t fit = hi[0] ? 0 : rings;
+        while (fit && hi[fit] > limit) --fit;
+        if (fit < at.least) continue;
         T.n = nt;
-        T.most = hi[0];
-        T.ext = (hi[0] + WAVE - 1) / WAVE * WAVE;
-        T.rings = rings;
+        T.most = hi[fit];
+        T.ext = (T.most + WAVE - 1) / WAVE * WAVE;
+        T.rings = fit;
         T.W2 = W2;
         break;
     }
@@ -323,30 +329,39 @@ int tiles_build(Tiles& T, const Off16& O, uint32_t wmax, const double2* xy, hipS
     // 128 -> 104, 700x350 158 -> 131, 800x400 196 -> 180; 1,024: 900x450 271 ->
     // 249, 1024x512 279 -> 268; 2048x1024 937 (979 in rounds of 512).  Longer
     // rows: 33k nodes 74.5 -> 73.8, 80k 151 -> 97, 136k 230 -> 127, 193k 325 ->
-    // 207.
+    // 207; 263k 320 against 437 with a step per launch; beyond, with three rings,
+    // 526k 878 against 657: a step per launch there.
     const bool six = O.width == 6;
+    if (!six && n > 512 * 528u) return NBX_OK;
     uint32_t tiles = 256;
     if (six && n > 98304) tiles = n <= 512 * 640 ? 512 : 1024;
     if (!six && n > 256 * 640) tiles = 512;
-    uint32_t own0 = std::max((n + tiles - 1) / tiles, 16u), rings0 = 3;
-    if (n > (six ? 1024 : 512) * 528u) {
+    uint32_t own0 = std::max((n + tiles - 1) / tiles, 16u), rings0 = 3, least = 3;
+    uint32_t limit = TILE_TB;
+    if (n > 1024 * 528u) {
         own0 = 256;
         tiles = (n + own0 - 1) / own0;
+        limit = 704;
     } else {
         // the rows of r rings around a square of own0 nodes of a triangle mesh
         auto rows = [&](uint32_t r) { return own0 + 4.0 * r * sqrt((double)own0) + 3.0 * r * r; };
         while (rings0 < 8 && rows(rings0 + 1) <= TILE_TB) ++rings0;
+        least = std::max(rings0 / 2, six || tiles <= 256 ? 2u : 3u);
     }
     const uint32_t cells0 = std::max(std::min(tiles, n / own0), 1u);
-    // A mesh of uneven density, or with wider rows, can outgrow TILE_TB in a
-    // few cells: fewer rings then, and more cells.
-    return tiles_cut(T, TileRows<uint8_t>{O.slice_ptr, O.rowlen, O.bcol}, n, wmax, xy,
-                     {{cells0, rings0},
-                      {cells0, rings0 - 1},
-                      {cells0, rings0 / 2},
-                      {2 * cells0, rings0 / 2},
-                      {4 * cells0, rings0 / 4}},
-                     TILE_TB, s);
+    // A mesh of uneven density, or with wider rows, can outgrow a tile in a few
+    // cells: fewer rings then, or (rows of six blocks, eight rings) twice the
+    // cells with four.  Every tile takes the threads of the fullest and most
+    // then own little, so more cells with fewer rings lose to a step per launch;
+    // us per outer iteration of 1024x512 (541), spacing growing to three, five
+    // times the first in x and y: 579, 904 with 2 and 4 times the cells and two
+    // rings; 512x256 (275-318), growing ten times: 429.  In the three rings of
+    // the largest meshes tiles of more than 704 rows do (1430x720, 834: of 664
+    // 741, of 747 832, of 829 877).
+    std::vector<TileAttempt> attempts{{cells0, rings0, least}};
+    if (six && rings0 == 8) attempts.push_back({2 * cells0, 4, 4});
+    return tiles_cut(T, TileRows<uint8_t>{O.slice_ptr, O.rowlen, O.bcol}, n, wmax, xy, attempts,
+                     limit, s);
 }
 
 int tiles_build(Tiles& T, const TileRows<uint16_t>& O, uint32_t n, uint32_t wmax, const double2* xy,

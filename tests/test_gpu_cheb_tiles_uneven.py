@@ -1,0 +1,52 @@
+"""Meshes on which tiles of several Chebyshev steps per launch do not pay (or
+that outgrow them) take a step per launch: an outer iteration of the device
+system is no slower than the sparse API's on the same matrix, which knows no
+node positions and never has tiles (20 % for the spread of the timings), and its
+result is the same to the bit.
+
+Spacing that grows along one side, and an unstructured mesh of even density
+with more than 512 * 528 nodes (rows of up to eleven blocks)."""
+import numpy as np
+import pytest
+
+from test_gpu_amg_bottom import delaunay
+
+pytestmark = pytest.mark.gpu
+
+
+def _graded(nx, ny):
+    """Four fifths of the rows of nodes in the lowest fifth of the height"""
+    from nbots_amd import synth
+    p = synth.cantilever_traction(nx, ny)
+    q = p.nod.reshape(-1, 2).copy()
+    t = q[:, 1] / ny
+    q[:, 1] = ny * np.where(t < 0.8, 0.25 * t, 0.2 + 4.0 * (t - 0.8))
+    p.nod = q.reshape(-1)
+    return p
+
+
+@pytest.mark.parametrize("kind,nx,ny", [("graded", 724, 362), ("delaunay", 740, 370)])
+def test_no_slower_than_single_steps(kind, nx, ny):
+    import nbots_amd as nb
+    from nbots_amd.fem import Fem, SOLVE_MIXED
+    p = _graded(nx, ny) if kind == "graded" else delaunay(nx, ny)
+    f = Fem.from_problem(p)
+    rp, col, val, F = f.system()
+    conn = p.conn.reshape(-1, 3).astype(np.int64)
+    e = np.concatenate([conn[:, [0, 1]], conn[:, [1, 2]], conn[:, [2, 0]]])
+    key = np.unique(np.concatenate([e, e[:, ::-1]]) @ np.array([p.N_nod, 1]))
+    deg = np.bincount(key // p.N_nod, minlength=p.N_nod)
+    A = nb.Sparse.from_graph(deg, np.split((key % p.N_nod).astype(np.uint32),
+                                           np.cumsum(deg)[:-1]), vars_per_node=2)
+    A.import_values(val)
+    ms = [np.inf, np.inf]
+    for _ in range(3):
+        x, ia = A.solve(F, mode=SOLVE_MIXED, tol=1e-14, max_iter=8)
+        i = f.solve(SOLVE_MIXED, tol=1e-14, max_iter=8)
+        assert i["iters"] == ia["iters"] == 8
+        ms = [min(ms[0], ia["ms"]), min(ms[1], i["ms"])]
+    print(kind, [1e3 * m / 8 for m in ms])
+    assert np.array_equal(f.displacement(), x)
+    assert ms[1] <= 1.2 * ms[0]
+    A.destroy()
+    f.destroy()
