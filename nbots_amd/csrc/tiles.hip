@@ -63,26 +63,46 @@ __device__ __forceinline__ uint32_t tile_cell(const TileGrid& g, double2 p) {
     const uint32_t cy = (uint32_t)fmin(fmax((p.y - g.y0) * g.iy, 0.0), (double)(g.ny - 1));
     return cy * g.nx + cx;
 }
+// A wavefront's lanes in runs of equal cells: one atomic a run instead of one a
+// lane, all on one address where a cell holds most of the mesh.
+struct CellRun {
+    unsigned first, len;   // the run's first lane and lanes
+};
+__device__ __forceinline__ CellRun cell_run(uint32_t cell) {
+    const unsigned lane = threadIdx.x % WAVE;
+    const uint32_t before = (uint32_t)__shfl_up((int)cell, 1, WAVE);
+    const uint64_t heads = __ballot(lane == 0 || cell != before);
+    const uint64_t upto = heads & ((2ull << lane) - 1), after = heads & ~((2ull << lane) - 1);
+    const unsigned first = WAVE - 1 - (unsigned)__clzll((long long)upto);
+    return {first, (after ? (unsigned)__ffsll((long long)after) - 1 : WAVE) - first};
+}
 __global__ void k_tile_count(TileGrid g, const double2* __restrict__ xy, uint32_t n,
                              uint32_t* __restrict__ cell, uint32_t* cnt) {
     const uint32_t v = blockIdx.x * BLOCK + threadIdx.x;
-    if (v >= n) return;
-    const uint32_t c = tile_cell(g, xy[v]);
-    cell[v] = c;
-    atomicAdd(&cnt[c], 1u);
+    const uint32_t c = v < n ? tile_cell(g, xy[v]) : NONE;
+    if (v < n) cell[v] = c;
+    const CellRun run = cell_run(c);
+    if (threadIdx.x % WAVE == run.first && c != NONE) atomicAdd(&cnt[c], run.len);
 }
 __global__ void k_tile_zero(uint32_t* p, uint32_t n) {
     const uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
     if (i < n) p[i] = 0u;
 }
-// each cell's nodes, in any order (the ring kernel sorts them)
+// Each cell's nodes, in any order (the ring kernel sorts them); info[0]: a cell
+// has more than `limit`.
 __global__ void k_tile_fill(const uint32_t* __restrict__ cell, uint32_t n,
                             const uint32_t* __restrict__ ptr, uint32_t* pos,
-                            uint32_t* __restrict__ own) {
+                            uint32_t* __restrict__ own, uint32_t limit, unsigned* info) {
     const uint32_t v = blockIdx.x * BLOCK + threadIdx.x;
-    if (v >= n) return;
-    const uint32_t c = cell[v];
-    own[ptr[c] + atomicAdd(&pos[c], 1u)] = v;
+    const uint32_t c = v < n ? cell[v] : NONE;
+    const CellRun run = cell_run(c);
+    uint32_t at = 0;
+    if (threadIdx.x % WAVE == run.first && c != NONE) {
+        at = atomicAdd(&pos[c], run.len);
+        if (at + run.len > limit) info[0] = 1u;
+    }
+    at = (uint32_t)__shfl((int)at, (int)run.first, WAVE) + threadIdx.x % WAVE - run.first;
+    if (c != NONE) own[ptr[c] + at] = v;
 }
 
 __device__ __forceinline__ uint32_t tile_hash(uint32_t id) {
@@ -120,9 +140,8 @@ __device__ void tile_sort(uint32_t* list, uint32_t* tmp, uint32_t b, uint32_t e)
     __syncthreads();
 }
 
-// One workgroup per tile.  ext = 0: only info[0], set by a tile that owns more
-// than `limit` rows, and info[r], r = 1 .. rings, the rows of the largest tile
-// of r rings (TOO_MANY: more than `limit`).  Otherwise the
+// One workgroup per tile.  ext = 0: only info[r], r = 1 .. rings, the rows of
+// the largest tile of r rings (TOO_MANY: more than `limit`).  Otherwise the
 // tile's list, ring offsets and columns (row i's block 2 q + h in half h of word
 // lcol[(t W2 + q) ext + i]; padding names the row itself).
 template <class Len>
@@ -139,11 +158,8 @@ __global__ __launch_bounds__(TILE_TB) void k_tile_rings(TileRows<Len> O,
     __shared__ uint16_t slot[TILE_HASH];
     __shared__ uint32_t cnt;
     const uint32_t t = blockIdx.x, tid = threadIdx.x;
+    if (info[0]) return;   // a cell has more than `limit` (set by the kernel before this one)
     const uint32_t o0 = ptr[t], c0 = ptr[t + 1] - o0;
-    if (c0 > limit) {
-        if (tid == 0) info[0] = 1u;
-        return;
-    }
     for (uint32_t i = tid; i < TILE_HASH; i += TILE_TB) keys[i] = NONE;
     __syncthreads();
     if (tid < c0) {
@@ -278,7 +294,8 @@ static int tiles_cut(Tiles& T, const TileRows<Len>& O, uint32_t n, uint32_t wmax
         const int rc = scan_u32(cnt, ptr, nt, s);
         if (rc) return done(rc);
         hipLaunchKernelGGL(k_tile_zero, dim3(grid_for(nt)), dim3(BLOCK), 0, s, cnt, nt);
-        hipLaunchKernelGGL(k_tile_fill, dim3(grid_for(n)), dim3(BLOCK), 0, s, cell, n, ptr, cnt, own);
+        hipLaunchKernelGGL(k_tile_fill, dim3(grid_for(n)), dim3(BLOCK), 0, s, cell, n, ptr, cnt, own,
+                           limit, info);
         hipLaunchKernelGGL(k_tile_rings<Len>, dim3(nt), dim3(TILE_TB), 0, s, O, ptr, own, limit, rings,
                            wmax, W2, 0u, (uint32_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr, info);
         unsigned hi[RINGS_MAX + 1];

@@ -50,3 +50,28 @@ def test_no_slower_than_single_steps(kind, nx, ny):
     assert ms[1] <= 1.2 * ms[0]
     A.destroy()
     f.destroy()
+
+
+def test_first_solve_of_a_crowded_mesh():
+    """Four fifths of the nodes in a 400th of the area, where no attempt fits:
+    finding that out takes the first solve no longer than cutting the even mesh
+    does (twice its time for the spread)."""
+    import time
+
+    from nbots_amd import synth
+    from nbots_amd.fem import Fem, SOLVE_MIXED
+    nx, ny = 1024, 512
+    best = {}
+    for even in (True, False, True, False):
+        p = synth.cantilever_traction(nx, ny)
+        if not even:
+            t = p.nod.reshape(-1, 2) / np.array([nx, ny])
+            t = np.where(t < 0.8, 0.0625 * t, 0.05 + 4.75 * (t - 0.8))
+            p.nod = (t * np.array([nx, ny])).reshape(-1)
+        f = Fem.from_problem(p)
+        t0 = time.perf_counter()
+        f.solve(SOLVE_MIXED, tol=1e-14, max_iter=1)
+        best[even] = min(best.get(even, np.inf), time.perf_counter() - t0)
+        f.destroy()
+    print(best)
+    assert best[False] <= 2.0 * best[True]
