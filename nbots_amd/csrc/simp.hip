@@ -477,23 +477,38 @@ int build_filter(Simp& o, FemSys& S) {
 
 }  // namespace
 
-// H and Hs as host CSR
+// H and Hs as host CSR.  On a stream of its own: the copies wait neither for
+// another handle's work (a plain hipMemcpy would, and would end a graph capture
+// of another thread) nor for the system's, which need not exist any more.
 int simp_filter_csr(const Simp& o, uint32_t* ptr, uint32_t* idx, double* val, double* Hs) {
     const DevFilter& H = o.H;
-    if (Hs) NBX_HIP(hipMemcpy(Hs, H.Hs, (size_t)H.ne * 8, hipMemcpyDeviceToHost));
-    if (!ptr && !idx && !val) return NBX_OK;
-    std::vector<uint32_t> sptr(H.n_slices + 1), ei(idx ? H.n_stored : 0);
-    std::vector<uint16_t> len(H.ne);
+    const bool rows = ptr || idx || val;
+    if (!rows && !Hs) return NBX_OK;
+    std::vector<uint32_t> sptr(rows ? H.n_slices + 1 : 0), ei(idx ? H.n_stored : 0);
+    std::vector<uint16_t> len(rows ? H.ne : 0);
     std::vector<double> ev(val ? H.n_stored : 0);
-    NBX_HIP(hipMemcpy(sptr.data(), H.slice_ptr, sptr.size() * 4, hipMemcpyDeviceToHost));
-    NBX_HIP(hipMemcpy(len.data(), H.rowlen, len.size() * 2, hipMemcpyDeviceToHost));
-    if (!ei.empty()) NBX_HIP(hipMemcpy(ei.data(), H.idx, ei.size() * 4, hipMemcpyDeviceToHost));
-    if (!ev.empty()) NBX_HIP(hipMemcpy(ev.data(), H.val, ev.size() * 8, hipMemcpyDeviceToHost));
+    struct Own {
+        hipStream_t s = nullptr;
+        ~Own() { if (s) (void)hipStreamDestroy(s); }
+    } own;
+    NBX_HIP(hipStreamCreateWithFlags(&own.s, hipStreamNonBlocking));
+    auto get = [&](void* to, const void* from, size_t bytes) {
+        return bytes ? hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToHost, own.s) : hipSuccess;
+    };
+    hipError_t e = Hs ? get(Hs, H.Hs, (size_t)H.ne * 8) : hipSuccess;
+    if (e == hipSuccess) e = get(sptr.data(), H.slice_ptr, sptr.size() * 4);
+    if (e == hipSuccess) e = get(len.data(), H.rowlen, len.size() * 2);
+    if (e == hipSuccess) e = get(ei.data(), H.idx, ei.size() * 4);
+    if (e == hipSuccess) e = get(ev.data(), H.val, ev.size() * 8);
+    const hipError_t done = hipStreamSynchronize(own.s);   // (before the arrays go, also after an error)
+    NBX_HIP(e);
+    NBX_HIP(done);
+    if (!rows) return NBX_OK;
     size_t at = 0;
-    for (uint32_t e = 0; e < H.ne; ++e) {
-        if (ptr) ptr[e] = (uint32_t)at;
-        size_t i = (size_t)sptr[e / SLICE] + e % SLICE;
-        for (uint32_t k = 0; k < len[e]; ++k, ++at, i += SLICE) {
+    for (uint32_t r = 0; r < H.ne; ++r) {
+        if (ptr) ptr[r] = (uint32_t)at;
+        size_t i = (size_t)sptr[r / SLICE] + r % SLICE;
+        for (uint32_t k = 0; k < len[r]; ++k, ++at, i += SLICE) {
             if (idx) idx[at] = ei[i];
             if (val) val[at] = ev[i];
         }
