@@ -1447,7 +1447,7 @@ __global__ __launch_bounds__(BLOCK) void k_fcg_p(const P* __restrict__ z,
 }
 
 // The flexible CG's outer iteration without one-workgroup kernels, up to
-// FCG2_MAX_NODES: k_cg_dir<.., FcgDir> (the direction and w = K p), this
+// cg2_nodes: k_cg_dir<.., FcgDir> (the direction and w = K p), this
 // update, the preconditioner, then k_fcg2_dots; 3 kernels in place of 7 around
 // the preconditioner (2-3 us each).  Every workgroup sums the partials of the
 // kernel before it, as in the two-kernel PCG, with the same results bit for
@@ -1835,16 +1835,32 @@ static bool sym_u3(const Sym2& y) {
 }
 
 // The iteration in two kernels (k_cg_dir, k_cg_update), with pcg_run's host
-// cadence.  Node systems with the symmetric copy take it up to 196,608 nodes:
-// us per iteration, five kernels -> two, 64x32 cantilever 17.8 -> 9.3, 256x128
-// 17 -> 9.1, 400x200 (80k nodes) 17 -> 10.4, 540x270 (147k) 22.3 -> 17.1,
-// 600x300 (181k) 23.3 -> 19.5, 640x320 (206k) 24.4 -> 24.7, 1024x512 (525k)
-// 40 -> 47: a row of the direction kernel gathers twice the bytes and holds
-// 138 VGPRs.  The full layout, with twice the blocks a row, stops at 131,072.
-// Scalar CSR takes it up to 262,144 rows (figures at k_cg_dir_csr).  Both keep
-// the partials, which every workgroup sums, at 1,024 a value at most.
-constexpr uint32_t FCG2_MAX_NODES = ALL_PARTS * BLOCK;
-constexpr uint32_t CG2_MAX_NODES = 196608, CG2_MAX_FULL = 131072, CG2_MAX_ROWS = 262144;
+// cadence, where one round of workgroups takes all rows: the direction kernel's
+// loads ahead are then under way in all of them at once, and it gathers twice
+// the bytes of a plain product.  us per iteration, five kernels -> two:
+// * rows of up to three lower and three upper blocks (142-149 VGPRs, three
+//   workgroups a CU) up to 196,608 nodes: 64x32 cantilever 17.8 -> 9.3, 256x128
+//   17 -> 9.1, 400x200 (80k nodes) 17 -> 10.4, 540x270 (147k) 22.3 -> 17.1,
+//   600x300 (181k) 23.3 -> 19.5, 640x320 (206k) 24.4 -> 24.7, 1024x512 (525k)
+//   40 -> 47;
+// * other symmetric rows (174 VGPRs, two a CU) up to 131,072: unstructured
+//   triangles 480x270 (130k) 26.8 -> 20.6, 512x256 (132k) 32.2 -> 31.2, 600x300
+//   32.9 -> 37.2; the same with nodes in random order 41.4 -> 41.3, 44.7 -> 48.4,
+//   57 -> 78; rows of 13 blocks, 125k 31.0 -> 24.4, 150k 33.5 -> 35.8;
+// * full rows up to 131,072 as well: 400x200 23 -> 14.6, 510x256 (131k) 25.5 ->
+//   20.0, in random order 480x270 28.6 -> 25.4.  (Rows of seven blocks in order
+//   gain beyond too: 600x300 27.4 -> 24.1, 640x320 29.4 -> 28.9.)
+// Scalar CSR takes it up to 262,144 rows (figures at k_cg_dir_csr; in random
+// order 90,000 rows of seven 24.2 -> 17.0, 250,000 34.1 -> 28.7).  All keep the
+// partials, which every workgroup sums, at 1,024 a value at most.
+constexpr uint32_t CG2_MAX_U3 = 196608, CG2_MAX_NODES = 131072, CG2_MAX_ROWS = 262144;
+// ... and the flexible CG's direction, which the launches it saves carry further
+// on rows of three and three: up to where its partials allow.
+constexpr uint32_t FCG2_MAX_U3 = ALL_PARTS * BLOCK;
+// most nodes for the two kernels (u3: where the rows are three and three)
+static uint32_t cg2_nodes(const DevMatrix& m, uint32_t u3) {
+    return m.has_sym && sym_u3(m.y) ? u3 : CG2_MAX_NODES;
+}
 template <class Op>
 static int pcg2_run(const Op& op, uint32_t nu, const double* diag_in, const typename Op::V* b,
                     typename Op::V* x, uint32_t max_iter, double tol, Workspace& w, hipStream_t s,
@@ -1960,13 +1976,14 @@ int pcg_jacobi(const DevMatrix& m, const double* b, double* x, uint32_t max_iter
                                                8.0 * (double)m.y.n_lower
                                          : 36.0 * (double)m.s.n_blocks;
     const bool stream = mat_bytes + 40.0 * (double)m.n > (double)INFINITY_CACHE_BYTES;
-    if (m.blocked && m.has_sym && m.s.n_nodes <= CG2_MAX_NODES)
+    const bool two = m.blocked && m.s.n_nodes <= cg2_nodes(m, CG2_MAX_U3);
+    if (two && m.has_sym)
         rc = sym_u3(m.y)
                  ? pcg2_run(OpSymU<3>{{m.y}}, m.s.n_nodes, diag, (const double2*)b, (double2*)x,
                             max_iter, tol, w, s, stats)
                  : pcg2_run(OpSymU<4>{{m.y}}, m.s.n_nodes, diag, (const double2*)b, (double2*)x,
                             max_iter, tol, w, s, stats);
-    else if (m.blocked && !m.has_sym && m.s.n_nodes <= CG2_MAX_FULL)
+    else if (two)
         rc = pcg2_run(OpS2{m.s}, m.s.n_nodes, diag, (const double2*)b, (double2*)x, max_iter, tol,
                       w, s, stats);
     else if (m.blocked && m.has_sym && stream)
@@ -2251,7 +2268,7 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
     OpSym ops{m.y};
     // three kernels around the preconditioner (k_fcg2_update) or seven; the
     // preconditioner's kernels test `done` in stp
-    const bool fold = !p64 && nu <= FCG2_MAX_NODES;
+    const bool fold = !p64 && nu <= cg2_nodes(m, FCG2_MAX_U3);
     PcgState* const stp = fold ? w.st + 1 : w.st;
     CgPair<double2>* const pair[2] = {(CgPair<double2>*)w.v64[1], (CgPair<double2>*)w.v64[6]};
     if (fold) wv = (double2*)w.v64[8];
