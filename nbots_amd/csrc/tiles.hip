@@ -27,6 +27,7 @@ constexpr uint32_t TILE_HASH = 4096;
 constexpr uint32_t NONE = 0xffffffffu;
 constexpr unsigned TOO_MANY = 0xffffffffu;
 constexpr uint32_t RINGS_MAX = 8;
+constexpr uint32_t RUNS = RINGS_MAX + 1, INFO = RUNS + 1;   // words of k_tile_rings's info
 
 // per workgroup: smallest and largest x and y
 __global__ __launch_bounds__(BLOCK) void k_tile_bbox(const double2* __restrict__ xy, uint32_t n,
@@ -141,7 +142,8 @@ __device__ void tile_sort(uint32_t* list, uint32_t* tmp, uint32_t b, uint32_t e)
 }
 
 // One workgroup per tile.  ext = 0: only info[r], r = 1 .. rings, the rows of
-// the largest tile of r rings (TOO_MANY: more than `limit`).  Otherwise the
+// the largest tile of r rings (TOO_MANY: more than `limit`), and info[RUNS], the
+// groups of 8 consecutive ids that the tiles' owned rows touch.  Otherwise the
 // tile's list, ring offsets and columns (row i's block 2 q + h in half h of word
 // lcol[(t W2 + q) ext + i]; padding names the row itself).
 template <class Len>
@@ -169,6 +171,11 @@ __global__ __launch_bounds__(TILE_TB) void k_tile_rings(TileRows<Len> O,
     }
     __syncthreads();
     tile_sort(list, tmp, 0, c0);
+    if (!ext) {
+        const bool head = tid < c0 && (tid == 0 || list[tid] / 8 != list[tid - 1] / 8);
+        const uint64_t heads = __ballot(head);
+        if (tid % WAVE == 0 && heads) atomicAdd(&info[RUNS], (unsigned)__popcll(heads));
+    }
     if (ext && tid == 0) roff[(size_t)t * (rings + 1)] = c0;
     uint32_t beg = 0, end = c0;
     for (uint32_t r = 1; r <= rings; ++r) {
@@ -231,12 +238,14 @@ void tiles_free(Tiles& T) {
 
 // Cuts the n rows at positions xy into the first of `attempts` whose tiles have
 // at most `limit` rows with `least` rings or more (as many of its `rings` as
-// fit).  Leaves T.n = 0 (nothing allocated) when none has, or
+// fit) and whose owned rows touch at most `most_runs` groups of 8 consecutive
+// ids.  Leaves T.n = 0 (nothing allocated) when none has, or
 // without device memory for them: the kernels that take one step per launch
 // then run.
 template <class Len>
 static int tiles_cut(Tiles& T, const TileRows<Len>& O, uint32_t n, uint32_t wmax, const double2* xy,
-                     const std::vector<TileAttempt>& attempts, uint32_t limit, hipStream_t s) {
+                     const std::vector<TileAttempt>& attempts, uint32_t limit, uint32_t most_runs,
+                     hipStream_t s) {
     uint32_t *cell = nullptr, *cnt = nullptr, *ptr = nullptr, *own = nullptr;
     unsigned* info = nullptr;
     double* bb = nullptr;
@@ -268,7 +277,7 @@ static int tiles_cut(Tiles& T, const TileRows<Len>& O, uint32_t n, uint32_t wmax
         return done(NBX_OK);
     if (hipMalloc(&cell, (size_t)n * 4) != hipSuccess ||
         hipMalloc(&own, (size_t)n * 4) != hipSuccess ||
-        hipMalloc(&info, (RINGS_MAX + 1) * sizeof(unsigned)) != hipSuccess)
+        hipMalloc(&info, INFO * sizeof(unsigned)) != hipSuccess)
         return no_memory();
     const uint32_t W2 = (wmax + 1) / 2;
     for (const auto& at : attempts) {
@@ -289,7 +298,7 @@ static int tiles_cut(Tiles& T, const TileRows<Len>& O, uint32_t n, uint32_t wmax
             hipMalloc(&ptr, ((size_t)nt + 1) * 4) != hipSuccess)
             return no_memory();
         hipLaunchKernelGGL(k_tile_zero, dim3(grid_for(nt)), dim3(BLOCK), 0, s, cnt, nt);
-        hipLaunchKernelGGL(k_tile_zero, dim3(1), dim3(BLOCK), 0, s, (uint32_t*)info, RINGS_MAX + 1);
+        hipLaunchKernelGGL(k_tile_zero, dim3(1), dim3(BLOCK), 0, s, (uint32_t*)info, INFO);
         hipLaunchKernelGGL(k_tile_count, dim3(grid_for(n)), dim3(BLOCK), 0, s, g, xy, n, cell, cnt);
         const int rc = scan_u32(cnt, ptr, nt, s);
         if (rc) return done(rc);
@@ -298,12 +307,13 @@ static int tiles_cut(Tiles& T, const TileRows<Len>& O, uint32_t n, uint32_t wmax
                            limit, info);
         hipLaunchKernelGGL(k_tile_rings<Len>, dim3(nt), dim3(TILE_TB), 0, s, O, ptr, own, limit, rings,
                            wmax, W2, 0u, (uint32_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr, info);
-        unsigned hi[RINGS_MAX + 1];
+        unsigned hi[INFO];
         if (hipGetLastError() != hipSuccess ||
             copy_on(hi, info, sizeof hi, hipMemcpyDeviceToHost, s) != hipSuccess) {
             set_last_error("tiles: halo rings");
             return done(NBX_ERR_HIP);
         }
+        if (hi[RUNS] > most_runs) return done(NBX_OK);
         uint32_t fit = hi[0] ? 0 : rings;
         while (fit && hi[fit] > limit) --fit;
         if (fit < at.least) continue;
@@ -377,15 +387,22 @@ int tiles_build(Tiles& T, const Off16& O, uint32_t wmax, const double2* xy, hipS
     // 741, of 747 832, of 829 877).
     std::vector<TileAttempt> attempts{{cells0, rings0, least}};
     if (six && rings0 == 8) attempts.push_back({2 * cells0, 4, 4});
+    // A tile reads its rows' blocks where the rows lie.  Where the matrix exceeds
+    // the caches and the numbering scatters a tile's rows, each block is a line of
+    // its own and the overlap costs more than the launches: nodes in random order,
+    // single steps -> tiles: 620x310 524 -> 486, 724x362 705 -> 675, 850x425 907 ->
+    // 948, 1024x512 1,332 -> 1,552, 1430x720 3,403 -> 4,227.  (In order 256 owned
+    // rows touch about 50 groups of 8, scattered ones 256.)
+    const uint32_t most_runs = n > 512 * 640 ? n / 2 : n;
     return tiles_cut(T, TileRows<uint8_t>{O.slice_ptr, O.rowlen, O.bcol}, n, wmax, xy, attempts,
-                     limit, s);
+                     limit, most_runs, s);
 }
 
 int tiles_build(Tiles& T, const TileRows<uint16_t>& O, uint32_t n, uint32_t wmax, const double2* xy,
                 const std::vector<TileAttempt>& attempts, uint32_t limit, hipStream_t s) {
     tiles_free(T);
     if (!xy || n == 0 || wmax == 0) return NBX_OK;
-    return tiles_cut(T, O, n, wmax, xy, attempts, std::min(limit, (uint32_t)TILE_TB), s);
+    return tiles_cut(T, O, n, wmax, xy, attempts, std::min(limit, (uint32_t)TILE_TB), n, s);
 }
 
 }  // namespace nbx

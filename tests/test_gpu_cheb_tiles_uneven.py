@@ -4,12 +4,14 @@ system is no slower than the sparse API's on the same matrix, which knows no
 node positions and never has tiles (20 % for the spread of the timings), and its
 result is the same to the bit.
 
-Spacing that grows along one side, and an unstructured mesh of even density
-with more than 512 * 528 nodes (rows of up to eleven blocks)."""
+Spacing that grows along one side, an unstructured mesh of even density with
+more than 512 * 528 nodes (rows of up to eleven blocks), and a large mesh whose
+nodes are numbered in random order (10 % there: it took 24 % longer)."""
 import numpy as np
 import pytest
 
 from test_gpu_amg_bottom import delaunay
+from test_gpu_cheb_tiles import _shuffled
 
 pytestmark = pytest.mark.gpu
 
@@ -25,11 +27,15 @@ def _graded(nx, ny):
     return p
 
 
-@pytest.mark.parametrize("kind,nx,ny", [("graded", 724, 362), ("delaunay", 740, 370)])
-def test_no_slower_than_single_steps(kind, nx, ny):
+MESHES = {"graded": _graded, "delaunay": delaunay, "shuffled": _shuffled}
+
+
+@pytest.mark.parametrize("kind,nx,ny,bar", [("graded", 724, 362, 1.2), ("delaunay", 740, 370, 1.2),
+                                            ("shuffled", 1430, 720, 1.1)])
+def test_no_slower_than_single_steps(kind, nx, ny, bar):
     import nbots_amd as nb
     from nbots_amd.fem import Fem, SOLVE_MIXED
-    p = _graded(nx, ny) if kind == "graded" else delaunay(nx, ny)
+    p = MESHES[kind](nx, ny)
     f = Fem.from_problem(p)
     rp, col, val, F = f.system()
     conn = p.conn.reshape(-1, 3).astype(np.int64)
@@ -47,7 +53,7 @@ def test_no_slower_than_single_steps(kind, nx, ny):
         ms = [min(ms[0], ia["ms"]), min(ms[1], i["ms"])]
     print(kind, [1e3 * m / 8 for m in ms])
     assert np.array_equal(f.displacement(), x)
-    assert ms[1] <= 1.2 * ms[0]
+    assert ms[1] <= bar * ms[0]
     A.destroy()
     f.destroy()
 
