@@ -78,7 +78,8 @@ struct AmgDev {
     double* pow_y = nullptr;
     double* scal = nullptr;         // [2 levels] 1 / norm and norm of the power iteration
     double* partials = nullptr;     // [MAX_GRID] reduction partials
-    double* dense = nullptr;        // the coarsest matrix, n x n
+    double* dense = nullptr;        // the coarsest matrix, its inverse, I - A A^-1, n x n each,
+                                    // and n flags
     size_t bytes = 0;
     // more than one level: the finest is smoothed on the matrix's fp16
     // scaled copy, in scaled variables, and its P values are stored as
@@ -254,19 +255,17 @@ __global__ __launch_bounds__(FIN) void k_amg_pow_fin(const double* partials, uns
 // sweeps (Goodnight 1979): sweeping k turns a_kk into -1 / a_kk, a_ik into
 // a_ik / a_kk and a_ij into a_ij - a_ik a_kj / a_kk; all swept, A is -A^-1.
 // The pivots are the Cholesky factor's, and an unknown whose pivot is not
-// above 1e-13 of the largest diagonal entry is dropped as amg_dense_inverse
-// drops it (zero row and column).  One workgroup holds the matrix in
-// registers, the lower half of its 32 x 32 blocks; a step passes column k
-// through LDS and costs one barrier.  Bound by its n steps of LDS reads, a
-// division and a barrier: 142 us at 162 unknowns (190 with all entries).  The
-// host function took 0.6 ms there besides
-// the copies and the wait; with the folded power iteration above, the numeric
-// phase went from 1.13 to 0.71 ms at 96x48 (162 unknowns), 0.95 -> 0.78 at
-// 150x75 (36), 1.74 -> 1.52 at 512x256 (24).  The same Cholesky factor and
-// products on the device, bit for bit the host's, take 445 us at 162.  Against
-// extended precision the inverse's error is as often below the host's as above
-// it (0.01 to 12 times, 0.8 on average over 18 elasticity matrices: 1e-14 to
-// 1e-10 at condition numbers of 1e4 to 1e9, FP32 rounding being 2e-8).
+// above 1e-13 of the largest diagonal entry is dropped (zero row and column).
+// One workgroup holds the matrix in registers, the lower half of its 32 x 32
+// blocks; a step passes column k through LDS and costs one barrier.  Bound by
+// its n steps of LDS reads, a division and a barrier: 142 us at 162 unknowns
+// (190 with all entries).  The sweeps' error is up to 84 times that of a
+// Cholesky factor's inverse in FP64 (3.0 on average over the coarsest levels of
+// 60 systems of 200 to 200,000 unknowns; with void elements, condition numbers
+// of 1e11, 4e-6 where FP32 rounds to 2e-8), so one step of Newton's iteration
+// X + X (I - A X) follows, its residual in doubled precision, over one workgroup
+// a row: then the stored inverse is A^-1 rounded to FP32 in all 60, which the
+// Cholesky inverse was in 52.
 constexpr int SWEEP_SIDE = 32, SWEEP_TB = SWEEP_SIDE * SWEEP_SIDE;
 constexpr int SWEEP_NB = (AMG_COARSEST + SWEEP_SIDE - 1) / SWEEP_SIDE;
 
@@ -284,13 +283,18 @@ __global__ __launch_bounds__(WAVE) void k_dense_rows(const uint32_t* __restrict_
     for (uint32_t j = threadIdx.x; j < n; j += WAVE) out[(size_t)i * n + j] = row[j];
 }
 
-// inv = A^-1 in FP32, of A symmetrised (P^T A P rounds slightly
-// unsymmetrically).  Thread (tx, ty) holds the entries (ty + 32 p, tx + 32 q)
+// entry (i, j) of A symmetrised (P^T A P rounds slightly unsymmetrically)
+__device__ __forceinline__ double dense_sym(const double* __restrict__ a, uint32_t n, uint32_t i,
+                                            uint32_t j) {
+    return i == j ? a[(size_t)i * n + i] : 0.5 * (a[(size_t)i * n + j] + a[(size_t)j * n + i]);
+}
+
+// inv = A^-1 by sweeps.  Thread (tx, ty) holds the entries (ty + 32 p, tx + 32 q)
 // with q <= p; column k is those of the column from row block k / 32 on and
 // those of row k before it.
 template <int NB>
 __global__ __launch_bounds__(SWEEP_TB) void k_dense_sweep(const double* __restrict__ a,
-                                                          float* __restrict__ inv, uint32_t n) {
+                                                          double* __restrict__ inv, uint32_t n) {
     __shared__ double colk[2][NB * SWEEP_SIDE], big[SWEEP_TB / WAVE];
     const uint32_t tx = threadIdx.x % SWEEP_SIDE, ty = threadIdx.x / SWEEP_SIDE;
     double v[NB][NB], dmax = 0.0;   // (the entries q > p are never used)
@@ -300,9 +304,7 @@ __global__ __launch_bounds__(SWEEP_TB) void k_dense_sweep(const double* __restri
         for (int q = 0; q <= p; ++q) {
             const uint32_t i = ty + p * SWEEP_SIDE, j = tx + q * SWEEP_SIDE;
             v[p][q] = 0.0;
-            if (i < n && j < n)
-                v[p][q] = i == j ? a[(size_t)i * n + i]
-                                 : 0.5 * (a[(size_t)i * n + j] + a[(size_t)j * n + i]);
+            if (i < n && j < n) v[p][q] = dense_sym(a, n, i, j);
             if (i == j) dmax = fmax(dmax, v[p][q]);
         }
     for (int off = WAVE / 2; off > 0; off >>= 1) dmax = fmax(dmax, __shfl_xor(dmax, off));
@@ -349,9 +351,48 @@ __global__ __launch_bounds__(SWEEP_TB) void k_dense_sweep(const double* __restri
             // (of a diagonal block's two entries that rounding may leave
             // different, the lower one for both)
             if (i < n && j <= i)
-                inv[(size_t)i * n + j] = inv[(size_t)j * n + i] = (float)-v[p][q];
+                inv[(size_t)i * n + j] = inv[(size_t)j * n + i] = -v[p][q];
         }
 }
+
+// R = I - A X by compensated dot products, a workgroup per row; far[i]: the row
+// is not small enough for a step of Newton's iteration (rows of dropped unknowns,
+// whose X is zero, do not count)
+__global__ __launch_bounds__(BLOCK) void k_dense_residual(const double* __restrict__ a,
+                                                          const double* __restrict__ x,
+                                                          double* __restrict__ r,
+                                                          uint32_t* __restrict__ far, uint32_t n) {
+    __shared__ double row[AMG_COARSEST], red[1][BLOCK / WAVE];
+    const uint32_t i = blockIdx.x, j = threadIdx.x;
+    if (j < n) row[j] = -dense_sym(a, n, i, j);
+    __syncthreads();
+    double acc[1] = {0.0};
+    if (j < n) {
+        double s = i == j ? 1.0 : 0.0, c = 0.0;
+        for (uint32_t p = 0; p < n; ++p) dot2_add(row[p], x[(size_t)p * n + j], s, c);
+        const double e = s + c;
+        r[(size_t)i * n + j] = e;
+        acc[0] = fabs(e);
+    }
+    block_sum<1>(acc, red);
+    if (j == 0) far[i] = x[(size_t)i * n + i] != 0.0 && !(acc[0] < 0.1);
+}
+// inv = X + X R in FP32 (X alone where a row of R is far from 0), a workgroup per row
+__global__ __launch_bounds__(BLOCK) void k_dense_refine(const double* __restrict__ x,
+                                                        const double* __restrict__ r,
+                                                        const uint32_t* __restrict__ far,
+                                                        float* __restrict__ inv, uint32_t n) {
+    __shared__ double row[AMG_COARSEST];
+    const uint32_t i = blockIdx.x, j = threadIdx.x;
+    if (j < n) row[j] = x[(size_t)i * n + j];
+    const bool skip = __syncthreads_or(j < n && far[j]);
+    if (j > i) return;
+    double s = 0.0;
+    if (!skip)
+        for (uint32_t p = 0; p < n; ++p) s += row[p] * r[(size_t)p * n + j];
+    inv[(size_t)i * n + j] = inv[(size_t)j * n + i] = (float)(row[j] + s);
+}
+static_assert(AMG_COARSEST <= BLOCK, "a thread per column");
 
 // P = T - omega D^-1 A T: SMOOTH_SLOTS threads per node, each taking every
 // SMOOTH_SLOTS-th aggregate column group of the node's P rows (its R rows
@@ -1575,7 +1616,7 @@ static int amg_symbolic(FemSys& S) {
     NBX_TRY(alloc(&A->pow_x, n, A->bytes));
     NBX_TRY(alloc(&A->pow_y, n, A->bytes));
     NBX_TRY(alloc(&A->scal, 2 * nl, A->bytes));
-    NBX_TRY(alloc(&A->dense, (size_t)nco * nco, A->bytes));
+    NBX_TRY(alloc(&A->dense, 3 * (size_t)nco * nco + nco, A->bytes));
     NBX_TRY(alloc(&A->partials, (size_t)MAX_GRID, A->bytes));
     std::vector<double> ones(n + 2, 1.0);
     NBX_HIP(hipMemcpy(A->ones, ones.data(), ones.size() * sizeof(double), hipMemcpyHostToDevice));
@@ -1650,7 +1691,8 @@ template <int NB>
 static void launch_sweep(AmgDev* A, uint32_t n, hipStream_t s) {
     if constexpr (NB < SWEEP_NB)
         if (n > NB * SWEEP_SIDE) return launch_sweep<NB + 1>(A, n, s);
-    hipLaunchKernelGGL(k_dense_sweep<NB>, dim3(1), dim3(SWEEP_TB), 0, s, A->dense, A->cinv, n);
+    hipLaunchKernelGGL(k_dense_sweep<NB>, dim3(1), dim3(SWEEP_TB), 0, s, A->dense,
+                       A->dense + (size_t)n * n, n);
 }
 static int coarsest_inverse(AmgDev* A, hipStream_t s) {
     const AmgDevLevel& L = A->lv.back();
@@ -1658,6 +1700,10 @@ static int coarsest_inverse(AmgDev* A, hipStream_t s) {
     hipLaunchKernelGGL(k_dense_rows, dim3(L.n), dim3(WAVE), 0, s, L.a_ptr, L.a_col, L.a64, A->dense,
                        L.n);
     launch_sweep<1>(A, L.n, s);
+    double *const x = A->dense + (size_t)L.n * L.n, *const r = x + (size_t)L.n * L.n;
+    uint32_t* const far = (uint32_t*)(r + (size_t)L.n * L.n);
+    hipLaunchKernelGGL(k_dense_residual, dim3(L.n), dim3(BLOCK), 0, s, A->dense, x, r, far, L.n);
+    hipLaunchKernelGGL(k_dense_refine, dim3(L.n), dim3(BLOCK), 0, s, x, r, far, A->cinv, L.n);
     NBX_HIP(hipGetLastError());
     return NBX_OK;
 }

@@ -207,6 +207,22 @@ __device__ __forceinline__ f32c cadd(f32c x, f32c y) {
     return {t.s, (x.c + y.c) + t.c};
 }
 
+// s + c += a x, the errors of the product and of the sum collected in c (Dot2 of
+// Ogita, Rump and Oishi 2005)
+__device__ __forceinline__ void two_sum64(double a, double b, double& s, double& e) {
+    s = a + b;
+    const double bb = s - a;
+    e = (a - (s - bb)) + (b - bb);
+}
+__device__ __forceinline__ void dot2_add(double a, double x, double& s, double& c) {
+    const double p = a * x;
+    const double pe = fma(a, x, -p);
+    double t, e;
+    two_sum64(s, p, t, e);
+    s = t;
+    c = c + (e + pe);
+}
+
 typedef unsigned uv2x __attribute__((ext_vector_type(2)));
 
 // ---- wavefront / workgroup reductions in a fixed order --------------------

@@ -930,19 +930,6 @@ __global__ __launch_bounds__(BLOCK) void k_residual64(Sell2 K, const double2* __
 // Oishi 2005: each product's rounding error from an FMA, each sum's from
 // TwoSum, the errors summed alongside), so r is accurate to about one
 // rounding of r itself instead of eps * sum |K_ij u_j|; partials of r.r.
-__device__ __forceinline__ void two_sum64(double a, double b, double& s, double& e) {
-    s = a + b;
-    const double bb = s - a;
-    e = (a - (s - bb)) + (b - bb);
-}
-__device__ __forceinline__ void dot2_add(double a, double x, double& s, double& c) {
-    const double p = a * x;
-    const double pe = fma(a, x, -p);
-    double t, e;
-    two_sum64(s, p, t, e);
-    s = t;
-    c = c + (e + pe);
-}
 __global__ __launch_bounds__(BLOCK) void k_residual_dot2(Sell2 K, const double2* __restrict__ F,
                                                          const double2* __restrict__ u,
                                                          double* partials, uint32_t n) {
