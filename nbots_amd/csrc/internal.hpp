@@ -79,9 +79,9 @@ struct DevMatrix {
 //                               v64[1..2] and v64[6..7] the (q, p) pairs
 //   flexible CG (CHEB_FCG):     v64[0] r, v64[1] p, v64[2] w; v32[0..3]
 //                               residual, two directions and z of the
-//                               Chebyshev steps, v32[4] the residual's second
-//                               buffer (several steps per launch); FP64
-//                               preconditioner: v64[5..8] instead
+//                               Chebyshev steps, v64[5] (as FP32) the
+//                               residual's second buffer (several steps per
+//                               launch); FP64 preconditioner: v64[5..8] instead
 //   FP32 CG (CG_RESTART/RELIABLE): v32[0..3]; a fallback to FP64 PCG takes
 //                               the FP64 slots above
 //   free for callers: v64[3], v64[4] (the drop-in's b and x, the system's
@@ -90,7 +90,7 @@ struct DevMatrix {
 struct Workspace {
     uint32_t n = 0;
     double* v64[9] = {};       // FP64 vectors
-    float* v32[5] = {};        // FP32 vectors
+    float* v32[4] = {};        // FP32 vectors
     double* partials = nullptr;
     float* partials32 = nullptr;
     PcgState* st = nullptr;    // device state (2 slots, which the two-kernel PCG alternates)

@@ -2393,7 +2393,7 @@ static int fcg_cheb_pass(const DevMatrix& m, const double* b, double* x, double 
         float2* din = da;
         float2* dout = db;
         if (tiled) {
-            float2 *rin = res, *rout = (float2*)w.v32[4];
+            float2 *rin = res, *rout = (float2*)w.v64[5];
             ChebSteps cs;
             cs.last = deg - 1;
             for (uint32_t k = 1; k < deg; k += cs.steps) {
