@@ -263,8 +263,8 @@ __global__ __launch_bounds__(FIN) void k_amg_pow_fin(const double* partials, uns
 // Cholesky factor's inverse in FP64 (3.0 on average over the coarsest levels of
 // 60 systems of 200 to 200,000 unknowns; with void elements, condition numbers
 // of 1e11, 4e-6 where FP32 rounds to 2e-8), so one step of Newton's iteration
-// X + X (I - A X) follows, its residual in doubled precision, over one workgroup
-// a row: then the stored inverse is A^-1 rounded to FP32 in all 60, which the
+// X + X (I - A X) follows, its residual in doubled precision, a workgroup a row
+// (9.6 + 7.9 us at 162 unknowns): then the stored inverse is A^-1 rounded to FP32 in all 60, which the
 // Cholesky inverse was in 52.
 constexpr int SWEEP_SIDE = 32, SWEEP_TB = SWEEP_SIDE * SWEEP_SIDE;
 constexpr int SWEEP_NB = (AMG_COARSEST + SWEEP_SIDE - 1) / SWEEP_SIDE;
@@ -355,41 +355,80 @@ __global__ __launch_bounds__(SWEEP_TB) void k_dense_sweep(const double* __restri
         }
 }
 
-// R = I - A X by compensated dot products, a workgroup per row; far[i]: the row
-// is not small enough for a step of Newton's iteration (rows of dropped unknowns,
-// whose X is zero, do not count)
-__global__ __launch_bounds__(BLOCK) void k_dense_residual(const double* __restrict__ a,
-                                                          const double* __restrict__ x,
-                                                          double* __restrict__ r,
-                                                          uint32_t* __restrict__ far, uint32_t n) {
-    __shared__ double row[AMG_COARSEST], red[1][BLOCK / WAVE];
-    const uint32_t i = blockIdx.x, j = threadIdx.x;
-    if (j < n) row[j] = -dense_sym(a, n, i, j);
-    __syncthreads();
-    double acc[1] = {0.0};
-    if (j < n) {
-        double s = i == j ? 1.0 : 0.0, c = 0.0;
-        for (uint32_t p = 0; p < n; ++p) dot2_add(row[p], x[(size_t)p * n + j], s, c);
-        const double e = s + c;
-        r[(size_t)i * n + j] = e;
-        acc[0] = fabs(e);
+// R = I - A X by compensated dot products, a workgroup per row, every column by
+// REFINE_PARTS threads with REFINE_AHEAD loads under way each (bound by the loads'
+// latency: one thread a column 18 and 16 us for the two kernels, four 14.7 and 11.6); far[i]: the row is not small enough for a step of Newton's iteration
+// (rows of dropped unknowns, whose X is zero, do not count)
+constexpr uint32_t REFINE_PARTS = 4, REFINE_AHEAD = 14;
+static_assert(AMG_COARSEST + REFINE_PARTS * REFINE_AHEAD <= BLOCK, "row[] is zero past n");
+// f(a row's entry p, column j's) for the p of a part, then for entries of 0
+template <class F>
+__device__ __forceinline__ void refine_dot(const double* row, const double* __restrict__ m,
+                                           uint32_t n, uint32_t j, uint32_t part, F&& f) {
+    for (uint32_t p0 = part; p0 < n; p0 += REFINE_PARTS * REFINE_AHEAD) {
+        double v[REFINE_AHEAD];
+#pragma unroll
+        for (uint32_t u = 0; u < REFINE_AHEAD; ++u) {
+            const uint32_t p = p0 + u * REFINE_PARTS;
+            v[u] = p < n ? m[(size_t)p * n + j] : 0.0;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < REFINE_AHEAD; ++u) f(row[p0 + u * REFINE_PARTS], v[u]);
     }
-    block_sum<1>(acc, red);
-    if (j == 0) far[i] = x[(size_t)i * n + i] != 0.0 && !(acc[0] < 0.1);
 }
-// inv = X + X R in FP32 (X alone where a row of R is far from 0), a workgroup per row
-__global__ __launch_bounds__(BLOCK) void k_dense_refine(const double* __restrict__ x,
-                                                        const double* __restrict__ r,
-                                                        const uint32_t* __restrict__ far,
-                                                        float* __restrict__ inv, uint32_t n) {
-    __shared__ double row[AMG_COARSEST];
-    const uint32_t i = blockIdx.x, j = threadIdx.x;
-    if (j < n) row[j] = x[(size_t)i * n + j];
-    const bool skip = __syncthreads_or(j < n && far[j]);
-    if (j > i) return;
-    double s = 0.0;
-    if (!skip)
-        for (uint32_t p = 0; p < n; ++p) s += row[p] * r[(size_t)p * n + j];
+__global__ __launch_bounds__(REFINE_PARTS * BLOCK) void k_dense_residual(
+    const double* __restrict__ a, const double* __restrict__ x, double* __restrict__ r,
+    uint32_t* __restrict__ far, uint32_t n) {
+    __shared__ double row[BLOCK], ps[REFINE_PARTS][BLOCK], pc[REFINE_PARTS][BLOCK],
+        red[BLOCK / WAVE];
+    const uint32_t i = blockIdx.x, j = threadIdx.x % BLOCK, part = threadIdx.x / BLOCK;
+    if (part == 0) row[j] = j < n ? -dense_sym(a, n, i, j) : 0.0;
+    __syncthreads();
+    if (j < n) {
+        double s = part == 0 && i == j ? 1.0 : 0.0, c = 0.0;
+        refine_dot(row, x, n, j, part, [&](double av, double xv) { dot2_add(av, xv, s, c); });
+        ps[part][j] = s;
+        pc[part][j] = c;
+    }
+    __syncthreads();
+    double e = 0.0;
+    if (part == 0 && j < n) {
+        double s = ps[0][j], c = pc[0][j];
+        for (uint32_t q = 1; q < REFINE_PARTS; ++q) {
+            double t, d;
+            two_sum64(s, ps[q][j], t, d);
+            s = t;
+            c += d + pc[q][j];
+        }
+        r[(size_t)i * n + j] = s + c;
+        e = fabs(s + c);
+    }
+    e = wave_sum(e);
+    if (part == 0 && j % WAVE == 0) red[j / WAVE] = e;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        e = 0.0;
+        for (int w = 0; w < BLOCK / WAVE; ++w) e += red[w];
+        far[i] = x[(size_t)i * n + i] != 0.0 && !(e < 0.1);
+    }
+}
+// inv = X + X R in FP32 (X alone where a row of R is far from 0), likewise
+__global__ __launch_bounds__(REFINE_PARTS * BLOCK) void k_dense_refine(
+    const double* __restrict__ x, const double* __restrict__ r, const uint32_t* __restrict__ far,
+    float* __restrict__ inv, uint32_t n) {
+    __shared__ double row[BLOCK], ps[REFINE_PARTS][BLOCK];
+    const uint32_t i = blockIdx.x, j = threadIdx.x % BLOCK, part = threadIdx.x / BLOCK;
+    if (part == 0) row[j] = j < n ? x[(size_t)i * n + j] : 0.0;
+    const bool skip = __syncthreads_or(part == 0 && j < n && far[j]);
+    if (j <= i) {
+        double s = 0.0;
+        if (!skip) refine_dot(row, r, n, j, part, [&](double xv, double rv) { s += xv * rv; });
+        ps[part][j] = s;
+    }
+    __syncthreads();
+    if (part != 0 || j > i) return;
+    double s = ps[0][j];
+    for (uint32_t q = 1; q < REFINE_PARTS; ++q) s += ps[q][j];
     inv[(size_t)i * n + j] = inv[(size_t)j * n + i] = (float)(row[j] + s);
 }
 static_assert(AMG_COARSEST <= BLOCK, "a thread per column");
@@ -1702,8 +1741,9 @@ static int coarsest_inverse(AmgDev* A, hipStream_t s) {
     launch_sweep<1>(A, L.n, s);
     double *const x = A->dense + (size_t)L.n * L.n, *const r = x + (size_t)L.n * L.n;
     uint32_t* const far = (uint32_t*)(r + (size_t)L.n * L.n);
-    hipLaunchKernelGGL(k_dense_residual, dim3(L.n), dim3(BLOCK), 0, s, A->dense, x, r, far, L.n);
-    hipLaunchKernelGGL(k_dense_refine, dim3(L.n), dim3(BLOCK), 0, s, x, r, far, A->cinv, L.n);
+    const dim3 rows(L.n), tb(REFINE_PARTS * BLOCK);
+    hipLaunchKernelGGL(k_dense_residual, rows, tb, 0, s, A->dense, x, r, far, L.n);
+    hipLaunchKernelGGL(k_dense_refine, rows, tb, 0, s, x, r, far, A->cinv, L.n);
     NBX_HIP(hipGetLastError());
     return NBX_OK;
 }

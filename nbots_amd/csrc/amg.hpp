@@ -149,7 +149,9 @@ inline double amg_sign(uint32_t i) {
 // In-place inverse of a dense symmetric positive semi-definite n x n matrix
 // (row-major, FP64) by Cholesky with a pivot guard: an unknown whose pivot
 // falls below 1e-13 times the largest diagonal entry is dropped (its row and
-// column of the inverse are 0).  Returns the number of dropped unknowns.
+// column of the inverse are 0).  Returns the number of dropped unknowns.  The
+// host check's FP64 hierarchy solves its coarsest level with it; a solve on the
+// device uses k_dense_sweep (amg.hip).
 int amg_dense_inverse(uint32_t n, double* a);
 
 }  // namespace nbx

@@ -169,8 +169,8 @@ struct Sym2 {
     uint8_t* l_rowlen = nullptr;     // [n_nodes]
     uint32_t* l_idx = nullptr;       // [2 * n_lower]: (w, upper position of (w, v))
     // > 0: every slice holds that many upper (lower) blocks per row, so row
-    // v's start at (v / 64) 64 width + v % 64; padding may be read (valid
-    // columns and positions, zero values) but is not part of a row
+    // v's start at (v / 64) 64 width + v % 64; padding may be read
+    // (valid columns and positions, any values) but is not part of a row
     uint32_t u_width = 0, l_width = 0;
 };
 

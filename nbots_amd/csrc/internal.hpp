@@ -189,11 +189,10 @@ int mat_prepare_mixed(DevMatrix& m, hipStream_t s, const MixedOpts& o);
 
 // exclusive scan: out[0..n) = scan of in, out[n] = total
 int scan_u32(const uint32_t* in, uint32_t* out, size_t n, hipStream_t s);
-// tiles of the off-diagonal pattern O, whose rows hold at most wmax blocks,
-// by the node positions xy (T.n = 0 when they do not fit)
-// Tiles of the fp16 copy's rows for the Chebyshev preconditioner, or (the second
-// form) of any sliced rows: the first of `attempts` (cells, rings) whose tiles
-// have at most `limit` rows; T.n = 0 when none has.
+// Tiles, by the node positions xy, of the fp16 copy's rows for the Chebyshev
+// preconditioner, or (the second form) of any sliced rows of at most wmax blocks:
+// the first of `attempts` whose tiles have at most `limit` rows.  T.n = 0 when none
+// has, or where a step per launch is the faster.
 int tiles_build(Tiles& T, const Off16& O, uint32_t wmax, const double2* xy, hipStream_t s);
 struct TileAttempt {
     uint32_t cells, rings, least;   // `rings` rings, or as many as fit but `least` at least

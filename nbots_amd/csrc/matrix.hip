@@ -96,7 +96,8 @@ __global__ void k_sym_count(Sell2 A, uint8_t* __restrict__ ulen, uint8_t* __rest
 // Upper columns, and for every lower block (v, w) the pair (w, position of
 // the upper block (w, v)); *bad when row w lacks column v.  Row v of the full
 // layout holds lo lower blocks, the diagonal block, then the upper ones.
-// Padding: upper (column v), lower (v, 0); never read.
+// Padding: upper (column v), lower (v, 0): loaded and gathered through where every
+// slice has one width (row64s, CgRow), never added.
 __global__ void k_sym_pattern(Sell2 A, Sym2 Y, unsigned* bad) {
     const uint32_t v = blockIdx.x * BLOCK + threadIdx.x;
     if (v >= A.n_nodes) return;
