@@ -12,19 +12,10 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def _hip():
-    """The HIP runtime that the library has loaded"""
-    from nbots_amd import load
-    load()
-    with open("/proc/self/maps") as f:
-        path = next(l.split()[-1] for l in f if "libamdhip64" in l)
-    return C.CDLL(path)
-
-
 def test_filter_waits_for_no_other_stream():
-    from nbots_amd import synth
+    from nbots_amd import load, synth
     from nbots_amd.fem import Fem, Simp
-    hip = _hip()
+    hip = load()   # (symbols are looked up in what the library is linked with, too)
     f = Fem.from_problem(synth.cantilever_point(32, 16, jitter=0.1))
     s = Simp(f, rmin=1.5)
     want = s.filter()
