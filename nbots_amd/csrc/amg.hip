@@ -264,8 +264,8 @@ __global__ __launch_bounds__(FIN) void k_amg_pow_fin(const double* partials, uns
 // 60 systems of 200 to 200,000 unknowns; with void elements, condition numbers
 // of 1e11, 4e-6 where FP32 rounds to 2e-8), so one step of Newton's iteration
 // X + X (I - A X) follows, its residual in doubled precision, a workgroup a row
-// (9.6 + 7.9 us at 162 unknowns): then the stored inverse is A^-1 rounded to FP32 in all 60, which the
-// Cholesky inverse was in 52.
+// (9.6 + 7.9 us at 162 unknowns): then the stored inverse is A^-1 rounded to FP32
+// in all 60, which the Cholesky inverse was in 53.
 constexpr int SWEEP_SIDE = 32, SWEEP_TB = SWEEP_SIDE * SWEEP_SIDE;
 constexpr int SWEEP_NB = (AMG_COARSEST + SWEEP_SIDE - 1) / SWEEP_SIDE;
 
