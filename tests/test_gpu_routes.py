@@ -102,7 +102,7 @@ CASES = [
 def routes():
     r = subprocess.run([sys.executable, "-u", "-c", CHILD,
                         json.dumps([c[:2] for c in CASES])], cwd=ROOT, capture_output=True,
-                       text=True, timeout=100, env=dict(os.environ))
+                       text=True, timeout=240, env=dict(os.environ))
     got = [json.loads(line[6:]) for line in r.stdout.splitlines() if line.startswith("ROUTE ")]
     assert r.returncode == 0 and len(got) == len(CASES), r.stdout[-2000:] + r.stderr[-2000:]
     return {(solver, tuple(case)): names for solver, case, names in got}
